@@ -31,6 +31,12 @@
 // v_sin_f32, v_sqrt_f32, v_rcp_f32: about 1 ulp, cos/sin to ~1e-6 absolute on [0, pi]).
 #include "fnet_internal.hpp"
 
+// The kernel instances are compiled in four translation units, side by side: this file (FP32
+// forward) and the three that include it with FNET_ACSF_PART set.
+#ifndef FNET_ACSF_PART
+#define FNET_ACSF_PART 0
+#endif
+
 namespace fnet {
 namespace {
 
@@ -725,6 +731,29 @@ __device__ __forceinline__ void pairs_adj_p(bool ipow, const Slice<T>& sl, int l
 // P^(2^m) for every slot and, as the running product, P^(2^m - 1) for the derivative: the same
 // straight-line code for every slot, with no per-member branch on the exponent.
 
+// Forward: radial-and-r_jk factor of one pair (0 when it does not exist or r_jk > rc), with the
+// pair weight, and its cos(theta).
+template <typename T, bool SAME, bool G4>
+__device__ __forceinline__ T pair_base(const JkConst<T>& K, const typename Vec4<T>::type& dj,
+                                       const typename Vec4<T>::type& pj,
+                                       const typename Vec4<T>::type& dk,
+                                       const typename Vec4<T>::type& pk, bool v, T& c) {
+  c = value_cos(dj, dk, pj.x, pk.x);
+  T base = (SAME ? (T)2 : (T)1) * pj.y * pk.y;
+  bool in = v;
+  if (G4) {
+    const T rx = dj.x - dk.x, ry = dj.y - dk.y, rz = dj.z - dk.z;
+    const T r2 = rx * rx + ry * ry + rz * rz;
+    const T rjk = fsqrt(r2);
+    T cx, sx;
+    K.cs(rjk, cx, sx);
+    const T fcjk = (T)0.5 * pj.z * pk.z * (cx + (T)1);
+    base *= K.ex(r2) * fcjk;
+    in = in && (rjk <= K.rc);
+  }
+  return in ? base : (T)0;
+}
+
 // Forward: off-diagonal pairs, two per step (PairWalk2), FP64 sums per slot; the two pairs'
 // terms are added in T before the conversion.
 template <typename T, int MX, int MASK, bool SAME, bool G4>
@@ -736,23 +765,6 @@ __device__ __forceinline__ void pairs_fwd_lad(const Slice<T>& sl, int lane, int 
   it.init(lane, A0, LA, B0, LB);
   int ej, ek1, ek2;
   bool v1, v2;
-  // radial-and-r_jk factor of one pair (0 when it does not exist or r_jk > rc) and its cos(theta)
-  auto pair_base = [&](const V& dj, const V& pj, const V& dk, const V& pk, bool v, T& c) {
-    c = value_cos(dj, dk, pj.x, pk.x);
-    T base = (SAME ? (T)2 : (T)1) * pj.y * pk.y;
-    bool in = v;
-    if (G4) {
-      const T rx = dj.x - dk.x, ry = dj.y - dk.y, rz = dj.z - dk.z;
-      const T r2 = rx * rx + ry * ry + rz * rz;
-      const T rjk = fsqrt(r2);
-      T cx, sx;
-      K.cs(rjk, cx, sx);
-      const T fcjk = (T)0.5 * pj.z * pk.z * (cx + (T)1);
-      base *= K.ex(r2) * fcjk;
-      in = in && (rjk <= K.rc);
-    }
-    return in ? base : (T)0;
-  };
   // G4: the slot sums go through partial sums that are added to the lane's sums every 16 steps
   // (water boxes: forward 1.13 -> 1.09 ms when the lane's sums were FP64; for the cheaper G5
   // pairs the extra registers cost more, so they add every step)
@@ -777,8 +789,8 @@ __device__ __forceinline__ void pairs_fwd_lad(const Slice<T>& sl, int lane, int 
     const V dk1 = sl.d[ek1], pk1 = sl.pa[ek1];
     const V dk2 = sl.d[ek2], pk2 = sl.pa[ek2];
     T c1, c2;
-    const T b1 = pair_base(dj, pj, dk1, pk1, v1, c1);
-    const T b2 = pair_base(dj, pj, dk2, pk2, v2, c2);
+    const T b1 = pair_base<T, SAME, G4>(K, dj, pj, dk1, pk1, v1, c1);
+    const T b2 = pair_base<T, SAME, G4>(K, dj, pj, dk2, pk2, v2, c2);
 #pragma unroll
     for (int l = 0; l < 2; ++l) {
       const T lam = l ? lam1 : lam0;
@@ -1009,7 +1021,6 @@ template <typename T, int MX, int MASK>
 __device__ void group_lad_pair_fwd(CGroup& ga, CGroup& gb, const Slice<T>& sl, int lane,
                                    long long i, int A0, int L1, int B0, int L2, double* G,
                                    int nG) {
-  using V = typename Vec4<T>::type;
   const T lam0 = (T)ga.lamv[0], lam1 = (T)ga.lamv[1];
   T acc[2][2][MX + 1];  // each lane's slot sums in T, as in group_lad
 #pragma unroll
@@ -1188,6 +1199,221 @@ __device__ __forceinline__ void lad_one(CGroup& grp, CGroup* pg,
   group_lad<T, ADJ, MX, MASK>(grp, sl, lane, i, A0, L1, B0, L2, rc, eta, pi, pirc, cG, G, nG);
 }
 
+// ---- progression groups ----
+// Every member has xi = x0 + k s (k < K) and one of two lambda values: the reference's automatic
+// scheme, whose steps are real numbers.  Per pair and lambda one P = 1 + lambda cos(theta), one
+// R = P^s and, for groups that start above xi = 1, one P^(x0 - 1) serve all members: a power
+// function per member and pair (two in the adjoint) bound the kernels before (256 Si cells, 18 113
+// atoms, 16 angular functions in steps of 15 / 7: whole FP32 step 3.50 -> 0.44 ms).
+
+template <typename T> struct ProgConst {
+  int sint, bint;
+  T sfrac, bfrac;
+};
+
+// P^(n + f), 0 <= f < 1: integer powers as products, the fraction through exp2 and log2 (FP64:
+// exp and log; P = 0 gives 0 for f > 0).  n and f are wave-uniform.
+__device__ __forceinline__ float pow_split(float P, int n, float f) {
+  float r = powi(P, n);
+  if (f != 0.0f) r *= __builtin_amdgcn_exp2f(f * __builtin_amdgcn_logf(P));
+  return r;
+}
+__device__ __forceinline__ double pow_split(double P, int n, double f) {
+  double r = powi(P, n);
+  if (f != 0.0) r *= exp(f * log(P));
+  return r;
+}
+
+// Forward: off-diagonal pairs, two per step, FP64 sums per slot; the two pairs' terms are added in
+// T before the conversion.
+template <typename T, int K, bool SAME, bool G4>
+__device__ __forceinline__ void pairs_fwd_prog(const Slice<T>& sl, int lane, int A0, int LA, int B0,
+                                               int LB, T lam0, T lam1, const JkConst<T>& J,
+                                               const ProgConst<T>& pc, double (&acc)[2][K]) {
+  using V = typename Vec4<T>::type;
+  PairWalk2<SAME> it;
+  it.init(lane, A0, LA, B0, LB);
+  int ej, ek1, ek2;
+  bool v1, v2;
+  while (it.next(ej, ek1, ek2, v1, v2)) {
+    const V dj = sl.d[ej], pj = sl.pa[ej];
+    const V dk1 = sl.d[ek1], pk1 = sl.pa[ek1];
+    const V dk2 = sl.d[ek2], pk2 = sl.pa[ek2];
+    T c1, c2;
+    const T b1 = pair_base<T, SAME, G4>(J, dj, pj, dk1, pk1, v1, c1);
+    const T b2 = pair_base<T, SAME, G4>(J, dj, pj, dk2, pk2, v2, c2);
+#pragma unroll
+    for (int l = 0; l < 2; ++l) {
+      const T lam = l ? lam1 : lam0;
+      const T P1 = (T)1 + lam * c1, P2 = (T)1 + lam * c2;
+      const T R1 = pow_split(P1, pc.sint, pc.sfrac), R2 = pow_split(P2, pc.sint, pc.sfrac);
+      T t1 = b1 * P1, t2 = b2 * P2;
+      if (pc.bint || pc.bfrac != (T)0) {
+        t1 *= pow_split(P1, pc.bint, pc.bfrac);
+        t2 *= pow_split(P2, pc.bint, pc.bfrac);
+      }
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        acc[l][k] += (double)(t1 + t2);
+        t1 *= R1;
+        t2 *= R2;
+      }
+    }
+  }
+}
+
+// Adjoint: with H0 = sum_k c0_k R^k and H1 = sum_k c1_k R^k (Horner), S0 = P^x0 H0 and its
+// derivative in cos(theta) S1 = P^(x0 - 1) H1; c0, c1 as in pairs_adj_lad.
+template <typename T, int K, bool SAME, bool G4>
+__device__ __forceinline__ void pairs_adj_prog(const Slice<T>& sl, int lane, int A0, int LA, int B0,
+                                               int LB, T lam0, T lam1, const T (&c0)[2][K],
+                                               const T (&c1)[2][K], const JkConst<T>& J,
+                                               const ProgConst<T>& pc) {
+  using V = typename Vec4<T>::type;
+  PairWalk2<SAME> it;
+  it.init(lane, A0, LA, B0, LB);
+  int ej, ek1, ek2;
+  bool v1, v2;
+  auto pair = [&](const V& dj, const V& pj, int ek, bool v, T& gx, T& gy, T& gz) {
+    const V dk = sl.d[ek], pk = sl.pa[ek];
+    T rr, c, H, Hq;
+    adj_geom_sel<T, G4>(dj, dk, pj, pk, J, v, rr, c, H, Hq);
+    T S0 = 0, S1 = 0;
+#pragma unroll
+    for (int l = 0; l < 2; ++l) {
+      const T P = (T)1 + (l ? lam1 : lam0) * c;
+      const T R = pow_split(P, pc.sint, pc.sfrac);
+      T h0 = c0[l][K - 1], h1 = c1[l][K - 1];
+#pragma unroll
+      for (int k = K - 2; k >= 0; --k) {
+        h0 = h0 * R + c0[l][k];
+        h1 = h1 * R + c1[l][k];
+      }
+      if (pc.bint || pc.bfrac != (T)0) {
+        const T B = pow_split(P, pc.bint, pc.bfrac);
+        h0 *= B;
+        h1 *= B;
+      }
+      S0 += P * h0;
+      S1 += h1;
+    }
+    T Pj, Pk, Q;
+    adj_coef<T, G4>(pj, pk, rr, c, H, Hq, S0, S1, Pj, Pk, Q);
+    gx += Pj * dj.x + Q * dk.x;
+    gy += Pj * dj.y + Q * dk.y;
+    gz += Pj * dj.z + Q * dk.z;
+    lds_f64* gk = sl.gs + __umul24(ek, 3);
+    lds_add(gk + 0, (double)(Pk * dk.x + Q * dj.x));
+    lds_add(gk + 1, (double)(Pk * dk.y + Q * dj.y));
+    lds_add(gk + 2, (double)(Pk * dk.z + Q * dj.z));
+  };
+  while (it.next(ej, ek1, ek2, v1, v2)) {
+    const V dj = sl.d[ej], pj = sl.pa[ej];
+    T gx = 0, gy = 0, gz = 0;
+    pair(dj, pj, ek1, v1, gx, gy, gz);
+    pair(dj, pj, ek2, v2, gx, gy, gz);
+    lds_f64* gj = sl.gs + __umul24(ej, 3);
+    lds_add(gj + 0, (double)gx);
+    lds_add(gj + 1, (double)gy);
+    lds_add(gj + 2, (double)gz);
+  }
+}
+
+// One progression group of one centre; K >= the group's exponents, the slots beyond them unused.
+template <typename T, bool ADJ, int K>
+__device__ __forceinline__ void group_prog(CGroup& grp, const Slice<T>& sl, int lane, long long i,
+                                           int A0, int L1, int B0, int L2, T rc, T eta, T pirc,
+                                           cdouble* cG, double* G, int nG) {
+  const bool g4 = grp.type == 4;
+  const bool same = grp.same != 0;
+  const T lam0 = uniform((T)grp.lamv[0]), lam1 = uniform((T)grp.lamv[1]);
+  JkConst<T> J;
+  J.set(uniform(rc), uniform(eta), uniform(pirc));
+  ProgConst<T> pc;
+  pc.sint = grp.sint;
+  pc.bint = grp.bint;
+  pc.sfrac = uniform((T)grp.sfrac);
+  pc.bfrac = uniform((T)grp.bfrac);
+  if constexpr (!ADJ) {
+    double acc[2][K];
+#pragma unroll
+    for (int l = 0; l < 2; ++l)
+#pragma unroll
+      for (int k = 0; k < K; ++k) acc[l][k] = 0.0;
+    if (same) {
+      // j == k terms (acsf.F90:1420-1432)
+      for (int e = lane; e < L1; e += 64) {
+        const auto pj = sl.pa[A0 + e];
+        T base = pj.y * pj.y;
+        if (g4) base *= pj.z * pj.z;
+        const T cjj = diag_cos(sl.d[A0 + e], (T)0);
+#pragma unroll
+        for (int l = 0; l < 2; ++l) {
+          const T P = (T)1 + (l ? lam1 : lam0) * cjj;
+          const T R = pow_split(P, pc.sint, pc.sfrac);
+          T t = base * P * pow_split(P, pc.bint, pc.bfrac);
+#pragma unroll
+          for (int k = 0; k < K; ++k) {
+            acc[l][k] += (double)t;
+            t *= R;
+          }
+        }
+      }
+      if (g4) pairs_fwd_prog<T, K, true, true>(sl, lane, A0, L1, B0, L2, lam0, lam1, J, pc, acc);
+      else pairs_fwd_prog<T, K, true, false>(sl, lane, A0, L1, B0, L2, lam0, lam1, J, pc, acc);
+    } else {
+      if (g4) pairs_fwd_prog<T, K, false, true>(sl, lane, A0, L1, B0, L2, lam0, lam1, J, pc, acc);
+      else pairs_fwd_prog<T, K, false, false>(sl, lane, A0, L1, B0, L2, lam0, lam1, J, pc, acc);
+    }
+    // the slot sums in one exchange; slot (l, k) has flat index l K + k
+    constexpr int NA = pow2_at_least(2 * K);
+    double v[NA];
+#pragma unroll
+    for (int q = 0; q < NA; ++q) v[q] = q < 2 * K ? acc[q / K][q % K] : 0.0;
+    int q;
+    const double s = wave_sum_scatter<NA>(v, lane, q);
+    if ((lane & (64 / NA - 1)) == 0 && q < 2 * K) {
+      const int l = q / K, k = q % K;
+      const int mem = k < grp.np ? grp.pmem[kProgLen * l + k] : -1;
+      if (mem >= 0) G[i * nG + grp.col[mem]] = s * grp.scale[mem];
+    }
+  } else {
+    T c0[2][K], c1[2][K];
+    T S0d = 0;
+    const T w = same ? (T)2 : (T)1;  // unordered pairs of one list count twice
+#pragma unroll
+    for (int l = 0; l < 2; ++l)
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const int mem = k < grp.np ? grp.pmem[kProgLen * l + k] : -1;
+        const T v = mem >= 0 ? (T)(cG[grp.col[mem]] * grp.scale[mem]) : (T)0;
+        const T xl = mem >= 0 ? (T)(grp.xi[mem] * grp.lam[mem]) : (T)0;
+        c0[l][k] = uniform(w * v);
+        c1[l][k] = uniform(w * v * xl);
+        S0d += mem >= 0 ? v * (T)grp.pdiag[mem] : (T)0;
+      }
+    S0d = uniform(S0d);
+    if (same) {
+      // j == k terms, as in group_lad (acsf.F90:1580-1585)
+      for (int e = lane; e < L1; e += 64) {
+        const int ej = A0 + e;
+        const auto dj = sl.d[ej];
+        const auto pj = sl.pa[ej];
+        const T H = g4 ? pj.z * pj.z : (T)1;
+        const T gsc = S0d * (T)2 * pj.y * pj.w * H;
+        sl.gs[3 * ej + 0] += gsc * dj.x;
+        sl.gs[3 * ej + 1] += gsc * dj.y;
+        sl.gs[3 * ej + 2] += gsc * dj.z;
+      }
+      if (g4) pairs_adj_prog<T, K, true, true>(sl, lane, A0, L1, B0, L2, lam0, lam1, c0, c1, J, pc);
+      else pairs_adj_prog<T, K, true, false>(sl, lane, A0, L1, B0, L2, lam0, lam1, c0, c1, J, pc);
+    } else {
+      if (g4) pairs_adj_prog<T, K, false, true>(sl, lane, A0, L1, B0, L2, lam0, lam1, c0, c1, J, pc);
+      else pairs_adj_prog<T, K, false, false>(sl, lane, A0, L1, B0, L2, lam0, lam1, c0, c1, J, pc);
+    }
+  }
+}
+
 // Forward value of one radial function (G1/G2/G3, acsf.F90:1287-1373) summed over the staged
 // entries e0, e0 + step, ... below e1, with the terms evaluated in U and summed in FP64.  U is the
 // kernel's T, or FP64 in an FP32 kernel whose model standardises some radial feature by a sigma
@@ -1225,11 +1451,12 @@ __device__ __forceinline__ double radial_sum(const AcsfArgs& a, const Slice<T>& 
   return acc;
 }
 
-// LAD: every angular group has the exponent-ladder form (AngGroup::lad > 0); MQ is then unused.
+// FORM: 1 every angular group has the exponent-ladder form (AngGroup::lad > 0), MQ is then unused;
+// 2 every group has it or the progression form, of at most MQ exponents; 0 the per-member loop.
 // PAIRS (ladder groups only): paired groups are evaluated together (own instance, so
 // that the kernels of models without pairs keep their register budget).  R64 (FP32 forward
 // only): radial terms in FP64 (radial_sum), also an instance of its own.
-template <typename T, bool ADJ, int MQ, bool LAD, bool PAIRS, bool R64 = false>
+template <typename T, bool ADJ, int MQ, int FORM, bool PAIRS, bool R64 = false>
 __device__ __forceinline__ void acsf_centre(const AcsfArgs& a, const long long i) {
   using V = typename Vec4<T>::type;
   extern __shared__ __align__(32) unsigned char smem[];
@@ -1458,11 +1685,11 @@ __device__ __forceinline__ void acsf_centre(const AcsfArgs& a, const long long i
       if constexpr (PAIRS && !ADJ) {
         if (grp.follower) continue;  // evaluated together with its partner
       }
-      T A[MQ];
+      T A[FORM ? 1 : MQ];
       if (ADJ) {
         // a group whose dE/dG are all zero adds nothing to the forces
         bool any = false;
-        if (LAD) {
+        if (FORM) {
           if (PAIRS && grp.follower) continue;  // evaluated together with its partner
           for (int q = 0; q < nm; ++q) any = any || (cG[grp.col[q]] != 0.0);
           if (PAIRS && grp.partner >= 0) {
@@ -1542,9 +1769,17 @@ __device__ __forceinline__ void acsf_centre(const AcsfArgs& a, const long long i
       }
       wave_sync();
 
-      if constexpr (LAD) {
+      if constexpr (FORM != 0) {
+        if constexpr (FORM == 2) {
+          if (grp.np) {
+            group_prog<T, ADJ, MQ>(grp, sl, lane, i, A0, L1, B0, L2, rc, eta, pirc, cG, a.G, a.nG);
+            wave_sync();
+            continue;
+          }
+        }
         switch (grp.lad) {
-          // exponent sets {1, 4} and {1, 2, 4, 16} have their own instances, others the full one
+          // exponent sets {1, 4}, {1, 16} and {1, 2, 4, 16} have their own instances, others the
+          // full one
           case 1: lad_one<T, ADJ, 1, 0x3>(grp, pg, sl, lane, i, A0, L1, B0, L2, rc, eta, pi, pirc, cG, a.G, a.nG); break;
           case 2:
             if (grp.lmask == 0x5) lad_one<T, ADJ, 2, 0x5>(grp, pg, sl, lane, i, A0, L1, B0, L2, rc, eta, pi, pirc, cG, a.G, a.nG);
@@ -1552,7 +1787,9 @@ __device__ __forceinline__ void acsf_centre(const AcsfArgs& a, const long long i
             break;
           case 3: lad_one<T, ADJ, 3, 0xf>(grp, pg, sl, lane, i, A0, L1, B0, L2, rc, eta, pi, pirc, cG, a.G, a.nG); break;
           default:
-            if (grp.lmask == 0x17) lad_one<T, ADJ, 4, 0x17>(grp, pg, sl, lane, i, A0, L1, B0, L2, rc, eta, pi, pirc, cG, a.G, a.nG);
+            // (the paired kernels have no registers left for one more instance)
+            if (!PAIRS && grp.lmask == 0x11) lad_one<T, ADJ, 4, PAIRS ? 0x1f : 0x11>(grp, pg, sl, lane, i, A0, L1, B0, L2, rc, eta, pi, pirc, cG, a.G, a.nG);
+            else if (grp.lmask == 0x17) lad_one<T, ADJ, 4, 0x17>(grp, pg, sl, lane, i, A0, L1, B0, L2, rc, eta, pi, pirc, cG, a.G, a.nG);
             else lad_one<T, ADJ, 4, 0x1f>(grp, pg, sl, lane, i, A0, L1, B0, L2, rc, eta, pi, pirc, cG, a.G, a.nG);
             break;
         }
@@ -1677,26 +1914,26 @@ __device__ __forceinline__ void acsf_centre(const AcsfArgs& a, const long long i
 // One wave per centre.  PERSIST: a grid of as many blocks as stay resident takes the centres in
 // strides of its wave count, restaging the slice for each (an instance of its own: the loop
 // around the body costs the one-centre kernels registers).
-template <typename T, bool ADJ, int MQ, bool LAD, bool PAIRS, bool R64 = false,
+template <typename T, bool ADJ, int MQ, int FORM, bool PAIRS, bool R64 = false,
           bool PERSIST = false>
 __device__ __forceinline__ void acsf_wave(const AcsfArgs& a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wpb = blockDim.x >> 6;
   long long i = a.a0 + (long long)blockIdx.x * wpb + wave;
   if constexpr (!PERSIST) {
-    if (i < a.a1) acsf_centre<T, ADJ, MQ, LAD, PAIRS, R64>(a, i);
+    if (i < a.a1) acsf_centre<T, ADJ, MQ, FORM, PAIRS, R64>(a, i);
   } else {
     const long long stride = (long long)gridDim.x * wpb;
     for (; i < a.a1; i += stride) {
-      acsf_centre<T, ADJ, MQ, LAD, PAIRS, R64>(a, i);
+      acsf_centre<T, ADJ, MQ, FORM, PAIRS, R64>(a, i);
       wave_sync();
     }
   }
 }
 
-template <typename T, bool ADJ, int MQ, bool LAD, bool PAIRS>
+template <typename T, bool ADJ, int MQ, int FORM, bool PAIRS>
 __global__ void __launch_bounds__(512) k_acsf(AcsfArgs a) {
-  acsf_wave<T, ADJ, MQ, LAD, PAIRS>(a);
+  acsf_wave<T, ADJ, MQ, FORM, PAIRS>(a);
 }
 
 // The FP32 exponent-ladder kernels, at least 5 waves per SIMD (the bound once kept them from the
@@ -1704,14 +1941,14 @@ __global__ void __launch_bounds__(512) k_acsf(AcsfArgs a) {
 template <bool ADJ>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(5)))
     k_acsf_lad32(AcsfArgs a) {
-  acsf_wave<float, ADJ, 1, true, false>(a);
+  acsf_wave<float, ADJ, 1, 1, false>(a);
 }
 
 // persistent grid of the same (the loop needs more than 96 registers: 4 waves per SIMD)
 template <bool ADJ>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
     k_acsf_lad32_persist(AcsfArgs a) {
-  acsf_wave<float, ADJ, 1, true, false, false, true>(a);
+  acsf_wave<float, ADJ, 1, 1, false, false, true>(a);
 }
 
 // FP32 ladder adjoint with paired groups (72 registers: 7 waves per SIMD; the persistent
@@ -1719,23 +1956,24 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
 template <bool PERSIST = false>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
     k_acsf_lad32_pairs(AcsfArgs a) {
-  acsf_wave<float, true, 1, true, true, false, PERSIST>(a);
+  acsf_wave<float, true, 1, 1, true, false, PERSIST>(a);
 }
 
 // FP32 ladder forward with paired groups, bounded to 64 registers (8 waves per SIMD), which its
 // FP32 slot sums per lane meet without spilling (66 unbounded, 7 waves)
+template <bool PAIRS = true>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8)))
     k_acsf_lad32_fpairs(AcsfArgs a) {
-  acsf_wave<float, false, 1, true, true>(a);
+  acsf_wave<float, false, 1, 1, PAIRS>(a);
 }
 
 // FP32 forward with the radial terms in FP64 (models with an ill-conditioned radial z-score)
-template <int MQ, bool LAD>
+template <int MQ, int FORM>
 __global__ void __launch_bounds__(512) k_acsf_fwd32_r64(AcsfArgs a) {
-  acsf_wave<float, false, MQ, LAD, false, true>(a);
+  acsf_wave<float, false, MQ, FORM, false, true>(a);
 }
 
-template <typename T, bool ADJ, int MQ, bool LAD>
+template <typename T, bool ADJ, int MQ, int FORM>
 hipError_t launch_mq(fnet_batch* b, const DevModel& m, long long a0, long long a1,
                      hipStream_t s) {
   const long long n = a1 - a0;
@@ -1745,7 +1983,7 @@ hipError_t launch_mq(fnet_batch* b, const DevModel& m, long long a0, long long a
   const size_t lmax = (size_t)b->ctx->lds_block;
   // paired ladder groups share one walk when the larger slice still fits a block (the forward
   // with an FP64 radial part and the persistent forward keep the unpaired kernels)
-  const int pairs = (LAD && m.has_pairs && slice_bytes<T, ADJ>(M, 1) <= lmax &&
+  const int pairs = (FORM == 1 && m.has_pairs && slice_bytes<T, ADJ>(M, 1) <= lmax &&
                      (ADJ || !(std::is_same<T, float>::value && (m.radial64 || tn.persist))))
                         ? 1 : 0;
   const size_t sb = slice_bytes<T, ADJ>(M, pairs);
@@ -1803,37 +2041,61 @@ hipError_t launch_mq(fnet_batch* b, const DevModel& m, long long a0, long long a
     return hipGetLastError();
   };
   const bool ps = a.persist != 0;
-  if constexpr (ADJ && LAD) {
+  if constexpr (ADJ && FORM == 1) {
     if (pairs) {
       if constexpr (std::is_same<T, float>::value)
         return ps ? go(k_acsf_lad32_pairs<true>, true) : go(k_acsf_lad32_pairs<false>, false);
-      else return go(k_acsf<T, true, 1, true, true>, false);
+      else return go(k_acsf<T, true, 1, 1, true>, false);
     }
   }
-  if constexpr (!ADJ && LAD) {
+  if constexpr (!ADJ && FORM == 1) {
     if (pairs) {
-      if constexpr (std::is_same<T, float>::value) return go(k_acsf_lad32_fpairs, false);
-      else return go(k_acsf<T, false, 1, true, true>, false);
+      if constexpr (std::is_same<T, float>::value) return go(k_acsf_lad32_fpairs<>, false);
+      else return go(k_acsf<T, false, 1, 1, true>, false);
     }
   }
   if constexpr (!ADJ && std::is_same<T, float>::value) {
-    if (m.radial64) return go(k_acsf_fwd32_r64<MQ, LAD>, false);
+    if (m.radial64) return go(k_acsf_fwd32_r64<MQ, FORM>, false);
   }
-  if constexpr (LAD && std::is_same<T, float>::value)
+  if constexpr (FORM == 1 && std::is_same<T, float>::value)
     return ps ? go(k_acsf_lad32_persist<ADJ>, true) : go(k_acsf_lad32<ADJ>, false);
-  else return go(k_acsf<T, ADJ, MQ, LAD, false>, false);
+  else return go(k_acsf<T, ADJ, MQ, FORM, false>, false);
 }
 
 template <typename T, bool ADJ>
 hipError_t launch(fnet_batch* b, const DevModel& m, long long a0, long long a1, hipStream_t s) {
-  if (m.all_lad) return launch_mq<T, ADJ, 1, true>(b, m, a0, a1, s);
-  if (m.maxmem <= 4) return launch_mq<T, ADJ, 4, false>(b, m, a0, a1, s);
-  if (m.maxmem <= 8) return launch_mq<T, ADJ, 8, false>(b, m, a0, a1, s);
-  if (m.maxmem <= 12) return launch_mq<T, ADJ, 12, false>(b, m, a0, a1, s);
-  return launch_mq<T, ADJ, kMaxMembers, false>(b, m, a0, a1, s);
+  if (m.form == 1) return launch_mq<T, ADJ, 1, 1>(b, m, a0, a1, s);
+  if (m.form == 2) {
+    if (m.maxprog <= 4) return launch_mq<T, ADJ, 4, 2>(b, m, a0, a1, s);
+    return launch_mq<T, ADJ, kProgLen, 2>(b, m, a0, a1, s);
+  }
+  if (m.maxmem <= 4) return launch_mq<T, ADJ, 4, 0>(b, m, a0, a1, s);
+  if (m.maxmem <= 8) return launch_mq<T, ADJ, 8, 0>(b, m, a0, a1, s);
+  if (m.maxmem <= 12) return launch_mq<T, ADJ, 12, 0>(b, m, a0, a1, s);
+  return launch_mq<T, ADJ, kMaxMembers, 0>(b, m, a0, a1, s);
 }
 
 }  // namespace
+
+#if FNET_ACSF_PART == 1
+hipError_t launch_acsf_adj32(fnet_batch* b, const DevModel& m, long long a0, long long a1,
+                             hipStream_t s) {
+  return launch<float, true>(b, m, a0, a1, s);
+}
+#elif FNET_ACSF_PART == 2
+hipError_t launch_acsf_fwd64(fnet_batch* b, const DevModel& m, long long a0, long long a1,
+                             hipStream_t s) {
+  return launch<double, false>(b, m, a0, a1, s);
+}
+#elif FNET_ACSF_PART == 3
+hipError_t launch_acsf_adj64(fnet_batch* b, const DevModel& m, long long a0, long long a1,
+                             hipStream_t s) {
+  return launch<double, true>(b, m, a0, a1, s);
+}
+#else
+hipError_t launch_acsf_adj32(fnet_batch*, const DevModel&, long long, long long, hipStream_t);
+hipError_t launch_acsf_fwd64(fnet_batch*, const DevModel&, long long, long long, hipStream_t);
+hipError_t launch_acsf_adj64(fnet_batch*, const DevModel&, long long, long long, hipStream_t);
 
 int acsf_slice_entries(int max_nb) { return slice_entries(max_nb); }
 
@@ -1846,12 +2108,13 @@ size_t lds_bytes_acsf(int max_nb, int nZ, int fp64, int adj) {
 
 hipError_t launch_acsf_fwd(fnet_batch* b, const DevModel& m, long long a0, long long a1, int fp64,
                            hipStream_t s) {
-  return fp64 ? launch<double, false>(b, m, a0, a1, s) : launch<float, false>(b, m, a0, a1, s);
+  return fp64 ? launch_acsf_fwd64(b, m, a0, a1, s) : launch<float, false>(b, m, a0, a1, s);
 }
 
 hipError_t launch_acsf_adj(fnet_batch* b, const DevModel& m, long long a0, long long a1, int fp64,
                            hipStream_t s) {
-  return fp64 ? launch<double, true>(b, m, a0, a1, s) : launch<float, true>(b, m, a0, a1, s);
+  return fp64 ? launch_acsf_adj64(b, m, a0, a1, s) : launch_acsf_adj32(b, m, a0, a1, s);
 }
+#endif
 
 }  // namespace fnet

@@ -139,6 +139,56 @@ void ladder_form(AngGroup& a) {
   a.lmask = mask;
 }
 
+// Fills the progression form of an angular group (np = 0 when it does not have it): at most two
+// lambda values, exponents x0 + k s with x0 >= 1 (P^(x0 - 1) stays finite at P = 0) and at most
+// kProgLen of them, each (lambda, xi) once.  The automatic ACSF scheme steps xi evenly from 1
+// (acsf.F90:276-363); a group split at kMaxMembers continues the steps from a larger x0.  The
+// largest exponent is bounded so that the padded slots of the kernels stay finite in FP32.
+void progression_form(AngGroup& a) {
+  a.np = a.sint = a.bint = 0;
+  a.sfrac = a.bfrac = 0.0;
+  for (int k = 0; k < 2 * kProgLen; ++k) a.pmem[k] = -1;
+  if (a.lad) return;
+  std::vector<double> lam(a.lam, a.lam + a.nmem), xi(a.xi, a.xi + a.nmem);
+  auto distinct = [](std::vector<double>& v) {
+    std::sort(v.begin(), v.end());
+    v.erase(std::unique(v.begin(), v.end()), v.end());
+  };
+  distinct(lam);
+  distinct(xi);
+  const int K = (int)xi.size();
+  if (lam.size() > 2 || K > kProgLen || K < 1 || !(xi[0] >= 1.0)) return;
+  const double s = K > 1 ? (xi[K - 1] - xi[0]) / (K - 1) : 0.0;
+  for (int k = 0; k < K; ++k)
+    if (std::fabs(xi[k] - (xi[0] + k * s)) > 1e-14 * xi[k]) return;
+  if (!(xi[0] + kProgLen * s <= 120.0)) return;
+  for (int q = 0; q < a.nmem; ++q) {
+    const int i = a.lam[q] == lam[0] ? 0 : 1;
+    const int k = (int)(std::lower_bound(xi.begin(), xi.end(), a.xi[q]) - xi.begin());
+    if (a.pmem[kProgLen * i + k] >= 0) {
+      a.pmem[0] = -1;
+      return;
+    }
+    a.pmem[kProgLen * i + k] = q;
+  }
+  a.lamv[0] = lam[0];
+  a.lamv[1] = lam.size() > 1 ? lam[1] : lam[0];
+  // an integer step (or base) within rounding is taken as one: products instead of a real power
+  auto split = [](double x, int& n, double& f) {
+    n = (int)std::floor(x);
+    f = x - n;
+    if (f > 1.0 - 1e-14) {
+      n += 1;
+      f = 0.0;
+    } else if (f < 1e-14) {
+      f = 0.0;
+    }
+  };
+  split(s, a.sint, a.sfrac);
+  split(xi[0] - 1.0, a.bint, a.bfrac);
+  a.np = K;
+}
+
 void invalidate(fnet_batch* b) {
   b->have_nl = b->have_G = b->have_E = b->have_F = false;
   b->have_mirror = false;
@@ -1007,12 +1057,15 @@ int fnet_model_upload(fnet_ctx* ctx, const fnet_model_desc* md) {
   m.nAG = (int)grp.size();
   m.maxmem = 1;
   for (const AngGroup& a : grp) m.maxmem = std::max(m.maxmem, a.nmem);
-  m.all_lad = 1;
+  m.form = 1;
+  m.maxprog = 0;
   for (AngGroup& a : grp) {
     ladder_form(a);
+    progression_form(a);
     a.partner = -1;
     a.follower = 0;
-    if (a.lad == 0) m.all_lad = 0;
+    m.maxprog = std::max(m.maxprog, a.np);
+    if (a.lad == 0) m.form = a.np && m.form ? 2 : 0;
   }
   // G5 ladder groups that differ only in eta share one pass of the adjoint
   m.has_pairs = 0;

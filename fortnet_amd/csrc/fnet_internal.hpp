@@ -16,6 +16,7 @@ constexpr int kMaxDim = 256;    // widest layer of the generic network kernels
 constexpr int kMaxMembers = 16; // functions sharing one angular neighbour-pair loop
 constexpr int kMaxZ = 16;       // distinct atomic numbers referenced by one model
 constexpr int kLadSlots = 10;   // (lambda, 2^m) slots of an exponent-ladder group: 2 x 5
+constexpr int kProgLen = 8;     // exponents per lambda of a progression group
 constexpr int kMaxOut = 8;      // network outputs (targets)
 constexpr double kPi = 3.14159265358979323846; // lib_dftbp/constants.F90:15
 
@@ -57,6 +58,14 @@ struct AngGroup {
   double lamv[2];
   int smem[kLadSlots];
   double lpdiag[kLadSlots]; // (1 + lamv[i])^(2^m)
+  // Progression form (np > 0, groups without the ladder form): the exponents are x0 + k s, k < np
+  // <= kProgLen, x0 >= 1, with the lambdas in lamv (the reference's automatic scheme); slot
+  // kProgLen i + k stands for (lamv[i], x0 + k s).  The powers of 1 + lambda cos(theta) then are
+  // P^(x0 - 1) and P R^k with R = P^s, both exponents split into integer and fraction.
+  int np;
+  int sint, bint;       // integer parts of s and x0 - 1
+  double sfrac, bfrac;  // their fractions
+  int pmem[2 * kProgLen];
   // Adjoint pass: a G5 ladder group and another one over the same lists with the same ladder
   // and lambdas but another eta are evaluated together (partner >= 0 on the first one,
   // follower = 1 on the second).
@@ -103,7 +112,9 @@ struct OptState {
 struct DevModel {
   int nG = 0, nR = 0, nAG = 0, nZ = 0;
   int maxmem = 1;               // largest angular group
-  int all_lad = 0;              // every angular group has the exponent-ladder form
+  int form = 0;                 // angular groups: 1 all exponent ladders, 2 ladders and
+                                // progressions, 0 some group has neither
+  int maxprog = 0;              // longest progression
   int has_pairs = 0;            // some angular groups are evaluated in pairs by the adjoint
   int radial_resolved = 0;      // some radial function is restricted to one neighbour element
   int radial64 = 0;             // FP32 modes sum the radial functions in FP64 (kRadial64Kappa)
