@@ -29,7 +29,7 @@
 // are accumulated in FP64 in both modes.  FP64 evaluates the elementary functions with libm in the
 // reference's operation order; FP32 uses the hardware instructions (v_exp_f32, v_cos_f32,
 // v_sin_f32, v_sqrt_f32, v_rcp_f32: about 1 ulp, cos/sin to ~1e-6 absolute on [0, pi]).
-#include "fnet_internal.hpp"
+#include "fnet_device.hpp"
 
 // The kernel instances are compiled in four translation units, side by side: this file (FP32
 // forward) and the three that include it with FNET_ACSF_PART set.
@@ -211,6 +211,7 @@ struct AcsfArgs {
                     // the neighbour's row that points back), or at its own index without one;
                     // FP64 values from the FP64 kernels, FP32 values from the FP32 ones
   const int* mir;   // [entries] mirror entries (-1: none)
+  unsigned long long* stamp;  // start time of the launch, when asked for
 };
 
 // Bytes of one wave's LDS slice (host and device agree on this layout).  Per entry, in element
@@ -1917,6 +1918,8 @@ __device__ __forceinline__ void acsf_centre(const AcsfArgs& a, const long long i
 template <typename T, bool ADJ, int MQ, int FORM, bool PAIRS, bool R64 = false,
           bool PERSIST = false>
 __device__ __forceinline__ void acsf_wave(const AcsfArgs& a) {
+  // (the paired forward has no register left for it: its boundary is the search's end)
+  if constexpr (ADJ) stamp(a.stamp);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wpb = blockDim.x >> 6;
   long long i = a.a0 + (long long)blockIdx.x * wpb + wave;
@@ -1975,7 +1978,7 @@ __global__ void __launch_bounds__(512) k_acsf_fwd32_r64(AcsfArgs a) {
 
 template <typename T, bool ADJ, int MQ, int FORM>
 hipError_t launch_mq(fnet_batch* b, const DevModel& m, long long a0, long long a1,
-                     hipStream_t s) {
+                     hipStream_t s, unsigned long long* stamp) {
   const long long n = a1 - a0;
   if (n <= 0) return hipSuccess;
   const Tune& tn = tune_of(b);
@@ -2022,6 +2025,7 @@ hipError_t launch_mq(fnet_batch* b, const DevModel& m, long long a0, long long a
   a.F = (double*)b->F;
   a.gvec = b->gvec;
   a.mir = b->mir;
+  a.stamp = stamp;
   const unsigned grid = (unsigned)((n + wpb - 1) / wpb);
   const size_t lds = sb * wpb;
   // persistent grids exist for the FP32 exponent-ladder kernels (the batched FP32 / BF16 path);
@@ -2063,39 +2067,43 @@ hipError_t launch_mq(fnet_batch* b, const DevModel& m, long long a0, long long a
 }
 
 template <typename T, bool ADJ>
-hipError_t launch(fnet_batch* b, const DevModel& m, long long a0, long long a1, hipStream_t s) {
-  if (m.form == 1) return launch_mq<T, ADJ, 1, 1>(b, m, a0, a1, s);
+hipError_t launch(fnet_batch* b, const DevModel& m, long long a0, long long a1, hipStream_t s,
+                  unsigned long long* stamp) {
+  if (m.form == 1) return launch_mq<T, ADJ, 1, 1>(b, m, a0, a1, s, stamp);
   if (m.form == 2) {
-    if (m.maxprog <= 4) return launch_mq<T, ADJ, 4, 2>(b, m, a0, a1, s);
-    return launch_mq<T, ADJ, kProgLen, 2>(b, m, a0, a1, s);
+    if (m.maxprog <= 4) return launch_mq<T, ADJ, 4, 2>(b, m, a0, a1, s, stamp);
+    return launch_mq<T, ADJ, kProgLen, 2>(b, m, a0, a1, s, stamp);
   }
-  if (m.maxmem <= 4) return launch_mq<T, ADJ, 4, 0>(b, m, a0, a1, s);
-  if (m.maxmem <= 8) return launch_mq<T, ADJ, 8, 0>(b, m, a0, a1, s);
-  if (m.maxmem <= 12) return launch_mq<T, ADJ, 12, 0>(b, m, a0, a1, s);
-  return launch_mq<T, ADJ, kMaxMembers, 0>(b, m, a0, a1, s);
+  if (m.maxmem <= 4) return launch_mq<T, ADJ, 4, 0>(b, m, a0, a1, s, stamp);
+  if (m.maxmem <= 8) return launch_mq<T, ADJ, 8, 0>(b, m, a0, a1, s, stamp);
+  if (m.maxmem <= 12) return launch_mq<T, ADJ, 12, 0>(b, m, a0, a1, s, stamp);
+  return launch_mq<T, ADJ, kMaxMembers, 0>(b, m, a0, a1, s, stamp);
 }
 
 }  // namespace
 
 #if FNET_ACSF_PART == 1
 hipError_t launch_acsf_adj32(fnet_batch* b, const DevModel& m, long long a0, long long a1,
-                             hipStream_t s) {
-  return launch<float, true>(b, m, a0, a1, s);
+                             hipStream_t s, unsigned long long* stamp) {
+  return launch<float, true>(b, m, a0, a1, s, stamp);
 }
 #elif FNET_ACSF_PART == 2
 hipError_t launch_acsf_fwd64(fnet_batch* b, const DevModel& m, long long a0, long long a1,
-                             hipStream_t s) {
-  return launch<double, false>(b, m, a0, a1, s);
+                             hipStream_t s, unsigned long long* stamp) {
+  return launch<double, false>(b, m, a0, a1, s, stamp);
 }
 #elif FNET_ACSF_PART == 3
 hipError_t launch_acsf_adj64(fnet_batch* b, const DevModel& m, long long a0, long long a1,
-                             hipStream_t s) {
-  return launch<double, true>(b, m, a0, a1, s);
+                             hipStream_t s, unsigned long long* stamp) {
+  return launch<double, true>(b, m, a0, a1, s, stamp);
 }
 #else
-hipError_t launch_acsf_adj32(fnet_batch*, const DevModel&, long long, long long, hipStream_t);
-hipError_t launch_acsf_fwd64(fnet_batch*, const DevModel&, long long, long long, hipStream_t);
-hipError_t launch_acsf_adj64(fnet_batch*, const DevModel&, long long, long long, hipStream_t);
+hipError_t launch_acsf_adj32(fnet_batch*, const DevModel&, long long, long long, hipStream_t,
+                             unsigned long long*);
+hipError_t launch_acsf_fwd64(fnet_batch*, const DevModel&, long long, long long, hipStream_t,
+                             unsigned long long*);
+hipError_t launch_acsf_adj64(fnet_batch*, const DevModel&, long long, long long, hipStream_t,
+                             unsigned long long*);
 
 int acsf_slice_entries(int max_nb) { return slice_entries(max_nb); }
 
@@ -2108,12 +2116,14 @@ size_t lds_bytes_acsf(int max_nb, int nZ, int fp64, int adj) {
 
 hipError_t launch_acsf_fwd(fnet_batch* b, const DevModel& m, long long a0, long long a1, int fp64,
                            hipStream_t s) {
-  return fp64 ? launch_acsf_fwd64(b, m, a0, a1, s) : launch<float, false>(b, m, a0, a1, s);
+  return fp64 ? launch_acsf_fwd64(b, m, a0, a1, s, nullptr)
+              : launch<float, false>(b, m, a0, a1, s, nullptr);
 }
 
 hipError_t launch_acsf_adj(fnet_batch* b, const DevModel& m, long long a0, long long a1, int fp64,
-                           hipStream_t s) {
-  return fp64 ? launch_acsf_adj64(b, m, a0, a1, s) : launch_acsf_adj32(b, m, a0, a1, s);
+                           hipStream_t s, unsigned long long* stamp) {
+  return fp64 ? launch_acsf_adj64(b, m, a0, a1, s, stamp)
+              : launch_acsf_adj32(b, m, a0, a1, s, stamp);
 }
 #endif
 

@@ -191,7 +191,7 @@ void progression_form(AngGroup& a) {
 
 void invalidate(fnet_batch* b) {
   b->have_nl = b->have_G = b->have_E = b->have_F = false;
-  b->have_mirror = false;
+  b->have_mirror = b->mir_clear = false;
   b->pending = false;
 }
 
@@ -377,6 +377,7 @@ int do_neighbours(fnet_batch* b) {
   const int fp64 = b->precision == FNET_FP64;
   HIPCHECK(ctx, launch_struct_prep(b, rc, s));
   HIPCHECK(ctx, launch_cell_bin(b, s));
+  b->mir_clear = false;
   // One pass into padded rows when the previous list gives a capacity (and the cell-list sort
   // of that capacity fits a block's LDS); a row longer than it sends the batch through the fill
   // pass below, with the counts this pass already made.
@@ -462,7 +463,12 @@ int do_acsf(fnet_batch* b) {
   return FNET_OK;
 }
 
-int do_mlp(fnet_batch* b, int gradin) {
+// Batches of up to this many atoms search their mirror entries in extra blocks of the networks
+// launch, which is latency-bound there and hides them; larger ones search them on the side stream
+// beside the ACSF forward.
+constexpr long long kMirrorInline = 16384;
+
+int do_mlp(fnet_batch* b, int gradin, bool mirror = false) {
   fnet_ctx* ctx = b->ctx;
   const DevModel& m = ctx->model;
   const int fp64 = net64(b->precision);
@@ -480,9 +486,9 @@ int do_mlp(fnet_batch* b, int gradin) {
       }
     }
   } else if (mfma) {
-    HIPCHECK(ctx, launch_mlp_mfma(b, m, 0, b->nmtiles, gradin, ctx->stream));
+    HIPCHECK(ctx, launch_mlp_mfma(b, m, 0, b->nmtiles, gradin, ctx->stream, mirror));
   } else {
-    HIPCHECK(ctx, launch_mlp_fwd(b, m, 0, b->ntiles, fp64, gradin, ctx->stream));
+    HIPCHECK(ctx, launch_mlp_fwd(b, m, 0, b->ntiles, fp64, gradin, ctx->stream, mirror));
   }
   return FNET_OK;
 }
@@ -494,7 +500,8 @@ int do_reduce(fnet_batch* b) {
     for (int st = 0; st < b->S; ++st)
       HIPCHECK(ctx, launch_energy_reduce(b, m, st, st + 1, ctx->stream));
   } else {
-    HIPCHECK(ctx, launch_energy_reduce(b, m, 0, b->S, ctx->stream));
+    HIPCHECK(ctx, launch_energy_reduce(b, m, 0, b->S, ctx->stream,
+                                       b->pending ? b->h_maxnb : nullptr));
   }
   b->have_E = true;
   return FNET_OK;
@@ -511,6 +518,7 @@ int ensure_force_buffers(fnet_batch* b) {
     dfree(b->mir);
     dfree(b->orph);
     b->mir = b->orph = nullptr;
+    b->mir_clear = false;
     const long long cap = entries + entries / 8 + 1024;
     HIPCHECK(ctx, dalloc(&b->mir, (size_t)cap));
     HIPCHECK(ctx, dalloc(&b->orph, (size_t)cap));
@@ -525,7 +533,10 @@ int ensure_force_buffers(fnet_batch* b) {
     b->gv_len = cap;
     b->gen++;
   }
-  if (!b->d_norph) HIPCHECK(ctx, dalloc(&b->d_norph, 1));
+  if (!b->d_norph) {
+    HIPCHECK(ctx, dalloc(&b->d_norph, 1));
+    HIPCHECK(ctx, launch_zero_int(b->d_norph, 1, ctx->stream));
+  }
   return FNET_OK;
 }
 
@@ -536,7 +547,8 @@ int do_mirror(fnet_batch* b) {
   int rc = ensure_force_buffers(b);
   if (rc) return rc;
   hipStream_t s = ctx->stream;
-  const long long entries = layout_entries(b);
+  const long long entries = b->mir_clear ? 0 : layout_entries(b);
+  b->mir_clear = false;
   if (b->launch == FNET_PER_STRUCT) {
     for (int st = 0; st < b->S; ++st)
       HIPCHECK(ctx, launch_mirror(b, b->h_off[st], b->h_off[st + 1], st == 0 ? entries : 0, s));
@@ -556,17 +568,16 @@ int do_adjoint(fnet_batch* b) {
   int rc = do_mirror(b);
   if (rc) return rc;
   hipStream_t s = ctx->stream;
-  HIPCHECK(ctx, launch_zero_int(b->d_norph, 1, s));
   if (b->launch == FNET_PER_STRUCT) {
     for (int st = 0; st < b->S; ++st) {
       HIPCHECK(ctx, launch_acsf_adj(b, m, b->h_off[st], b->h_off[st + 1], fp64, s));
-      HIPCHECK(ctx, launch_force_gather(b, m.nout, b->h_off[st], b->h_off[st + 1], s));
+      HIPCHECK(ctx, launch_force_gather(b, m, b->h_off[st], b->h_off[st + 1], false, s));
     }
   } else {
     HIPCHECK(ctx, launch_acsf_adj(b, m, 0, b->N, fp64, s));
-    HIPCHECK(ctx, launch_force_gather(b, m.nout, 0, b->N, s));
+    HIPCHECK(ctx, launch_force_gather(b, m, 0, b->N, false, s));
   }
-  HIPCHECK(ctx, launch_force_orphans(b, m.nout, s));
+  HIPCHECK(ctx, launch_force_finish(b, m, false, s));
   b->have_F = true;
   return FNET_OK;
 }
@@ -577,11 +588,14 @@ int do_adjoint(fnet_batch* b) {
 // the direct scan (per centre: 27 bins of n / (nb_0 nb_1 nb_2) atoms, against n atoms in each of
 // the ~(1 + 2 w_a) images per axis that the scan's image pruning keeps, w_a = rc / width_a);
 // any other structure takes the direct scan.
-int setup_cells(fnet_batch* b, const double* lat, const int* per) {
+// `fresh`: the device tables hold nothing of this batch yet (else equal tables stay as they are).
+int setup_cells(fnet_batch* b, const double* lat, const int* per, bool fresh) {
   fnet_ctx* ctx = b->ctx;
   const double rc = ctx->model.rcmax;
   std::vector<int> info(4 * (size_t)b->S, 0), coff(b->S + 1, 0);
-  long long total = 0;
+  long long total = 0, bins = 0;
+  int used = 0;
+  bool in_prep = true;  // every cell-list structure fits one struct-prep block
   for (int s = 0; s < b->S; ++s) {
     coff[s] = (int)total;
     const long long n = b->h_off[s + 1] - b->h_off[s];
@@ -616,11 +630,19 @@ int setup_cells(fnet_batch* b, const double* lat, const int* per) {
     info[4 * s + 1] = nb[1];
     info[4 * s + 2] = nb[2];
     info[4 * s + 3] = 1;
-    total += (long long)nb[0] * nb[1] * nb[2];
+    // one more than the bins: the end of the structure's last bin
+    const long long nbins = (long long)nb[0] * nb[1] * nb[2];
+    total += nbins + 1;
+    bins = std::max(bins, nbins);
+    in_prep = in_prep && n <= kPrepBinAtoms && nbins <= kPrepBins;
+    ++used;
   }
+  b->n_cell_struct = used;
+  b->bin_lds = used && in_prep ? (int)bins : 0;
   coff[b->S] = (int)total;
   if (total >= (1LL << 30)) return fail(ctx, FNET_ERR_CAPACITY, "too many cells");
   hipStream_t s = ctx->stream;
+  if (!fresh && info == b->h_cellinfo) return FNET_OK;
   if (!b->cellinfo) {
     HIPCHECK(ctx, dalloc(&b->cellinfo, (size_t)b->S));
     HIPCHECK(ctx, dalloc(&b->cell_off, (size_t)b->S + 1));
@@ -636,6 +658,7 @@ int setup_cells(fnet_batch* b, const double* lat, const int* per) {
     HIPCHECK(ctx, dalloc(&b->cell_count, (size_t)total));
     HIPCHECK(ctx, dalloc(&b->cell_start, (size_t)total + 1));
     HIPCHECK(ctx, dalloc(&b->cell_scan_tmp, (size_t)scan_tmp_size(total)));
+    HIPCHECK(ctx, launch_zero_int(b->cell_count, (int)total, s));
     b->ncells = total;
     b->gen++;
   }
@@ -655,6 +678,7 @@ int run_sync_step(fnet_batch* b) {
   fnet_ctx* ctx = b->ctx;
   invalidate(b);
   b->last_graph = 0;
+  ctx->stamped = false;
   ev_record(ctx, 0);
   int rc = do_neighbours(b);
   if (rc) return rc;
@@ -675,10 +699,10 @@ int run_sync_step(fnet_batch* b) {
   return FNET_OK;
 }
 
-// A batched step can skip every host read-back once a previous list gave the row capacity of the
-// one-pass search (nb_cap) and the longest row the ACSF slices are sized for (max_nb); buffers
+// A batched list can skip every host read-back once a previous list gave the row capacity of the
+// one-pass search (nb_cap) and the longest row the ACSF slices are sized for (max_nb); its buffers
 // are sized here, outside any capture.
-bool fast_step_ready(fnet_batch* b) {
+bool fast_list_ready(fnet_batch* b) {
   fnet_ctx* ctx = b->ctx;
   const DevModel& m = ctx->model;
   if (b->launch != FNET_BATCHED || b->N <= 0 || b->nb_cap <= 0 || b->max_nb <= 0) return false;
@@ -689,13 +713,6 @@ bool fast_step_ready(fnet_batch* b) {
       cells_lds_bytes(b->nb_cap, b->precision == FNET_FP64) > (size_t)ctx->lds_block)
     return false;
   if (!ensure_padded(b)) return false;
-  const bool was = b->nl_padded;
-  b->nl_padded = true;
-  if (ensure_force_buffers(b)) {
-    b->nl_padded = was;
-    (void)hipGetLastError();
-    return false;
-  }
   if (!b->h_maxnb) {
     if (hipHostMalloc((void**)&b->h_maxnb, sizeof(int), hipHostMallocDefault) != hipSuccess) {
       b->h_maxnb = nullptr;
@@ -707,47 +724,66 @@ bool fast_step_ready(fnet_batch* b) {
   return true;
 }
 
+// ... and a whole step, with the buffers of the force assembly.
+bool fast_step_ready(fnet_batch* b) {
+  if (!fast_list_ready(b)) return false;
+  const bool was = b->nl_padded;
+  b->nl_padded = true;
+  if (ensure_force_buffers(b)) {
+    b->nl_padded = was;
+    (void)hipGetLastError();
+    return false;
+  }
+  return true;
+}
+
+// The padded list without a read-back: row i at i * nb_cap, the longest row raised on the device
+// by the search.  The search clears the mirror slot of every entry it writes when the mirror array
+// is there, so the mirror search needs no fill of the whole padded array first.
+int enqueue_list(fnet_batch* b, unsigned long long* stamps) {
+  fnet_ctx* ctx = b->ctx;
+  hipStream_t s = ctx->stream;
+  const double rc = ctx->model.rcmax;
+  const int fp64 = b->precision == FNET_FP64;
+  int* mir = b->mir && b->gv_entries >= (long long)b->N * b->nb_cap ? b->mir : nullptr;
+  HIPCHECK(ctx, launch_struct_prep(b, rc, s, stamps));
+  HIPCHECK(ctx, launch_cell_bin(b, s));
+  HIPCHECK(ctx, launch_neigh_pad(b, rc, fp64, s, mir, stamps ? stamps + 1 : nullptr));
+  HIPCHECK(ctx, launch_cells_pad(b, rc, fp64, s, mir, stamps ? stamps + 1 : nullptr));
+  b->mir_clear = mir != nullptr;
+  return FNET_OK;
+}
+
 // Kernels of one steady-state step: no host read-back, no allocation and no memset, so the
 // sequence runs eagerly or as a captured HIP graph.  The padded rows are searched with capacity
 // nb_cap and every row is cut to the ACSF slice of the previous longest row; the longest row of
-// this list is reduced on the device and copied to pinned memory with the step (validate_step).
-int enqueue_fast_step(fnet_batch* b, bool events) {
+// this list goes to pinned memory with the energies (validate_step).
+int enqueue_fast_step(fnet_batch* b) {
   fnet_ctx* ctx = b->ctx;
   const DevModel& m = ctx->model;
   hipStream_t s = ctx->stream;
-  const double rc = m.rcmax;
   const int fp64 = b->precision == FNET_FP64;
-  if (events) ev_record(ctx, 0);
-  HIPCHECK(ctx, launch_struct_prep(b, rc, s));
-  HIPCHECK(ctx, launch_cell_bin(b, s));
-  // the search clears the mirror slot of every entry it writes, so the mirror search needs no fill
-  // of the whole padded array first
-  HIPCHECK(ctx, launch_neigh_pad(b, rc, fp64, s, b->mir));
-  HIPCHECK(ctx, launch_cells_pad(b, rc, fp64, s, b->mir));
-  HIPCHECK(ctx, launch_row_max(b->cnt, b->N, b->d_maxnb, s));
-  // The mirror entries need only the list: their search (latency-bound) runs on the side stream
-  // beside the ACSF forward and the networks (VALU- and matrix-bound), and the adjoint waits for
-  // it.  Under graph capture the event pair becomes a fork and a join of the graph.
-  HIPCHECK(ctx, hipEventRecord(ctx->fork_ev, s));
-  HIPCHECK(ctx, hipStreamWaitEvent(ctx->side, ctx->fork_ev, 0));
-  HIPCHECK(ctx, launch_mirror(b, 0, b->N, 0, ctx->side));
-  HIPCHECK(ctx, hipEventRecord(ctx->join_ev, ctx->side));
-  if (events) ev_record(ctx, 1);
+  unsigned long long* ts = ctx->stamps;
+  const int rc = enqueue_list(b, ts);
+  if (rc) return rc;
+  // The mirror entries need only the list: on a large batch their search (latency-bound) runs on
+  // the side stream beside the ACSF forward and the networks (VALU- and matrix-bound), and the
+  // adjoint waits for it.  Under graph capture the event pair becomes a fork and a join.
+  const bool in_line = b->N <= kMirrorInline;
+  if (!in_line) {
+    HIPCHECK(ctx, hipEventRecord(ctx->fork_ev, s));
+    HIPCHECK(ctx, hipStreamWaitEvent(ctx->side, ctx->fork_ev, 0));
+    HIPCHECK(ctx, launch_mirror(b, 0, b->N, 0, ctx->side));
+    HIPCHECK(ctx, hipEventRecord(ctx->join_ev, ctx->side));
+  }
   HIPCHECK(ctx, launch_acsf_fwd(b, m, 0, b->N, fp64, s));
-  if (events) ev_record(ctx, 2);
   const bool mfma = !net64(b->precision) && m.wpack && b->mtile_waves > 0;
-  if (mfma) HIPCHECK(ctx, launch_mlp_mfma(b, m, 0, b->nmtiles, 1, s));
-  else HIPCHECK(ctx, launch_mlp_fwd(b, m, 0, b->ntiles, net64(b->precision), 1, s));
-  if (events) ev_record(ctx, 3);
-  HIPCHECK(ctx, hipStreamWaitEvent(s, ctx->join_ev, 0));
-  HIPCHECK(ctx, launch_acsf_adj(b, m, 0, b->N, fp64, s));
-  HIPCHECK(ctx, launch_zero_int(b->d_norph, 1, s));
-  HIPCHECK(ctx, launch_force_gather(b, m.nout, 0, b->N, s));
-  HIPCHECK(ctx, launch_force_orphans(b, m.nout, s));
-  if (events) ev_record(ctx, 4);
-  HIPCHECK(ctx, launch_energy_reduce(b, m, 0, b->S, s));
-  if (events) ev_record(ctx, 5);
-  HIPCHECK(ctx, hipMemcpyAsync(b->h_maxnb, b->d_maxnb, sizeof(int), hipMemcpyDeviceToHost, s));
+  if (mfma) HIPCHECK(ctx, launch_mlp_mfma(b, m, 0, b->nmtiles, 1, s, in_line, ts + 2));
+  else HIPCHECK(ctx, launch_mlp_fwd(b, m, 0, b->ntiles, net64(b->precision), 1, s, in_line, ts + 2));
+  if (!in_line) HIPCHECK(ctx, hipStreamWaitEvent(s, ctx->join_ev, 0));
+  HIPCHECK(ctx, launch_acsf_adj(b, m, 0, b->N, fp64, s, ts + 3));
+  HIPCHECK(ctx, launch_force_gather(b, m, 0, b->N, true, s));
+  HIPCHECK(ctx, launch_force_finish(b, m, true, s, ts + 4));
   return FNET_OK;
 }
 
@@ -764,7 +800,7 @@ std::vector<long long> graph_key(const fnet_batch* b) {
   const fnet_ctx* ctx = b->ctx;
   const Tune& t = tune_of(b);
   return {b->gen, ctx->model_gen, b->precision, b->launch, b->nb_cap, b->max_nb, b->ncells,
-          b->N, b->S, b->ntiles, b->nmtiles, t.fwd_wpb, t.adj_wpb, t.mlp_waves, t.rbal,
+          b->N, b->S, b->ntiles, b->nmtiles, b->n_cell_struct, b->bin_lds, t.fwd_wpb, t.adj_wpb, t.mlp_waves, t.rbal,
           t.persist};
 }
 
@@ -780,7 +816,7 @@ int run_fast_step(fnet_batch* b) {
       drop_graph(b);
       HIPCHECK(ctx, hipStreamSynchronize(s));
       hipError_t e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
-      int rc = e == hipSuccess ? enqueue_fast_step(b, false) : FNET_ERR_HIP;
+      int rc = e == hipSuccess ? enqueue_fast_step(b) : FNET_ERR_HIP;
       hipGraph_t g = nullptr;
       const hipError_t e2 = hipStreamEndCapture(s, &g);
       if (e == hipSuccess && rc == FNET_OK && e2 == hipSuccess && g) {
@@ -799,40 +835,102 @@ int run_fast_step(fnet_batch* b) {
       }
     }
     if (b->gexec) {
-      ev_record(ctx, 0);
       HIPCHECK(ctx, hipGraphLaunch(b->gexec, s));
-      ev_record(ctx, 1);
       ctx->n_ev = 2;
       b->last_graph = 1;
     }
   }
   if (!b->last_graph) {
-    const int rc = enqueue_fast_step(b, true);
+    const int rc = enqueue_fast_step(b);
     if (rc) return rc;
     ctx->n_ev = 6;
   }
+  ctx->stamped = true;
   b->have_nl = b->have_G = b->have_E = b->have_F = true;
   b->have_mirror = true;
+  b->mir_clear = false;
   b->result_precision = b->precision;
   b->pending = true;
+  b->pending_level = 3;
   return FNET_OK;
 }
 
-// Checks the longest row of a steady-state step once it has run.  A row longer than the ACSF
-// slice (or the row capacity) was cut, so that step is recomputed on the synchronous path, which
-// also raises the capacities for the next steps; a list that shrank well below its slice lowers
-// the slice.
-int validate_step(fnet_batch* b) {
+// The current list: with the previous list's capacities and no read-back where that can be done
+// (`pending` until its longest row has been checked), else through the host.
+int ensure_list(fnet_batch* b) {
+  if (b->have_nl && b->result_precision == b->precision) return FNET_OK;
+  if (!fast_list_ready(b)) return do_neighbours(b);
+  const int rc = enqueue_list(b, nullptr);
+  if (rc) return rc;
+  b->nl_padded = b->have_nl = true;
+  b->have_mirror = false;
+  b->result_precision = b->precision;
+  b->pending = true;
+  b->pending_level = 1;
+  return FNET_OK;
+}
+
+// What a call needs: 1 features, 2 energies, 3 forces.
+int evaluate(fnet_batch* b, int level) {
+  int rc = FNET_OK;
+  if (!b->have_G || b->result_precision != b->precision) {
+    b->have_E = b->have_F = false;
+    rc = ensure_list(b);
+    if (!rc) rc = do_acsf(b);
+    if (rc) return rc;
+  }
+  if (level == 2 && !b->have_E) {
+    rc = do_mlp(b, 0);
+    if (!rc) rc = do_reduce(b);
+  } else if (level == 3 && !b->have_F) {
+    // the networks with their input gradient; energies that are there already are the same.  A
+    // small batch whose cleared list waits for its mirror search has it in the same launch.
+    const bool mirror = b->launch == FNET_BATCHED && b->N <= kMirrorInline && !b->have_mirror &&
+                        b->mir_clear && b->nl_padded && b->N > 0 &&
+                        !ensure_force_buffers(b) && b->mir_clear;
+    rc = do_mlp(b, 1, mirror);
+    if (rc) return rc;
+    if (mirror) {
+      b->have_mirror = true;
+      b->mir_clear = false;
+    }
+    if (!b->have_E) rc = do_reduce(b);
+    if (!rc) rc = do_adjoint(b);
+  }
+  if (b->pending) b->pending_level = std::max(b->pending_level, level);
+  return rc;
+}
+
+// Checks the longest row of a list built without a read-back, once its stream has run.  A row
+// longer than the ACSF slice (or the row capacity) was cut, so what was computed on the list is
+// recomputed through the host, which also raises the capacities for the next lists; a list that
+// shrank well below its slice lowers the slice.  *redone: the results are being recomputed.
+int settle_list(fnet_batch* b, bool* redone) {
+  if (redone) *redone = false;
   if (!b->pending) return FNET_OK;
-  fnet_ctx* ctx = b->ctx;
-  HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
   b->pending = false;
   const int mx = *b->h_maxnb;
   if (mx <= acsf_slice_entries(b->max_nb) && mx <= b->nb_cap) {
     if (mx + 16 < b->max_nb) b->max_nb = mx;
     return FNET_OK;
   }
-  return run_sync_step(b);
+  if (redone) *redone = true;
+  const int level = b->pending_level;
+  if (level == 3) return run_sync_step(b);
+  invalidate(b);
+  const int rc = do_neighbours(b);
+  return rc ? rc : evaluate(b, level);
+}
+
+int validate_step(fnet_batch* b) {
+  if (!b->pending) return FNET_OK;
+  fnet_ctx* ctx = b->ctx;
+  // features alone: nothing after them took the longest row to the host
+  if (b->pending_level == 1)
+    HIPCHECK(ctx, hipMemcpyAsync(b->h_maxnb, b->d_maxnb, sizeof(int), hipMemcpyDeviceToHost,
+                                 ctx->stream));
+  HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
+  return settle_list(b, nullptr);
 }
 
 int check_ready(fnet_ctx* ctx, fnet_batch* b) {
@@ -857,17 +955,9 @@ int check_ready(fnet_ctx* ctx, fnet_batch* b) {
   return ensure_results(b);
 }
 
-int download_T(fnet_ctx* ctx, const void* dsrc, int fp64, size_t n, double* out) {
-  if (fp64) {
-    HIPCHECK(ctx, hipMemcpyAsync(out, dsrc, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
-  } else {
-    std::vector<float> tmp(n);
-    HIPCHECK(ctx, hipMemcpyAsync(tmp.data(), dsrc, sizeof(float) * n, hipMemcpyDeviceToHost,
-                                 ctx->stream));
-    HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
-    for (size_t k = 0; k < n; ++k) out[k] = (double)tmp[k];
-  }
+int download(fnet_ctx* ctx, const void* dsrc, size_t n, double* out) {
+  HIPCHECK(ctx, hipMemcpyAsync(out, dsrc, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->stream));
+  HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
   return FNET_OK;
 }
 
@@ -901,6 +991,13 @@ int fnet_ctx_create(int device, fnet_ctx** out) {
     return FNET_ERR_HIP;
   }
   for (int k = 0; k < 8; ++k) (void)hipEventCreate(&ctx->ev[k]);
+  int khz = 0;
+  if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) != hipSuccess) khz = 0;
+  ctx->stamp_khz = khz;
+  if (dalloc(&ctx->stamps, 8) != hipSuccess) {
+    fnet_ctx_destroy(ctx);
+    return FNET_ERR_HIP;
+  }
   if (hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreateWithFlags(&ctx->fork_ev, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&ctx->join_ev, hipEventDisableTiming) != hipSuccess) {
@@ -920,6 +1017,7 @@ void fnet_ctx_destroy(fnet_ctx* ctx) {
   dfree(ctx->opt_vecs);
   dfree(ctx->opt_states);
   dfree(ctx->opt_conv);
+  dfree(ctx->stamps);
   for (int k = 0; k < 8; ++k) (void)hipEventDestroy(ctx->ev[k]);
   if (ctx->side) {
     (void)hipStreamSynchronize(ctx->side);
@@ -1312,6 +1410,9 @@ int load_batch(fnet_ctx* ctx, fnet_batch* b, const fnet_batch_desc* d) {
       b->epart_len = need;
     }
     b->nchunks = (int)cs.size();
+    b->single_chunks = 1;
+    for (int st = 0; st < S; ++st)
+      if (cf[st + 1] - cf[st] != 1) b->single_chunks = 0;
     b->h_chunk_first = cf;
   }
   if (N) HIPCHECK(ctx, hipMemcpyAsync(b->xyz, d->coords, sizeof(double) * 3 * N,
@@ -1342,7 +1443,7 @@ int load_batch(fnet_ctx* ctx, fnet_batch* b, const fnet_batch_desc* d) {
   b->tile_atoms = 0;  // species layout changed: rebuild the network tiles
   b->result_precision = -1;
   b->gen++;
-  return setup_cells(b, lat.data(), per.data());
+  return setup_cells(b, lat.data(), per.data(), true);
 }
 
 }  // namespace
@@ -1416,7 +1517,7 @@ int fnet_batch_update_coords(fnet_batch* b, const double* coords, const double* 
                                  hipMemcpyHostToDevice, ctx->stream));
     for (int q = 0; q < 9 * b->S; ++q)
       if (b->h_periodic[q / 9]) b->h_lat[q] = latvecs[q];
-    const int crc = setup_cells(b, b->h_lat.data(), b->h_periodic.data());
+    const int crc = setup_cells(b, b->h_lat.data(), b->h_periodic.data(), false);
     if (crc) return crc;
   }
   HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
@@ -1505,14 +1606,21 @@ int fnet_acsf_forward(fnet_ctx* ctx, fnet_batch* b, double* G_out) {
   rc = validate_step(b);
   if (rc) return rc;
   if (!b->have_nl || b->result_precision != b->precision) {
-    rc = do_neighbours(b);
+    rc = ensure_list(b);
     if (rc) return rc;
   }
   rc = do_acsf(b);
-  if (rc) return rc;
-  if (G_out)
-    return download_T(ctx, b->G, 1, (size_t)b->N * ctx->model.nG, G_out);
-  return FNET_OK;
+  if (rc || !G_out) return rc;
+  for (;;) {
+    if (b->pending && b->pending_level == 1)
+      HIPCHECK(ctx, hipMemcpyAsync(b->h_maxnb, b->d_maxnb, sizeof(int), hipMemcpyDeviceToHost,
+                                   ctx->stream));
+    rc = download(ctx, b->G, (size_t)b->N * ctx->model.nG, G_out);
+    if (rc) return rc;
+    bool redone;
+    rc = settle_list(b, &redone);
+    if (rc || !redone) return rc;
+  }
 }
 
 int fnet_energy(fnet_ctx* ctx, fnet_batch* b, double* E_struct, double* E_atom) {
@@ -1520,25 +1628,21 @@ int fnet_energy(fnet_ctx* ctx, fnet_batch* b, double* E_struct, double* E_atom) 
   if (rc) return rc;
   rc = validate_step(b);
   if (rc) return rc;
-  if (!b->have_G || b->result_precision != b->precision) {
-    rc = fnet_acsf_forward(ctx, b, nullptr);
-    if (rc) return rc;
-  }
-  if (!b->have_E) {
-    rc = do_mlp(b, 0);
-    if (rc) return rc;
-    rc = do_reduce(b);
-    if (rc) return rc;
-  }
+  rc = evaluate(b, 2);
   const DevModel& m = ctx->model;
-  if (E_struct)
-    HIPCHECK(ctx, hipMemcpyAsync(E_struct, b->Estruct, sizeof(double) * b->S * m.nout,
-                                 hipMemcpyDeviceToHost, ctx->stream));
-  if (E_atom)
-    HIPCHECK(ctx, hipMemcpyAsync(E_atom, b->Eatom, sizeof(double) * b->N * m.nout,
-                                 hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
-  return FNET_OK;
+  for (;;) {
+    if (rc) return rc;
+    if (E_struct)
+      HIPCHECK(ctx, hipMemcpyAsync(E_struct, b->Estruct, sizeof(double) * b->S * m.nout,
+                                   hipMemcpyDeviceToHost, ctx->stream));
+    if (E_atom)
+      HIPCHECK(ctx, hipMemcpyAsync(E_atom, b->Eatom, sizeof(double) * b->N * m.nout,
+                                   hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
+    bool redone;
+    rc = settle_list(b, &redone);
+    if (!rc && !redone) return FNET_OK;
+  }
 }
 
 int fnet_forces(fnet_ctx* ctx, fnet_batch* b, double* F) {
@@ -1546,21 +1650,15 @@ int fnet_forces(fnet_ctx* ctx, fnet_batch* b, double* F) {
   if (rc) return rc;
   rc = validate_step(b);
   if (rc) return rc;
-  if (!b->have_G || b->result_precision != b->precision) {
-    rc = fnet_acsf_forward(ctx, b, nullptr);
+  rc = evaluate(b, 3);
+  if (rc || !F) return rc;
+  for (;;) {
+    rc = download(ctx, b->F, (size_t)b->N * ctx->model.nout * 3, F);
     if (rc) return rc;
+    bool redone;
+    rc = settle_list(b, &redone);
+    if (rc || !redone) return rc;
   }
-  if (!b->have_F) {
-    rc = do_mlp(b, 1);
-    if (rc) return rc;
-    rc = do_reduce(b);
-    if (rc) return rc;
-    rc = do_adjoint(b);
-    if (rc) return rc;
-  }
-  if (F)
-    return download_T(ctx, b->F, 1, (size_t)b->N * ctx->model.nout * 3, F);
-  return FNET_OK;
 }
 
 int fnet_run(fnet_ctx* ctx, fnet_batch* b) {
@@ -1588,15 +1686,28 @@ int fnet_set_graph(fnet_ctx* ctx, int enable) {
   return FNET_OK;
 }
 
+// Time between stage boundaries k0 and k1 of the last step (the stream has run).
+static int stage_ms(fnet_ctx* ctx, int k0, int k1, double* ms) {
+  if (ctx->stamped) {
+    unsigned long long t[8];
+    HIPCHECK(ctx, hipMemcpy(t, ctx->stamps, sizeof(t), hipMemcpyDeviceToHost));
+    // a replayed graph tells its total only
+    if (ctx->n_ev == 2) k1 = k1 == 1 ? 5 : k1;
+    *ms = ctx->stamp_khz > 0.0 ? (double)(long long)(t[k1] - t[k0]) / ctx->stamp_khz : 0.0;
+    return FNET_OK;
+  }
+  float t = 0.f;
+  HIPCHECK(ctx, hipEventElapsedTime(&t, ctx->ev[k0], ctx->ev[k1]));
+  *ms = t;
+  return FNET_OK;
+}
+
 int fnet_step_time(fnet_ctx* ctx, double* ms) {
   if (!ctx || !ms) return FNET_ERR_ARG;
   HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
   *ms = 0.0;
   if (ctx->n_ev < 2) return FNET_OK;
-  float t = 0.f;
-  HIPCHECK(ctx, hipEventElapsedTime(&t, ctx->ev[0], ctx->ev[ctx->n_ev - 1]));
-  *ms = t;
-  return FNET_OK;
+  return stage_ms(ctx, 0, ctx->n_ev - 1, ms);
 }
 
 int fnet_batch_step_info(const fnet_batch* b, int* graph) {
@@ -1610,9 +1721,8 @@ int fnet_stage_times(fnet_ctx* ctx, double* ms, int n) {
   HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
   int k = 0;
   for (; k < n && k + 1 < ctx->n_ev; ++k) {
-    float t = 0.f;
-    HIPCHECK(ctx, hipEventElapsedTime(&t, ctx->ev[k], ctx->ev[k + 1]));
-    ms[k] = t;
+    const int rc = stage_ms(ctx, k, k + 1, ms + k);
+    if (rc) return rc;
   }
   return FNET_OK;
 }
@@ -1671,9 +1781,10 @@ int fnet_autotune(fnet_ctx* ctx, fnet_batch* b, int reps, double* ms, int* knobs
       e = validate_step(b);
       if (e) return e;
       if (!eager) continue;
-      float t = 0.f;
-      HIPCHECK(ctx, hipEventElapsedTime(&t, ctx->ev[k0], ctx->ev[k1]));
-      best = std::min(best, (double)t);
+      double t = 0.0;
+      e = stage_ms(ctx, k0, k1, &t);
+      if (e) return e;
+      best = std::min(best, t);
     }
     *out = best;
     return FNET_OK;
@@ -1740,10 +1851,9 @@ int fnet_train_gradients(fnet_ctx* ctx, fnet_batch* b, int n_global, const doubl
   if (n_global < 0 || n_global > m.nout) return fail(ctx, FNET_ERR_ARG, "invalid n_global");
   if (n_global > 0 && !g_targets) return fail(ctx, FNET_ERR_ARG, "g_targets missing");
   if (n_global < m.nout && !a_targets) return fail(ctx, FNET_ERR_ARG, "a_targets missing");
-  if (!b->have_G || b->result_precision != b->precision) {
-    rc = fnet_acsf_forward(ctx, b, nullptr);
-    if (rc) return rc;
-  }
+  rc = evaluate(b, 1);
+  if (!rc) rc = validate_step(b);
+  if (rc) return rc;
   rc = do_mlp(b, 0);
   if (rc) return rc;
   rc = do_reduce(b);

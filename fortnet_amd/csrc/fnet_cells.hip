@@ -10,7 +10,7 @@
 // (dynneighlist.F90:291-294).  The hits of one centre are then sorted in LDS by (lattice image in
 // the reference's lexicographic order, (j - i) mod n), which is the order in which
 // TNeighIterator_getNextNeighbours (dynneighlist.F90:233-320) emits them.
-#include "fnet_internal.hpp"
+#include "fnet_device.hpp"
 
 namespace fnet {
 namespace {
@@ -35,33 +35,23 @@ __global__ void k_cell_bin(const double* __restrict__ xyz, const int* __restrict
   const int s = atom_struct[i];
   const int4 ci = cellinfo[s];
   if (!ci.w) return;
-  const StructInfo& si = sinfo[s];
-  const double x = xyz[3 * i], y = xyz[3 * i + 1], z = xyz[3 * i + 2];
-  const int nb[3] = {ci.x, ci.y, ci.z};
-  int m[3], bn[3];
-  for (int a = 0; a < 3; ++a) {
-    const double f = si.inv[0 * 3 + a] * x + si.inv[1 * 3 + a] * y + si.inv[2 * 3 + a] * z;
-    const double fl = floor(f);
-    m[a] = (int)fl;
-    int b = (int)((f - fl) * nb[a]);
-    bn[a] = b < 0 ? 0 : (b >= nb[a] ? nb[a] - 1 : b);
-  }
-  const int local = (bn[0] * nb[1] + bn[1]) * nb[2] + bn[2];
-  const int cell = cell_off[s] + local;
+  const int4 m = bin_of(sinfo[s], xyz + 3 * i, ci);
+  const int cell = cell_off[s] + m.w;
   atom_cell[i] = cell;
-  atom_m[i] = make_int4(m[0], m[1], m[2], local);
+  atom_m[i] = m;
   atomicAdd(&cell_count[cell], 1);
 }
 
+// Counts the cells back down to zero, so that the next search finds them cleared.
 __global__ void k_cell_scatter(const int* __restrict__ atom_struct,
                                const int4* __restrict__ cellinfo, long long a0, long long a1,
                                const int* __restrict__ atom_cell, const int* __restrict__ cell_start,
-                               int* __restrict__ cell_cursor, int* __restrict__ cell_atoms) {
+                               int* __restrict__ cell_count, int* __restrict__ cell_atoms) {
   const long long i = a0 + (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= a1) return;
   if (!cellinfo[atom_struct[i]].w) return;
   const int c = atom_cell[i];
-  cell_atoms[cell_start[c] + atomicAdd(&cell_cursor[c], 1)] = (int)i;
+  cell_atoms[cell_start[c] + atomicSub(&cell_count[c], 1) - 1] = (int)i;
 }
 
 struct CellArgs {
@@ -85,6 +75,8 @@ struct CellArgs {
   int* nimg;
   void* nd;
   int* mir;  // padded rows: each entry's mirror slot set to -1 when given
+  int* maxnb;  // padded rows: longest row
+  unsigned long long* t_end;
 };
 
 // MODE: 0 writes the row lengths; 1 writes the sorted rows at their CSR offsets; 2 writes row i
@@ -100,6 +92,7 @@ __global__ void __launch_bounds__(256) k_neigh_cells(CellArgs a) {
   if (i >= a.a1) return;
   const int s = a.atom_struct[i];
   const int4 ci = a.cellinfo[s];
+  if (MODE == 2 && blockIdx.x == gridDim.x - 1 && lane == 0) stamp_now(a.t_end);
   if (!ci.w) return;
   const int K = a.K;
   // LDS slice of this wave (fill pass only)
@@ -257,7 +250,10 @@ __global__ void __launch_bounds__(256) k_neigh_cells(CellArgs a) {
   }
   const long long rb = MODE == 2 ? i * a.cap : (long long)a.rowptr[i];
   const int mw = MODE == 2 ? (m < a.cap ? m : a.cap) : m;
-  if (MODE == 2 && lane == 0) a.cnt[i] = count;
+  if (MODE == 2 && lane == 0) {
+    a.cnt[i] = count;
+    raise_max(a.maxnb, count);
+  }
   V* out = (V*)a.nd;
   for (int e = lane; e < mw; e += 64) {
     const int q = slot[e];
@@ -270,7 +266,7 @@ __global__ void __launch_bounds__(256) k_neigh_cells(CellArgs a) {
 
 template <int MODE, typename V>
 hipError_t launch_cells_t(fnet_batch* b, double rc, long long a0, long long a1, hipStream_t s,
-                          int* mir = nullptr) {
+                          int* mir = nullptr, unsigned long long* stamp = nullptr) {
   constexpr bool WRITE = MODE != 0;
   const long long n = a1 - a0;
   if (n <= 0) return hipSuccess;
@@ -297,6 +293,8 @@ hipError_t launch_cells_t(fnet_batch* b, double rc, long long a0, long long a1, 
   a.nimg = MODE == 2 ? b->pnimg : b->nimg;
   a.nd = MODE == 2 ? b->pnd : b->nd;
   a.mir = MODE == 2 ? mir : nullptr;
+  a.maxnb = b->d_maxnb;
+  a.t_end = stamp;
   size_t lds = 0;
   int wpb = 4;
   if (WRITE) {
@@ -313,15 +311,12 @@ hipError_t launch_cells_t(fnet_batch* b, double rc, long long a0, long long a1, 
 }  // namespace
 
 hipError_t launch_cell_bin(fnet_batch* b, hipStream_t s) {
-  if (b->ncells == 0 || b->N == 0) return hipSuccess;
-  // fill kernels rather than memsets: this sequence is also captured into a HIP graph
-  FNET_HIP_TRY(launch_zero_int(b->cell_count, (int)b->ncells, s));
+  if (b->ncells == 0 || b->N == 0 || b->bin_lds > 0) return hipSuccess;
   const unsigned grid = (unsigned)((b->N + 255) / 256);
   k_cell_bin<<<grid, 256, 0, s>>>(b->xyz, b->atom_struct, b->sinfo, b->cellinfo, b->cell_off, 0,
                                   b->N, b->atom_cell, b->atom_m, b->cell_count);
   FNET_HIP_TRY(hipGetLastError());
   FNET_HIP_TRY(launch_scan(b->cell_count, b->cell_start, b->ncells, b->cell_scan_tmp, s, nullptr));
-  FNET_HIP_TRY(launch_zero_int(b->cell_count, (int)b->ncells, s));
   k_cell_scatter<<<grid, 256, 0, s>>>(b->atom_struct, b->cellinfo, 0, b->N, b->atom_cell,
                                       b->cell_start, b->cell_count, b->cell_atoms);
   return hipGetLastError();
@@ -351,10 +346,11 @@ hipError_t launch_cells_fill(fnet_batch* b, double rc, long long a0, long long a
               : launch_cells_t<1, float4>(b, rc, a0, a1, s);
 }
 
-hipError_t launch_cells_pad(fnet_batch* b, double rc, int fp64, hipStream_t s, int* mir) {
+hipError_t launch_cells_pad(fnet_batch* b, double rc, int fp64, hipStream_t s, int* mir,
+                            unsigned long long* stamp) {
   if (b->ncells == 0) return hipSuccess;
-  return fp64 ? launch_cells_t<2, double4>(b, rc, 0, b->N, s, mir)
-              : launch_cells_t<2, float4>(b, rc, 0, b->N, s, mir);
+  return fp64 ? launch_cells_t<2, double4>(b, rc, 0, b->N, s, mir, stamp)
+              : launch_cells_t<2, float4>(b, rc, 0, b->N, s, mir, stamp);
 }
 
 }  // namespace fnet

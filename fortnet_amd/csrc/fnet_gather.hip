@@ -25,14 +25,14 @@
 // The distance test is evaluated as coords(j) + L n - coords(i) in FP64, whose mirror expression
 // rounds differently; a pair exactly at the cutoff can therefore be in one row and not in the
 // other.  Such an entry has no mirror: the gather puts it on an orphan list and its -g is added to
-// its neighbour's force afterwards (k_force_orphans, the only atomic update left, for pairs within
+// its neighbour's force afterwards (k_force_finish, the only atomic update left, for pairs within
 // an ulp of the cutoff).
 #include <algorithm>
 #include <mutex>
 #include <string>
 
 #include "../../include/fnet_hip.h"
-#include "fnet_internal.hpp"
+#include "fnet_device.hpp"
 
 // Scratch of fnet_forces_noalloc: per-entry gradient vectors, mirror entries, the orphan list and
 // its counter of one force assembly, for callers that cannot allocate.  Each GPU holds its own
@@ -43,84 +43,28 @@ static __device__ __align__(256) unsigned char scratch[fnet::kNoallocScratchByte
 namespace fnet {
 namespace {
 
-struct RowLayout {
-  const int* rowptr;  // CSR rows (cap == 0)
-  const int* cnt;     // padded rows: row i at i * cap with cnt[i] entries
-  int cap;
-  __device__ __forceinline__ long long base(long long i) const {
-    return cap ? i * (long long)cap : (long long)rowptr[i];
-  }
-  __device__ __forceinline__ int len(long long i) const {
-    return cap ? min(cnt[i], cap) : rowptr[i + 1] - rowptr[i];
-  }
-};
-
-__device__ __forceinline__ int mod_n(int x, int n) {
-  x %= n;
-  return x < 0 ? x + n : x;
-}
-
-// One wave per centre; lanes over the centre's entries.  The entries store their keys
-// (image + 1) n + (j - i) mod n.  Each mirror pair is searched once, from the entry with i < j (or,
-// for the centre's own images, from the one with the lower image index), which writes both
-// directions; entries left at -1 (filled before) have no mirror.
-__global__ void __launch_bounds__(256)
-    k_mirror(RowLayout rl, const int* __restrict__ nj, const int* __restrict__ key,
-             const long long* __restrict__ off, const int* __restrict__ atom_struct,
-             const StructInfo* __restrict__ sinfo, long long a0, long long a1,
-             int* __restrict__ mir) {
-  const int lane = threadIdx.x & 63;
-  const long long i = a0 + ((long long)blockIdx.x * blockDim.x + threadIdx.x) / 64;
-  if (i >= a1) return;
-  const int s = atom_struct[i];
-  const long long o = off[s];
-  const int n = (int)(off[s + 1] - o);
-  const StructInfo& si = sinfo[s];
-  const int nimages =
-      si.periodic ? (si.hi[0] - si.lo[0] + 1) * (si.hi[1] - si.lo[1] + 1) *
-                            (si.hi[2] - si.lo[2] + 1) - 1
-                  : 0;
-  const int li = (int)(i - o);
-  const long long bi = rl.base(i);
-  const int len = rl.len(i);
-  for (int e = lane; e < len; e += 64) {
-    const int k = key[bi + e];
-    const int j = nj[bi + e];
-    const int lj = j - (int)o;
-    const int img = k / n - 1;
-    const int t = k - (img + 1) * n;  // (j - i) mod n
-    const int mimg = img < 0 ? -1 : nimages - 1 - img;
-    if (!(li < lj || (li == lj && img < mimg))) continue;
-    const int target = (mimg + 1) * n + (t == 0 ? 0 : n - t);
-    const long long bj = rl.base(j);
-    const int lenj = rl.len(j);
-    int lo = 0, hi = lenj;
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (key[bj + mid] < target) lo = mid + 1;
-      else hi = mid;
-    }
-    if (lo < lenj && key[bj + lo] == target) {
-      mir[bi + e] = (int)(bj + lo);
-      mir[bj + lo] = (int)(bi + e);
-    }
-  }
-}
-
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
-  return v;
+__global__ void __launch_bounds__(256) k_mirror(MirrorArgs a) {
+  mirror_centre(a, a.a0 + ((long long)blockIdx.x * blockDim.x + threadIdx.x) / 64,
+                threadIdx.x & 63);
 }
 
 // F_i += -sum over row i's slots of g (each holding the gradient of the slot's mirror entry), per
 // output, in row order, in FP64; entries of row i without a mirror (whose slot holds their own
 // gradient) go to the orphan list.  G: the type the adjoint stored g in (its own precision).
+// Blocks from ngather on sum the batch's energy chunks instead: both only wait for the kernels
+// before, and on small batches a launch costs as much as either.
 template <typename G>
 __global__ void __launch_bounds__(256)
     k_force_gather(RowLayout rl, const int* __restrict__ mir, const G* __restrict__ gvec,
                    long long a0, long long a1, int nout, double* __restrict__ F,
-                   int* __restrict__ orph, int* __restrict__ norph) {
+                   int* __restrict__ orph, int* __restrict__ norph, unsigned ngather,
+                   EnergyArgs en) {
+  __shared__ double ws[4];
+  if (blockIdx.x >= ngather) {
+    if (blockIdx.x == ngather && threadIdx.x == 0 && en.h_maxnb) *en.h_maxnb = *en.maxnb;
+    energy_chunk(en, (int)(blockIdx.x - ngather), ws);
+    return;
+  }
   const int lane = threadIdx.x & 63;
   const long long i = a0 + ((long long)blockIdx.x * blockDim.x + threadIdx.x) / 64;
   if (i >= a1) return;
@@ -151,12 +95,18 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// Entries without a mirror: -g to the neighbour's force.
+// Entries without a mirror: -g to the neighbour's force (block 0, which leaves the counter at zero
+// for the next gather); the other blocks add the chunk sums of structures of several chunks.
 template <typename G>
 __global__ void __launch_bounds__(256)
-    k_force_orphans(const int* __restrict__ norph, const int* __restrict__ orph,
-                    const int* __restrict__ nj, const G* __restrict__ gvec, int nout,
-                    double* __restrict__ F) {
+    k_force_finish(int* __restrict__ norph, const int* __restrict__ orph,
+                   const int* __restrict__ nj, const G* __restrict__ gvec, int nout,
+                   double* __restrict__ F, EnergyArgs en, int S, unsigned long long* ts) {
+  stamp(ts);
+  if (blockIdx.x > 0) {
+    energy_total(en, (long long)(blockIdx.x - 1) * 256 + threadIdx.x, 0, S);
+    return;
+  }
   const int cnt = *norph;
   for (int q = threadIdx.x; q < cnt; q += blockDim.x) {
     const long long e = orph[q];
@@ -165,6 +115,9 @@ __global__ void __launch_bounds__(256)
       for (int c = 0; c < 3; ++c)
         unsafeAtomicAdd(&F[(j * nout + t) * 3 + c], -(double)gvec[(e * nout + t) * 3 + c]);
   }
+  __syncthreads();
+  if (threadIdx.x == 0 && cnt) *norph = 0;
+  stamp(ts ? ts + 1 : nullptr);
 }
 
 __global__ void k_zero_int(int* __restrict__ p, int n) {
@@ -195,31 +148,32 @@ hipError_t launch_zero_int(int* p, int n, hipStream_t s) {
 
 // Mirror entries of atoms [a0, a1); `entries` > 0 first fills the whole mirror array with -1
 // (a range of atoms whose rows are alone in their structures may skip it after the first, and the
-// steady-state step skips it: its padded search sets every written entry's slot to -1).
+// padded search of a steady-state step clears the slots it writes).
 hipError_t launch_mirror(fnet_batch* b, long long a0, long long a1, long long entries,
                          hipStream_t s) {
   if (entries > 0)
     k_fill_int<<<(unsigned)((entries + 255) / 256), 256, 0, s>>>(b->mir, entries, -1);
   const long long n = a1 - a0;
   if (n <= 0) return hipGetLastError();
-  const int* nj = b->nl_padded ? b->pnj : b->nj;
-  const int* key = b->nl_padded ? b->pnimg : b->nimg;
-  k_mirror<<<(unsigned)((n + 3) / 4), 256, 0, s>>>(layout_of(b), nj, key, b->off, b->atom_struct,
-                                                   b->sinfo, a0, a1, b->mir);
+  k_mirror<<<(unsigned)((n + 3) / 4), 256, 0, s>>>(mirror_args(b, a0, a1));
   return hipGetLastError();
 }
 
-hipError_t launch_force_gather(fnet_batch* b, int nout, long long a0, long long a1,
-                               hipStream_t s) {
+hipError_t launch_force_gather(fnet_batch* b, const DevModel& m, long long a0, long long a1,
+                               bool energies, hipStream_t s) {
   const long long n = a1 - a0;
-  if (n <= 0) return hipSuccess;
-  const unsigned grid = (unsigned)((n + 3) / 4);
+  const unsigned ng = n > 0 ? (unsigned)((n + 3) / 4) : 0u;
+  const unsigned grid = ng + (energies ? (unsigned)b->nchunks : 0u);
+  if (grid == 0) return hipSuccess;
+  EnergyArgs en = energy_args(b, m);
+  if (energies) en.h_maxnb = b->h_maxnb;
   if (b->precision == FNET_FP64)
-    k_force_gather<double><<<grid, 256, 0, s>>>(layout_of(b), b->mir, b->gvec, a0, a1, nout,
-                                                (double*)b->F, b->orph, b->d_norph);
+    k_force_gather<double><<<grid, 256, 0, s>>>(layout_of(b), b->mir, b->gvec, a0, a1, m.nout,
+                                                (double*)b->F, b->orph, b->d_norph, ng, en);
   else
     k_force_gather<float><<<grid, 256, 0, s>>>(layout_of(b), b->mir, (const float*)b->gvec, a0,
-                                               a1, nout, (double*)b->F, b->orph, b->d_norph);
+                                               a1, m.nout, (double*)b->F, b->orph, b->d_norph, ng,
+                                               en);
   return hipGetLastError();
 }
 
@@ -247,14 +201,18 @@ void* scratch_ptr(int device) {
   return g_scratch_ptr[device];
 }
 
-hipError_t launch_force_orphans(fnet_batch* b, int nout, hipStream_t s) {
+hipError_t launch_force_finish(fnet_batch* b, const DevModel& m, bool energies, hipStream_t s,
+                               unsigned long long* stamps) {
   const int* nj = b->nl_padded ? b->pnj : b->nj;
+  const EnergyArgs en = energy_args(b, m);
+  const unsigned grid =
+      1u + (energies && !en.single ? (unsigned)(((long long)b->S * m.nout + 255) / 256) : 0u);
   if (b->precision == FNET_FP64)
-    k_force_orphans<double><<<1, 256, 0, s>>>(b->d_norph, b->orph, nj, b->gvec, nout,
-                                               (double*)b->F);
+    k_force_finish<double><<<grid, 256, 0, s>>>(b->d_norph, b->orph, nj, b->gvec, m.nout,
+                                                (double*)b->F, en, b->S, stamps);
   else
-    k_force_orphans<float><<<1, 256, 0, s>>>(b->d_norph, b->orph, nj, (const float*)b->gvec,
-                                              nout, (double*)b->F);
+    k_force_finish<float><<<grid, 256, 0, s>>>(b->d_norph, b->orph, nj, (const float*)b->gvec,
+                                               m.nout, (double*)b->F, en, b->S, stamps);
   return hipGetLastError();
 }
 
@@ -337,13 +295,13 @@ extern "C" int fnet_forces_noalloc(fnet_ctx* ctx, fnet_batch* b) {
     if (b->launch == FNET_PER_STRUCT) {
       for (int st = 0; st < b->S && e == hipSuccess; ++st) {
         e = launch_acsf_adj(b, m, b->h_off[st], b->h_off[st + 1], fp64, s);
-        if (e == hipSuccess) e = launch_force_gather(b, m.nout, b->h_off[st], b->h_off[st + 1], s);
+        if (e == hipSuccess) e = launch_force_gather(b, m, b->h_off[st], b->h_off[st + 1], false, s);
       }
     } else {
       if (e == hipSuccess) e = launch_acsf_adj(b, m, 0, b->N, fp64, s);
-      if (e == hipSuccess) e = launch_force_gather(b, m.nout, 0, b->N, s);
+      if (e == hipSuccess) e = launch_force_gather(b, m, 0, b->N, false, s);
     }
-    if (e == hipSuccess) e = launch_force_orphans(b, m.nout, s);
+    if (e == hipSuccess) e = launch_force_finish(b, m, false, s);
   }
   if (e != hipSuccess) {
     ctx->err = std::string("fnet_forces_noalloc: ") + hipGetErrorString(e);

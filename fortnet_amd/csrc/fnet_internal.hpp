@@ -159,11 +159,6 @@ struct Tune {
   }
 };
 
-struct Timer {
-  hipEvent_t ev[8];
-  bool made = false;
-};
-
 }  // namespace fnet
 
 struct fnet_batch;
@@ -179,7 +174,11 @@ struct fnet_ctx {
   fnet::DevModel model;
   hipEvent_t ev[8] = {};
   int n_ev = 0;
-  double stage_ms[8] = {};
+  // stage boundaries of the last steady-state step, written by its kernels (an event between two
+  // kernels costs a barrier packet each); stamped: the last step's times are these
+  unsigned long long* stamps = nullptr;
+  double stamp_khz = 0.0;
+  bool stamped = false;
   double* d_grad = nullptr; // [nspecies][nparams] FP64 gradient of the last train call
   long long grad_cap = 0;
   bool have_grad = false;
@@ -273,7 +272,10 @@ struct fnet_batch {
   int* atom_cell = nullptr;    // [N]
   int4* atom_m = nullptr;      // [N] integer part of the fractional coordinates, local bin
   int* cell_scan_tmp = nullptr;
-  long long ncells = 0;
+  long long ncells = 0;        // cells of the structures with cell lists, one more per structure
+  int n_cell_struct = 0;       // structures with cell lists
+  int bin_lds = 0;             // > 0: every such structure is binned by its struct-prep block, with
+                               // this many LDS bins; 0: binning kernels over all atoms
   std::vector<int> h_cellinfo; // [4*S]
   std::vector<double> h_lat;   // [S][9]
   std::vector<int> h_periodic; // [S]
@@ -293,12 +295,14 @@ struct fnet_batch {
   long long gv_entries = 0;    // allocated entries of mir / orph
   long long gv_len = 0;        // allocated doubles of gvec
   bool have_mirror = false;
+  bool mir_clear = false;      // every entry of the current padded list has its mirror slot at -1
   // energy reduction in fixed-size chunks of atoms (two passes, fixed order)
   int* chunk_struct = nullptr; // [nchunks]
   int* chunk_first = nullptr;  // [S+1]
   double* Epart = nullptr;     // [nchunks][nout]
   std::vector<int> h_chunk_first;
   int nchunks = 0;
+  int single_chunks = 0;       // every structure has exactly one chunk
   long long epart_len = 0;
   // weight gradient: one FP64 partial vector per network tile, reduced in tile order
   double* gpart = nullptr;
@@ -307,6 +311,7 @@ struct fnet_batch {
   // copied to pinned host memory with the step and checked when results are next read
   int* h_maxnb = nullptr;
   bool pending = false;
+  int pending_level = 0;        // what was computed on that list: 1 features, 2 energies, 3 forces
   long long gen = 0;            // bumped whenever a buffer the step uses is reallocated
   // HIP graph of the steady-state step and the launch parameters it was captured with
   hipGraph_t graph = nullptr;
@@ -341,20 +346,23 @@ __device__ __forceinline__ double entry_r(double w) { return sqrt(w); }
 __device__ __forceinline__ float entry_r(float w) { return sqrtf(w); }
 
 // launchers (fnet_neigh.hip)
-hipError_t launch_struct_prep(fnet_batch* b, double rc, hipStream_t s);
+// lattices, extents and (bin_lds > 0) cell bins; clears the batch's row maximum
+hipError_t launch_struct_prep(fnet_batch* b, double rc, hipStream_t s,
+                              unsigned long long* stamp = nullptr);
+constexpr int kPrepBins = 4096;      // LDS bins of one struct-prep block
+constexpr int kPrepBinAtoms = 8192;  // largest structure a struct-prep block bins
 hipError_t launch_neigh_count(fnet_batch* b, double rc, long long a0, long long a1, hipStream_t s);
 hipError_t launch_neigh_fill(fnet_batch* b, double rc, long long a0, long long a1, int fp64,
                              hipStream_t s);
 // padded rows; a non-null mir (sized for the padded layout) gets -1 at every entry written
+// (stamp: end of the launch)
 hipError_t launch_neigh_pad(fnet_batch* b, double rc, int fp64, hipStream_t s,
-                            int* mir = nullptr);
+                            int* mir = nullptr, unsigned long long* stamp = nullptr);
 hipError_t launch_cells_pad(fnet_batch* b, double rc, int fp64, hipStream_t s,
-                            int* mir = nullptr);
+                            int* mir = nullptr, unsigned long long* stamp = nullptr);
 hipError_t launch_compact_rows(fnet_batch* b, int fp64, hipStream_t s);
 hipError_t launch_scan(int* cnt, int* rowptr, long long n, int* tmp, hipStream_t s,
                        int* maxout);
-// *out = max(cnt[0..n)) (graph-safe: zeroed by a kernel)
-hipError_t launch_row_max(const int* cnt, long long n, int* out, hipStream_t s);
 long long scan_tmp_size(long long n);
 
 // launchers (fnet_cells.hip)
@@ -394,21 +402,28 @@ void* scratch_ptr(int device);
 hipError_t launch_zero_int(int* p, int n, hipStream_t s);
 hipError_t launch_mirror(fnet_batch* b, long long a0, long long a1, long long fill_entries,
                          hipStream_t s);
-hipError_t launch_force_gather(fnet_batch* b, int nout, long long a0, long long a1,
-                               hipStream_t s);
-hipError_t launch_force_orphans(fnet_batch* b, int nout, hipStream_t s);
+// energies: also the energy chunks of the whole batch, in blocks of their own
+hipError_t launch_force_gather(fnet_batch* b, const DevModel& m, long long a0, long long a1,
+                               bool energies, hipStream_t s);
+// the orphans' part of the forces (and their counter reset); energies: also the sums over the
+// chunks; stamps: {start, end} of the launch
+hipError_t launch_force_finish(fnet_batch* b, const DevModel& m, bool energies, hipStream_t s,
+                               unsigned long long* stamps = nullptr);
 
 // launchers (fnet_acsf.hip)
 hipError_t launch_acsf_fwd(fnet_batch* b, const DevModel& m, long long a0, long long a1, int fp64,
                            hipStream_t s);
 hipError_t launch_acsf_adj(fnet_batch* b, const DevModel& m, long long a0, long long a1, int fp64,
-                           hipStream_t s);
+                           hipStream_t s, unsigned long long* stamp = nullptr);
 
 // launchers (fnet_mlp.hip)
+// mirror: extra blocks of the launch search the mirror entries of the whole batch
 hipError_t launch_mlp_fwd(fnet_batch* b, const DevModel& m, int first_tile, int ntiles, int fp64,
-                          int want_grad_in, hipStream_t s);
+                          int want_grad_in, hipStream_t s, bool mirror = false,
+                          unsigned long long* stamp = nullptr);
 constexpr int kEnergyChunk = 2048;  // atoms per block of the energy reduction
-hipError_t launch_energy_reduce(fnet_batch* b, const DevModel& m, int s0, int s1, hipStream_t s);
+hipError_t launch_energy_reduce(fnet_batch* b, const DevModel& m, int s0, int s1, hipStream_t s,
+                                int* h_maxnb = nullptr);
 hipError_t launch_lossgrad(fnet_batch* b, const DevModel& m, int n_global, const double* gt,
                            const double* at, const double* aw, const double* dpw, double inv_wsum,
                            int loss, hipStream_t s);
@@ -442,7 +457,8 @@ void pack_bf16_weights(const NetShape& sh, int nspecies, const double* params,
                        std::vector<uint16_t>& out, long long& stride, long long* bfw,
                        long long* brw, long long* bsz);
 hipError_t launch_mlp_mfma(fnet_batch* b, const DevModel& m, int first_tile, int ntiles,
-                           int want_grad_in, hipStream_t s);
+                           int want_grad_in, hipStream_t s, bool mirror = false,
+                           unsigned long long* stamp = nullptr);
 hipError_t launch_to_float(const double* in, float* out, long long n, hipStream_t s);
 
 size_t lds_bytes_acsf(int max_nb, int nZ, int fp64, int adj);

@@ -6,7 +6,7 @@
 // bpnn.F90:692-702).  Per-structure energies and weight gradients are reduced in FP64.
 #include <algorithm>
 
-#include "fnet_internal.hpp"
+#include "fnet_device.hpp"
 
 namespace fnet {
 namespace {
@@ -69,6 +69,9 @@ struct MlpArgs {
   double* cG;         // [N][nout][nG]
   const double* lossgrad; // [N][nout]
   double* grad;       // [nspecies][nparams]
+  int ntiles;         // blocks beyond the tiles search mirror entries
+  MirrorArgs mr;
+  unsigned long long* stamp;
 };
 
 // LDS per tile: input x [TA][d0], activations of every layer [TA][d_l], f'(z) of hidden layers,
@@ -136,6 +139,12 @@ __device__ __forceinline__ size_t mlp_lds_floats(const NetShape& sh, int TA) {
 template <typename T, bool GRADIN>
 __global__ void __launch_bounds__(256) k_mlp_fwd(MlpArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
+  stamp(a.stamp);
+  if ((int)blockIdx.x >= a.ntiles) {
+    mirror_centre(a.mr, (long long)((int)blockIdx.x - a.ntiles) * 4 + (threadIdx.x >> 6),
+                  threadIdx.x & 63);
+    return;
+  }
   const int tile = a.first_tile + blockIdx.x;
   const int sp = a.tile_sp[tile], start = a.tile_start[tile], cnt = a.tile_cnt[tile];
   const int nl = a.sh.nl;
@@ -307,46 +316,14 @@ __global__ void k_grad_reduce(const double* __restrict__ gchunk, int nchunks, lo
   grad[q] = v;
 }
 
-// Per-structure sums of the atomic outputs (predictBatch sums, bpnn.F90:1040-1047;
-// forces.F90:381-385) in FP64, in two passes with a fixed order: each block sums one chunk of
-// kEnergyChunk atoms of one structure (thread t takes atoms t, t + 256, ... in order; the four
-// wave sums combine in a fixed order), then one thread per (structure, output) adds its chunks'
-// partials in chunk order.  The result does not depend on scheduling, and a large cell is spread
-// over many blocks instead of one.
-__global__ void __launch_bounds__(256) k_energy_partial(const double* __restrict__ Eatom,
-                                                       const long long* __restrict__ off,
-                                                       const int* __restrict__ chunk_struct,
-                                                       const int* __restrict__ chunk_first,
-                                                       int c0, int nout,
-                                                       double* __restrict__ Epart) {
+__global__ void __launch_bounds__(256) k_energy_partial(EnergyArgs a, int c0) {
   __shared__ double ws[4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int c = c0 + blockIdx.x;
-  const int s = chunk_struct[c];
-  const long long a0 = off[s] + (long long)(c - chunk_first[s]) * kEnergyChunk;
-  const long long a1 = min(a0 + (long long)kEnergyChunk, off[s + 1]);
-  for (int t = 0; t < nout; ++t) {
-    double v = 0.0;
-    for (long long i = a0 + threadIdx.x; i < a1; i += 256) v += Eatom[i * nout + t];
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
-    if (lane == 0) ws[wave] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) Epart[(long long)c * nout + t] = (ws[0] + ws[1]) + (ws[2] + ws[3]);
-    __syncthreads();
-  }
+  if (blockIdx.x == 0 && threadIdx.x == 0 && a.h_maxnb) *a.h_maxnb = *a.maxnb;
+  energy_chunk(a, c0 + (int)blockIdx.x, ws);
 }
 
-__global__ void k_energy_final(const double* __restrict__ Epart,
-                               const int* __restrict__ chunk_first, int s0, int s1, int nout,
-                               double* __restrict__ Estruct) {
-  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long long s = s0 + q / nout;
-  const int t = (int)(q % nout);
-  if (s >= s1) return;
-  double v = 0.0;
-  for (int c = chunk_first[s]; c < chunk_first[s + 1]; ++c) v += Epart[(long long)c * nout + t];
-  Estruct[s * nout + t] = v;
+__global__ void k_energy_final(EnergyArgs a, int s0, int s1) {
+  energy_total(a, (long long)blockIdx.x * blockDim.x + threadIdx.x, s0, s1);
 }
 
 // Loss-gradient functions of loss.F90:217-281, elementwise on (prediction, target):
@@ -591,6 +568,9 @@ MlpArgs make_args(fnet_batch* b, const DevModel& m, int first_tile) {
   a.cG = (double*)b->cG;
   a.lossgrad = b->lossgrad;
   a.grad = nullptr;
+  a.ntiles = b->ntiles;
+  a.mr = mirror_args(b, 0, b->N);
+  a.stamp = nullptr;
   return a;
 }
 
@@ -605,32 +585,38 @@ int mlp_tile_atoms(const NetShape& sh, int fp64) {
 }
 
 hipError_t launch_mlp_fwd(fnet_batch* b, const DevModel& m, int first_tile, int ntiles, int fp64,
-                          int want_grad_in, hipStream_t s) {
+                          int want_grad_in, hipStream_t s, bool mirror,
+                          unsigned long long* stamp) {
   if (ntiles <= 0) return hipSuccess;
+  auto go = [&](auto* grad, auto* plain, MlpArgs a, size_t lds) {
+    a.ntiles = ntiles;
+    a.stamp = stamp;
+    const unsigned grid = ntiles + (mirror ? (unsigned)((b->N + 3) / 4) : 0u);
+    if (want_grad_in) grad<<<grid, 256, lds, s>>>(a);
+    else plain<<<grid, 256, lds, s>>>(a);
+  };
   if (fp64) {
     MlpArgs a = make_args<double>(b, m, first_tile);
-    const size_t lds = host_lds<double>(m.shape, a.TA);
-    if (want_grad_in) k_mlp_fwd<double, true><<<ntiles, 256, lds, s>>>(a);
-    else k_mlp_fwd<double, false><<<ntiles, 256, lds, s>>>(a);
+    go(k_mlp_fwd<double, true>, k_mlp_fwd<double, false>, a, host_lds<double>(m.shape, a.TA));
   } else {
     MlpArgs a = make_args<float>(b, m, first_tile);
-    const size_t lds = host_lds<float>(m.shape, a.TA);
-    if (want_grad_in) k_mlp_fwd<float, true><<<ntiles, 256, lds, s>>>(a);
-    else k_mlp_fwd<float, false><<<ntiles, 256, lds, s>>>(a);
+    go(k_mlp_fwd<float, true>, k_mlp_fwd<float, false>, a, host_lds<float>(m.shape, a.TA));
   }
   return hipGetLastError();
 }
 
-hipError_t launch_energy_reduce(fnet_batch* b, const DevModel& m, int s0, int s1, hipStream_t s) {
+hipError_t launch_energy_reduce(fnet_batch* b, const DevModel& m, int s0, int s1, hipStream_t s,
+                                int* h_maxnb) {
   const int n = s1 - s0;
   if (n <= 0) return hipSuccess;
+  EnergyArgs a = energy_args(b, m);
+  a.h_maxnb = h_maxnb;
   const int c0 = b->h_chunk_first[s0], nc = b->h_chunk_first[s1] - c0;
-  if (nc > 0)
-    k_energy_partial<<<nc, 256, 0, s>>>(b->Eatom, b->off, b->chunk_struct, b->chunk_first, c0,
-                                        m.nout, b->Epart);
-  const long long q = (long long)n * m.nout;
-  k_energy_final<<<(unsigned)((q + 255) / 256), 256, 0, s>>>(b->Epart, b->chunk_first, s0, s1,
-                                                            m.nout, b->Estruct);
+  if (nc > 0) k_energy_partial<<<nc, 256, 0, s>>>(a, c0);
+  if (!a.single) {
+    const long long q = (long long)n * m.nout;
+    k_energy_final<<<(unsigned)((q + 255) / 256), 256, 0, s>>>(a, s0, s1);
+  }
   return hipGetLastError();
 }
 

@@ -28,7 +28,7 @@
 #include <cstring>
 
 #include "../../include/fnet_hip.h"
-#include "fnet_internal.hpp"
+#include "fnet_device.hpp"
 
 namespace fnet {
 namespace {
@@ -125,6 +125,9 @@ struct MfmaArgs {
   int wave_floats;
   double* Eatom;  // [N][nout]
   double* cG;     // [N][nout][nG]
+  int ntiles;     // blocks beyond the tiles search mirror entries
+  MirrorArgs mr;
+  unsigned long long* stamp;
 };
 
 // Row stride and per-wave LDS (floats) for a network shape: 16 activation rows of the widest
@@ -244,6 +247,11 @@ __global__ void __launch_bounds__(256) k_mlp_mfma(MfmaArgs a) {
   extern __shared__ __align__(16) float smf[];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int g = lane >> 4, j = lane & 15;
+  stamp(a.stamp);
+  if ((int)blockIdx.x >= a.ntiles) {
+    mirror_centre(a.mr, (long long)((int)blockIdx.x - a.ntiles) * (blockDim.x >> 6) + w, lane);
+    return;
+  }
   const int tile = a.first_tile + blockIdx.x;
   const int sp = a.tile_sp[tile], start = a.tile_start[tile], cnt = a.tile_cnt[tile];
   const int a0 = 16 * w;
@@ -817,7 +825,8 @@ hipError_t launch_mlp_grad_mfma(fnet_batch* b, const DevModel& m, hipStream_t s)
 }
 
 hipError_t launch_mlp_mfma(fnet_batch* b, const DevModel& m, int first_tile, int ntiles,
-                           int want_grad_in, hipStream_t s) {
+                           int want_grad_in, hipStream_t s, bool mirror,
+                           unsigned long long* stamp) {
   if (ntiles <= 0) return hipSuccess;
   MfmaArgs a;
   a.sh = m.shape;
@@ -856,7 +865,11 @@ hipError_t launch_mlp_mfma(fnet_batch* b, const DevModel& m, int first_tile, int
                : (b->precision == FNET_BF16_FAST && m.bpack) ? 1 : 0;
   const int waves = b->mtile_waves;
   const size_t lds = (size_t)waves * a.wave_floats * sizeof(float);
-  const dim3 grid(ntiles), block(64 * waves);
+  a.ntiles = ntiles;
+  a.mr = mirror_args(b, 0, b->N);
+  a.stamp = stamp;
+  const dim3 grid((unsigned)(ntiles + (mirror ? (b->N + waves - 1) / waves : 0))),
+      block(64 * waves);
   if (want_grad_in) {
     if (bf == 3) k_mlp_mfma<true, 3><<<grid, block, lds, s>>>(a);
     else if (bf == 1) k_mlp_mfma<true, 1><<<grid, block, lds, s>>>(a);
