@@ -296,7 +296,7 @@ class Context:
     def optimizer_step(self):
         """``fnet_optimizer_step`` on the gradient of the last train call: (new params,
         converged flag of the last network)."""
-        out = np.zeros_like(self.model.params)
+        out = np.empty_like(self.model.params)
         conv = ctypes.c_int(0)
         check(self.h, self.lib.fnet_optimizer_step(self.h, self._opt, ptr(out),
                                                    ctypes.byref(conv)), "fnet_optimizer_step")
@@ -305,7 +305,7 @@ class Context:
 
     def sd_step(self, lr, max_disp=1e4, tol=0.0):
         """``fnet_optimizer_step_sd`` on the gradient of the last train call."""
-        out = np.zeros_like(self.model.params)
+        out = np.empty_like(self.model.params)
         conv = ctypes.c_int(0)
         check(self.h, self.lib.fnet_optimizer_step_sd(self.h, lr, max_disp, tol, ptr(out),
                                                       ctypes.byref(conv)), "fnet_optimizer_step_sd")
@@ -411,7 +411,7 @@ class Batch:
 
     def acsf(self):
         """Unstandardised ACSF values [N, nG] (``TAcsf%calculate``)."""
-        G = np.zeros((self.N, len(self.ctx.model.g)))
+        G = np.empty((self.N, len(self.ctx.model.g)))
         check(self.ctx.h, self.lib.fnet_acsf_forward(self.ctx.h, self.h, ptr(G)),
               "fnet_acsf_forward")
         return G
@@ -419,14 +419,14 @@ class Batch:
     def energy(self):
         """(E_struct [S, nOut], E_atom [N, nOut])."""
         no = self.ctx.model.n_out
-        Es = np.zeros((self.S, no))
-        Ea = np.zeros((self.N, no))
+        Es = np.empty((self.S, no))
+        Ea = np.empty((self.N, no))
         check(self.ctx.h, self.lib.fnet_energy(self.ctx.h, self.h, ptr(Es), ptr(Ea)), "fnet_energy")
         return Es, Ea
 
     def forces(self):
         """F [N, 3*nOut] in the fnetout layout (F[k, 3t + c])."""
-        F = np.zeros((self.N, 3 * self.ctx.model.n_out))
+        F = np.empty((self.N, 3 * self.ctx.model.n_out))
         check(self.ctx.h, self.lib.fnet_forces(self.ctx.h, self.h, ptr(F)), "fnet_forces")
         return F
 
@@ -480,8 +480,8 @@ class Batch:
             at = _f64(a_targets).reshape(self.N, m.n_out - ng)
         aw = None if atomic_weights is None else _f64(atomic_weights).reshape(self.N)
         dw = None if dp_weights is None else _f64(dp_weights).reshape(self.S)
-        grad = np.zeros_like(m.params)
-        pred = np.zeros((self.N, m.n_out))
+        grad = np.empty_like(m.params)
+        pred = np.empty((self.N, m.n_out))
         loss = np.zeros(1)
         check(self.ctx.h, self.lib.fnet_train_gradients(self.ctx.h, self.h, ng, ptr(gt), ptr(at),
                                                         ptr(aw), ptr(dw), ptr(grad), ptr(pred),

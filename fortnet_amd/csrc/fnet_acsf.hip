@@ -212,6 +212,7 @@ struct AcsfArgs {
                     // FP64 values from the FP64 kernels, FP32 values from the FP32 ones
   const int* mir;   // [entries] mirror entries (-1: none)
   unsigned long long* stamp;  // start time of the launch, when asked for
+  int* norph;       // adjoint: counter of the gather's orphans, cleared here (or null)
 };
 
 // Bytes of one wave's LDS slice (host and device agree on this layout).  Per entry, in element
@@ -1919,7 +1920,10 @@ template <typename T, bool ADJ, int MQ, int FORM, bool PAIRS, bool R64 = false,
           bool PERSIST = false>
 __device__ __forceinline__ void acsf_wave(const AcsfArgs& a) {
   // (the paired forward has no register left for it: its boundary is the search's end)
-  if constexpr (ADJ) stamp(a.stamp);
+  if constexpr (ADJ) {
+    stamp(a.stamp);
+    if (a.norph && blockIdx.x == 0 && threadIdx.x == 0) *a.norph = 0;
+  }
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wpb = blockDim.x >> 6;
   long long i = a.a0 + (long long)blockIdx.x * wpb + wave;
@@ -1978,7 +1982,7 @@ __global__ void __launch_bounds__(512) k_acsf_fwd32_r64(AcsfArgs a) {
 
 template <typename T, bool ADJ, int MQ, int FORM>
 hipError_t launch_mq(fnet_batch* b, const DevModel& m, long long a0, long long a1,
-                     hipStream_t s, unsigned long long* stamp) {
+                     hipStream_t s, int* norph, unsigned long long* stamp) {
   const long long n = a1 - a0;
   if (n <= 0) return hipSuccess;
   const Tune& tn = tune_of(b);
@@ -2026,6 +2030,7 @@ hipError_t launch_mq(fnet_batch* b, const DevModel& m, long long a0, long long a
   a.gvec = b->gvec;
   a.mir = b->mir;
   a.stamp = stamp;
+  a.norph = norph;
   const unsigned grid = (unsigned)((n + wpb - 1) / wpb);
   const size_t lds = sb * wpb;
   // persistent grids exist for the FP32 exponent-ladder kernels (the batched FP32 / BF16 path);
@@ -2068,42 +2073,41 @@ hipError_t launch_mq(fnet_batch* b, const DevModel& m, long long a0, long long a
 
 template <typename T, bool ADJ>
 hipError_t launch(fnet_batch* b, const DevModel& m, long long a0, long long a1, hipStream_t s,
-                  unsigned long long* stamp) {
-  if (m.form == 1) return launch_mq<T, ADJ, 1, 1>(b, m, a0, a1, s, stamp);
+                  int* norph = nullptr, unsigned long long* stamp = nullptr) {
+  if (m.form == 1) return launch_mq<T, ADJ, 1, 1>(b, m, a0, a1, s, norph, stamp);
   if (m.form == 2) {
-    if (m.maxprog <= 4) return launch_mq<T, ADJ, 4, 2>(b, m, a0, a1, s, stamp);
-    return launch_mq<T, ADJ, kProgLen, 2>(b, m, a0, a1, s, stamp);
+    if (m.maxprog <= 4) return launch_mq<T, ADJ, 4, 2>(b, m, a0, a1, s, norph, stamp);
+    return launch_mq<T, ADJ, kProgLen, 2>(b, m, a0, a1, s, norph, stamp);
   }
-  if (m.maxmem <= 4) return launch_mq<T, ADJ, 4, 0>(b, m, a0, a1, s, stamp);
-  if (m.maxmem <= 8) return launch_mq<T, ADJ, 8, 0>(b, m, a0, a1, s, stamp);
-  if (m.maxmem <= 12) return launch_mq<T, ADJ, 12, 0>(b, m, a0, a1, s, stamp);
-  return launch_mq<T, ADJ, kMaxMembers, 0>(b, m, a0, a1, s, stamp);
+  if (m.maxmem <= 4) return launch_mq<T, ADJ, 4, 0>(b, m, a0, a1, s, norph, stamp);
+  if (m.maxmem <= 8) return launch_mq<T, ADJ, 8, 0>(b, m, a0, a1, s, norph, stamp);
+  if (m.maxmem <= 12) return launch_mq<T, ADJ, 12, 0>(b, m, a0, a1, s, norph, stamp);
+  return launch_mq<T, ADJ, kMaxMembers, 0>(b, m, a0, a1, s, norph, stamp);
 }
 
 }  // namespace
 
 #if FNET_ACSF_PART == 1
 hipError_t launch_acsf_adj32(fnet_batch* b, const DevModel& m, long long a0, long long a1,
-                             hipStream_t s, unsigned long long* stamp) {
-  return launch<float, true>(b, m, a0, a1, s, stamp);
+                             hipStream_t s, int* norph, unsigned long long* stamp) {
+  return launch<float, true>(b, m, a0, a1, s, norph, stamp);
 }
 #elif FNET_ACSF_PART == 2
 hipError_t launch_acsf_fwd64(fnet_batch* b, const DevModel& m, long long a0, long long a1,
-                             hipStream_t s, unsigned long long* stamp) {
-  return launch<double, false>(b, m, a0, a1, s, stamp);
+                             hipStream_t s) {
+  return launch<double, false>(b, m, a0, a1, s);
 }
 #elif FNET_ACSF_PART == 3
 hipError_t launch_acsf_adj64(fnet_batch* b, const DevModel& m, long long a0, long long a1,
-                             hipStream_t s, unsigned long long* stamp) {
-  return launch<double, true>(b, m, a0, a1, s, stamp);
+                             hipStream_t s, int* norph, unsigned long long* stamp) {
+  return launch<double, true>(b, m, a0, a1, s, norph, stamp);
 }
 #else
+hipError_t launch_acsf_fwd64(fnet_batch*, const DevModel&, long long, long long, hipStream_t);
 hipError_t launch_acsf_adj32(fnet_batch*, const DevModel&, long long, long long, hipStream_t,
-                             unsigned long long*);
-hipError_t launch_acsf_fwd64(fnet_batch*, const DevModel&, long long, long long, hipStream_t,
-                             unsigned long long*);
+                             int*, unsigned long long*);
 hipError_t launch_acsf_adj64(fnet_batch*, const DevModel&, long long, long long, hipStream_t,
-                             unsigned long long*);
+                             int*, unsigned long long*);
 
 int acsf_slice_entries(int max_nb) { return slice_entries(max_nb); }
 
@@ -2116,14 +2120,13 @@ size_t lds_bytes_acsf(int max_nb, int nZ, int fp64, int adj) {
 
 hipError_t launch_acsf_fwd(fnet_batch* b, const DevModel& m, long long a0, long long a1, int fp64,
                            hipStream_t s) {
-  return fp64 ? launch_acsf_fwd64(b, m, a0, a1, s, nullptr)
-              : launch<float, false>(b, m, a0, a1, s, nullptr);
+  return fp64 ? launch_acsf_fwd64(b, m, a0, a1, s) : launch<float, false>(b, m, a0, a1, s);
 }
 
 hipError_t launch_acsf_adj(fnet_batch* b, const DevModel& m, long long a0, long long a1, int fp64,
-                           hipStream_t s, unsigned long long* stamp) {
-  return fp64 ? launch_acsf_adj64(b, m, a0, a1, s, stamp)
-              : launch_acsf_adj32(b, m, a0, a1, s, stamp);
+                           hipStream_t s, int* norph, unsigned long long* stamp) {
+  return fp64 ? launch_acsf_adj64(b, m, a0, a1, s, norph, stamp)
+              : launch_acsf_adj32(b, m, a0, a1, s, norph, stamp);
 }
 #endif
 

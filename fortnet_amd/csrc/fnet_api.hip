@@ -34,7 +34,10 @@ const Tune& tune_of(const fnet_batch* b) {
 namespace {
 
 int fail(fnet_ctx* ctx, int code, const std::string& msg) {
-  if (ctx) ctx->err = msg;
+  if (ctx) {
+    ctx->err = msg;
+    ctx->segs.n = 0;  // copies of a call that did not get through are not made
+  }
   return code;
 }
 
@@ -61,11 +64,10 @@ void dfree(void* p) {
 }
 
 template <typename T>
-hipError_t upload(T** p, const T* h, size_t count, hipStream_t s) {
+hipError_t upload(fnet_ctx* ctx, T** p, const T* h, size_t count) {
   hipError_t e = dalloc(p, count);
   if (e != hipSuccess) return e;
-  if (count && h) return hipMemcpyAsync(*p, h, sizeof(T) * count, hipMemcpyHostToDevice, s);
-  return hipSuccess;
+  return h ? stage_in(ctx, *p, h, sizeof(T) * count) : hipSuccess;
 }
 
 void free_model(DevModel& m) {
@@ -191,6 +193,7 @@ void progression_form(AngGroup& a) {
 
 void invalidate(fnet_batch* b) {
   b->have_nl = b->have_G = b->have_E = b->have_F = false;
+  b->host_E = b->host_F = false;
   b->have_mirror = b->mir_clear = false;
   b->pending = false;
 }
@@ -210,34 +213,8 @@ int upload_zcode(fnet_batch* b) {
   }
   b->zone = one;
   b->zcode_gen = ctx->model_gen;
-  if (N)
-    HIPCHECK(ctx, hipMemcpyAsync(b->zcode, zc.data(), sizeof(int) * N, hipMemcpyHostToDevice,
-                                 ctx->stream));
-  // the copy reads zc before this function returns
-  HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
-  return FNET_OK;
-}
-
-// Packs the host copy of the parameters into MFMA fragments and uploads them (FP32 networks on
-// the matrix cores); a model whose shape the MFMA kernel does not take keeps wpack empty.
-int upload_wpack(fnet_ctx* ctx, DevModel& m, hipStream_t s) {
-  if (!mlp_mfma_waves(m.shape)) return FNET_OK;
-  std::vector<float> pk;
-  pack_mfma_weights(m.shape, m.nspecies, m.h_params.data(), pk, m.pk_stride, m.pk_fw, m.pk_rw,
-                    m.pk_b);
-  if (!m.wpack) HIPCHECK(ctx, dalloc(&m.wpack, pk.size()));
-  HIPCHECK(ctx, hipMemcpyAsync(m.wpack, pk.data(), sizeof(float) * pk.size(),
-                               hipMemcpyHostToDevice, s));
-  // BF16 fragments of the hidden-to-hidden layers (none for networks with one hidden layer)
-  std::vector<uint16_t> bk;
-  pack_bf16_weights(m.shape, m.nspecies, m.h_params.data(), bk, m.bk_stride, m.bk_fw, m.bk_rw,
-                    m.bk_sz);
-  if (!bk.empty()) {
-    if (!m.bpack) HIPCHECK(ctx, dalloc(&m.bpack, bk.size()));
-    HIPCHECK(ctx, hipMemcpyAsync(m.bpack, bk.data(), sizeof(uint16_t) * bk.size(),
-                                 hipMemcpyHostToDevice, s));
-  }
-  HIPCHECK(ctx, hipStreamSynchronize(s));
+  HIPCHECK(ctx, stage_in(ctx, b->zcode, zc.data(), sizeof(int) * N));
+  HIPCHECK(ctx, stage_flush(ctx));
   return FNET_OK;
 }
 
@@ -251,68 +228,70 @@ int ensure_tiles(fnet_batch* b) {
   if (MW && tune_of(b).mlp_waves > 0) MW = std::min(MW, tune_of(b).mlp_waves);
   if (b->tile_atoms == TA && b->mtile_waves == MW && b->tile_launch == b->launch && b->tile_sp)
     return FNET_OK;
-  std::vector<int> perm, tsp, tstart, tcnt, msp, mstart, mcnt;
-  perm.reserve(b->N);
+  // atoms by element in perm, structure after structure for the per-structure launches; each run of
+  // one element is cut into tiles
+  const int nsp = m.nspecies;
+  const bool per = b->launch == FNET_PER_STRUCT;
+  const int runs = per ? b->S : 1;
   b->h_tile_first.assign(b->S + 1, 0);
   b->h_mtile_first.assign(b->S + 1, 0);
-  auto add_tiles = [&](int sp, const std::vector<int>& atoms) {
-    const int p0 = (int)perm.size();
-    for (size_t k = 0; k < atoms.size(); k += TA) {
-      tsp.push_back(sp);
-      tstart.push_back((int)perm.size());
-      const int c = (int)std::min<size_t>(TA, atoms.size() - k);
-      tcnt.push_back(c);
-      for (int q = 0; q < c; ++q) perm.push_back(atoms[k + q]);
+  std::vector<int> count(nsp), at(nsp), tiles, mtiles;  // tiles: (element, first, atoms) each
+  std::vector<int>& tab = b->h_tab;
+  tab.resize((size_t)b->N);
+  for (int r = 0; r < runs; ++r) {
+    const long long i0 = per ? b->h_off[r] : 0, i1 = per ? b->h_off[r + 1] : b->N;
+    b->h_tile_first[r] = (int)tiles.size() / 3;
+    b->h_mtile_first[r] = (int)mtiles.size() / 3;
+    std::fill(count.begin(), count.end(), 0);
+    for (long long i = i0; i < i1; ++i) ++count[b->h_species[i]];
+    int p = (int)i0;
+    for (int sp = 0; sp < nsp; ++sp) {
+      at[sp] = p;
+      const int n = count[sp];
+      for (int k = 0; k < n; k += TA) tiles.insert(tiles.end(), {sp, p + k, std::min(TA, n - k)});
+      if (MW)
+        for (int k = 0; k < n; k += 16 * MW)
+          mtiles.insert(mtiles.end(), {sp, p + k, std::min(16 * MW, n - k)});
+      p += n;
     }
-    if (MW)
-      for (size_t k = 0; k < atoms.size(); k += 16 * MW) {
-        msp.push_back(sp);
-        mstart.push_back(p0 + (int)k);
-        mcnt.push_back((int)std::min<size_t>(16 * MW, atoms.size() - k));
-      }
-  };
-  if (b->launch == FNET_PER_STRUCT) {
-    for (int s = 0; s < b->S; ++s) {
-      b->h_tile_first[s] = (int)tsp.size();
-      b->h_mtile_first[s] = (int)msp.size();
-      for (int sp = 0; sp < m.nspecies; ++sp) {
-        std::vector<int> atoms;
-        for (long long i = b->h_off[s]; i < b->h_off[s + 1]; ++i)
-          if (b->h_species[i] == sp) atoms.push_back((int)i);
-        add_tiles(sp, atoms);
-      }
+    for (long long i = i0; i < i1; ++i) tab[at[b->h_species[i]]++] = (int)i;
+  }
+  const int nt = (int)tiles.size() / 3, nm = (int)mtiles.size() / 3;
+  if (per) {
+    b->h_tile_first[b->S] = nt;
+    b->h_mtile_first[b->S] = nm;
+  }
+  // the seven tables in one allocation, each on a 64-byte boundary
+  auto up16 = [](size_t n) { return (n + 15) & ~size_t(15); };
+  const size_t need = up16(b->N) + 3 * up16(nt) + 3 * up16(nm);
+  tab.resize(need);
+  size_t o = up16(b->N);
+  int** dst[2][3] = {{&b->tile_sp, &b->tile_start, &b->tile_cnt},
+                     {&b->mtile_sp, &b->mtile_start, &b->mtile_cnt}};
+  if (need > b->tab_cap || !b->tab) {
+    dfree(b->tab);
+    b->tab = nullptr;
+    b->tab_cap = 0;
+    const size_t cap = need + need / 4 + 256;
+    HIPCHECK(ctx, dalloc(&b->tab, cap));
+    b->tab_cap = cap;
+  }
+  b->perm = b->tab;
+  for (int w = 0; w < 2; ++w) {
+    const std::vector<int>& t = w ? mtiles : tiles;
+    const int n = w ? nm : nt;
+    for (int c = 0; c < 3; ++c) {
+      for (int k = 0; k < n; ++k) tab[o + k] = t[3 * k + c];
+      *dst[w][c] = b->tab + o;
+      o += up16(n);
     }
-    b->h_tile_first[b->S] = (int)tsp.size();
-    b->h_mtile_first[b->S] = (int)msp.size();
-  } else {
-    std::vector<std::vector<int>> by(m.nspecies);
-    for (long long i = 0; i < b->N; ++i) by[b->h_species[i]].push_back((int)i);
-    for (int sp = 0; sp < m.nspecies; ++sp) add_tiles(sp, by[sp]);
   }
-  dfree(b->perm);
-  dfree(b->tile_sp);
-  dfree(b->tile_start);
-  dfree(b->tile_cnt);
-  dfree(b->mtile_sp);
-  dfree(b->mtile_start);
-  dfree(b->mtile_cnt);
-  b->perm = b->tile_sp = b->tile_start = b->tile_cnt = nullptr;
-  b->mtile_sp = b->mtile_start = b->mtile_cnt = nullptr;
-  hipStream_t s = ctx->stream;
-  HIPCHECK(ctx, upload(&b->perm, perm.data(), perm.size(), s));
-  HIPCHECK(ctx, upload(&b->tile_sp, tsp.data(), tsp.size(), s));
-  HIPCHECK(ctx, upload(&b->tile_start, tstart.data(), tstart.size(), s));
-  HIPCHECK(ctx, upload(&b->tile_cnt, tcnt.data(), tcnt.size(), s));
-  if (MW) {
-    HIPCHECK(ctx, upload(&b->mtile_sp, msp.data(), msp.size(), s));
-    HIPCHECK(ctx, upload(&b->mtile_start, mstart.data(), mstart.size(), s));
-    HIPCHECK(ctx, upload(&b->mtile_cnt, mcnt.data(), mcnt.size(), s));
-  }
-  HIPCHECK(ctx, hipStreamSynchronize(s));
+  HIPCHECK(ctx, stage_in(ctx, b->tab, tab.data(), sizeof(int) * need));
+  HIPCHECK(ctx, stage_flush(ctx));
   b->gen++;
-  b->nmtiles = (int)msp.size();
+  b->nmtiles = nm;
   b->mtile_waves = MW;
-  b->ntiles = (int)tsp.size();
+  b->ntiles = nt;
   b->tile_atoms = TA;
   b->tile_launch = b->launch;
   return FNET_OK;
@@ -321,6 +300,30 @@ int ensure_tiles(fnet_batch* b) {
 int ensure_results(fnet_batch* b) {
   fnet_ctx* ctx = b->ctx;
   const DevModel& m = ctx->model;
+  // pinned copies of the results of a small batch: room for its energies and forces
+  const size_t need = (size_t)((b->S + 4 * b->N) * m.nout);
+  if (b->N * m.nout > kHostAtoms || b->S * m.nout > kHostAtoms) {
+    if (b->h_res) {
+      HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
+      (void)hipHostFree(b->h_res);
+      b->gen++;
+    }
+    b->h_res = nullptr;
+    b->h_res_cap = 0;
+  } else if (need > b->h_res_cap) {
+    HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
+    if (b->h_res) (void)hipHostFree(b->h_res);
+    const size_t cap = need + need / 4 + 64;
+    b->gen++;
+    b->host_E = b->host_F = false;
+    if (hipHostMalloc((void**)&b->h_res, sizeof(double) * cap, hipHostMallocDefault) !=
+        hipSuccess) {
+      // the copy commands serve such a batch
+      (void)hipGetLastError();
+      b->h_res = nullptr;
+    }
+    b->h_res_cap = b->h_res ? cap : 0;
+  }
   if (b->G && b->res_N >= b->N && b->res_S >= b->S && b->res_nG == m.nG && b->res_nout == m.nout)
     return FNET_OK;
   void* pr[] = {b->G, b->cG, b->Eatom, b->Estruct, b->F, b->lossgrad};
@@ -464,9 +467,10 @@ int do_acsf(fnet_batch* b) {
 }
 
 // Batches of up to this many atoms search their mirror entries in extra blocks of the networks
-// launch, which is latency-bound there and hides them; larger ones search them on the side stream
-// beside the ACSF forward.
-constexpr long long kMirrorInline = 16384;
+// launch, which is latency-bound there and hides them (18 113 atoms: 396 -> 382 us per step); larger
+// ones (38 400 atoms: 1587 -> 1537 us, 130 000: 2941 -> 2682) on the side stream beside the ACSF
+// forward.
+constexpr long long kMirrorInline = 24576;
 
 int do_mlp(fnet_batch* b, int gradin, bool mirror = false) {
   fnet_ctx* ctx = b->ctx;
@@ -498,12 +502,12 @@ int do_reduce(fnet_batch* b) {
   const DevModel& m = ctx->model;
   if (b->launch == FNET_PER_STRUCT) {
     for (int st = 0; st < b->S; ++st)
-      HIPCHECK(ctx, launch_energy_reduce(b, m, st, st + 1, ctx->stream));
+      HIPCHECK(ctx, launch_energy_reduce(b, m, st, st + 1, ctx->stream, true));
   } else {
-    HIPCHECK(ctx, launch_energy_reduce(b, m, 0, b->S, ctx->stream,
-                                       b->pending ? b->h_maxnb : nullptr));
+    HIPCHECK(ctx, launch_energy_reduce(b, m, 0, b->S, ctx->stream, true));
   }
   b->have_E = true;
+  b->host_E = b->h_res != nullptr;
   return FNET_OK;
 }
 
@@ -568,17 +572,21 @@ int do_adjoint(fnet_batch* b) {
   int rc = do_mirror(b);
   if (rc) return rc;
   hipStream_t s = ctx->stream;
+  int* norph = b->d_norph;  // cleared by the first launch of the adjoint
   if (b->launch == FNET_PER_STRUCT) {
     for (int st = 0; st < b->S; ++st) {
-      HIPCHECK(ctx, launch_acsf_adj(b, m, b->h_off[st], b->h_off[st + 1], fp64, s));
+      if (b->h_off[st + 1] == b->h_off[st]) continue;
+      HIPCHECK(ctx, launch_acsf_adj(b, m, b->h_off[st], b->h_off[st + 1], fp64, s, norph));
+      norph = nullptr;
       HIPCHECK(ctx, launch_force_gather(b, m, b->h_off[st], b->h_off[st + 1], false, s));
     }
   } else {
-    HIPCHECK(ctx, launch_acsf_adj(b, m, 0, b->N, fp64, s));
+    HIPCHECK(ctx, launch_acsf_adj(b, m, 0, b->N, fp64, s, norph));
     HIPCHECK(ctx, launch_force_gather(b, m, 0, b->N, false, s));
   }
-  HIPCHECK(ctx, launch_force_finish(b, m, false, s));
+  HIPCHECK(ctx, launch_force_finish(b, m, false, s, b->h_res != nullptr));
   b->have_F = true;
+  b->host_F = b->h_res != nullptr;
   return FNET_OK;
 }
 
@@ -641,7 +649,6 @@ int setup_cells(fnet_batch* b, const double* lat, const int* per, bool fresh) {
   b->bin_lds = used && in_prep ? (int)bins : 0;
   coff[b->S] = (int)total;
   if (total >= (1LL << 30)) return fail(ctx, FNET_ERR_CAPACITY, "too many cells");
-  hipStream_t s = ctx->stream;
   if (!fresh && info == b->h_cellinfo) return FNET_OK;
   if (!b->cellinfo) {
     HIPCHECK(ctx, dalloc(&b->cellinfo, (size_t)b->S));
@@ -650,7 +657,7 @@ int setup_cells(fnet_batch* b, const double* lat, const int* per, bool fresh) {
     HIPCHECK(ctx, dalloc(&b->atom_m, (size_t)b->N));
     HIPCHECK(ctx, dalloc(&b->cell_atoms, (size_t)b->N));
   }
-  if (total != b->ncells) {
+  if (total > b->cell_cap) {
     dfree(b->cell_count);
     dfree(b->cell_start);
     dfree(b->cell_scan_tmp);
@@ -658,16 +665,15 @@ int setup_cells(fnet_batch* b, const double* lat, const int* per, bool fresh) {
     HIPCHECK(ctx, dalloc(&b->cell_count, (size_t)total));
     HIPCHECK(ctx, dalloc(&b->cell_start, (size_t)total + 1));
     HIPCHECK(ctx, dalloc(&b->cell_scan_tmp, (size_t)scan_tmp_size(total)));
-    HIPCHECK(ctx, launch_zero_int(b->cell_count, (int)total, s));
-    b->ncells = total;
+    HIPCHECK(ctx, launch_zero_int(b->cell_count, (int)total, ctx->stream));
+    b->cell_cap = total;
     b->gen++;
   }
+  b->ncells = total;
   b->h_cellinfo = info;
-  HIPCHECK(ctx, hipMemcpyAsync(b->cellinfo, info.data(), sizeof(int) * info.size(),
-                               hipMemcpyHostToDevice, s));
-  HIPCHECK(ctx, hipMemcpyAsync(b->cell_off, coff.data(), sizeof(int) * coff.size(),
-                               hipMemcpyHostToDevice, s));
-  HIPCHECK(ctx, hipStreamSynchronize(s));
+  HIPCHECK(ctx, stage_in(ctx, b->cellinfo, info.data(), sizeof(int) * info.size()));
+  HIPCHECK(ctx, stage_in(ctx, b->cell_off, coff.data(), sizeof(int) * coff.size()));
+  HIPCHECK(ctx, stage_flush(ctx));
   return FNET_OK;
 }
 
@@ -781,9 +787,9 @@ int enqueue_fast_step(fnet_batch* b) {
   if (mfma) HIPCHECK(ctx, launch_mlp_mfma(b, m, 0, b->nmtiles, 1, s, in_line, ts + 2));
   else HIPCHECK(ctx, launch_mlp_fwd(b, m, 0, b->ntiles, net64(b->precision), 1, s, in_line, ts + 2));
   if (!in_line) HIPCHECK(ctx, hipStreamWaitEvent(s, ctx->join_ev, 0));
-  HIPCHECK(ctx, launch_acsf_adj(b, m, 0, b->N, fp64, s, ts + 3));
+  HIPCHECK(ctx, launch_acsf_adj(b, m, 0, b->N, fp64, s, b->d_norph, ts + 3));
   HIPCHECK(ctx, launch_force_gather(b, m, 0, b->N, true, s));
-  HIPCHECK(ctx, launch_force_finish(b, m, true, s, ts + 4));
+  HIPCHECK(ctx, launch_force_finish(b, m, true, s, b->h_res != nullptr, ts + 4));
   return FNET_OK;
 }
 
@@ -849,6 +855,7 @@ int run_fast_step(fnet_batch* b) {
   b->have_nl = b->have_G = b->have_E = b->have_F = true;
   b->have_mirror = true;
   b->mir_clear = false;
+  b->host_E = b->host_F = b->h_res != nullptr;
   b->result_precision = b->precision;
   b->pending = true;
   b->pending_level = 3;
@@ -874,7 +881,7 @@ int ensure_list(fnet_batch* b) {
 int evaluate(fnet_batch* b, int level) {
   int rc = FNET_OK;
   if (!b->have_G || b->result_precision != b->precision) {
-    b->have_E = b->have_F = false;
+    b->have_E = b->have_F = b->host_E = b->host_F = false;
     rc = ensure_list(b);
     if (!rc) rc = do_acsf(b);
     if (rc) return rc;
@@ -949,16 +956,10 @@ int check_ready(fnet_ctx* ctx, fnet_batch* b) {
       if (rc) return rc;
     }
   } else if (b->seen_params_gen != ctx->params_gen) {
-    b->have_E = b->have_F = false;
+    b->have_E = b->have_F = b->host_E = b->host_F = false;
   }
   b->seen_params_gen = ctx->params_gen;
   return ensure_results(b);
-}
-
-int download(fnet_ctx* ctx, const void* dsrc, size_t n, double* out) {
-  HIPCHECK(ctx, hipMemcpyAsync(out, dsrc, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
-  return FNET_OK;
 }
 
 }  // namespace
@@ -1018,6 +1019,7 @@ void fnet_ctx_destroy(fnet_ctx* ctx) {
   dfree(ctx->opt_states);
   dfree(ctx->opt_conv);
   dfree(ctx->stamps);
+  if (ctx->ring) (void)hipHostFree(ctx->ring);
   for (int k = 0; k < 8; ++k) (void)hipEventDestroy(ctx->ev[k]);
   if (ctx->side) {
     (void)hipStreamSynchronize(ctx->side);
@@ -1217,25 +1219,23 @@ int fnet_model_upload(fnet_ctx* ctx, const fnet_model_desc* md) {
     ext_in[k] = md->ext_in_idx[k] - 1;
   }
   const size_t np = (size_t)sh.nparams * md->n_species;
-  m.h_params.assign(md->params, md->params + np);
-  m.h_species_z.assign(md->species_z, md->species_z + md->n_species);
-  hipStream_t s = ctx->stream;
-  HIPCHECK(ctx, upload(&m.radial, rad.data(), rad.size(), s));
-  HIPCHECK(ctx, upload(&m.groups, grp.data(), grp.size(), s));
-  HIPCHECK(ctx, upload(&m.zmean, zmean.data(), zmean.size(), s));
-  HIPCHECK(ctx, upload(&m.zinv, zinv.data(), zinv.size(), s));
-  HIPCHECK(ctx, upload(&m.ext_in, ext_in.data(), ext_in.size(), s));
-  HIPCHECK(ctx, upload(&m.params, m.h_params.data(), np, s));
+  HIPCHECK(ctx, upload(ctx, &m.radial, rad.data(), rad.size()));
+  HIPCHECK(ctx, upload(ctx, &m.groups, grp.data(), grp.size()));
+  HIPCHECK(ctx, upload(ctx, &m.zmean, zmean.data(), zmean.size()));
+  HIPCHECK(ctx, upload(ctx, &m.zinv, zinv.data(), zinv.size()));
+  HIPCHECK(ctx, upload(ctx, &m.ext_in, ext_in.data(), ext_in.size()));
+  HIPCHECK(ctx, upload(ctx, &m.params, md->params, np));
   HIPCHECK(ctx, dalloc(&m.params_f, np));
-  HIPCHECK(ctx, launch_to_float(m.params, m.params_f, (long long)np, s));
-  HIPCHECK(ctx, hipStreamSynchronize(s));
-  {
-    const int prc = upload_wpack(ctx, m, s);
-    if (prc) {
-      free_model(m);
-      return prc;
-    }
+  // a model whose shape the MFMA kernels do not take keeps wpack empty
+  if (mlp_mfma_waves(m.shape)) {
+    size_t floats = 0, halves = 0;
+    mfma_layout(m, &floats, &halves);
+    HIPCHECK(ctx, dalloc(&m.wpack, floats));
+    if (halves) HIPCHECK(ctx, dalloc(&m.bpack, halves));
   }
+  HIPCHECK(ctx, stage_flush(ctx));
+  HIPCHECK(ctx, launch_model_params(m, ctx->stream));
+  HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
   m.valid = true;
   free_model(ctx->model);
   ctx->model = m;
@@ -1252,13 +1252,11 @@ int fnet_params_upload(fnet_ctx* ctx, const double* params) {
   DevModel& m = ctx->model;
   const size_t np = (size_t)m.shape.nparams * m.nspecies;
   HIPCHECK(ctx, hipSetDevice(ctx->device));
-  m.h_params.assign(params, params + np);
-  HIPCHECK(ctx, hipMemcpyAsync(m.params, params, sizeof(double) * np, hipMemcpyHostToDevice,
-                               ctx->stream));
-  HIPCHECK(ctx, launch_to_float(m.params, m.params_f, (long long)np, ctx->stream));
-  HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
+  HIPCHECK(ctx, stage_in(ctx, m.params, params, sizeof(double) * np));
+  HIPCHECK(ctx, stage_flush(ctx));
+  HIPCHECK(ctx, launch_model_params(m, ctx->stream));
   ctx->params_gen++;
-  return upload_wpack(ctx, m, ctx->stream);
+  return FNET_OK;
 }
 
 }  // extern "C"
@@ -1335,19 +1333,49 @@ int load_batch(fnet_ctx* ctx, fnet_batch* b, const fnet_batch_desc* d) {
     for (long long i = d->offsets[s]; i < d->offsets[s + 1]; ++i) astruct[i] = s;
   }
   int zone = m.nZ == 1;
+  int last_z = 0, last_c = zcode_of(m, 0);  // runs of one element look its slot up once
   for (long long i = 0; i < N; ++i) {
     if (d->species[i] < 0 || d->species[i] >= m.nspecies)
       return fail(ctx, FNET_ERR_ARG, "species index out of range");
-    zc[i] = zcode_of(m, d->atnum[i]);
-    zone = zone && zc[i] == 0;
+    if (d->atnum[i] != last_z) {
+      last_z = d->atnum[i];
+      last_c = zcode_of(m, last_z);
+    }
+    zc[i] = last_c;
+    zone = zone && last_c == 0;
   }
-  hipStream_t s = ctx->stream;
-  HIPCHECK(ctx, hipStreamSynchronize(s));
-  // capacity: atoms
-  if (N > b->capN || !b->xyz) {
+  const hipStream_t s = ctx->stream;
+  // chunks of the energy reduction: kEnergyChunk atoms of one structure each
+  std::vector<int> chunks(S + 1, 0);  // chunk_first, then (padded) chunk_struct
+  for (int st = 0; st < S; ++st) {
+    const long long na = d->offsets[st + 1] - d->offsets[st];
+    chunks[st + 1] = chunks[st] + (int)((na + kEnergyChunk - 1) / kEnergyChunk);
+  }
+  const int nchunks = chunks[S];
+  b->h_chunk_first = chunks;
+  b->single_chunks = 1;
+  const size_t first_len = ((size_t)S + 16) & ~size_t(15);
+  chunks.resize(first_len + nchunks);
+  for (int st = 0; st < S; ++st) {
+    const int c0 = b->h_chunk_first[st], c1 = b->h_chunk_first[st + 1];
+    if (c1 - c0 != 1) b->single_chunks = 0;
+    for (int c = c0; c < c1; ++c) chunks[first_len + c] = st;
+  }
+  const long long need_part = std::max<long long>(nchunks, 1) * kMaxOut;
+  // capacities: the buffers of an earlier load may still be in use by what was enqueued on it
+  const bool grow_n = N > b->capN || !b->xyz, grow_s = S > b->capS || !b->lat,
+             grow_e = N * d->n_ext > b->capExt || !b->ext,
+             grow_c = chunks.size() > b->chunk_cap || !b->chunk_tab,
+             grow_p = need_part > b->epart_len;
+  if (grow_n || grow_s || grow_e || grow_c || grow_p) HIPCHECK(ctx, hipStreamSynchronize(s));
+  if (grow_n) {
     void* pa[] = {b->xyz, b->atom_struct, b->species, b->zcode, b->cnt, b->rowptr, b->scan_tmp,
                   b->atom_cell, b->atom_m, b->cell_atoms};
     for (void* p : pa) dfree(p);
+    b->xyz = nullptr;
+    b->atom_struct = b->species = b->zcode = b->cnt = b->rowptr = b->scan_tmp = nullptr;
+    b->atom_cell = b->cell_atoms = nullptr;
+    b->atom_m = nullptr;
     const long long cap = std::max<long long>(N, 1);
     HIPCHECK(ctx, dalloc(&b->xyz, (size_t)3 * cap));
     HIPCHECK(ctx, dalloc(&b->atom_struct, (size_t)cap));
@@ -1361,15 +1389,20 @@ int load_batch(fnet_ctx* ctx, fnet_batch* b, const fnet_batch_desc* d) {
     HIPCHECK(ctx, dalloc(&b->cell_atoms, (size_t)cap));
     b->capN = cap;
   }
-  if (N * d->n_ext > b->capExt || !b->ext) {
+  if (grow_e) {
     dfree(b->ext);
+    b->ext = nullptr;
     b->capExt = std::max<long long>(N * d->n_ext, 1);
     HIPCHECK(ctx, dalloc(&b->ext, (size_t)b->capExt));
   }
-  // capacity: structures
-  if (S > b->capS || !b->lat) {
+  if (grow_s) {
     void* ps[] = {b->lat, b->periodic, b->off, b->sinfo, b->cellinfo, b->cell_off};
     for (void* p : ps) dfree(p);
+    b->lat = nullptr;
+    b->periodic = b->cell_off = nullptr;
+    b->off = nullptr;
+    b->sinfo = nullptr;
+    b->cellinfo = nullptr;
     const long long cap = std::max(S, 1);
     HIPCHECK(ctx, dalloc(&b->lat, (size_t)9 * cap));
     HIPCHECK(ctx, dalloc(&b->periodic, (size_t)cap));
@@ -1379,6 +1412,21 @@ int load_batch(fnet_ctx* ctx, fnet_batch* b, const fnet_batch_desc* d) {
     HIPCHECK(ctx, dalloc(&b->cell_off, (size_t)cap + 1));
     b->capS = cap;
   }
+  if (grow_c) {
+    dfree(b->chunk_tab);
+    b->chunk_tab = nullptr;
+    b->chunk_cap = 0;
+    const size_t cap = chunks.size() + chunks.size() / 4 + 64;
+    HIPCHECK(ctx, dalloc(&b->chunk_tab, cap));
+    b->chunk_cap = cap;
+  }
+  if (grow_p) {
+    dfree(b->Epart);
+    b->Epart = nullptr;
+    b->epart_len = 0;
+    HIPCHECK(ctx, dalloc(&b->Epart, (size_t)need_part));
+    b->epart_len = need_part;
+  }
   if (!b->d_maxnb) HIPCHECK(ctx, dalloc(&b->d_maxnb, 1));
   b->S = S;
   b->N = N;
@@ -1387,63 +1435,29 @@ int load_batch(fnet_ctx* ctx, fnet_batch* b, const fnet_batch_desc* d) {
   b->h_species.assign(d->species, d->species + N);
   b->h_lat = lat;
   b->h_periodic = per;
-  // chunks of the energy reduction: kEnergyChunk atoms of one structure each (the host tables
-  // live until the stream synchronisation below: the copies may read them late)
-  std::vector<int> cs, cf(S + 1, 0);
-  {
-    for (int st = 0; st < S; ++st) {
-      cf[st] = (int)cs.size();
-      const long long na = d->offsets[st + 1] - d->offsets[st];
-      for (long long q = 0; q < na; q += kEnergyChunk) cs.push_back(st);
-    }
-    cf[S] = (int)cs.size();
-    dfree(b->chunk_struct);
-    dfree(b->chunk_first);
-    b->chunk_struct = b->chunk_first = nullptr;
-    HIPCHECK(ctx, upload(&b->chunk_struct, cs.data(), cs.size(), s));
-    HIPCHECK(ctx, upload(&b->chunk_first, cf.data(), cf.size(), s));
-    const long long need = std::max<long long>((long long)cs.size(), 1) * kMaxOut;
-    if (need > b->epart_len) {
-      dfree(b->Epart);
-      b->Epart = nullptr;
-      HIPCHECK(ctx, dalloc(&b->Epart, (size_t)need));
-      b->epart_len = need;
-    }
-    b->nchunks = (int)cs.size();
-    b->single_chunks = 1;
-    for (int st = 0; st < S; ++st)
-      if (cf[st + 1] - cf[st] != 1) b->single_chunks = 0;
-    b->h_chunk_first = cf;
-  }
-  if (N) HIPCHECK(ctx, hipMemcpyAsync(b->xyz, d->coords, sizeof(double) * 3 * N,
-                                      hipMemcpyHostToDevice, s));
-  if (S) {
-    HIPCHECK(ctx, hipMemcpyAsync(b->lat, lat.data(), sizeof(double) * lat.size(),
-                                 hipMemcpyHostToDevice, s));
-    HIPCHECK(ctx, hipMemcpyAsync(b->periodic, per.data(), sizeof(int) * S, hipMemcpyHostToDevice,
-                                 s));
-  }
-  HIPCHECK(ctx, hipMemcpyAsync(b->off, d->offsets, sizeof(long long) * (S + 1),
-                               hipMemcpyHostToDevice, s));
-  if (N) {
-    HIPCHECK(ctx, hipMemcpyAsync(b->atom_struct, astruct.data(), sizeof(int) * N,
-                                 hipMemcpyHostToDevice, s));
-    HIPCHECK(ctx, hipMemcpyAsync(b->species, d->species, sizeof(int) * N, hipMemcpyHostToDevice,
-                                 s));
-    HIPCHECK(ctx, hipMemcpyAsync(b->zcode, zc.data(), sizeof(int) * N, hipMemcpyHostToDevice, s));
-  }
+  b->nchunks = nchunks;
+  b->chunk_first = b->chunk_tab;
+  b->chunk_struct = b->chunk_tab + first_len;
   b->h_atnum.assign(d->atnum, d->atnum + N);
   b->zone = zone;
   b->zcode_gen = ctx->model_gen;
-  if (N * d->n_ext)
-    HIPCHECK(ctx, hipMemcpyAsync(b->ext, d->ext, sizeof(double) * N * d->n_ext,
-                                 hipMemcpyHostToDevice, s));
-  HIPCHECK(ctx, hipStreamSynchronize(s));
+  HIPCHECK(ctx, stage_in(ctx, b->xyz, d->coords, sizeof(double) * 3 * N));
+  HIPCHECK(ctx, stage_in(ctx, b->lat, lat.data(), sizeof(double) * lat.size()));
+  HIPCHECK(ctx, stage_in(ctx, b->periodic, per.data(), sizeof(int) * S));
+  HIPCHECK(ctx, stage_in(ctx, b->off, d->offsets, sizeof(long long) * (S + 1)));
+  HIPCHECK(ctx, stage_in(ctx, b->atom_struct, astruct.data(), sizeof(int) * N));
+  HIPCHECK(ctx, stage_in(ctx, b->species, d->species, sizeof(int) * N));
+  HIPCHECK(ctx, stage_in(ctx, b->zcode, zc.data(), sizeof(int) * N));
+  HIPCHECK(ctx, stage_in(ctx, b->chunk_tab, chunks.data(), sizeof(int) * chunks.size()));
+  HIPCHECK(ctx, stage_in(ctx, b->ext, d->ext, sizeof(double) * N * d->n_ext));
   invalidate(b);
   b->tile_atoms = 0;  // species layout changed: rebuild the network tiles
   b->result_precision = -1;
   b->gen++;
-  return setup_cells(b, lat.data(), per.data(), true);
+  const int rc = setup_cells(b, lat.data(), per.data(), true);
+  if (rc) return rc;
+  HIPCHECK(ctx, stage_flush(ctx));
+  return FNET_OK;
 }
 
 }  // namespace
@@ -1483,17 +1497,17 @@ void fnet_batch_destroy(fnet_batch* b) {
   (void)hipSetDevice(b->ctx->device);
   (void)hipStreamSynchronize(b->ctx->stream);
   void* ptrs[] = {b->xyz, b->lat, b->periodic, b->off, b->atom_struct, b->species, b->zcode,
-                  b->ext, b->sinfo, b->perm, b->tile_sp, b->tile_start, b->tile_cnt, b->cnt,
+                  b->ext, b->sinfo, b->tab, b->cnt,
                   b->rowptr, b->scan_tmp, b->nj, b->nimg, b->nd, b->d_maxnb, b->G, b->cG,
                   b->Eatom, b->Estruct, b->F, b->lossgrad, b->d_targets, b->cellinfo,
                   b->cell_off, b->cell_count, b->cell_start, b->cell_atoms, b->atom_cell,
-                  b->atom_m, b->cell_scan_tmp, b->mtile_sp, b->mtile_start, b->mtile_cnt,
+                  b->atom_m, b->cell_scan_tmp,
                   b->pnj, b->pnimg, b->pnd, b->gvec, b->mir, b->orph, b->d_norph,
-                  b->chunk_struct, b->chunk_first, b->Epart, b->gpart};
+                  b->chunk_tab, b->Epart, b->gpart};
   for (void* p : ptrs) dfree(p);
   drop_graph(b);
   if (b->h_maxnb) (void)hipHostFree(b->h_maxnb);
-  if (b->ctx->last_train_batch == b) b->ctx->last_train_batch = nullptr;
+  if (b->h_res) (void)hipHostFree(b->h_res);
   delete b;
 }
 
@@ -1510,17 +1524,15 @@ int fnet_batch_update_coords(fnet_batch* b, const double* coords, const double* 
         if (lrc) return lrc;
       }
   HIPCHECK(ctx, hipSetDevice(ctx->device));
-  HIPCHECK(ctx, hipMemcpyAsync(b->xyz, coords, sizeof(double) * 3 * b->N, hipMemcpyHostToDevice,
-                               ctx->stream));
+  HIPCHECK(ctx, stage_in(ctx, b->xyz, coords, sizeof(double) * 3 * b->N));
   if (latvecs) {
-    HIPCHECK(ctx, hipMemcpyAsync(b->lat, latvecs, sizeof(double) * 9 * b->S,
-                                 hipMemcpyHostToDevice, ctx->stream));
+    HIPCHECK(ctx, stage_in(ctx, b->lat, latvecs, sizeof(double) * 9 * b->S));
     for (int q = 0; q < 9 * b->S; ++q)
       if (b->h_periodic[q / 9]) b->h_lat[q] = latvecs[q];
     const int crc = setup_cells(b, b->h_lat.data(), b->h_periodic.data(), false);
     if (crc) return crc;
   }
-  HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
+  HIPCHECK(ctx, stage_flush(ctx));
   invalidate(b);
   return FNET_OK;
 }
@@ -1612,11 +1624,10 @@ int fnet_acsf_forward(fnet_ctx* ctx, fnet_batch* b, double* G_out) {
   rc = do_acsf(b);
   if (rc || !G_out) return rc;
   for (;;) {
-    if (b->pending && b->pending_level == 1)
-      HIPCHECK(ctx, hipMemcpyAsync(b->h_maxnb, b->d_maxnb, sizeof(int), hipMemcpyDeviceToHost,
-                                   ctx->stream));
-    rc = download(ctx, b->G, (size_t)b->N * ctx->model.nG, G_out);
-    if (rc) return rc;
+    const StageOut out[2] = {
+        {G_out, b->G, sizeof(double) * b->N * ctx->model.nG},
+        {b->pending && b->pending_level == 1 ? b->h_maxnb : nullptr, b->d_maxnb, sizeof(int)}};
+    HIPCHECK(ctx, stage_out(ctx, out, 2));
     bool redone;
     rc = settle_list(b, &redone);
     if (rc || !redone) return rc;
@@ -1632,13 +1643,15 @@ int fnet_energy(fnet_ctx* ctx, fnet_batch* b, double* E_struct, double* E_atom) 
   const DevModel& m = ctx->model;
   for (;;) {
     if (rc) return rc;
-    if (E_struct)
-      HIPCHECK(ctx, hipMemcpyAsync(E_struct, b->Estruct, sizeof(double) * b->S * m.nout,
-                                   hipMemcpyDeviceToHost, ctx->stream));
-    if (E_atom)
-      HIPCHECK(ctx, hipMemcpyAsync(E_atom, b->Eatom, sizeof(double) * b->N * m.nout,
-                                   hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
+    const size_t ns = sizeof(double) * b->S * m.nout, na = sizeof(double) * b->N * m.nout;
+    if (b->host_E) {
+      HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
+      if (E_struct && ns) std::memcpy(E_struct, host_Estruct(b), ns);
+      if (E_atom && na) std::memcpy(E_atom, host_Eatom(b), na);
+    } else {
+      const StageOut out[2] = {{E_struct, b->Estruct, ns}, {E_atom, b->Eatom, na}};
+      HIPCHECK(ctx, stage_out(ctx, out, 2));
+    }
     bool redone;
     rc = settle_list(b, &redone);
     if (!rc && !redone) return FNET_OK;
@@ -1653,8 +1666,13 @@ int fnet_forces(fnet_ctx* ctx, fnet_batch* b, double* F) {
   rc = evaluate(b, 3);
   if (rc || !F) return rc;
   for (;;) {
-    rc = download(ctx, b->F, (size_t)b->N * ctx->model.nout * 3, F);
-    if (rc) return rc;
+    const StageOut out = {F, b->F, sizeof(double) * b->N * ctx->model.nout * 3};
+    if (b->host_F) {
+      HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
+      if (out.bytes) std::memcpy(F, host_F(b), out.bytes);
+    } else {
+      HIPCHECK(ctx, stage_out(ctx, &out, 1));
+    }
     bool redone;
     rc = settle_list(b, &redone);
     if (rc || !redone) return rc;
@@ -1876,21 +1894,17 @@ int fnet_train_gradients(fnet_ctx* ctx, fnet_batch* b, int n_global, const doubl
   double* dpw = aw + b->N;
   double wsum = 0.0;
   if (n_global > 0)
-    HIPCHECK(ctx, hipMemcpyAsync(gt, g_targets, sizeof(double) * b->S * n_global,
-                                 hipMemcpyHostToDevice, s));
-  if (na > 0)
-    HIPCHECK(ctx, hipMemcpyAsync(at, a_targets, sizeof(double) * b->N * na, hipMemcpyHostToDevice,
-                                 s));
-  if (atomic_weights)
-    HIPCHECK(ctx, hipMemcpyAsync(aw, atomic_weights, sizeof(double) * b->N,
-                                 hipMemcpyHostToDevice, s));
+    HIPCHECK(ctx, stage_in(ctx, gt, g_targets, sizeof(double) * b->S * n_global));
+  if (na > 0) HIPCHECK(ctx, stage_in(ctx, at, a_targets, sizeof(double) * b->N * na));
+  if (atomic_weights) HIPCHECK(ctx, stage_in(ctx, aw, atomic_weights, sizeof(double) * b->N));
   if (dp_weights) {
-    HIPCHECK(ctx, hipMemcpyAsync(dpw, dp_weights, sizeof(double) * b->S, hipMemcpyHostToDevice, s));
+    HIPCHECK(ctx, stage_in(ctx, dpw, dp_weights, sizeof(double) * b->S));
     for (int k = 0; k < b->S; ++k) wsum += dp_weights[k];
   } else {
     wsum = (double)b->S;
   }
   if (!(wsum > 0.0)) return fail(ctx, FNET_ERR_ARG, "datapoint weights sum to zero");
+  HIPCHECK(ctx, stage_flush(ctx));
   HIPCHECK(ctx, launch_lossgrad(b, m, n_global, gt, at, atomic_weights ? aw : nullptr,
                                 dp_weights ? dpw : nullptr, 1.0 / wsum, ctx->loss, s));
   const long long np = m.shape.nparams * m.nspecies;
@@ -1919,18 +1933,17 @@ int fnet_train_gradients(fnet_ctx* ctx, fnet_batch* b, int n_global, const doubl
   HIPCHECK(ctx, launch_loss(b, m, n_global, gt, at, atomic_weights ? aw : nullptr,
                             dp_weights ? dpw : nullptr, ctx->loss, dloss, dloss + 2,
                             dloss + 2 + 2LL * b->S, s));
-  if (grad)
-    HIPCHECK(ctx, hipMemcpyAsync(grad, ctx->d_grad, sizeof(double) * np, hipMemcpyDeviceToHost, s));
-  if (pred)
-    HIPCHECK(ctx, hipMemcpyAsync(pred, b->Eatom, sizeof(double) * b->N * m.nout,
-                                 hipMemcpyDeviceToHost, s));
   double lv = 0.0;
-  HIPCHECK(ctx, hipMemcpyAsync(&lv, dloss, sizeof(double), hipMemcpyDeviceToHost, s));
-  HIPCHECK(ctx, hipStreamSynchronize(s));
+  const bool host = b->host_E;  // a small batch's outputs are in pinned memory already
+  const size_t npred = sizeof(double) * b->N * m.nout;
+  const StageOut out[3] = {{grad, ctx->d_grad, sizeof(double) * np},
+                           {&lv, dloss, sizeof(double)},
+                           {host ? nullptr : pred, b->Eatom, npred}};
+  HIPCHECK(ctx, stage_out(ctx, out, 3));
+  if (pred && host && npred) std::memcpy(pred, host_Eatom(b), npred);
   if (loss) *loss = lv;
   ctx->last_loss = lv;
   ctx->have_grad = true;
-  ctx->last_train_batch = b;
   return FNET_OK;
 }
 
@@ -1964,18 +1977,11 @@ int fnet_optimizer_step_sd(fnet_ctx* ctx, double lr, double max_disp, double tol
   HIPCHECK(ctx, launch_sd_step(m.params, ctx->d_grad, m.shape.nparams, lr, max_disp, tol, gmax,
                                m.nspecies, ctx->stream));
   ctx->params_gen++;
-  HIPCHECK(ctx, launch_to_float(m.params, m.params_f, np, ctx->stream));
+  HIPCHECK(ctx, launch_model_params(m, ctx->stream));
   std::vector<double> gm(m.nspecies);
-  HIPCHECK(ctx, hipMemcpyAsync(m.h_params.data(), m.params, sizeof(double) * np,
-                               hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHECK(ctx, hipMemcpyAsync(gm.data(), gmax, sizeof(double) * m.nspecies,
-                               hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
-  {
-    const int prc = upload_wpack(ctx, m, ctx->stream);
-    if (prc) return prc;
-  }
-  if (params_out) std::memcpy(params_out, m.h_params.data(), sizeof(double) * np);
+  const StageOut out[2] = {{params_out, m.params, sizeof(double) * np},
+                           {gm.data(), gmax, sizeof(double) * m.nspecies}};
+  HIPCHECK(ctx, stage_out(ctx, out, 2));
   if (converged) {
     int c = 1;
     for (double v : gm) c = c && (v < tol);
@@ -2052,18 +2058,11 @@ int fnet_optimizer_step(fnet_ctx* ctx, int kind, double* params_out, int* conver
   HIPCHECK(ctx, launch_opt_step(ctx->opt_states, m.params, ctx->d_grad, ctx->opt_vecs, n,
                                 ctx->opt_vstride, ctx->last_loss, ctx->opt_conv, m.nspecies, s));
   ctx->params_gen++;
-  HIPCHECK(ctx, launch_to_float(m.params, m.params_f, np, s));
+  HIPCHECK(ctx, launch_model_params(m, s));
   std::vector<int> conv(m.nspecies, 0);
-  HIPCHECK(ctx, hipMemcpyAsync(m.h_params.data(), m.params, sizeof(double) * np,
-                               hipMemcpyDeviceToHost, s));
-  HIPCHECK(ctx, hipMemcpyAsync(conv.data(), ctx->opt_conv, sizeof(int) * m.nspecies,
-                               hipMemcpyDeviceToHost, s));
-  HIPCHECK(ctx, hipStreamSynchronize(s));
-  {
-    const int prc = upload_wpack(ctx, m, s);
-    if (prc) return prc;
-  }
-  if (params_out) std::memcpy(params_out, m.h_params.data(), sizeof(double) * np);
+  const StageOut out[2] = {{params_out, m.params, sizeof(double) * np},
+                           {conv.data(), ctx->opt_conv, sizeof(int) * m.nspecies}};
+  HIPCHECK(ctx, stage_out(ctx, out, 2));
   if (converged) *converged = conv[m.nspecies - 1];
   ctx->have_grad = false;
   return FNET_OK;

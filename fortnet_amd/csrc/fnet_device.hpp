@@ -124,6 +124,8 @@ struct EnergyArgs {
   double* Estruct;
   const int* maxnb;  // longest row of the list, handed to the host with the energies
   int* h_maxnb;      // pinned host memory, or null
+  double* h_Eatom;   // pinned copies of the energies, or null
+  double* h_Estruct;
 };
 
 // chunk c by a block of 256 threads
@@ -134,15 +136,23 @@ __device__ __forceinline__ void energy_chunk(const EnergyArgs& a, int c, double*
   const long long a1 = min(a0 + (long long)kEnergyChunk, a.off[s + 1]);
   for (int t = 0; t < a.nout; ++t) {
     double v = 0.0;
-    for (long long i = a0 + threadIdx.x; i < a1; i += 256) v += a.Eatom[i * a.nout + t];
+    for (long long i = a0 + threadIdx.x; i < a1; i += 256) {
+      const double e = a.Eatom[i * a.nout + t];
+      if (a.h_Eatom) a.h_Eatom[i * a.nout + t] = e;
+      v += e;
+    }
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
     if (lane == 0) ws[wave] = v;
     __syncthreads();
     if (threadIdx.x == 0) {
       const double e = (ws[0] + ws[1]) + (ws[2] + ws[3]);
-      if (a.single) a.Estruct[(long long)s * a.nout + t] = e;
-      else a.Epart[(long long)c * a.nout + t] = e;
+      if (a.single) {
+        a.Estruct[(long long)s * a.nout + t] = e;
+        if (a.h_Estruct) a.h_Estruct[(long long)s * a.nout + t] = e;
+      } else {
+        a.Epart[(long long)c * a.nout + t] = e;
+      }
     }
     __syncthreads();
   }
@@ -157,9 +167,11 @@ __device__ __forceinline__ void energy_total(const EnergyArgs& a, long long q, i
   for (int c = a.chunk_first[s]; c < a.chunk_first[s + 1]; ++c)
     v += a.Epart[(long long)c * a.nout + t];
   a.Estruct[s * a.nout + t] = v;
+  if (a.h_Estruct) a.h_Estruct[s * a.nout + t] = v;
 }
 
-inline EnergyArgs energy_args(const fnet_batch* b, const DevModel& m) {
+// host: with the pinned copies
+inline EnergyArgs energy_args(const fnet_batch* b, const DevModel& m, bool host) {
   EnergyArgs e;
   e.Eatom = b->Eatom;
   e.off = b->off;
@@ -170,7 +182,9 @@ inline EnergyArgs energy_args(const fnet_batch* b, const DevModel& m) {
   e.Epart = b->Epart;
   e.Estruct = b->Estruct;
   e.maxnb = b->d_maxnb;
-  e.h_maxnb = nullptr;
+  e.h_maxnb = host ? b->h_maxnb : nullptr;
+  e.h_Eatom = host && b->h_res ? host_Eatom(b) : nullptr;
+  e.h_Estruct = host && b->h_res ? host_Estruct(b) : nullptr;
   return e;
 }
 

@@ -95,19 +95,26 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// Entries without a mirror: -g to the neighbour's force (block 0, which leaves the counter at zero
-// for the next gather); the other blocks add the chunk sums of structures of several chunks.
+// Entries without a mirror: -g to the neighbour's force (block 0); the next nen blocks add the
+// chunk sums of structures of several chunks, the others copy the forces to pinned host memory
+// (hF; when there are orphans, block 0 does that after them).
 template <typename G>
 __global__ void __launch_bounds__(256)
-    k_force_finish(int* __restrict__ norph, const int* __restrict__ orph,
-                   const int* __restrict__ nj, const G* __restrict__ gvec, int nout,
-                   double* __restrict__ F, EnergyArgs en, int S, unsigned long long* ts) {
+    k_force_finish(const int* __restrict__ norph, const int* __restrict__ orph,
+                   const int* __restrict__ nj, const G* __restrict__ gvec, int nout, double* F,
+                   EnergyArgs en, int S, unsigned nen, double* __restrict__ hF, long long nf,
+                   unsigned long long* ts) {
   stamp(ts);
-  if (blockIdx.x > 0) {
+  if (blockIdx.x > 0 && blockIdx.x <= nen) {
     energy_total(en, (long long)(blockIdx.x - 1) * 256 + threadIdx.x, 0, S);
     return;
   }
   const int cnt = *norph;
+  if (blockIdx.x > 0) {
+    const long long k = (long long)(blockIdx.x - 1 - nen) * 256 + threadIdx.x;
+    if (cnt == 0 && k < nf) hF[k] = F[k];
+    return;
+  }
   for (int q = threadIdx.x; q < cnt; q += blockDim.x) {
     const long long e = orph[q];
     const long long j = nj[e];
@@ -115,8 +122,12 @@ __global__ void __launch_bounds__(256)
       for (int c = 0; c < 3; ++c)
         unsafeAtomicAdd(&F[(j * nout + t) * 3 + c], -(double)gvec[(e * nout + t) * 3 + c]);
   }
-  __syncthreads();
-  if (threadIdx.x == 0 && cnt) *norph = 0;
+  if (hF && cnt) {
+    __threadfence();
+    __syncthreads();
+    for (long long k = threadIdx.x; k < nf; k += blockDim.x)
+      hF[k] = __hip_atomic_load(&F[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
   stamp(ts ? ts + 1 : nullptr);
 }
 
@@ -165,8 +176,7 @@ hipError_t launch_force_gather(fnet_batch* b, const DevModel& m, long long a0, l
   const unsigned ng = n > 0 ? (unsigned)((n + 3) / 4) : 0u;
   const unsigned grid = ng + (energies ? (unsigned)b->nchunks : 0u);
   if (grid == 0) return hipSuccess;
-  EnergyArgs en = energy_args(b, m);
-  if (energies) en.h_maxnb = b->h_maxnb;
+  const EnergyArgs en = energy_args(b, m, energies);
   if (b->precision == FNET_FP64)
     k_force_gather<double><<<grid, 256, 0, s>>>(layout_of(b), b->mir, b->gvec, a0, a1, m.nout,
                                                 (double*)b->F, b->orph, b->d_norph, ng, en);
@@ -202,17 +212,20 @@ void* scratch_ptr(int device) {
 }
 
 hipError_t launch_force_finish(fnet_batch* b, const DevModel& m, bool energies, hipStream_t s,
-                               unsigned long long* stamps) {
+                               bool host, unsigned long long* stamps) {
   const int* nj = b->nl_padded ? b->pnj : b->nj;
-  const EnergyArgs en = energy_args(b, m);
-  const unsigned grid =
-      1u + (energies && !en.single ? (unsigned)(((long long)b->S * m.nout + 255) / 256) : 0u);
+  const EnergyArgs en = energy_args(b, m, energies);
+  const unsigned nen =
+      energies && !en.single ? (unsigned)(((long long)b->S * m.nout + 255) / 256) : 0u;
+  const long long nf = 3 * b->N * m.nout;
+  double* hF = host ? host_F(b) : nullptr;
+  const unsigned grid = 1u + nen + (hF ? (unsigned)((nf + 255) / 256) : 0u);
   if (b->precision == FNET_FP64)
     k_force_finish<double><<<grid, 256, 0, s>>>(b->d_norph, b->orph, nj, b->gvec, m.nout,
-                                                (double*)b->F, en, b->S, stamps);
+                                                (double*)b->F, en, b->S, nen, hF, nf, stamps);
   else
     k_force_finish<float><<<grid, 256, 0, s>>>(b->d_norph, b->orph, nj, (const float*)b->gvec,
-                                               m.nout, (double*)b->F, en, b->S, stamps);
+                                               m.nout, (double*)b->F, en, b->S, nen, hF, nf, stamps);
   return hipGetLastError();
 }
 
@@ -291,22 +304,26 @@ extern "C" int fnet_forces_noalloc(fnet_ctx* ctx, fnet_batch* b) {
     } else {
       e = launch_mirror(b, 0, b->N, entries, s);
     }
-    if (e == hipSuccess) e = launch_zero_int(norph, 1, s);
+    int* clear = norph;  // cleared by the first launch of the adjoint
+    if (b->N == 0 && e == hipSuccess) e = launch_zero_int(norph, 1, s);
     if (b->launch == FNET_PER_STRUCT) {
       for (int st = 0; st < b->S && e == hipSuccess; ++st) {
-        e = launch_acsf_adj(b, m, b->h_off[st], b->h_off[st + 1], fp64, s);
+        if (b->h_off[st + 1] == b->h_off[st]) continue;
+        e = launch_acsf_adj(b, m, b->h_off[st], b->h_off[st + 1], fp64, s, clear);
+        clear = nullptr;
         if (e == hipSuccess) e = launch_force_gather(b, m, b->h_off[st], b->h_off[st + 1], false, s);
       }
     } else {
-      if (e == hipSuccess) e = launch_acsf_adj(b, m, 0, b->N, fp64, s);
+      if (e == hipSuccess) e = launch_acsf_adj(b, m, 0, b->N, fp64, s, norph);
       if (e == hipSuccess) e = launch_force_gather(b, m, 0, b->N, false, s);
     }
-    if (e == hipSuccess) e = launch_force_finish(b, m, false, s);
+    if (e == hipSuccess) e = launch_force_finish(b, m, false, s, false);
   }
   if (e != hipSuccess) {
     ctx->err = std::string("fnet_forces_noalloc: ") + hipGetErrorString(e);
     return FNET_ERR_HIP;
   }
   b->have_F = true;
+  b->host_F = false;
   return FNET_OK;
 }

@@ -140,8 +140,6 @@ struct DevModel {
   uint16_t* bpack = nullptr;
   long long bk_stride = 0;
   long long bk_fw[kMaxLayers] = {}, bk_rw[kMaxLayers] = {}, bk_sz[kMaxLayers] = {};
-  std::vector<double> h_params;
-  std::vector<int> h_species_z;
   bool valid = false;
 };
 
@@ -159,6 +157,23 @@ struct Tune {
   }
 };
 
+// Host I/O through pinned memory (fnet_stage.hip): segments that one kernel copies.
+constexpr int kStageSegs = 24;
+constexpr size_t kStageRing = 2u << 20;  // pinned bytes of one context
+constexpr size_t kStageMax = 512u << 10; // larger arrays keep their own copy command
+struct StageSegs {
+  int n = 0;
+  unsigned first[kStageSegs];
+  const void* src[kStageSegs];
+  void* dst[kStageSegs];
+  size_t bytes[kStageSegs];
+};
+struct StageOut {
+  void* host;
+  const void* dev;
+  size_t bytes;
+};
+
 }  // namespace fnet
 
 struct fnet_batch;
@@ -171,6 +186,10 @@ struct fnet_ctx {
   hipStream_t side = nullptr;
   hipEvent_t fork_ev = nullptr, join_ev = nullptr;
   std::string err;
+  char* ring = nullptr;      // pinned ring of the staged copies
+  size_t ring_at = 0;
+  fnet::StageSegs segs;      // copies in that have not been launched yet
+  bool stage_direct = false; // ... and a copy command was enqueued beside them
   fnet::DevModel model;
   hipEvent_t ev[8] = {};
   int n_ev = 0;
@@ -182,7 +201,6 @@ struct fnet_ctx {
   double* d_grad = nullptr; // [nspecies][nparams] FP64 gradient of the last train call
   long long grad_cap = 0;
   bool have_grad = false;
-  fnet_batch* last_train_batch = nullptr;
   int loss = 0;               // fnet_loss of the training gradient and loss value
   int use_graph = 0;          // fnet_run replays a captured HIP graph of its steady-state step
   double last_loss = 0.0;     // loss of the last training-gradient call
@@ -227,7 +245,10 @@ struct fnet_batch {
   unsigned long long zcode_gen = 0;  // model generation zcode was derived with
   double* ext = nullptr;       // [N][next]
   fnet::StructInfo* sinfo = nullptr; // [S]
-  // per-species tiles of the network kernels
+  // per-species tiles of the network kernels; the tables share one allocation (tab)
+  int* tab = nullptr;
+  size_t tab_cap = 0;
+  std::vector<int> h_tab;
   int* perm = nullptr;         // [N] atoms grouped by species
   int* tile_sp = nullptr;      // [ntiles]
   int* tile_start = nullptr;   // [ntiles] into perm
@@ -273,6 +294,7 @@ struct fnet_batch {
   int4* atom_m = nullptr;      // [N] integer part of the fractional coordinates, local bin
   int* cell_scan_tmp = nullptr;
   long long ncells = 0;        // cells of the structures with cell lists, one more per structure
+  long long cell_cap = 0;      // allocated cells
   int n_cell_struct = 0;       // structures with cell lists
   int bin_lds = 0;             // > 0: every such structure is binned by its struct-prep block, with
                                // this many LDS bins; 0: binning kernels over all atoms
@@ -297,6 +319,8 @@ struct fnet_batch {
   bool have_mirror = false;
   bool mir_clear = false;      // every entry of the current padded list has its mirror slot at -1
   // energy reduction in fixed-size chunks of atoms (two passes, fixed order)
+  int* chunk_tab = nullptr;    // allocation of the two tables
+  size_t chunk_cap = 0;
   int* chunk_struct = nullptr; // [nchunks]
   int* chunk_first = nullptr;  // [S+1]
   double* Epart = nullptr;     // [nchunks][nout]
@@ -310,6 +334,11 @@ struct fnet_batch {
   // steady-state step of fnet_run (no host read-back): the longest row of the list it built is
   // copied to pinned host memory with the step and checked when results are next read
   int* h_maxnb = nullptr;
+  // small batches: pinned copies of the results, written by the kernels that produce them
+  // (kHostAtoms), and which of them hold the current results
+  double* h_res = nullptr;
+  size_t h_res_cap = 0;
+  bool host_E = false, host_F = false;
   bool pending = false;
   int pending_level = 0;        // what was computed on that list: 1 features, 2 energies, 3 forces
   long long gen = 0;            // bumped whenever a buffer the step uses is reallocated
@@ -344,6 +373,19 @@ __device__ __forceinline__ void entry_d2(double4& v, double d2) { v.w = d2; }
 __device__ __forceinline__ void entry_d2(float4& v, double d2) { v.w = (float)d2; }
 __device__ __forceinline__ double entry_r(double w) { return sqrt(w); }
 __device__ __forceinline__ float entry_r(float w) { return sqrtf(w); }
+
+// staged host I/O (fnet_stage.hip), on the context's stream: stage_in copies `src` now and to the
+// device with the next stage_flush; stage_out brings n results to the host and waits for them
+hipError_t stage_in(fnet_ctx* ctx, void* dst, const void* src, size_t bytes);
+hipError_t stage_flush(fnet_ctx* ctx);
+hipError_t stage_out(fnet_ctx* ctx, const StageOut* out, int n);
+
+// Batches of up to this many outputs have their energies and forces written to pinned host memory
+// as they are formed.
+constexpr long long kHostAtoms = 8192;
+inline double* host_Estruct(const fnet_batch* b);
+inline double* host_Eatom(const fnet_batch* b);
+inline double* host_F(const fnet_batch* b);
 
 // launchers (fnet_neigh.hip)
 // lattices, extents and (bin_lds > 0) cell bins; clears the batch's row maximum
@@ -405,16 +447,17 @@ hipError_t launch_mirror(fnet_batch* b, long long a0, long long a1, long long fi
 // energies: also the energy chunks of the whole batch, in blocks of their own
 hipError_t launch_force_gather(fnet_batch* b, const DevModel& m, long long a0, long long a1,
                                bool energies, hipStream_t s);
-// the orphans' part of the forces (and their counter reset); energies: also the sums over the
-// chunks; stamps: {start, end} of the launch
+// the orphans' part of the forces; energies: also the sums over the chunks; host: also the pinned
+// copy of the forces; stamps: {start, end} of the launch
 hipError_t launch_force_finish(fnet_batch* b, const DevModel& m, bool energies, hipStream_t s,
-                               unsigned long long* stamps = nullptr);
+                               bool host, unsigned long long* stamps = nullptr);
 
 // launchers (fnet_acsf.hip)
 hipError_t launch_acsf_fwd(fnet_batch* b, const DevModel& m, long long a0, long long a1, int fp64,
                            hipStream_t s);
+// norph: orphan counter that the launch clears, or null
 hipError_t launch_acsf_adj(fnet_batch* b, const DevModel& m, long long a0, long long a1, int fp64,
-                           hipStream_t s, unsigned long long* stamp = nullptr);
+                           hipStream_t s, int* norph, unsigned long long* stamp = nullptr);
 
 // launchers (fnet_mlp.hip)
 // mirror: extra blocks of the launch search the mirror entries of the whole batch
@@ -422,8 +465,9 @@ hipError_t launch_mlp_fwd(fnet_batch* b, const DevModel& m, int first_tile, int 
                           int want_grad_in, hipStream_t s, bool mirror = false,
                           unsigned long long* stamp = nullptr);
 constexpr int kEnergyChunk = 2048;  // atoms per block of the energy reduction
+// host: also the pinned copies (longest row, energies of small batches)
 hipError_t launch_energy_reduce(fnet_batch* b, const DevModel& m, int s0, int s1, hipStream_t s,
-                                int* h_maxnb = nullptr);
+                                bool host = false);
 hipError_t launch_lossgrad(fnet_batch* b, const DevModel& m, int n_global, const double* gt,
                            const double* at, const double* aw, const double* dpw, double inv_wsum,
                            int loss, hipStream_t s);
@@ -450,16 +494,13 @@ int grad_chunks(int ntiles);  // chunks of the weight-gradient reduction
 
 // launchers (fnet_mlp_mfma.hip): FP32 element networks on MFMA 16x16x4 f32
 int mlp_mfma_waves(const NetShape& sh);  // waves per block, 0 if the shape is not supported
-void pack_mfma_weights(const NetShape& sh, int nspecies, const double* params,
-                       std::vector<float>& out, long long& stride, long long* fw, long long* rw,
-                       long long* pb);
-void pack_bf16_weights(const NetShape& sh, int nspecies, const double* params,
-                       std::vector<uint16_t>& out, long long& stride, long long* bfw,
-                       long long* brw, long long* bsz);
+// sizes of the packed fragments (floats, bf16 values) and where each layer's lie
+void mfma_layout(DevModel& m, size_t* floats, size_t* halves);
 hipError_t launch_mlp_mfma(fnet_batch* b, const DevModel& m, int first_tile, int ntiles,
                            int want_grad_in, hipStream_t s, bool mirror = false,
                            unsigned long long* stamp = nullptr);
-hipError_t launch_to_float(const double* in, float* out, long long n, hipStream_t s);
+// FP32 copy of the resident parameters and, for networks on the matrix cores, their fragments
+hipError_t launch_model_params(const DevModel& m, hipStream_t s);
 
 size_t lds_bytes_acsf(int max_nb, int nZ, int fp64, int adj);
 int acsf_slice_entries(int max_nb);  // entries of one wave's LDS slice for rows up to max_nb
@@ -473,6 +514,9 @@ int acsf_slice_entries(int max_nb);  // entries of one wave's LDS slice for rows
   } while (0)
 
 namespace fnet {
+inline double* host_Estruct(const fnet_batch* b) { return b->h_res; }
+inline double* host_Eatom(const fnet_batch* b) { return b->h_res + b->S * b->ctx->model.nout; }
+inline double* host_F(const fnet_batch* b) { return host_Eatom(b) + b->N * b->ctx->model.nout; }
 inline long long layout_entries(const fnet_batch* b) {
   return b->nl_padded ? (long long)b->N * b->nb_cap : b->npairs;
 }

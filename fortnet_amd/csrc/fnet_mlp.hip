@@ -526,11 +526,6 @@ __global__ void __launch_bounds__(256) k_sd_step(double* __restrict__ x,
   }
 }
 
-__global__ void k_to_float(const double* __restrict__ in, float* __restrict__ out, long long n) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = (float)in[i];
-}
-
 template <typename T>
 size_t host_lds(const NetShape& sh, int TA) {
   size_t s = 0;
@@ -606,11 +601,10 @@ hipError_t launch_mlp_fwd(fnet_batch* b, const DevModel& m, int first_tile, int 
 }
 
 hipError_t launch_energy_reduce(fnet_batch* b, const DevModel& m, int s0, int s1, hipStream_t s,
-                                int* h_maxnb) {
+                                bool host) {
   const int n = s1 - s0;
   if (n <= 0) return hipSuccess;
-  EnergyArgs a = energy_args(b, m);
-  a.h_maxnb = h_maxnb;
+  const EnergyArgs a = energy_args(b, m, host);
   const int c0 = b->h_chunk_first[s0], nc = b->h_chunk_first[s1] - c0;
   if (nc > 0) k_energy_partial<<<nc, 256, 0, s>>>(a, c0);
   if (!a.single) {
@@ -699,12 +693,6 @@ hipError_t launch_sd_step(double* params, const double* grad, long long n, doubl
                           double max_disp, double tol, double* scratch, int nspecies,
                           hipStream_t s) {
   k_sd_step<<<nspecies, 256, 0, s>>>(params, grad, n, lr, max_disp, tol, scratch);
-  return hipGetLastError();
-}
-
-hipError_t launch_to_float(const double* in, float* out, long long n, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
-  k_to_float<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(in, out, n);
   return hipGetLastError();
 }
 

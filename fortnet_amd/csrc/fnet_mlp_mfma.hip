@@ -25,7 +25,6 @@
 // takes hi.hi only (8 bits; its errors are reported, not gated).  The input layer (z-scored
 // features, which can be ill-conditioned) and the output layer stay FP32.
 #include <algorithm>
-#include <cstring>
 
 #include "../../include/fnet_hip.h"
 #include "fnet_device.hpp"
@@ -616,126 +615,154 @@ int mlp_mfma_waves(const NetShape& sh) {
   return waves;
 }
 
-// Packs the FP32 weights of every species into MFMA A-operand fragments (see the header comment),
-// every layer width padded to a multiple of 32.  Forward fragment of layer l: index
-// ((ob * Kc + c) * 4 + s) * 64 + lane, lane = 16 g + i, holds ww_l(k = 16 c + 4 g + s,
-// o = 16 ob + i); reverse fragment: ((ib * Oc + c) * 4 + s) * 64 + lane holds
-// ww_l(k = 16 ib + i, o = 16 c + 4 g + s); zero outside the layer's dimensions.
-void pack_mfma_weights(const NetShape& sh, int nspecies, const double* params,
-                       std::vector<float>& out, long long& stride, long long* fw, long long* rw,
-                       long long* pb) {
+void mfma_layout(DevModel& m, size_t* floats, size_t* halves) {
+  const NetShape& sh = m.shape;
   long long o = 0;
   for (int l = 0; l + 1 < sh.nl; ++l) {
     const long long sz = (long long)r32(sh.dims[l]) * r32(sh.dims[l + 1]);
-    fw[l] = o;
+    m.pk_fw[l] = o;
     o += sz;
-    rw[l] = o;
+    m.pk_rw[l] = o;
     o += sz;
-    pb[l] = o;
+    m.pk_b[l] = o;
     o += r32(sh.dims[l + 1]);
   }
-  stride = (o + 63) & ~63LL;
-  out.assign((size_t)stride * nspecies, 0.0f);
-  for (int sp = 0; sp < nspecies; ++sp) {
-    const double* P = params + (long long)sp * sh.nparams;
-    float* D = out.data() + (long long)sp * stride;
-    for (int l = 0; l + 1 < sh.nl; ++l) {
-      const int din = sh.dims[l], dout = sh.dims[l + 1];
-      const int Kc = r32(din) / 16, Oc = r32(dout) / 16;
-      auto ww = [&](int k, int oo) -> float {
-        return (k < din && oo < dout) ? (float)P[sh.woff[l] + (long long)oo * din + k] : 0.0f;
-      };
-      for (int ob = 0; ob < Oc; ++ob)
-        for (int c = 0; c < Kc; ++c)
-          for (int s = 0; s < 4; ++s)
-            for (int lane = 0; lane < 64; ++lane) {
-              const int g = lane / 16, i = lane % 16;
-              D[fw[l] + ((long long)(ob * Kc + c) * 4 + s) * 64 + lane] =
-                  ww(16 * c + 4 * g + s, 16 * ob + i);
-            }
-      for (int ib = 0; ib < Kc; ++ib)
-        for (int c = 0; c < Oc; ++c)
-          for (int s = 0; s < 4; ++s)
-            for (int lane = 0; lane < 64; ++lane) {
-              const int g = lane / 16, i = lane % 16;
-              D[rw[l] + ((long long)(ib * Oc + c) * 4 + s) * 64 + lane] =
-                  ww(16 * ib + i, 16 * c + 4 * g + s);
-            }
-      for (int q = 0; q < dout; ++q) D[pb[l] + q] = (float)P[sh.boff[l + 1] + q];
-    }
+  m.pk_stride = (o + 63) & ~63LL;
+  *floats = (size_t)m.pk_stride * m.nspecies;
+  // BF16 fragments of the hidden-to-hidden layers (none for networks with one hidden layer)
+  long long h = 0;
+  for (int l = 0; l < kMaxLayers; ++l) m.bk_fw[l] = m.bk_rw[l] = m.bk_sz[l] = 0;
+  for (int l = 1; l + 2 < sh.nl; ++l) {
+    const long long sz = (long long)r32(sh.dims[l]) * r32(sh.dims[l + 1]) / 8;
+    m.bk_sz[l] = sz;
+    m.bk_fw[l] = h;
+    h += 2 * sz;
+    m.bk_rw[l] = h;
+    h += 2 * sz;
   }
+  m.bk_stride = h;
+  *halves = (size_t)(h * 8 * m.nspecies);
 }
 
 namespace {
+
 // float -> bf16 bits, round to nearest even (finite values)
-uint16_t to_bf16(float x) {
-  uint32_t u;
-  std::memcpy(&u, &x, 4);
+__device__ __forceinline__ uint16_t to_bf16(float x) {
+  uint32_t u = __float_as_uint(x);
   u += 0x7fffu + ((u >> 16) & 1u);
   return (uint16_t)(u >> 16);
 }
-float from_bf16(uint16_t h) {
-  const uint32_t u = (uint32_t)h << 16;
-  float x;
-  std::memcpy(&x, &u, 4);
-  return x;
+
+struct PackArgs {
+  NetShape sh;
+  int nspecies;
+  const double* params;
+  float* params_f;
+  float* wpack;  // null: no matrix-core networks
+  uint16_t* bpack;
+  long long pk_stride, bk_stride;
+  long long fw[kMaxLayers], rw[kMaxLayers], pb[kMaxLayers];
+  long long bfw[kMaxLayers], brw[kMaxLayers], bsz[kMaxLayers];
+};
+
+// The FP32 copy of the parameters and the MFMA fragments of every species, one thread per value:
+// after a parameter update nothing has to come to the host to be packed.
+//
+// A-operand fragments of FP32 layers, every width padded to a multiple of 32 with zeros.  Forward
+// fragment of layer l: index ((ob * Kc + c) * 4 + s) * 64 + lane, lane = 16 g + i, holds
+// ww_l(k = 16 c + 4 g + s, o = 16 ob + i); reverse fragment: ((ib * Oc + c) * 4 + s) * 64 + lane
+// holds ww_l(k = 16 ib + i, o = 16 c + 4 g + s); then the layer's biases.
+//
+// BF16 fragments (hi, then lo = bf16(w - hi)) of the hidden-to-hidden layers for
+// v_mfma_f32_16x16x32_bf16.  Forward: element ((ob * Kc32 + c) * 64 + lane) * 8 + e holds
+// ww_l(k = 32 c + 8 g + e, o = 16 ob + i); reverse: ((ib * Oc32 + c) * 64 + lane) * 8 + e holds
+// ww_l(k = 16 ib + i, o = 32 c + 8 g + e).  Offsets and sizes are in units of 8 values.
+__global__ void __launch_bounds__(256) k_model_params(PackArgs a) {
+  long long q = (long long)blockIdx.x * 256 + threadIdx.x;
+  const long long np = a.sh.nparams * a.nspecies;
+  if (q < np) {
+    a.params_f[q] = (float)a.params[q];
+    return;
+  }
+  q -= np;
+  if (!a.wpack) return;
+  const bool half = q >= a.pk_stride * a.nspecies;
+  if (half) q -= a.pk_stride * a.nspecies;
+  const long long stride = half ? 8 * a.bk_stride : a.pk_stride;
+  if (stride == 0 || q >= stride * a.nspecies) return;
+  const long long sp = q / stride, e = q - sp * stride;
+  const double* P = a.params + sp * a.sh.nparams;
+  float w = 0.0f;
+  bool lo = false;
+  for (int l = 0; l + 1 < a.sh.nl; ++l) {
+    const int din = a.sh.dims[l], dout = a.sh.dims[l + 1];
+    const long long sz = (long long)r32(din) * r32(dout);
+    int k = -1, o = -1;
+    if (half) {
+      if (a.bsz[l] == 0) continue;
+      const long long tf = e - 8 * a.bfw[l], tr = e - 8 * a.brw[l];
+      const bool fwd = tf >= 0 && tf < 2 * sz, rev = tr >= 0 && tr < 2 * sz;
+      if (!fwd && !rev) continue;
+      long long t = fwd ? tf : tr;
+      lo = t >= sz;
+      if (lo) t -= sz;
+      const int u = (int)(t & 7), lane = (int)(t >> 3) & 63, g = lane >> 4, i = lane & 15;
+      const int nc = r32(fwd ? din : dout) >> 5, blk = (int)(t >> 9);
+      const int ob = blk / nc, c = blk - ob * nc;
+      k = fwd ? 32 * c + 8 * g + u : 16 * ob + i;
+      o = fwd ? 16 * ob + i : 32 * c + 8 * g + u;
+    } else {
+      const long long tf = e - a.fw[l], tr = e - a.rw[l], tb = e - a.pb[l];
+      if (tb >= 0 && tb < r32(dout)) {
+        if (tb < dout) w = (float)P[a.sh.boff[l + 1] + tb];
+        break;
+      }
+      const bool fwd = tf >= 0 && tf < sz, rev = tr >= 0 && tr < sz;
+      if (!fwd && !rev) continue;
+      const long long t = fwd ? tf : tr;
+      const int lane = (int)t & 63, g = lane >> 4, i = lane & 15, s = (int)(t >> 6) & 3;
+      const int nc = r32(fwd ? din : dout) >> 4, blk = (int)(t >> 8);
+      const int ob = blk / nc, c = blk - ob * nc;
+      k = fwd ? 16 * c + 4 * g + s : 16 * ob + i;
+      o = fwd ? 16 * ob + i : 16 * c + 4 * g + s;
+    }
+    if (k < din && o < dout) w = (float)P[a.sh.woff[l] + (long long)o * din + k];
+    break;
+  }
+  if (!half) {
+    a.wpack[q] = w;
+  } else {
+    const uint16_t h = to_bf16(w);
+    a.bpack[q] = lo ? to_bf16(w - __uint_as_float((uint32_t)h << 16)) : h;
+  }
 }
+
 }  // namespace
 
-// BF16 fragments (hi, then lo = bf16(w - hi)) of the hidden-to-hidden layers for
-// v_mfma_f32_16x16x32_bf16.  Forward fragment of layer l: element
-// ((ob * Kc32 + c) * 64 + lane) * 8 + e, lane = 16 g + i, holds ww_l(k = 32 c + 8 g + e,
-// o = 16 ob + i); reverse: ((ib * Oc32 + c) * 64 + lane) * 8 + e holds
-// ww_l(k = 16 ib + i, o = 32 c + 8 g + e).  Offsets and sizes are in units of 8 values.
-void pack_bf16_weights(const NetShape& sh, int nspecies, const double* params,
-                       std::vector<uint16_t>& out, long long& stride, long long* bfw,
-                       long long* brw, long long* bsz) {
-  long long o = 0;
-  for (int l = 0; l < kMaxLayers; ++l) bfw[l] = brw[l] = bsz[l] = 0;
-  for (int l = 1; l + 2 < sh.nl; ++l) {
-    const long long sz = (long long)r32(sh.dims[l]) * r32(sh.dims[l + 1]) / 8;
-    bsz[l] = sz;
-    bfw[l] = o;
-    o += 2 * sz;
-    brw[l] = o;
-    o += 2 * sz;
+hipError_t launch_model_params(const DevModel& m, hipStream_t s) {
+  PackArgs a;
+  a.sh = m.shape;
+  a.nspecies = m.nspecies;
+  a.params = m.params;
+  a.params_f = m.params_f;
+  a.wpack = m.wpack;
+  a.bpack = m.bpack;
+  a.pk_stride = m.pk_stride;
+  a.bk_stride = m.bk_stride;
+  for (int l = 0; l < kMaxLayers; ++l) {
+    a.fw[l] = m.pk_fw[l];
+    a.rw[l] = m.pk_rw[l];
+    a.pb[l] = m.pk_b[l];
+    a.bfw[l] = m.bk_fw[l];
+    a.brw[l] = m.bk_rw[l];
+    a.bsz[l] = m.bk_sz[l];
   }
-  stride = o;
-  out.assign((size_t)(stride * 8 * nspecies), 0);
-  for (int sp = 0; sp < nspecies; ++sp) {
-    const double* P = params + (long long)sp * sh.nparams;
-    uint16_t* D = out.data() + (long long)sp * stride * 8;
-    for (int l = 1; l + 2 < sh.nl; ++l) {
-      const int din = sh.dims[l], dout = sh.dims[l + 1];
-      const int Kc32 = r32(din) / 32, Oc32 = r32(dout) / 32;
-      const int Kb = r32(din) / 16, Ob = r32(dout) / 16;
-      const long long sz8 = bsz[l] * 8;
-      auto put = [&](long long base, long long idx, float w) {
-        const uint16_t h = to_bf16(w);
-        D[base + idx] = h;
-        D[base + sz8 + idx] = to_bf16(w - from_bf16(h));
-      };
-      auto ww = [&](int k, int oo) -> float {
-        return (k < din && oo < dout) ? (float)P[sh.woff[l] + (long long)oo * din + k] : 0.0f;
-      };
-      for (int ob = 0; ob < Ob; ++ob)
-        for (int c = 0; c < Kc32; ++c)
-          for (int lane = 0; lane < 64; ++lane)
-            for (int e = 0; e < 8; ++e) {
-              const int g = lane / 16, i = lane % 16;
-              put(bfw[l] * 8, (((long long)ob * Kc32 + c) * 64 + lane) * 8 + e,
-                  ww(32 * c + 8 * g + e, 16 * ob + i));
-            }
-      for (int ib = 0; ib < Kb; ++ib)
-        for (int c = 0; c < Oc32; ++c)
-          for (int lane = 0; lane < 64; ++lane)
-            for (int e = 0; e < 8; ++e) {
-              const int g = lane / 16, i = lane % 16;
-              put(brw[l] * 8, (((long long)ib * Oc32 + c) * 64 + lane) * 8 + e,
-                  ww(16 * ib + i, 32 * c + 8 * g + e));
-            }
-    }
-  }
+  long long n = m.shape.nparams;
+  if (m.wpack) n += m.pk_stride + 8 * m.bk_stride;
+  n *= m.nspecies;
+  if (n <= 0) return hipSuccess;
+  k_model_params<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(a);
+  return hipGetLastError();
 }
 
 namespace {

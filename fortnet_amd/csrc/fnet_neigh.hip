@@ -73,8 +73,8 @@ __device__ void lattice_setup(const double* L, double rc, StructInfo& si) {
 // One block per structure: lattice set-up by thread 0, then the extent of the fractional
 // coordinates (it only serves the image pruning of the direct search) or, for a structure with
 // cell lists that fits one block (bin_lds), its bins: an LDS histogram, its prefix sums and the
-// scatter, in place of seven launches over all atoms (24 ternary cells of 16 - 4096 atoms: 75 us
-// of launches -> 20 us).  Block 0 clears the row maximum that the search raises.
+// scatter, in place of seven launches over all atoms (24 ternary cells of 16 - 4096 atoms: eight
+// launches and 99 us -> one of 13 us).  Block 0 clears the row maximum that the search raises.
 struct PrepArgs {
   const double* xyz;
   const double* lat;
