@@ -124,7 +124,8 @@ struct MfmaArgs {
   int wave_floats;
   double* Eatom;  // [N][nout]
   double* cG;     // [N][nout][nG]
-  int ntiles;     // blocks beyond the tiles search mirror entries
+  int nsub;       // 16-atom parts of a tile (blocks per tile when the waves share them)
+  int ntiles;     // blocks beyond the tiles' search mirror entries
   MirrorArgs mr;
   unsigned long long* stamp;
 };
@@ -179,6 +180,29 @@ __device__ __forceinline__ void gemm_pair(const float* __restrict__ Af, int ob0,
       c0 = __builtin_amdgcn_mfma_f32_16x16x4f32(u0[s], xb[s], c0, 0, 0, 0);
       c1 = __builtin_amdgcn_mfma_f32_16x16x4f32(u1[s], xb[s], c1, 0, 0, 0);
     }
+  }
+}
+
+// One output block of the same product (the same sums in the same order): the fragments of four
+// chunks are fetched before the first is used, since a block that runs alone has nothing else to
+// hide their latency behind.
+__device__ __forceinline__ void gemm_one(const float* __restrict__ Af, int ob, int Kc,
+                                         const float* X, int ldx, int lane, int j, int g, f4& c0) {
+  const float* A0 = Af + (long long)ob * Kc * 256 + lane;
+  for (int c = 0; c < Kc; c += 4) {
+    float u[4][4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) u[d][s] = c + d < Kc ? A0[((c + d) * 4 + s) * 64] : 0.0f;
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+      if (c + d < Kc) {
+        const f4 xb = *(const f4*)(X + j * ldx + 16 * (c + d) + 4 * g);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+          c0 = __builtin_amdgcn_mfma_f32_16x16x4f32(u[d][s], xb[s], c0, 0, 0, 0);
+      }
   }
 }
 
@@ -238,10 +262,43 @@ __device__ __forceinline__ void gemm_pair_bf(const bf8* __restrict__ Ah, long lo
   }
 }
 
+// ... and one block of it
+template <int BF>
+__device__ __forceinline__ void gemm_one_bf(const bf8* __restrict__ Ah, long long bsz, int ob,
+                                            int Kc32, const float* X, int ldx, int lane, int j,
+                                            int g, f4& c0) {
+  const bf8* A0 = Ah + (long long)ob * Kc32 * 64 + lane;
+  for (int c = 0; c < Kc32; c += 2) {
+    bf8 a[2], lo[2];
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+      if (c + d < Kc32) {
+        a[d] = A0[(c + d) * 64];
+        if (BF == 3) lo[d] = A0[bsz + (c + d) * 64];
+      }
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+      if (c + d < Kc32) {
+        const float* xr = X + j * ldx + 32 * (c + d) + 8 * g;
+        bf8 xh, xl;
+        split8(*(const f4*)xr, *(const f4*)(xr + 4), xh, xl);
+        c0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d], xh, c0, 0, 0, 0);
+        if (BF == 3) {
+          c0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d], xl, c0, 0, 0, 0);
+          c0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo[d], xh, c0, 0, 0, 0);
+        }
+      }
+  }
+}
+
 // layer l (ww(d_l, d_{l+1})) maps a hidden layer to a hidden layer
 __device__ __forceinline__ bool hidden_hidden(int l, int nl) { return l >= 1 && l + 1 <= nl - 2; }
 
-template <bool GRADIN, int BF>
+// SPLIT: the four waves of a block share 16 atoms, each taking every fourth output block, instead
+// of running 16 atoms each through all of them: a batch that leaves most of the chip idle waits
+// for one wave's chain of loads, products and activations, which this cuts to about a third.  The
+// sums are the same either way.
+template <bool GRADIN, int BF, bool SPLIT>
 __global__ void __launch_bounds__(256) k_mlp_mfma(MfmaArgs a) {
   extern __shared__ __align__(16) float smf[];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -251,15 +308,21 @@ __global__ void __launch_bounds__(256) k_mlp_mfma(MfmaArgs a) {
     mirror_centre(a.mr, (long long)((int)blockIdx.x - a.ntiles) * (blockDim.x >> 6) + w, lane);
     return;
   }
-  const int tile = a.first_tile + blockIdx.x;
+  // waves a layer's blocks (and an activation's rows) are dealt to, and this one's number
+  const int nw = SPLIT ? 4 : 1, me = SPLIT ? w : 0;
+  const int tile = a.first_tile + (SPLIT ? (int)blockIdx.x / a.nsub : (int)blockIdx.x);
+  const int a0 = 16 * (SPLIT ? (int)blockIdx.x % a.nsub : w);
   const int sp = a.tile_sp[tile], start = a.tile_start[tile], cnt = a.tile_cnt[tile];
-  const int a0 = 16 * w;
-  if (a0 >= cnt) return;  // whole wave
+  if (a0 >= cnt) return;  // whole wave (SPLIT: whole block)
+  auto sync = [] {
+    if constexpr (SPLIT) __syncthreads();
+    else wave_sync();
+  };
   const int nv = min(16, cnt - a0);
   const int nl = a.sh.nl;
   const int act = a.sh.act[sp];
   const int ldx = a.ldx;
-  float* X = smf + (size_t)w * a.wave_floats;
+  float* X = smf + (SPLIT ? 0 : (size_t)w * a.wave_floats);
   float* FP = X + 16 * ldx;
   const float* WP = a.wpack + (long long)sp * a.pk_stride;
   const bool valid = j < nv;
@@ -267,7 +330,7 @@ __global__ void __launch_bounds__(256) k_mlp_mfma(MfmaArgs a) {
 
   // input rows: standardised features (and external features), zero beyond d0 and nv
   const int d0 = a.sh.dims[0], K0 = r32(d0);
-  for (int idx = lane; idx < 16 * K0; idx += 64) {
+  for (int idx = SPLIT ? (int)threadIdx.x : lane; idx < 16 * K0; idx += 64 * nw) {
     const int r = idx / K0, k = idx - r * K0;
     float v = 0.0f;
     if (r < nv && k < d0) {
@@ -277,8 +340,16 @@ __global__ void __launch_bounds__(256) k_mlp_mfma(MfmaArgs a) {
     }
     X[r * ldx + k] = v;
   }
-  wave_sync();
+  sync();
 
+  // linear output layer (nout <= 16): lane group g holds outputs 4 g + r of atom j
+  auto write_out = [&](const f4& c) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int o = 4 * g + r;
+      if (o < a.nout) a.Eatom[atom * a.nout + o] = (double)c[r];
+    }
+  };
   for (int l = 0; l < nl - 1; ++l) {
     const int Kc = r32(a.sh.dims[l]) >> 4, Nb = r32(a.sh.dims[l + 1]) >> 4;
     const float* Wf = WP + a.fw[l];
@@ -286,33 +357,37 @@ __global__ void __launch_bounds__(256) k_mlp_mfma(MfmaArgs a) {
     const bool hidden = l < nl - 2;
     float* zs = FP + a.fpoff[l + 1];
     const bool bf = BF && hidden_hidden(l, nl);
-    for (int ob0 = 0; ob0 < Nb; ob0 += 2) {
-      f4 c0 = *(const f4*)(Bp + 16 * ob0 + 4 * g);
-      f4 c1 = *(const f4*)(Bp + 16 * ob0 + 16 + 4 * g);
-      if (bf)
-        gemm_pair_bf<BF>(a.bpack + (long long)sp * a.bk_stride + a.bfw[l], a.bsz[l], ob0, Kc >> 1,
-                         X, ldx, lane, j, g, c0, c1);
-      else
-        gemm_pair(Wf, ob0, Kc, X, ldx, lane, j, g, c0, c1);
-      if (hidden) {
-        *(f4*)(zs + (ob0 * 64 + lane) * 4) = c0;
-        *(f4*)(zs + ((ob0 + 1) * 64 + lane) * 4) = c1;
-      } else if (valid) {
-        // linear output layer (nout <= 16): lane group g holds outputs 4 g + r of atom j
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int o = 4 * g + r;
-          if (o < a.nout) a.Eatom[atom * a.nout + o] = (double)c0[r];
+    const bf8* Bf = a.bpack + (long long)sp * a.bk_stride + a.bfw[l];
+    if constexpr (SPLIT) {
+      // the output layer's second block holds no output
+      for (int ob = me; ob < (hidden ? Nb : 1); ob += nw) {
+        f4 c0 = *(const f4*)(Bp + 16 * ob + 4 * g);
+        if (bf) gemm_one_bf<BF ? BF : 1>(Bf, a.bsz[l], ob, Kc >> 1, X, ldx, lane, j, g, c0);
+        else gemm_one(Wf, ob, Kc, X, ldx, lane, j, g, c0);
+        if (hidden) *(f4*)(zs + (ob * 64 + lane) * 4) = c0;
+        else if (valid) write_out(c0);
+      }
+    } else {
+      for (int ob0 = 0; ob0 < Nb; ob0 += 2) {
+        f4 c0 = *(const f4*)(Bp + 16 * ob0 + 4 * g);
+        f4 c1 = *(const f4*)(Bp + 16 * ob0 + 16 + 4 * g);
+        if (bf) gemm_pair_bf<BF>(Bf, a.bsz[l], ob0, Kc >> 1, X, ldx, lane, j, g, c0, c1);
+        else gemm_pair(Wf, ob0, Kc, X, ldx, lane, j, g, c0, c1);
+        if (hidden) {
+          *(f4*)(zs + (ob0 * 64 + lane) * 4) = c0;
+          *(f4*)(zs + ((ob0 + 1) * 64 + lane) * 4) = c1;
+        } else if (valid) {
+          write_out(c0);
         }
       }
     }
-    wave_sync();  // every lane has read this layer's rows before they are overwritten
+    sync();  // every lane has read this layer's rows before they are overwritten
     if (hidden) {
       // activation: z in the fragment slots -> next rows y = f(z), slots <- f'(z); four at a
       // time, so that their LDS reads and transcendentals overlap (the kernel's occupancy is
       // set by its LDS, not by these registers)
 #pragma unroll 4
-      for (int q = 0; q < 4 * Nb; ++q) {
+      for (int q = me; q < 4 * Nb; q += nw) {
         const int ob = q >> 2, r = q & 3;
         float* slot = zs + (ob * 64 + lane) * 4 + r;
         const float z = *slot;
@@ -321,7 +396,7 @@ __global__ void __launch_bounds__(256) k_mlp_mfma(MfmaArgs a) {
         X[j * ldx + 16 * ob + 4 * g + r] = f;
         *slot = d;
       }
-      wave_sync();
+      sync();
     }
   }
   if (!GRADIN) return;
@@ -336,58 +411,69 @@ __global__ void __launch_bounds__(256) k_mlp_mfma(MfmaArgs a) {
     if (m >= 1) {
       float* sl = FP + a.fpoff[m];
 #pragma unroll 4
-      for (int q = 0; q < 4 * Kb; ++q) {
+      for (int q = me; q < 4 * Kb; q += nw) {
         const int ib = q >> 2, r = q & 3, k = 16 * ib + 4 * g + r;
         float* slot = sl + (ib * 64 + lane) * 4 + r;
         const float d = (k < dm ? col[k] : 0.0f) * *slot;
         *slot = d;
         X[j * ldx + k] = d;
       }
-      wave_sync();
+      sync();
     } else if (valid) {
-      for (int k = 4 * g; k < a.nG; k += 16)
+      for (int k = 4 * g + 16 * me; k < a.nG; k += 16 * nw)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           if (k + r < a.nG) out[k + r] = (double)col[k + r] * a.zinv[k + r];
     }
   }
-  // delta_{m-1}^T = W_{m-1} . delta_m^T (rows in X), times f'(z_{m-1}) for hidden layers
+  // delta_{m-1}^T = W_{m-1} . delta_m^T (rows in X), times f'(z_{m-1}) for hidden layers; the
+  // input layer: the ACSF part of d out / d x feeds the force adjoint (FP64, z-score factor)
+  auto write_in = [&](const f4& c, int ib) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int f = 16 * ib + 4 * g + r;
+      if (f < a.nG) out[f] = (double)c[r] * a.zinv[f];
+    }
+  };
   for (; m >= 1; --m) {
     const int Mb = r32(a.sh.dims[m - 1]) >> 4, Kc = r32(a.sh.dims[m]) >> 4;
     const float* Rf = WP + a.rw[m - 1];
     float* sl = FP + a.fpoff[m - 1];
     const bool bf = BF && hidden_hidden(m - 1, nl);
-    for (int ib0 = 0; ib0 < Mb; ib0 += 2) {
-      f4 c0 = {0.0f, 0.0f, 0.0f, 0.0f}, c1 = {0.0f, 0.0f, 0.0f, 0.0f};
-      if (bf)
-        gemm_pair_bf<BF>(a.bpack + (long long)sp * a.bk_stride + a.brw[m - 1], a.bsz[m - 1], ib0,
-                         Kc >> 1, X, ldx, lane, j, g, c0, c1);
-      else
-        gemm_pair(Rf, ib0, Kc, X, ldx, lane, j, g, c0, c1);
+    const bf8* Br = a.bpack + (long long)sp * a.bk_stride + a.brw[m - 1];
+    auto put = [&](const f4& c, int ib) {
       if (m - 1 >= 1) {
-        f4* s0 = (f4*)(sl + (ib0 * 64 + lane) * 4);
-        f4* s1 = (f4*)(sl + ((ib0 + 1) * 64 + lane) * 4);
-        *s0 = c0 * *s0;
-        *s1 = c1 * *s1;
+        f4* s0 = (f4*)(sl + (ib * 64 + lane) * 4);
+        *s0 = c * *s0;
       } else if (valid) {
-        // input layer: the ACSF part of d out / d x feeds the force adjoint (FP64, z-score factor)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int f0 = 16 * ib0 + 4 * g + r, f1 = f0 + 16;
-          if (f0 < a.nG) out[f0] = (double)c0[r] * a.zinv[f0];
-          if (f1 < a.nG) out[f1] = (double)c1[r] * a.zinv[f1];
-        }
+        write_in(c, ib);
+      }
+    };
+    if constexpr (SPLIT) {
+      for (int ib = me; ib < Mb; ib += nw) {
+        f4 c0 = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (bf) gemm_one_bf<BF ? BF : 1>(Br, a.bsz[m - 1], ib, Kc >> 1, X, ldx, lane, j, g, c0);
+        else gemm_one(Rf, ib, Kc, X, ldx, lane, j, g, c0);
+        put(c0, ib);
+      }
+    } else {
+      for (int ib0 = 0; ib0 < Mb; ib0 += 2) {
+        f4 c0 = {0.0f, 0.0f, 0.0f, 0.0f}, c1 = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (bf) gemm_pair_bf<BF>(Br, a.bsz[m - 1], ib0, Kc >> 1, X, ldx, lane, j, g, c0, c1);
+        else gemm_pair(Rf, ib0, Kc, X, ldx, lane, j, g, c0, c1);
+        put(c0, ib0);
+        put(c1, ib0 + 1);
       }
     }
-    wave_sync();
+    sync();
     if (m - 1 >= 1) {
       // delta_{m-1} fragments -> rows for the next product
 #pragma unroll 4
-      for (int q = 0; q < 4 * Mb; ++q) {
+      for (int q = me; q < 4 * Mb; q += nw) {
         const int ib = q >> 2, r = q & 3;
         X[j * ldx + 16 * ib + 4 * g + r] = sl[(ib * 64 + lane) * 4 + r];
       }
-      wave_sync();
+      sync();
     }
   }
 }
@@ -851,6 +937,9 @@ hipError_t launch_mlp_grad_mfma(fnet_batch* b, const DevModel& m, hipStream_t s)
   return hipGetLastError();
 }
 
+// 16-atom parts up to which the waves of a block share one (SPLIT)
+constexpr long long kSplitTiles = 1024;
+
 hipError_t launch_mlp_mfma(fnet_batch* b, const DevModel& m, int first_tile, int ntiles,
                            int want_grad_in, hipStream_t s, bool mirror,
                            unsigned long long* stamp) {
@@ -891,20 +980,26 @@ hipError_t launch_mlp_mfma(fnet_batch* b, const DevModel& m, int first_tile, int
   const int bf = (b->precision == FNET_BF16 && m.bpack) ? 3
                : (b->precision == FNET_BF16_FAST && m.bpack) ? 1 : 0;
   const int waves = b->mtile_waves;
-  const size_t lds = (size_t)waves * a.wave_floats * sizeof(float);
-  a.ntiles = ntiles;
+  a.nsub = waves;
   a.mr = mirror_args(b, 0, b->N);
   a.stamp = stamp;
-  const dim3 grid((unsigned)(ntiles + (mirror ? (b->N + waves - 1) / waves : 0))),
-      block(64 * waves);
+  const bool split = (long long)ntiles * waves <= kSplitTiles;
+  const int bw = split ? 4 : waves;  // waves per block
+  a.ntiles = split ? ntiles * waves : ntiles;
+  const size_t lds = (size_t)(split ? 1 : waves) * a.wave_floats * sizeof(float);
+  const dim3 grid((unsigned)(a.ntiles + (mirror ? (b->N + bw - 1) / bw : 0))), block(64 * bw);
+  auto go = [&](auto* sp, auto* one) {
+    if (split) sp<<<grid, block, lds, s>>>(a);
+    else one<<<grid, block, lds, s>>>(a);
+  };
   if (want_grad_in) {
-    if (bf == 3) k_mlp_mfma<true, 3><<<grid, block, lds, s>>>(a);
-    else if (bf == 1) k_mlp_mfma<true, 1><<<grid, block, lds, s>>>(a);
-    else k_mlp_mfma<true, 0><<<grid, block, lds, s>>>(a);
+    if (bf == 3) go(k_mlp_mfma<true, 3, true>, k_mlp_mfma<true, 3, false>);
+    else if (bf == 1) go(k_mlp_mfma<true, 1, true>, k_mlp_mfma<true, 1, false>);
+    else go(k_mlp_mfma<true, 0, true>, k_mlp_mfma<true, 0, false>);
   } else {
-    if (bf == 3) k_mlp_mfma<false, 3><<<grid, block, lds, s>>>(a);
-    else if (bf == 1) k_mlp_mfma<false, 1><<<grid, block, lds, s>>>(a);
-    else k_mlp_mfma<false, 0><<<grid, block, lds, s>>>(a);
+    if (bf == 3) go(k_mlp_mfma<false, 3, true>, k_mlp_mfma<false, 3, false>);
+    else if (bf == 1) go(k_mlp_mfma<false, 1, true>, k_mlp_mfma<false, 1, false>);
+    else go(k_mlp_mfma<false, 0, true>, k_mlp_mfma<false, 0, false>);
   }
   return hipGetLastError();
 }
