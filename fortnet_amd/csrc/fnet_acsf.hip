@@ -26,8 +26,8 @@
 //    dense array, but without forming it and with periodic images summed exactly.
 //
 // Arithmetic is T (double or float); sums over neighbours and pairs, the values G and the forces
-// are accumulated in FP64 in both modes.  FP64 evaluates the elementary functions with libm in the
-// reference's operation order; FP32 uses the hardware instructions (v_exp_f32, v_cos_f32,
+// are accumulated in FP64 in both modes.  FP64 evaluates exp and the cutoff's cos and sin to within
+// 3e-16 (fexp, cut_cs), roots, quotients and real powers with libm; FP32 uses the hardware instructions (v_exp_f32, v_cos_f32,
 // v_sin_f32, v_sqrt_f32, v_rcp_f32: about 1 ulp, cos/sin to ~1e-6 absolute on [0, pi]).
 #include "fnet_device.hpp"
 
@@ -55,7 +55,36 @@ __device__ __forceinline__ unsigned long long lanemask_lt(int lane) {
 }
 
 __device__ __forceinline__ float fexp(float x) { return __expf(x); }
-__device__ __forceinline__ double fexp(double x) { return exp(x); }
+// A literal that stays in two scalar moves where it is used: hoisted out of the loops, the
+// polynomials' coefficients took 60 vector registers and two waves per SIMD.
+__device__ __forceinline__ double lit(double c) {
+  __asm__ volatile("" : "+s"(c));
+  return c;
+}
+// FP64 exp from its definition: x = n ln 2 + r with ln 2 in two parts, the Taylor polynomial of
+// degree 13 on |r| <= ln 2 / 2 (remainder 4e-18), scaled by 2^n; 1.4e-16 relative.  20 instructions
+// without branches or large temporaries; libm's exp and cos took the FP64 kernels to 177 and 148
+// registers (now 112 and 100: 16 water boxes forward 194 -> 155 us, adjoint 327 -> 253 us).
+__device__ __forceinline__ double fexp(double x) {
+  const double n = rint(x * 1.4426950408889634);
+  double r = fma(-n, 0.6931471805599453, x);
+  r = fma(-n, 2.3190468138462996e-17, r);
+  double p = lit(1.0 / 6227020800.0);
+  p = fma(p, r, lit(1.0 / 479001600.0));
+  p = fma(p, r, lit(1.0 / 39916800.0));
+  p = fma(p, r, lit(1.0 / 3628800.0));
+  p = fma(p, r, lit(1.0 / 362880.0));
+  p = fma(p, r, lit(1.0 / 40320.0));
+  p = fma(p, r, lit(1.0 / 5040.0));
+  p = fma(p, r, lit(1.0 / 720.0));
+  p = fma(p, r, lit(1.0 / 120.0));
+  p = fma(p, r, lit(1.0 / 24.0));
+  p = fma(p, r, lit(1.0 / 6.0));
+  p = fma(p, r, 0.5);
+  p = fma(p, r, 1.0);
+  p = fma(p, r, 1.0);
+  return ldexp(p, __double2int_rn(n));
+}
 __device__ __forceinline__ float fcos(float x) { return __cosf(x); }
 __device__ __forceinline__ double fcos(double x) { return cos(x); }
 __device__ __forceinline__ float fsin(float x) { return __sinf(x); }
@@ -77,12 +106,43 @@ __device__ __forceinline__ void dist_inv(double r2, double& r, double& ir) {
   ir = 1.0 / r;
 }
 __device__ __forceinline__ double fdiv(double x, double y) { return x / y; }
-// argument pi r / rc of the cosine cutoff (FP32: with the wave-uniform pi / rc hoisted)
-__device__ __forceinline__ float cutarg(float r, float pi, float rc, float pirc) {
-  return r * pirc;
+// cos and sin of the cosine cutoff's argument x = pi r / rc for r in [0, rc] (finite beyond; the
+// callers discard those).  FP32: the hardware instructions on r (pi / rc).  FP64: with
+// u = x / 2 - pi / 4 = (pi / 4)(2 r / rc - 1), |u| <= pi / 4, cos x = -2 sin u cos u and
+// sin x = 1 - 2 sin^2 u, both from Taylor polynomials (remainders 5e-17 and 2e-18) and one rounding
+// of 2 r / rc - 1 in place of those of pi r and its quotient: as close to the exact value as libm's
+// cos of the rounded argument.
+__device__ __forceinline__ void cut_cs(float r, float rc, float pirc, float& c, float& s) {
+  c = fcos(r * pirc);
+  s = fsin(r * pirc);
 }
-__device__ __forceinline__ double cutarg(double r, double pi, double rc, double pirc) {
-  return pi * r / rc;
+__device__ __forceinline__ void cut_cs(double r, double rc, double pirc, double& c, double& s) {
+  const double u = fma(r, 2.0 / rc, -1.0) * 0.78539816339744831, z = u * u;
+  double a = lit(-1.0 / 1307674368000.0);
+  a = fma(a, z, lit(1.0 / 6227020800.0));
+  a = fma(a, z, lit(-1.0 / 39916800.0));
+  a = fma(a, z, lit(1.0 / 362880.0));
+  a = fma(a, z, lit(-1.0 / 5040.0));
+  a = fma(a, z, lit(1.0 / 120.0));
+  a = fma(a, z, lit(-1.0 / 6.0));
+  const double sn = fma(a * z, u, u);
+  double b = lit(1.0 / 20922789888000.0);
+  b = fma(b, z, lit(-1.0 / 87178291200.0));
+  b = fma(b, z, lit(1.0 / 479001600.0));
+  b = fma(b, z, lit(-1.0 / 3628800.0));
+  b = fma(b, z, lit(1.0 / 40320.0));
+  b = fma(b, z, lit(-1.0 / 720.0));
+  b = fma(b, z, lit(1.0 / 24.0));
+  b = fma(b, z, -0.5);
+  const double cs = fma(b, z, 1.0);
+  c = -2.0 * sn * cs;
+  s = fma(-2.0 * sn, sn, 1.0);
+}
+template <typename T>
+__device__ __forceinline__ T cut_cos(T r, T rc, T pirc) {
+  T c, s;
+  cut_cs(r, rc, pirc, c, s);
+  return c;
 }
 
 // A wave-uniform value moved to scalar registers (values converted from FP64 on the vector
@@ -527,7 +587,7 @@ __device__ __forceinline__ void pairs_fwd(const Slice<T>& sl, int lane, int A0, 
       const T rx = dj.x - dk.x, ry = dj.y - dk.y, rz = dj.z - dk.z;
       const T r2 = rx * rx + ry * ry + rz * rz;
       const T rjk = fsqrt(r2);
-      const T fcjk = (T)0.5 * pj.z * pk.z * (fcos(cutarg(rjk, pi, rc, pirc)) + (T)1);
+      const T fcjk = (T)0.5 * pj.z * pk.z * (cut_cos(rjk, rc, pirc) + (T)1);
       const T f = fexp(-eta * r2) * fcjk;
       base = (rjk <= rc) ? base * f : (T)0;
     }
@@ -560,10 +620,11 @@ __device__ __forceinline__ bool adj_geom(const typename Vec4<T>::type& dj,
     dist_inv(r2, rjk, irjk);
     if (!(rjk <= rc)) return false;
     const T qq = pj.z * pk.z;
-    const T x = cutarg(rjk, pi, rc, pirc);
+    T cx, sx;
+    cut_cs(rjk, rc, pirc, cx, sx);
     const T ex = fexp(-eta * r2);
-    const T fc = (T)0.5 * qq * (fcos(x) + (T)1);
-    const T dfc = -(T)0.5 * qq * pirc * fsin(x);
+    const T fc = (T)0.5 * qq * (cx + (T)1);
+    const T dfc = -(T)0.5 * qq * pirc * sx;
     H = ex * fc;
     Hq = ex * (dfc - (T)2 * eta * rjk * fc) * irjk;
   }
@@ -572,7 +633,7 @@ __device__ __forceinline__ bool adj_geom(const typename Vec4<T>::type& dj,
 
 // Wave-uniform constants of a group's r_jk factor exp(-eta r^2) fc(r).  FP32: -eta log2(e) and
 // pi / (2 pi rc) prepared for v_exp_f32 (2^x) and v_cos_f32 / v_sin_f32 (argument in turns);
-// FP64: libm in the reference's operation order.
+// FP64: fexp and cut_cs.
 template <typename T> struct JkConst;
 template <> struct JkConst<float> {
   float rc, eta, pirc, el2, prev;
@@ -597,11 +658,9 @@ template <> struct JkConst<double> {
     eta = eta_;
     pirc = pirc_;
   }
-  __device__ __forceinline__ double ex(double r2) const { return exp(-eta * r2); }
+  __device__ __forceinline__ double ex(double r2) const { return fexp(-eta * r2); }
   __device__ __forceinline__ void cs(double r, double& c, double& sn) const {
-    const double x = kPi * r / rc;
-    c = cos(x);
-    sn = sin(x);
+    cut_cs(r, rc, pirc, c, sn);
   }
 };
 
@@ -1441,7 +1500,7 @@ __device__ __forceinline__ double radial_sum(const AcsfArgs& a, const Slice<T>& 
         fcv = (U)sl.fc[e];
       } else {
         const U qj = (U)ext_q(a.ext, a.next, fn.atomid, sl.j[e]);
-        fcv = (U)0.5 * qi * qj * (fcos(cutarg(r, pi, rc, pirc)) + (U)1);
+        fcv = (U)0.5 * qi * qj * (cut_cos(r, rc, pirc) + (U)1);
       }
       U term;
       if (fn.type == 1) term = fcv;
@@ -1488,7 +1547,7 @@ __device__ __forceinline__ void acsf_centre(const AcsfArgs& a, const long long i
     sl.d[pos] = d;
     sl.j[pos] = ADJ ? e : jj;  // adjoint: the entry's index in its row, for the output
     sl.zc[pos] = key < nZ ? key : -1;
-    if (!ADJ) sl.fc[pos] = (T)0.5 * (fcos(cutarg(d.w, pi, rcl, pircl)) + (T)1);
+    if (!ADJ) sl.fc[pos] = (T)0.5 * (cut_cos(d.w, rcl, pircl) + (T)1);
   };
   if (a.zone) {
     if (lane < 2) {
@@ -1626,8 +1685,9 @@ __device__ __forceinline__ void acsf_centre(const AcsfArgs& a, const long long i
         const int zc = sl.zc[e];
         const T r = d.w;
         // list-cutoff fc and fc' of the entry (recomputed rather than kept in LDS)
-        const T xl = cutarg(r, pi, rcl, pircl);
-        const T fcl = (T)0.5 * (fcos(xl) + (T)1), dfcl = -(T)0.5 * pircl * fsin(xl);
+        T cl, snl;
+        cut_cs(r, rcl, pircl, cl, snl);
+        const T fcl = (T)0.5 * (cl + (T)1), dfcl = -(T)0.5 * pircl * snl;
         T s = 0;
         for (int f = 0; f < a.nR; ++f) {
           // the whole record, held in scalar registers from here on (the empty asm takes every
@@ -1656,9 +1716,10 @@ __device__ __forceinline__ void acsf_centre(const AcsfArgs& a, const long long i
             const T pirc = pi / rc;
             const T qq = (T)(ext_q(a.ext, a.next, fn.atomid, i) *
                              ext_q(a.ext, a.next, fn.atomid, nbr(e)));
-            const T x = cutarg(r, pi, rc, pirc);
-            fc = (T)0.5 * qq * (fcos(x) + (T)1);
-            dfc = -(T)0.5 * qq * pirc * fsin(x);
+            T cx, sx;
+            cut_cs(r, rc, pirc, cx, sx);
+            fc = (T)0.5 * qq * (cx + (T)1);
+            dfc = -(T)0.5 * qq * pirc * sx;
           }
           T g;
           if (fn.type == 1) {
@@ -1732,18 +1793,20 @@ __device__ __forceinline__ void acsf_centre(const AcsfArgs& a, const long long i
           T fc, dfc;
           if (shared) {
             if (ADJ) {
-              const T x = cutarg(r, pi, rcl, pircl);
-              fc = (T)0.5 * (fcos(x) + (T)1);
-              dfc = -(T)0.5 * pircl * fsin(x);
+              T cx, sx;
+              cut_cs(r, rcl, pircl, cx, sx);
+              fc = (T)0.5 * (cx + (T)1);
+              dfc = -(T)0.5 * pircl * sx;
             } else {
               fc = sl.fc[e];
               dfc = 0;
             }
           } else {
             qj = (T)ext_q(a.ext, a.next, grp.atomid, nbr(e));
-            const T x = cutarg(r, pi, rc, pirc);
-            fc = (T)0.5 * qi * qj * (fcos(x) + (T)1);
-            dfc = -(T)0.5 * qi * qj * pirc * fsin(x);
+            T cx, sx;
+            cut_cs(r, rc, pirc, cx, sx);
+            fc = (T)0.5 * qi * qj * (cx + (T)1);
+            dfc = -(T)0.5 * qi * qj * pirc * sx;
           }
           const T ex = fexp(-eta * r * r);
           E = ex * fc;
@@ -1974,10 +2037,12 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8)))
   acsf_wave<float, false, 1, 1, PAIRS>(a);
 }
 
-// FP32 forward with the radial terms in FP64 (models with an ill-conditioned radial z-score)
-template <int MQ, int FORM>
+// FP32 forward with the radial terms in FP64 (models with an ill-conditioned radial z-score); 96
+// registers, 5 waves per SIMD (130 000 Si atoms, 12 G2 + 20 G5: 780 -> 570 us with the paired groups
+// in one walk and the polynomial exp and cos)
+template <int MQ, int FORM, bool PAIRS>
 __global__ void __launch_bounds__(512) k_acsf_fwd32_r64(AcsfArgs a) {
-  acsf_wave<float, false, MQ, FORM, false, true>(a);
+  acsf_wave<float, false, MQ, FORM, PAIRS, true>(a);
 }
 
 template <typename T, bool ADJ, int MQ, int FORM>
@@ -1988,10 +2053,10 @@ hipError_t launch_mq(fnet_batch* b, const DevModel& m, long long a0, long long a
   const Tune& tn = tune_of(b);
   const int M = slice_entries(b->max_nb);
   const size_t lmax = (size_t)b->ctx->lds_block;
-  // paired ladder groups share one walk when the larger slice still fits a block (the forward
-  // with an FP64 radial part and the persistent forward keep the unpaired kernels)
+  // paired ladder groups share one walk when the larger slice still fits a block (the persistent
+  // forward keeps the unpaired kernel)
   const int pairs = (FORM == 1 && m.has_pairs && slice_bytes<T, ADJ>(M, 1) <= lmax &&
-                     (ADJ || !(std::is_same<T, float>::value && (m.radial64 || tn.persist))))
+                     (ADJ || !(std::is_same<T, float>::value && tn.persist && !m.radial64)))
                         ? 1 : 0;
   const size_t sb = slice_bytes<T, ADJ>(M, pairs);
   // waves per block: the tuned value, else 1 (adjoint) / 2 (forward) (water boxes: adjoint
@@ -2059,12 +2124,14 @@ hipError_t launch_mq(fnet_batch* b, const DevModel& m, long long a0, long long a
   }
   if constexpr (!ADJ && FORM == 1) {
     if (pairs) {
-      if constexpr (std::is_same<T, float>::value) return go(k_acsf_lad32_fpairs<>, false);
+      if constexpr (std::is_same<T, float>::value)
+        return m.radial64 ? go(k_acsf_fwd32_r64<1, 1, true>, false)
+                          : go(k_acsf_lad32_fpairs<>, false);
       else return go(k_acsf<T, false, 1, 1, true>, false);
     }
   }
   if constexpr (!ADJ && std::is_same<T, float>::value) {
-    if (m.radial64) return go(k_acsf_fwd32_r64<MQ, FORM>, false);
+    if (m.radial64) return go(k_acsf_fwd32_r64<MQ, FORM, false>, false);
   }
   if constexpr (FORM == 1 && std::is_same<T, float>::value)
     return ps ? go(k_acsf_lad32_persist<ADJ>, true) : go(k_acsf_lad32<ADJ>, false);

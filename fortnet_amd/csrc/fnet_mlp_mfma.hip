@@ -937,8 +937,9 @@ hipError_t launch_mlp_grad_mfma(fnet_batch* b, const DevModel& m, hipStream_t s)
   return hipGetLastError();
 }
 
-// 16-atom parts up to which the waves of a block share one (SPLIT)
-constexpr long long kSplitTiles = 1024;
+// 16-atom parts up to which the waves of a block share one (SPLIT): 1132 parts 26.2 -> 24.7 us,
+// 2400 parts 27.1 -> 26.2 us; beyond that every CU has its fill of the other kind
+constexpr long long kSplitTiles = 2560;
 
 hipError_t launch_mlp_mfma(fnet_batch* b, const DevModel& m, int first_tile, int ntiles,
                            int want_grad_in, hipStream_t s, bool mirror,
