@@ -1481,12 +1481,13 @@ __device__ __forceinline__ void group_prog(CGroup& grp, const Slice<T>& sl, int 
 // far below its mean (R64, DevModel::radial64): the z-score divides G - mean by that sigma, and the FP32
 // sums' relative error (~4e-7 over a few dozen neighbours) would reach the network input, and
 // through it the forces, amplified by |mean| / sigma.  The FP32 distance is then widened exactly,
-// and the cutoff value is recomputed in FP64 instead of read from the FP32 slice.
+// and the list cutoff's values are FP64 too, one per entry in the place of the angular groups'
+// factors (pa), which are formed later.
 template <typename U, typename T>
 __device__ __forceinline__ double radial_sum(const AcsfArgs& a, const Slice<T>& sl,
                                              const RadialFn& fn, long long i, int e0, int e1,
                                              int step) {
-  const bool shared = std::is_same<U, T>::value && fn.rc == a.rclist && fn.atomid == 0;
+  const bool shared = fn.rc == a.rclist && fn.atomid == 0;
   const U pi = (U)kPi;
   const U rc = (U)fn.rc, eta = (U)fn.eta, rs = (U)fn.rs, kap = (U)fn.kappa;
   const U pirc = pi / rc;
@@ -1496,8 +1497,10 @@ __device__ __forceinline__ double radial_sum(const AcsfArgs& a, const Slice<T>& 
     const U r = (U)sl.d[e].w;
     if (r <= rc) {
       U fcv;
-      if (shared) {
+      if (shared && std::is_same<U, T>::value) {
         fcv = (U)sl.fc[e];
+      } else if (shared) {
+        fcv = (U)*(const double*)(sl.pa + e);
       } else {
         const U qj = (U)ext_q(a.ext, a.next, fn.atomid, sl.j[e]);
         fcv = (U)0.5 * qi * qj * (cut_cos(r, rc, pirc) + (U)1);
@@ -1616,6 +1619,12 @@ __device__ __forceinline__ void acsf_centre(const AcsfArgs& a, const long long i
 
     // ---- radial functions ----
     if (!ADJ) {
+      if constexpr (R64) {
+        for (int e = lane; e < n; e += 64)
+          *(double*)(sl.pa + e) =
+              0.5 * (cut_cos((double)sl.d[e].w, a.rclist, kPi / a.rclist) + 1.0);
+        wave_sync();
+      }
       // Lanes are (function, share of its element range) pairs.  When the functions fit one
       // wave and some are species-resolved, each gets lanes in proportion to the length of its
       // range (on the water boxes the H functions walk twice as many entries as the O ones:
