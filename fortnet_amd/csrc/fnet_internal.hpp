@@ -489,8 +489,16 @@ hipError_t launch_regularize(const DevModel& m, double* grad, double scale, doub
 hipError_t launch_sd_step(double* params, const double* grad, long long n, double lr,
                           double max_disp, double tol, double* scratch, int nspecies,
                           hipStream_t s);
-int mlp_tile_atoms(const NetShape& sh, int fp64);
+// atoms per generic tile of a batch of n_atoms
+int mlp_tile_atoms(const NetShape& sh, int fp64, long long n_atoms);
 int grad_chunks(int ntiles);  // chunks of the weight-gradient reduction
+
+// launchers (fnet_mlp_f64.hip): FP64 element networks on MFMA 16x16x4 f64.  Atoms per tile for a
+// batch of n_atoms (a multiple of 16), 0 if the network is too wide for a block's LDS
+int mlp_f64_tile_atoms(const NetShape& sh, long long n_atoms);
+hipError_t launch_mlp_f64(fnet_batch* b, const DevModel& m, int first_tile, int ntiles,
+                          int want_grad_in, hipStream_t s, bool mirror, unsigned long long* stamp);
+hipError_t launch_mlp_grad_f64(fnet_batch* b, const DevModel& m, hipStream_t s);
 
 // launchers (fnet_mlp_mfma.hip): FP32 element networks on MFMA 16x16x4 f32
 int mlp_mfma_waves(const NetShape& sh);  // waves per block, 0 if the shape is not supported

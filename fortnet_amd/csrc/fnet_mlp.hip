@@ -573,7 +573,9 @@ MlpArgs make_args(fnet_batch* b, const DevModel& m, int first_tile) {
 
 int grad_chunks(int ntiles) { return std::max(1, (ntiles + kGradChunk - 1) / kGradChunk); }
 
-int mlp_tile_atoms(const NetShape& sh, int fp64) {
+int mlp_tile_atoms(const NetShape& sh, int fp64, long long n_atoms) {
+  if (fp64)
+    if (const int ta = mlp_f64_tile_atoms(sh, n_atoms)) return ta;
   int TA = 64;
   while (TA > 1 && (fp64 ? host_lds<double>(sh, TA) : host_lds<float>(sh, TA)) > 64 * 1024) TA >>= 1;
   return TA;
@@ -583,6 +585,8 @@ hipError_t launch_mlp_fwd(fnet_batch* b, const DevModel& m, int first_tile, int 
                           int want_grad_in, hipStream_t s, bool mirror,
                           unsigned long long* stamp) {
   if (ntiles <= 0) return hipSuccess;
+  if (fp64 && mlp_f64_tile_atoms(m.shape, b->N))
+    return launch_mlp_f64(b, m, first_tile, ntiles, want_grad_in, s, mirror, stamp);
   auto go = [&](auto* grad, auto* plain, MlpArgs a, size_t lds) {
     a.ntiles = ntiles;
     a.stamp = stamp;
@@ -663,7 +667,10 @@ hipError_t launch_mlp_grad(fnet_batch* b, const DevModel& m, int fp64, double* g
     const hipError_t e = launch_mlp_grad_mfma(b, m, s);
     if (e != hipSuccess) return e;
   } else if (b->ntiles > 0) {
-    if (fp64) {
+    if (fp64 && mlp_f64_tile_atoms(m.shape, b->N)) {
+      const hipError_t e = launch_mlp_grad_f64(b, m, s);
+      if (e != hipSuccess) return e;
+    } else if (fp64) {
       MlpArgs a = make_args<double>(b, m, 0);
       a.grad = b->gpart;
       k_mlp_grad<double><<<b->ntiles, 256, host_lds<double>(m.shape, a.TA), s>>>(a);
