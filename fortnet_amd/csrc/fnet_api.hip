@@ -1877,11 +1877,11 @@ int fnet_train_gradients(fnet_ctx* ctx, fnet_batch* b, int n_global, const doubl
   rc = do_reduce(b);
   if (rc) return rc;
   hipStream_t s = ctx->stream;
-  // stage inputs: gt [S*ng], at [N*na], aw [N], dpw [S]; then the loss, a pad, the
-  // per-structure loss terms [2 S] and the per-chunk partial sums [3 nchunks]
+  // stage inputs: gt [S*ng], at [N*na], aw [N], dpw [S]; then the loss, a pad and the per-chunk
+  // partial sums [3 nchunks]
   const long long na = m.nout - n_global;
   const long long need =
-      (long long)b->S * n_global + b->N * na + b->N + 3LL * b->S + 3LL * b->nchunks + 4;
+      (long long)b->S * n_global + b->N * na + b->N + b->S + 3LL * b->nchunks + 4;
   if (need > b->targets_cap) {
     dfree(b->d_targets);
     b->d_targets = nullptr;
@@ -1905,8 +1905,10 @@ int fnet_train_gradients(fnet_ctx* ctx, fnet_batch* b, int n_global, const doubl
   }
   if (!(wsum > 0.0)) return fail(ctx, FNET_ERR_ARG, "datapoint weights sum to zero");
   HIPCHECK(ctx, stage_flush(ctx));
-  HIPCHECK(ctx, launch_lossgrad(b, m, n_global, gt, at, atomic_weights ? aw : nullptr,
-                                dp_weights ? dpw : nullptr, 1.0 / wsum, ctx->loss, s));
+  double* dloss = dpw + b->S;
+  const LossInput li = {n_global, ctx->loss, gt, at, atomic_weights ? aw : nullptr,
+                        dp_weights ? dpw : nullptr, 1.0 / wsum, dloss + 2, dloss};
+  HIPCHECK(ctx, launch_lossgrad(b, m, li, s));
   const long long np = m.shape.nparams * m.nspecies;
   if (np > ctx->grad_cap) {
     dfree(ctx->d_grad);
@@ -1926,13 +1928,9 @@ int fnet_train_gradients(fnet_ctx* ctx, fnet_batch* b, int n_global, const doubl
       b->gpart_len = need;
     }
   }
-  HIPCHECK(ctx, launch_mlp_grad(b, m, net64(b->precision), ctx->d_grad, s));
+  HIPCHECK(ctx, launch_mlp_grad(b, m, net64(b->precision), ctx->d_grad, li, s));
   if (ctx->reg_strength > 0.0)
     HIPCHECK(ctx, launch_regularize(m, ctx->d_grad, ctx->reg_strength / wsum, ctx->reg_alpha, s));
-  double* dloss = dpw + b->S;
-  HIPCHECK(ctx, launch_loss(b, m, n_global, gt, at, atomic_weights ? aw : nullptr,
-                            dp_weights ? dpw : nullptr, ctx->loss, dloss, dloss + 2,
-                            dloss + 2 + 2LL * b->S, s));
   double lv = 0.0;
   const bool host = b->host_E;  // a small batch's outputs are in pinned memory already
   const size_t npred = sizeof(double) * b->N * m.nout;

@@ -468,21 +468,29 @@ constexpr int kEnergyChunk = 2048;  // atoms per block of the energy reduction
 // host: also the pinned copies (longest row, energies of small batches)
 hipError_t launch_energy_reduce(fnet_batch* b, const DevModel& m, int s0, int s1, hipStream_t s,
                                 bool host = false);
-hipError_t launch_lossgrad(fnet_batch* b, const DevModel& m, int n_global, const double* gt,
-                           const double* at, const double* aw, const double* dpw, double inv_wsum,
-                           int loss, hipStream_t s);
-// weight gradient: per-tile partials into b->gpart, then their sum in tile order into grad
-hipError_t launch_mlp_grad(fnet_batch* b, const DevModel& m, int fp64, double* grad, hipStream_t s);
+// Training targets and weights on the device, and where the loss goes: part [3 nchunks] (per energy
+// chunk), out [1]
+struct LossInput {
+  int n_global, loss;
+  const double* gt;
+  const double* at;
+  const double* aw;   // null: 1
+  const double* dpw;  // null: 1
+  double inv_wsum;
+  double* part;
+  double* out;
+};
+// loss gradient of every atomic output and the loss of every chunk
+hipError_t launch_lossgrad(fnet_batch* b, const DevModel& m, const LossInput& in, hipStream_t s);
+// weight gradient: per-tile partials into b->gpart, then their sum in a fixed order into grad; with
+// it the loss, from the chunks of launch_lossgrad
+hipError_t launch_mlp_grad(fnet_batch* b, const DevModel& m, int fp64, double* grad,
+                           const LossInput& in, hipStream_t s);
 // number of weight-gradient partial vectors launch_mlp_grad writes into b->gpart
 int grad_parts(const fnet_batch* b, const DevModel& m, int fp64);
 // MFMA weight gradient (FP32 / BF16 modes): blocks per MFMA tile, 0 without an MFMA path
 int mlp_grad_subtiles(const NetShape& sh, int tile_waves);
 hipError_t launch_mlp_grad_mfma(fnet_batch* b, const DevModel& m, hipStream_t s);
-// loss into out[0]; scratch: terms [2 S] (per-structure loss and weight), part [3 nchunks]
-// (per energy chunk; the chunk tables of the energy reduction must be set up)
-hipError_t launch_loss(fnet_batch* b, const DevModel& m, int n_global, const double* gt,
-                       const double* at, const double* aw, const double* dpw, int loss,
-                       double* out, double* terms, double* part, hipStream_t s);
 // elastic-net term (scale = strength / sum of datapoint weights) added to the device gradient
 hipError_t launch_regularize(const DevModel& m, double* grad, double scale, double alpha,
                              hipStream_t s);

@@ -284,34 +284,79 @@ __global__ void __launch_bounds__(256) k_mlp_grad(MlpArgs a) {
   }
 }
 
-// grad[sp][k] = sum over the tiles of species sp, in tile order, of the tiles' partials, in two
-// fixed-order levels: chunks of kGradChunk tiles (one thread per (chunk, species, k)), then the
-// chunks in order.
+// grad[sp][k] = sum over the tiles of species sp of the tiles' partials, in fixed-order levels:
+// chunks of kGradChunk partials (four waves take a quarter each, in order, with all its loads in
+// flight; then the quarters), then the chunks in order.
 constexpr int kGradChunk = 64;
 
 // Partial t belongs to tile t / nsub (the MFMA path writes nsub FP32 partials per tile; their
 // values are FP32 sums, so FP32 storage loses nothing, and they are added in FP64 from here on).
+// One thread per value that walked a chunk's 64 partials one load after the other took 22 us.
 template <typename P>
-__global__ void k_grad_chunks(const P* __restrict__ gpart, const int* __restrict__ tile_sp,
-                              int nparts, int nsub, long long nparams, int nspecies,
-                              double* __restrict__ gchunk) {
-  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nparams * nspecies) return;
+__global__ void __launch_bounds__(256)
+    k_grad_chunks(const P* __restrict__ gpart, const int* __restrict__ tile_sp, int nparts,
+                  int nsub, long long nparams, int nspecies, double* __restrict__ gchunk) {
+  constexpr int kQuarter = kGradChunk / 4;
+  __shared__ double quarter[4][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const long long q = (long long)blockIdx.x * 64 + lane;
+  const bool in = q < nparams * nspecies;
   const int c = blockIdx.y;
-  const int sp = (int)(q / nparams);
-  const long long k = q - (long long)sp * nparams;
-  const int t0 = c * kGradChunk, t1 = min(nparts, t0 + kGradChunk);
+  const int sp = in ? (int)(q / nparams) : 0;
+  const long long k = in ? q - (long long)sp * nparams : 0;
+  const int t0 = c * kGradChunk + w * kQuarter;
+  P x[kQuarter];
+#pragma unroll
+  for (int u = 0; u < kQuarter; ++u) {
+    const int t = min(t0 + u, nparts - 1);
+    x[u] = gpart[(long long)t * nparams + k];
+  }
   double v = 0.0;
-  for (int t = t0; t < t1; ++t)
-    if (tile_sp[t / nsub] == sp) v += (double)gpart[(long long)t * nparams + k];
-  gchunk[(long long)c * nparams * nspecies + q] = v;
+#pragma unroll
+  for (int u = 0; u < kQuarter; ++u) {
+    const int t = t0 + u;
+    if (t < nparts && tile_sp[t / nsub] == sp) v += (double)x[u];
+  }
+  quarter[w][lane] = v;
+  __syncthreads();
+  if (w == 0 && in)
+    gchunk[(long long)c * nparams * nspecies + q] =
+        (quarter[0][lane] + quarter[1][lane]) + (quarter[2][lane] + quarter[3][lane]);
 }
 
-__global__ void k_grad_reduce(const double* __restrict__ gchunk, int nchunks, long long n,
-                              double* __restrict__ grad) {
+// The loss of a batch (launch_loss): inputs of the chunk kernel and of the sum over structures.
+struct LossArgs {
+  const double* Eatom;
+  const double* Estruct;
+  const long long* off;
+  const int* chunk_struct;
+  const int* chunk_first;
+  int S, nout, nglob, loss;
+  const double* gt;
+  const double* at;
+  const double* aw;
+  const double* dpw;
+  double inv_wsum;
+  double* part;      // [nchunks][3]
+  double* lossgrad;  // [N][nout]
+  double* out;
+};
+
+__device__ void loss_sum(const LossArgs& a);
+
+// The chunks in order, one thread per value; the last block sums the loss (it needs only the loss
+// chunks, and would be three launches of its own).
+__global__ void __launch_bounds__(256) k_grad_reduce(const double* __restrict__ gchunk, int nchunks,
+                                                     long long n, double* __restrict__ grad,
+                                                     LossArgs ls) {
+  if (blockIdx.x == gridDim.x - 1) {
+    loss_sum(ls);
+    return;
+  }
   const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= n) return;
   double v = 0.0;
+#pragma unroll 8
   for (int c = 0; c < nchunks; ++c) v += gchunk[(long long)c * n + q];
   grad[q] = v;
 }
@@ -339,28 +384,6 @@ __device__ __forceinline__ double loss_grad(int loss, double p, double t) {
   }
 }
 
-// Loss gradient of every atomic output with the sysTrain scaling (bpnn.F90:677-700) and the
-// datapoint weight / normalisation of updateGradients + update (bpnn.F90:445-448,766).
-__global__ void k_lossgrad(const double* __restrict__ Eatom, const double* __restrict__ Estruct,
-                           const int* __restrict__ atom_struct, const long long* __restrict__ off,
-                           long long N, int nout, int nglob, const double* __restrict__ gt,
-                           const double* __restrict__ at, const double* __restrict__ aw,
-                           const double* __restrict__ dpw, double inv_wsum, int loss,
-                           double* __restrict__ lg) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= N) return;
-  const int s = atom_struct[i];
-  const double natom = (double)(off[s + 1] - off[s]);
-  const double sc = (aw ? aw[i] : 1.0) / natom * (dpw ? dpw[s] : 1.0) * inv_wsum;
-  const int natomic = nout - nglob;
-  for (int t = 0; t < nout; ++t) {
-    double v;
-    if (t < nglob) v = loss_grad(loss, Estruct[(long long)s * nout + t], gt[(long long)s * nglob + t]);
-    else v = loss_grad(loss, Eatom[i * nout + t], at[i * natomic + (t - nglob)]);
-    lg[i * nout + t] = v * sc;
-  }
-}
-
 // Per-item loss of loss.F90:285-366 over the targets of one item (a datapoint's global targets
 // or one atom's atomic targets): mean (t - p)^2, mean |t - p|, 100 mean |(t - p) / t|, or the
 // root of the mean square.
@@ -374,43 +397,50 @@ __device__ __forceinline__ double item_loss(int loss, double sum_sq, double sum_
   }
 }
 
-// Loss of the batch (maLoss / mapLoss / msLoss / rmsLoss, loss.F90:370-700) in FP64: global
-// targets weighted by w_s * sum(atomic weights of s), atomic targets by w_s * atomic weight; the
-// result is divided by the summed weights.  Three fixed-order levels: k_loss_chunks sums each
-// 2048-atom chunk of the energy reduction (one block: thread t takes atoms t, t + 256, ... in
-// order, then a fixed tree) into (atomic loss, atomic weight, summed atomic weights);
-// k_loss_terms adds a structure's chunks in order and its global term; k_loss_sum adds the
-// structures (thread t takes t, t + 256, ..., then a fixed tree).
-__global__ void __launch_bounds__(256) k_loss_chunks(const double* __restrict__ Eatom,
-                                                     const long long* __restrict__ off,
-                                                     const int* __restrict__ chunk_struct,
-                                                     const int* __restrict__ chunk_first,
-                                                     int nout, int nglob,
-                                                     const double* __restrict__ at,
-                                                     const double* __restrict__ aw,
-                                                     const double* __restrict__ dpw, int loss,
-                                                     double* __restrict__ part) {
+// Loss gradient and loss of the batch in FP64.
+//
+// Gradient: of every atomic output with the sysTrain scaling (bpnn.F90:677-700) and the datapoint
+// weight / normalisation of updateGradients + update (bpnn.F90:445-448,766).
+//
+// Loss (maLoss / mapLoss / msLoss / rmsLoss, loss.F90:370-700): global targets weighted by w_s *
+// sum(atomic weights of s), atomic targets by w_s * atomic weight; the result is divided by the
+// summed weights.  Fixed-order levels: k_loss_chunks sums each 2048-atom chunk of the energy
+// reduction (one block: thread t takes atoms t, t + 256, ... in order, then a fixed tree) into
+// (atomic loss, atomic weight, summed atomic weights); loss_sum adds a structure's chunks in order
+// and its global term, and the structures (thread t takes t, t + 256, ..., then a fixed tree).
+__global__ void __launch_bounds__(256) k_loss_chunks(LossArgs a) {
   __shared__ double r0[256], r1[256], r2[256];
   const int c = blockIdx.x;
-  const int s = chunk_struct[c];
-  const long long a0 = off[s] + (long long)(c - chunk_first[s]) * kEnergyChunk;
-  const long long a1 = min(a0 + (long long)kEnergyChunk, off[s + 1]);
-  const double w = dpw ? dpw[s] : 1.0;
-  const int natomic = nout - nglob;
+  const int s = a.chunk_struct[c];
+  const long long o0 = a.off[s], o1 = a.off[s + 1];
+  const long long a0 = o0 + (long long)(c - a.chunk_first[s]) * kEnergyChunk;
+  const long long a1 = min(a0 + (long long)kEnergyChunk, o1);
+  const double w = a.dpw ? a.dpw[s] : 1.0;
+  const double natom = (double)(o1 - o0);
+  const int natomic = a.nout - a.nglob;
   double l = 0.0, nv = 0.0, saw = 0.0;
   for (long long i = a0 + threadIdx.x; i < a1; i += blockDim.x) {
-    const double awi = aw ? aw[i] : 1.0;
+    const double awi = a.aw ? a.aw[i] : 1.0;
     saw += awi;
+    const double sc = awi / natom * w * a.inv_wsum;
+    for (int t = 0; t < a.nout; ++t) {
+      double v;
+      if (t < a.nglob)
+        v = loss_grad(a.loss, a.Estruct[(long long)s * a.nout + t],
+                      a.gt[(long long)s * a.nglob + t]);
+      else v = loss_grad(a.loss, a.Eatom[i * a.nout + t], a.at[i * natomic + (t - a.nglob)]);
+      a.lossgrad[i * a.nout + t] = v * sc;
+    }
     if (natomic > 0) {
-      double q = 0.0, a = 0.0, r = 0.0;
+      double q = 0.0, ab = 0.0, r = 0.0;
       for (int o = 0; o < natomic; ++o) {
-        const double tv = at[i * natomic + o];
-        const double d = tv - Eatom[i * nout + nglob + o];
+        const double tv = a.at[i * natomic + o];
+        const double d = tv - a.Eatom[i * a.nout + a.nglob + o];
         q += d * d;
-        a += fabs(d);
+        ab += fabs(d);
         r += fabs(d / tv);
       }
-      l += w * awi * item_loss(loss, q, a, r, natomic);
+      l += w * awi * item_loss(a.loss, q, ab, r, natomic);
       nv += w * awi;
     }
   }
@@ -427,52 +457,41 @@ __global__ void __launch_bounds__(256) k_loss_chunks(const double* __restrict__ 
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    part[3 * (long long)c] = r0[0];
-    part[3 * (long long)c + 1] = r1[0];
-    part[3 * (long long)c + 2] = r2[0];
+    a.part[3 * (long long)c] = r0[0];
+    a.part[3 * (long long)c + 1] = r1[0];
+    a.part[3 * (long long)c + 2] = r2[0];
   }
 }
 
-__global__ void k_loss_terms(const double* __restrict__ Estruct,
-                             const int* __restrict__ chunk_first, int S, int nout, int nglob,
-                             const double* __restrict__ gt, const double* __restrict__ dpw,
-                             int loss, const double* __restrict__ part,
-                             double* __restrict__ terms) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= S) return;
-  double l = 0.0, nv = 0.0, saw = 0.0;
-  for (int c = chunk_first[s]; c < chunk_first[s + 1]; ++c) {
-    l += part[3 * (long long)c];
-    nv += part[3 * (long long)c + 1];
-    saw += part[3 * (long long)c + 2];
-  }
-  if (nglob > 0) {
-    const double w = dpw ? dpw[s] : 1.0;
-    double q = 0.0, a = 0.0, r = 0.0;
-    for (int o = 0; o < nglob; ++o) {
-      const double tv = gt[(long long)s * nglob + o];
-      const double d = tv - Estruct[(long long)s * nout + o];
-      q += d * d;
-      a += fabs(d);
-      r += fabs(d / tv);
-    }
-    l += w * saw * item_loss(loss, q, a, r, nglob);
-    nv += w * saw;
-  }
-  terms[2 * (long long)s] = l;
-  terms[2 * (long long)s + 1] = nv;
-}
-
-__global__ void __launch_bounds__(256) k_loss_sum(const double* __restrict__ terms, int S,
-                                                  double* __restrict__ out) {
+// by one block of 256 threads
+__device__ void loss_sum(const LossArgs& a) {
   __shared__ double rl[256], rn[256];
-  double l = 0.0, nv = 0.0;
-  for (int s = threadIdx.x; s < S; s += blockDim.x) {
-    l += terms[2 * (long long)s];
-    nv += terms[2 * (long long)s + 1];
+  double lt = 0.0, nt = 0.0;
+  for (int s = threadIdx.x; s < a.S; s += 256) {
+    double l = 0.0, nv = 0.0, saw = 0.0;
+    for (int c = a.chunk_first[s]; c < a.chunk_first[s + 1]; ++c) {
+      l += a.part[3 * (long long)c];
+      nv += a.part[3 * (long long)c + 1];
+      saw += a.part[3 * (long long)c + 2];
+    }
+    if (a.nglob > 0) {
+      const double w = a.dpw ? a.dpw[s] : 1.0;
+      double q = 0.0, ab = 0.0, r = 0.0;
+      for (int o = 0; o < a.nglob; ++o) {
+        const double tv = a.gt[(long long)s * a.nglob + o];
+        const double d = tv - a.Estruct[(long long)s * a.nout + o];
+        q += d * d;
+        ab += fabs(d);
+        r += fabs(d / tv);
+      }
+      l += w * saw * item_loss(a.loss, q, ab, r, a.nglob);
+      nv += w * saw;
+    }
+    lt += l;
+    nt += nv;
   }
-  rl[threadIdx.x] = l;
-  rn[threadIdx.x] = nv;
+  rl[threadIdx.x] = lt;
+  rn[threadIdx.x] = nt;
   __syncthreads();
   for (int st = 128; st > 0; st >>= 1) {
     if (threadIdx.x < st) {
@@ -481,7 +500,7 @@ __global__ void __launch_bounds__(256) k_loss_sum(const double* __restrict__ ter
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[0] = rl[0] / rn[0];
+  if (threadIdx.x == 0) a.out[0] = rl[0] / rn[0];
 }
 
 // Elastic-net term of the weight gradients (TWeightDerivs_elasticNetRegularization,
@@ -618,26 +637,31 @@ hipError_t launch_energy_reduce(fnet_batch* b, const DevModel& m, int s0, int s1
   return hipGetLastError();
 }
 
-hipError_t launch_lossgrad(fnet_batch* b, const DevModel& m, int n_global, const double* gt,
-                           const double* at, const double* aw, const double* dpw, double inv_wsum,
-                           int loss, hipStream_t s) {
-  if (b->N == 0) return hipSuccess;
-  k_lossgrad<<<(unsigned)((b->N + 255) / 256), 256, 0, s>>>(b->Eatom, b->Estruct, b->atom_struct,
-                                                            b->off, b->N, m.nout, n_global, gt, at,
-                                                            aw, dpw, inv_wsum, loss, b->lossgrad);
-  return hipGetLastError();
+static LossArgs loss_args(const fnet_batch* b, const DevModel& m, const LossInput& in) {
+  LossArgs a;
+  a.Eatom = b->Eatom;
+  a.Estruct = b->Estruct;
+  a.off = b->off;
+  a.chunk_struct = b->chunk_struct;
+  a.chunk_first = b->chunk_first;
+  a.S = b->S;
+  a.nout = m.nout;
+  a.nglob = in.n_global;
+  a.loss = in.loss;
+  a.gt = in.gt;
+  a.at = in.at;
+  a.aw = in.aw;
+  a.dpw = in.dpw;
+  a.inv_wsum = in.inv_wsum;
+  a.part = in.part;
+  a.lossgrad = b->lossgrad;
+  a.out = in.out;
+  return a;
 }
 
-hipError_t launch_loss(fnet_batch* b, const DevModel& m, int n_global, const double* gt,
-                       const double* at, const double* aw, const double* dpw, int loss,
-                       double* out, double* terms, double* part, hipStream_t s) {
-  if (b->nchunks > 0)
-    k_loss_chunks<<<b->nchunks, 256, 0, s>>>(b->Eatom, b->off, b->chunk_struct, b->chunk_first,
-                                             m.nout, n_global, at, aw, dpw, loss, part);
-  if (b->S > 0)
-    k_loss_terms<<<(b->S + 255) / 256, 256, 0, s>>>(b->Estruct, b->chunk_first, b->S, m.nout,
-                                                    n_global, gt, dpw, loss, part, terms);
-  k_loss_sum<<<1, 256, 0, s>>>(terms, b->S, out);
+hipError_t launch_lossgrad(fnet_batch* b, const DevModel& m, const LossInput& in, hipStream_t s) {
+  if (b->nchunks <= 0) return hipSuccess;
+  k_loss_chunks<<<b->nchunks, 256, 0, s>>>(loss_args(b, m, in));
   return hipGetLastError();
 }
 
@@ -659,7 +683,7 @@ int grad_parts(const fnet_batch* b, const DevModel& m, int fp64) {
 }
 
 hipError_t launch_mlp_grad(fnet_batch* b, const DevModel& m, int fp64, double* grad,
-                           hipStream_t s) {
+                           const LossInput& in, hipStream_t s) {
   const long long np = m.shape.nparams * m.nspecies;
   const int nsub = fp64 || !m.wpack ? 0 : mlp_grad_subtiles(m.shape, b->mtile_waves);
   const int nparts = nsub ? b->nmtiles * nsub : b->ntiles;
@@ -683,7 +707,7 @@ hipError_t launch_mlp_grad(fnet_batch* b, const DevModel& m, int fp64, double* g
   const int nchunks = grad_chunks(nparts);
   double* gchunk = b->gpart + (long long)std::max(nparts, 1) * m.shape.nparams;
   if (nparts > 0) {
-    const dim3 grid((unsigned)((np + 255) / 256), (unsigned)nchunks);
+    const dim3 grid((unsigned)((np + 63) / 64), (unsigned)nchunks);
     if (nsub)
       k_grad_chunks<float><<<grid, 256, 0, s>>>((const float*)b->gpart, b->mtile_sp, nparts, nsub,
                                                 m.shape.nparams, m.nspecies, gchunk);
@@ -691,8 +715,8 @@ hipError_t launch_mlp_grad(fnet_batch* b, const DevModel& m, int fp64, double* g
       k_grad_chunks<double><<<grid, 256, 0, s>>>(b->gpart, b->tile_sp, nparts, 1,
                                                  m.shape.nparams, m.nspecies, gchunk);
   }
-  k_grad_reduce<<<(unsigned)((np + 255) / 256), 256, 0, s>>>(gchunk, nparts > 0 ? nchunks : 0, np,
-                                                             grad);
+  k_grad_reduce<<<(unsigned)((np + 255) / 256) + 1, 256, 0, s>>>(
+      gchunk, nparts > 0 ? nchunks : 0, np, grad, loss_args(b, m, in));
   return hipGetLastError();
 }
 
