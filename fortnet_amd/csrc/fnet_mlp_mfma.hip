@@ -938,7 +938,10 @@ hipError_t launch_mlp_grad_mfma(fnet_batch* b, const DevModel& m, hipStream_t s)
 }
 
 // 16-atom parts up to which the waves of a block share one (SPLIT): 1132 parts 26.2 -> 24.7 us,
-// 2400 parts 27.1 -> 26.2 us; beyond that every CU has its fill of the other kind
+// 2400 parts 27.1 -> 26.2 us; beyond that every CU has its fill of the other kind (6000 parts of
+// 32-32-32: 26.7 -> 33 us).  Networks whose rows and f'(z) let fewer than four waves of their own into
+// 64 KB share at every size: the other kind has 6 waves on a CU there (130 000 atoms of 32-128-128-1 in
+// split BF16: 294 -> 178 us).
 constexpr long long kSplitTiles = 2560;
 
 hipError_t launch_mlp_mfma(fnet_batch* b, const DevModel& m, int first_tile, int ntiles,
@@ -984,7 +987,8 @@ hipError_t launch_mlp_mfma(fnet_batch* b, const DevModel& m, int first_tile, int
   a.nsub = waves;
   a.mr = mirror_args(b, 0, b->N);
   a.stamp = stamp;
-  const bool split = (long long)ntiles * waves <= kSplitTiles;
+  const bool split = (long long)ntiles * waves <= kSplitTiles ||
+                     4 * a.wave_floats * sizeof(float) > 64 * 1024;
   const int bw = split ? 4 : waves;  // waves per block
   a.ntiles = split ? ntiles * waves : ntiles;
   const size_t lds = (size_t)(split ? 1 : waves) * a.wave_floats * sizeof(float);
