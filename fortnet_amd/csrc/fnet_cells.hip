@@ -7,7 +7,7 @@
 // integer part of the fractional coordinates and sigma the periodic wrap of the stencil bin.
 // Candidates whose image lies outside the reference's image ranges (latpointiter.F90:226-253) are
 // dropped, as the reference never visits them; the rest pass the reference's FP64 distance test
-// (dynneighlist.F90:291-294).  The hits of one centre are then sorted in LDS by (lattice image in
+// (dynneighlist.F90:291-294).  The hits of one centre are then put in the order of (lattice image in
 // the reference's lexicographic order, (j - i) mod n), which is the order in which
 // TNeighIterator_getNextNeighbours (dynneighlist.F90:233-320) emits them.
 #include "fnet_device.hpp"
@@ -54,6 +54,15 @@ __global__ void k_cell_scatter(const int* __restrict__ atom_struct,
   cell_atoms[cell_start[c] + atomicSub(&cell_count[c], 1) - 1] = (int)i;
 }
 
+// Rows are put in order by ranks up to this capacity (m^2 / 64 broadcasts), by a bitonic network
+// beyond it.
+constexpr int kRankMax = 256;
+// LDS bytes per hit of the writing passes
+template <typename V>
+__host__ __device__ constexpr size_t hit_bytes(int K) {
+  return sizeof(V) + (K <= kRankMax ? 2 : 3) * sizeof(int);
+}
+
 struct CellArgs {
   const double* xyz;
   const long long* off;
@@ -95,13 +104,12 @@ __global__ void __launch_bounds__(256) k_neigh_cells(CellArgs a) {
   if (MODE == 2 && blockIdx.x == gridDim.x - 1 && lane == 0) stamp_now(a.t_end);
   if (!ci.w) return;
   const int K = a.K;
-  // LDS slice of this wave (fill pass only)
-  unsigned char* base = smem + (size_t)wave * K * (sizeof(unsigned long long) + 3 * sizeof(int) + sizeof(V));
-  unsigned long long* key = (unsigned long long*)base;
-  V* pnd = (V*)(key + K);
-  int* slot = (int*)(pnd + K);
-  int* pj = slot + K;
-  int* pimg = pj + K;
+  // LDS slice of this wave (writing passes only): displacement, neighbour and key of each hit, and
+  // for rows that are sorted rather than ranked the slots that move with the keys
+  V* pnd = (V*)(smem + (size_t)wave * K * hit_bytes<V>(K));
+  int* pj = (int*)(pnd + K);
+  int* key = pj + K;
+  int* slot = key + K;
 
   const StructInfo& si = a.sinfo[s];
   const long long o = a.off[s];
@@ -158,9 +166,9 @@ __global__ void __launch_bounds__(256) k_neigh_cells(CellArgs a) {
     const int c0 = __shfl(bc0, bb, 64), e0b = __shfl(bex, bb, 64), sg = __shfl(bsg, bb, 64);
     const int s0 = sg / 9 - 1, s1 = (sg / 3) % 3 - 1, s2 = sg % 3 - 1;
     bool hit = false;
-    int lj = 0, img = -1;
+    int lj = 0;
     double nd0 = 0, nd1 = 0, nd2 = 0, dd = 0;
-    unsigned long long k = 0;
+    int k = 0;
     if (p < total) {
       const int j = a.cell_atoms[c0 + (p - e0b)];
       lj = (int)(j - o);
@@ -195,10 +203,9 @@ __global__ void __launch_bounds__(256) k_neigh_cells(CellArgs a) {
           lex = ((n0 - si.lo[0]) * N1 + (n1 - si.lo[1])) * N2 + (n2 - si.lo[2]);
           if (lex > origin) lex -= 1;
         }
-        img = lex;
         int t = lj - li;
         if (t < 0) t += n;
-        k = (unsigned long long)(lex + 1) * (unsigned long long)n + (unsigned long long)t;
+        k = (lex + 1) * n + t;  // below 2^31 (checked when the lattice is loaded)
       }
     }
     const unsigned long long mask = __ballot(hit);
@@ -206,7 +213,6 @@ __global__ void __launch_bounds__(256) k_neigh_cells(CellArgs a) {
       const int q = count + __popcll(mask & lanemask_lt(lane));
       if (q < K) {
         key[q] = k;
-        slot[q] = q;
         pj[q] = (int)(o + lj);
         V v;
         v.x = nd0;
@@ -223,8 +229,40 @@ __global__ void __launch_bounds__(256) k_neigh_cells(CellArgs a) {
     return;
   }
   const int m = count < K ? count : K;
-  for (int e = m + lane; e < K; e += 64) {
-    key[e] = ~0ull;
+  const long long rb = MODE == 2 ? i * a.cap : (long long)a.rowptr[i];
+  const int mw = MODE == 2 ? (m < a.cap ? m : a.cap) : m;
+  if (MODE == 2 && lane == 0) {
+    a.cnt[i] = count;
+    raise_max(a.maxnb, count);
+  }
+  V* out = (V*)a.nd;
+  // hit q of the LDS list goes to place e of the row
+  auto put = [&](int q, int e, int k) {
+    a.nj[rb + e] = pj[q];
+    a.nimg[rb + e] = k;  // the entry's key (image + 1) n + (j - i) mod n
+    out[rb + e] = pnd[q];
+    if (MODE == 2 && a.mir) a.mir[rb + e] = -1;
+  };
+  wave_sync();
+  if (K <= kRankMax) {
+    // a hit's place is the number of smaller keys (the keys of a row differ): every key is broadcast
+    // to the wave once for each 64 hits.  A row of 45 takes 45 broadcasts, compares and adds; the
+    // bitonic network on 128 slots took 28 rounds through LDS (130 000 Si atoms: search 460 -> 322 us).
+    for (int q0 = 0; q0 < m; q0 += 64) {
+      const int q = q0 + lane;
+      const int mine = q < m ? key[q] : 0;
+      int rank = 0;
+      for (int c0 = 0; c0 < m; c0 += 64) {
+        const int theirs = c0 + lane < m ? key[c0 + lane] : 0;
+        const int nc = min(64, m - c0);
+        for (int l = 0; l < nc; ++l) rank += __builtin_amdgcn_readlane(theirs, l) < mine ? 1 : 0;
+      }
+      if (q < m && rank < mw) put(q, rank, mine);
+    }
+    return;
+  }
+  for (int e = lane; e < K; e += 64) {
+    if (e >= m) key[e] = 0x7fffffff;
     slot[e] = e;
   }
   wave_sync();
@@ -235,7 +273,7 @@ __global__ void __launch_bounds__(256) k_neigh_cells(CellArgs a) {
         const int x = e ^ jj;
         if (x > e) {
           const bool up = (e & kk) == 0;
-          const unsigned long long ke = key[e], kx = key[x];
+          const int ke = key[e], kx = key[x];
           if ((ke > kx) == up) {
             key[e] = kx;
             key[x] = ke;
@@ -248,20 +286,7 @@ __global__ void __launch_bounds__(256) k_neigh_cells(CellArgs a) {
       wave_sync();
     }
   }
-  const long long rb = MODE == 2 ? i * a.cap : (long long)a.rowptr[i];
-  const int mw = MODE == 2 ? (m < a.cap ? m : a.cap) : m;
-  if (MODE == 2 && lane == 0) {
-    a.cnt[i] = count;
-    raise_max(a.maxnb, count);
-  }
-  V* out = (V*)a.nd;
-  for (int e = lane; e < mw; e += 64) {
-    const int q = slot[e];
-    a.nj[rb + e] = pj[q];
-    a.nimg[rb + e] = (int)key[e];  // the entry's key (image + 1) n + (j - i) mod n
-    out[rb + e] = pnd[q];
-    if (MODE == 2 && a.mir) a.mir[rb + e] = -1;
-  }
+  for (int e = lane; e < mw; e += 64) put(slot[e], e, key[e]);
 }
 
 template <int MODE, typename V>
@@ -298,7 +323,7 @@ hipError_t launch_cells_t(fnet_batch* b, double rc, long long a0, long long a1, 
   size_t lds = 0;
   int wpb = 4;
   if (WRITE) {
-    const size_t per = (size_t)K * (sizeof(unsigned long long) + 3 * sizeof(int) + sizeof(V));
+    const size_t per = (size_t)K * hit_bytes<V>(K);
     while (wpb > 1 && per * wpb > 64 * 1024) wpb >>= 1;
     if (per * wpb > (size_t)b->ctx->lds_block) return hipErrorInvalidConfiguration;
     lds = per * wpb;
@@ -329,8 +354,8 @@ int cells_sort_capacity(int need) {
 }
 
 size_t cells_lds_bytes(int need, int fp64) {
-  const size_t v = fp64 ? sizeof(double4) : sizeof(float4);
-  return (size_t)cells_sort_capacity(need) * (sizeof(unsigned long long) + 3 * sizeof(int) + v);
+  const int K = cells_sort_capacity(need);
+  return (size_t)K * (fp64 ? hit_bytes<double4>(K) : hit_bytes<float4>(K));
 }
 
 hipError_t launch_cells_count(fnet_batch* b, double rc, long long a0, long long a1,
