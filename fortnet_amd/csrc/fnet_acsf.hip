@@ -1520,7 +1520,10 @@ __device__ __forceinline__ double radial_sum(const AcsfArgs& a, const Slice<T>& 
 // PAIRS (ladder groups only): paired groups are evaluated together (own instance, so
 // that the kernels of models without pairs keep their register budget).  R64 (FP32 forward
 // only): radial terms in FP64 (radial_sum), also an instance of its own.
-template <typename T, bool ADJ, int MQ, int FORM, bool PAIRS, bool R64 = false>
+// SPLIT: the block's waves share the centre, each with a slice of its own: wave 0 takes the radial
+// functions, the angular groups are dealt to the waves in turn, and the adjoint adds the waves'
+// entry gradients at the end.
+template <typename T, bool ADJ, int MQ, int FORM, bool PAIRS, bool R64 = false, bool SPLIT = false>
 __device__ __forceinline__ void acsf_centre(const AcsfArgs& a, const long long i) {
   using V = typename Vec4<T>::type;
   extern __shared__ __align__(32) unsigned char smem[];
@@ -1618,7 +1621,12 @@ __device__ __forceinline__ void acsf_centre(const AcsfArgs& a, const long long i
     cdouble* cG = ADJ ? (cdouble*)a.cG + (i * a.nout + t) * a.nG : nullptr;
 
     // ---- radial functions ----
-    if (!ADJ) {
+    if (SPLIT && wave != 0) {
+      if (ADJ) {
+        for (int e = lane; e < 3 * n; e += 64) sl.gs[e] = 0.0;
+        wave_sync();
+      }
+    } else if (!ADJ) {
       if constexpr (R64) {
         for (int e = lane; e < n; e += 64)
           *(double*)(sl.pa + e) =
@@ -1751,11 +1759,15 @@ __device__ __forceinline__ void acsf_centre(const AcsfArgs& a, const long long i
     }
 
     // ---- angular groups ----
+    int unit = 0;  // SPLIT: shares of the centre dealt so far (0: the radial functions)
     for (int g = 0; g < a.nAG; ++g) {
       CGroup& grp = ((CGroup*)a.groups)[g];
       const int nm = grp.nmem;
-      if constexpr (PAIRS && !ADJ) {
+      if constexpr (PAIRS && (!ADJ || SPLIT)) {
         if (grp.follower) continue;  // evaluated together with its partner
+      }
+      if constexpr (SPLIT) {
+        if (++unit % (int)(blockDim.x >> 6) != wave) continue;
       }
       T A[FORM ? 1 : MQ];
       if (ADJ) {
@@ -1949,7 +1961,18 @@ __device__ __forceinline__ void acsf_centre(const AcsfArgs& a, const long long i
     // the entry's mirror, in the neighbour's own row, so that the gather reads its row
     // contiguously instead of one scattered 24-byte record per entry.  The centre side (+sum of
     // the centre's entries) is written here.
-    if (ADJ) {
+    if constexpr (ADJ && SPLIT) {
+      __syncthreads();
+      if (wave == 0) {
+        const long long slice = slice_bytes<T, ADJ>(M, PAIRS);
+        for (int w = 1; w < (int)(blockDim.x >> 6); ++w) {
+          lds_f64* gw = (lds_f64*)((__attribute__((address_space(3))) unsigned char*)sl.gs + slice * w);
+          for (int e = lane; e < 3 * n; e += 64) sl.gs[e] += gw[e];
+        }
+        wave_sync();
+      }
+    }
+    if (ADJ && (!SPLIT || wave == 0)) {
       double sx = 0, sy = 0, sz = 0;
       for (int e0 = 0; e0 < n; e0 += 64) {
         const int e = e0 + lane;
@@ -1982,6 +2005,9 @@ __device__ __forceinline__ void acsf_centre(const AcsfArgs& a, const long long i
       if ((lane & 15) == 0 && c < 3) a.F[(i * a.nout + t) * 3 + c] = sc;
       wave_sync();
     }
+    if constexpr (ADJ && SPLIT) {
+      if (t + 1 < nouts) __syncthreads();  // wave 0 has read the others' slices
+    }
   }
 }
 
@@ -2008,6 +2034,16 @@ __device__ __forceinline__ void acsf_wave(const AcsfArgs& a) {
       wave_sync();
     }
   }
+}
+
+// The waves of a block share one centre (SPLIT of acsf_centre).
+template <typename T, bool ADJ, int MQ, int FORM, bool PAIRS, bool R64>
+__global__ void __launch_bounds__(512) k_acsf_split(AcsfArgs a) {
+  if constexpr (ADJ) {
+    stamp(a.stamp);
+    if (a.norph && blockIdx.x == 0 && threadIdx.x == 0) *a.norph = 0;
+  }
+  acsf_centre<T, ADJ, MQ, FORM, PAIRS, R64, true>(a, a.a0 + blockIdx.x);
 }
 
 template <typename T, bool ADJ, int MQ, int FORM, bool PAIRS>
@@ -2053,6 +2089,14 @@ template <int MQ, int FORM, bool PAIRS>
 __global__ void __launch_bounds__(512) k_acsf_fwd32_r64(AcsfArgs a) {
   acsf_wave<float, false, MQ, FORM, PAIRS, true>(a);
 }
+
+// Waves up to which a batch's centres are split, eight for each SIMD: a wave's serial chain over all
+// functions bounds a small launch (192 water atoms: forward 38 -> 18 us, adjoint 60 -> 28 us; 209
+// serving atoms 21 -> 10 and 31 -> 14 us), and with up to 4096 centres the launch is still short of
+// waves.  Against 2048: 3072 atoms of an FP64 force call 494 -> 449 us, a serving batch
+// 572 -> 574 us; with 32768 the doubled staging shows (the same calls 472 and 600 us, FP64 features
+// of 9600 atoms 234 -> 261 us).
+constexpr long long kSplitWaves = 8192;
 
 template <typename T, bool ADJ, int MQ, int FORM>
 hipError_t launch_mq(fnet_batch* b, const DevModel& m, long long a0, long long a1,
@@ -2123,6 +2167,30 @@ hipError_t launch_mq(fnet_batch* b, const DevModel& m, long long a0, long long a
     hipLaunchKernelGGL(kern, dim3(g), dim3(64 * wpb), lds, s, a);
     return hipGetLastError();
   };
+  // A batch of few centres gives each several waves: one for the radial functions and one for each
+  // angular group (the forward takes paired groups one by one then, with the same sums).  A grid this small is
+  // resident at once, persistent or not.
+  if constexpr (FORM == 1) {
+    const int units = 1 + m.nAG - (ADJ && pairs ? m.n_followers : 0);
+    const size_t ssb = slice_bytes<T, ADJ>(M, ADJ ? pairs : 0);
+    int w = (int)std::min<long long>(std::min(units, 8), kSplitWaves / n);
+    while (w > 1 && ssb * w > 64 * 1024) --w;
+    if (w > 1) {
+      auto split = [&](void (*kern)(AcsfArgs)) -> hipError_t {
+        hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(64 * w), ssb * w, s, a);
+        return hipGetLastError();
+      };
+      if constexpr (ADJ) {
+        return pairs ? split(k_acsf_split<T, true, 1, 1, true, false>)
+                     : split(k_acsf_split<T, true, 1, 1, false, false>);
+      } else if constexpr (std::is_same<T, float>::value) {
+        return m.radial64 ? split(k_acsf_split<T, false, 1, 1, false, true>)
+                          : split(k_acsf_split<T, false, 1, 1, false, false>);
+      } else {
+        return split(k_acsf_split<T, false, 1, 1, false, false>);
+      }
+    }
+  }
   const bool ps = a.persist != 0;
   if constexpr (ADJ && FORM == 1) {
     if (pairs) {

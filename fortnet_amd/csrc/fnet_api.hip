@@ -1182,6 +1182,7 @@ int fnet_model_upload(fnet_ctx* ctx, const fnet_model_desc* md) {
       a.partner = (int)q;
       b.follower = 1;
       m.has_pairs = 1;
+      m.n_followers++;
       break;
     }
   }

@@ -116,6 +116,7 @@ struct DevModel {
                                 // progressions, 0 some group has neither
   int maxprog = 0;              // longest progression
   int has_pairs = 0;            // some angular groups are evaluated in pairs by the adjoint
+  int n_followers = 0;          // ... second groups of them
   int radial_resolved = 0;      // some radial function is restricted to one neighbour element
   int radial64 = 0;             // FP32 modes sum the radial functions in FP64 (kRadial64Kappa)
   int need_ext = 0;             // external feature columns the model reads
