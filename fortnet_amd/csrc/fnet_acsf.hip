@@ -216,6 +216,10 @@ __device__ __forceinline__ int wave_excl_scan_i(int v, int lane) {
   return x - v;
 }
 
+// x clamped to [-1, 1] (FP32: one v_med3_f32 in place of a maximum and a minimum)
+__device__ __forceinline__ float clamp1(float x) { return __builtin_amdgcn_fmed3f(x, -1.0f, 1.0f); }
+__device__ __forceinline__ double clamp1(double x) { return fmin(fmax(x, -1.0), 1.0); }
+
 // cos(theta) of an off-diagonal pair in the G4/G5 values, clamped to [-1, 1].  FP64 follows the
 // reference's value formula dot / (r_j r_k + 1e-13) (theta, acsf.F90:1159-1176; its
 // cos(acos(x)) round trip moves x by about an ulp): the regulariser lowers every cosine by a
@@ -224,12 +228,12 @@ __device__ __forceinline__ int wave_excl_scan_i(int v, int lane) {
 template <typename V>
 __device__ __forceinline__ float value_cos(const V& dj, const V& dk, float irj, float irk) {
   const float c = (dj.x * dk.x + dj.y * dk.y + dj.z * dk.z) * irj * irk;
-  return fminf(fmaxf(c, -1.0f), 1.0f);
+  return clamp1(c);
 }
 template <typename V>
 __device__ __forceinline__ double value_cos(const V& dj, const V& dk, double irj, double irk) {
   const double c = (dj.x * dk.x + dj.y * dk.y + dj.z * dk.z) / (dj.w * dk.w + 1e-13);
-  return fmin(fmax(c, -1.0), 1.0);
+  return clamp1(c);
 }
 
 // cos(theta) of the j == k term of a value: 1 in FP32; in FP64 the reference's
@@ -610,7 +614,7 @@ __device__ __forceinline__ bool adj_geom(const typename Vec4<T>::type& dj,
                                          const typename Vec4<T>::type& pk, T rc, T eta, T pi,
                                          T pirc, T& rr, T& c, T& H, T& Hq) {
   rr = pj.x * pk.x;
-  c = fmin(fmax((dj.x * dk.x + dj.y * dk.y + dj.z * dk.z) * rr, (T)-1), (T)1);
+  c = clamp1((dj.x * dk.x + dj.y * dk.y + dj.z * dk.z) * rr);
   H = 1;
   Hq = 0;
   if (G4) {
@@ -675,7 +679,7 @@ __device__ __forceinline__ void adj_geom_sel(const typename Vec4<T>::type& dj,
                                              const JkConst<T>& K, bool v, T& rr, T& c, T& H,
                                              T& Hq) {
   rr = pj.x * pk.x;
-  c = fmin(fmax((dj.x * dk.x + dj.y * dk.y + dj.z * dk.z) * rr, (T)-1), (T)1);
+  c = clamp1((dj.x * dk.x + dj.y * dk.y + dj.z * dk.z) * rr);
   H = v ? (T)1 : (T)0;
   Hq = 0;
   if (G4) {
@@ -733,6 +737,62 @@ __device__ __forceinline__ void adj_scatter(const Slice<T>& sl, int ej, int ek,
   lds_add(gk + 0, (double)(Pk * dk.x + Q * dj.x));
   lds_add(gk + 1, (double)(Pk * dk.y + Q * dj.y));
   lds_add(gk + 2, (double)(Pk * dk.z + Q * dj.z));
+}
+
+// adj_coef / adj_scatter for two pairs that share j (the walks with two offsets per step): the j
+// side is summed over them and the factors of j alone are applied once,
+//   g_j = (E'_j / r_j sum U E_k + sum h - sum(c t) / r_j^2) d_j + sum Q d_k,
+// and the ladder takes c0 P^(2^m) as P (c0 P^(2^m - 1)) from the powers the derivative needs: the
+// loops are bound by their vector instructions with the LDS close behind (95 % and 83 % busy in
+// the paired G5 loop), and lose 4 to 8 % of them here (two pairs of xi = 1 ... 8, two etas
+// 222 -> 210, of G4 xi = 1, 4 210 -> 201).  38 400 water atoms 797 -> 788 us in the adjoint, whole
+// step 1525 -> 1505; three pairs to a j were slower (fewer waves; 131 072 Si atoms 2155 -> 2195).
+template <typename T>
+struct JSide {
+  T ue = 0, h = 0, ct = 0, x = 0, y = 0, z = 0;
+};
+
+// One pair: its k side to the accumulator of ek, its j side to js.
+template <typename T, bool G4>
+__device__ __forceinline__ void adj_pair(const Slice<T>& sl, int ek,
+                                         const typename Vec4<T>::type& dj,
+                                         const typename Vec4<T>::type& pj,
+                                         const typename Vec4<T>::type& dk,
+                                         const typename Vec4<T>::type& pk, T rr, T c, T H, T Hq,
+                                         bool v, T S0, T S1, JSide<T>& js) {
+  const T EE = pj.y * pk.y;
+  T t, U, h = 0;
+  if (G4) {
+    t = S1 * EE * H;
+    U = S0 * H;
+    h = S0 * EE * Hq;
+  } else {
+    t = v ? S1 * EE : (T)0;
+    U = v ? S0 : (T)0;
+  }
+  const T Q = G4 ? t * rr - h : t * rr;
+  const T ct = c * t;
+  js.ue += U * pk.y;
+  js.ct += ct;
+  if (G4) js.h += h;
+  js.x += Q * dk.x;
+  js.y += Q * dk.y;
+  js.z += Q * dk.z;
+  const T Pk = U * pj.y * pk.w + h - ct * (pk.x * pk.x);
+  lds_f64* gk = sl.gs + __umul24(ek, 3);
+  lds_add(gk + 0, (double)(Pk * dk.x + Q * dj.x));
+  lds_add(gk + 1, (double)(Pk * dk.y + Q * dj.y));
+  lds_add(gk + 2, (double)(Pk * dk.z + Q * dj.z));
+}
+
+// The j side with coefficient P of d_j.
+template <typename T>
+__device__ __forceinline__ void adj_j(const Slice<T>& sl, int ej,
+                                      const typename Vec4<T>::type& dj, T P, const JSide<T>& js) {
+  lds_f64* gj = sl.gs + __umul24(ej, 3);
+  lds_add(gj + 0, (double)(P * dj.x + js.x));
+  lds_add(gj + 1, (double)(P * dj.y + js.y));
+  lds_add(gj + 2, (double)(P * dj.z + js.z));
 }
 
 // Adjoint: off-diagonal pairs of one group, gradients accumulated per entry in sl.gs.
@@ -886,46 +946,35 @@ __device__ __forceinline__ void pairs_adj_lad(const Slice<T>& sl, int lane, int 
   it.init(lane, A0, LA, B0, LB);
   int ej, ek1, ek2;
   bool v1, v2;
-  // one pair: adds its k-side gradient to the accumulator of ek, returns the j-side in g
-  auto pair = [&](const V& dj, const V& pj, int ek, bool v, T& gx, T& gy, T& gz) {
+  auto pair = [&](const V& dj, const V& pj, int ek, bool v, JSide<T>& js) {
     const V dk = sl.d[ek], pk = sl.pa[ek];
     T rr, c, H, Hq;
     adj_geom_sel<T, G4>(dj, dk, pj, pk, K, v, rr, c, H, Hq);
+    // sum of c0 P^(2^m) as P times the sum of c0 P^(2^m - 1), whose powers S1 needs
     T S0 = 0, S1 = c1const;
 #pragma unroll
     for (int l = 0; l < 2; ++l) {
-      T p = (T)1 + (l ? lam1 : lam0) * c;
-      T pm = (T)1;
-      if (MASK & 1) S0 += c0[l][0] * p;
+      const T P = (T)1 + (l ? lam1 : lam0) * c;
+      T p = P, pm = (T)1, s = MASK & 1 ? c0[l][0] : (T)0;
 #pragma unroll
       for (int m = 1; m <= MX; ++m) {
         pm = pm * p;
         p = p * p;
         if (MASK & (1 << m)) {
-          S0 += c0[l][m] * p;
+          s += c0[l][m] * pm;
           S1 += c1[l][m] * pm;
         }
       }
+      S0 += P * s;
     }
-    T Pj, Pk, Q;
-    adj_coef<T, G4>(pj, pk, rr, c, H, Hq, S0, S1, Pj, Pk, Q);
-    gx += Pj * dj.x + Q * dk.x;
-    gy += Pj * dj.y + Q * dk.y;
-    gz += Pj * dj.z + Q * dk.z;
-    lds_f64* gk = sl.gs + __umul24(ek, 3);
-    lds_add(gk + 0, (double)(Pk * dk.x + Q * dj.x));
-    lds_add(gk + 1, (double)(Pk * dk.y + Q * dj.y));
-    lds_add(gk + 2, (double)(Pk * dk.z + Q * dj.z));
+    adj_pair<T, G4>(sl, ek, dj, pj, dk, pk, rr, c, H, Hq, v, S0, S1, js);
   };
   while (it.next(ej, ek1, ek2, v1, v2)) {
     const V dj = sl.d[ej], pj = sl.pa[ej];
-    T gx = 0, gy = 0, gz = 0;
-    pair(dj, pj, ek1, v1, gx, gy, gz);
-    pair(dj, pj, ek2, v2, gx, gy, gz);
-    lds_f64* gj = sl.gs + __umul24(ej, 3);
-    lds_add(gj + 0, (double)gx);
-    lds_add(gj + 1, (double)gy);
-    lds_add(gj + 2, (double)gz);
+    JSide<T> js;
+    pair(dj, pj, ek1, v1, js);
+    pair(dj, pj, ek2, v2, js);
+    adj_j(sl, ej, dj, js.ue * pj.w + js.h - js.ct * (pj.x * pj.x), js);
   }
 }
 
@@ -1144,62 +1193,57 @@ __device__ __forceinline__ void pairs_adj_lad2(const Slice<T>& sl, int lane, int
                                                const T (&c1)[2][2][MX + 1],
                                                const T (&c1const)[2]) {
   using V = typename Vec4<T>::type;
-  PairWalk2<SAME> it;
-  it.init(lane, A0, LA, B0, LB);
-  int ej, ek1, ek2;
-  bool v1, v2;
-  auto pair = [&](const V& dj, const V& pj, const V& qj, int ek, bool v, T& gx, T& gy, T& gz) {
+  auto pair = [&](const V& dj, const V& pj, const V& qj, int ek, bool v, JSide<T>& js) {
     const V dk = sl.d[ek], pk = sl.pa[ek], qk = sl.pb[ek];
     const T rr = pj.x * pk.x;
-    const T c = fmin(fmax((dj.x * dk.x + dj.y * dk.y + dj.z * dk.z) * rr, (T)-1), (T)1);
+    const T c = clamp1((dj.x * dk.x + dj.y * dk.y + dj.z * dk.z) * rr);
     T S0a = 0, S1a = c1const[0], S0b = 0, S1b = c1const[1];
 #pragma unroll
     for (int l = 0; l < 2; ++l) {
-      T p = (T)1 + (l ? lam1 : lam0) * c;
-      T pm = (T)1;
-      if (MASK & 1) {
-        S0a += c0[0][l][0] * p;
-        S0b += c0[1][l][0] * p;
-      }
+      const T P = (T)1 + (l ? lam1 : lam0) * c;
+      T p = P, pm = (T)1, sa = MASK & 1 ? c0[0][l][0] : (T)0, sb = MASK & 1 ? c0[1][l][0] : (T)0;
 #pragma unroll
       for (int m = 1; m <= MX; ++m) {
         pm = pm * p;
         p = p * p;
         if (MASK & (1 << m)) {
-          S0a += c0[0][l][m] * p;
+          sa += c0[0][l][m] * pm;
           S1a += c1[0][l][m] * pm;
-          S0b += c0[1][l][m] * p;
+          sb += c0[1][l][m] * pm;
           S1b += c1[1][l][m] * pm;
         }
       }
+      S0a += P * sa;
+      S0b += P * sb;
     }
     // a pair that does not exist adds nothing
     S0a = v ? S0a : (T)0;
-    S1a = v ? S1a : (T)0;
     S0b = v ? S0b : (T)0;
-    S1b = v ? S1b : (T)0;
-    const T t = S1a * (pj.y * pk.y) + S1b * (qj.y * qk.y);
+    const T t = v ? S1a * (pj.y * pk.y) + S1b * (qj.y * qk.y) : (T)0;
     const T Q = t * rr;
     const T ct = c * t;
-    const T Pj = S0a * pk.y * pj.w + S0b * qk.y * qj.w - ct * (pj.x * pj.x);
+    js.ue += S0a * pk.y;
+    js.h += S0b * qk.y;  // (G5 has no h: the sum of the partner)
+    js.ct += ct;
+    js.x += Q * dk.x;
+    js.y += Q * dk.y;
+    js.z += Q * dk.z;
     const T Pk = S0a * pj.y * pk.w + S0b * qj.y * qk.w - ct * (pk.x * pk.x);
-    gx += Pj * dj.x + Q * dk.x;
-    gy += Pj * dj.y + Q * dk.y;
-    gz += Pj * dj.z + Q * dk.z;
     lds_f64* gk = sl.gs + __umul24(ek, 3);
     lds_add(gk + 0, (double)(Pk * dk.x + Q * dj.x));
     lds_add(gk + 1, (double)(Pk * dk.y + Q * dj.y));
     lds_add(gk + 2, (double)(Pk * dk.z + Q * dj.z));
   };
+  PairWalk2<SAME> it;
+  it.init(lane, A0, LA, B0, LB);
+  int ej, ek1, ek2;
+  bool v1, v2;
   while (it.next(ej, ek1, ek2, v1, v2)) {
     const V dj = sl.d[ej], pj = sl.pa[ej], qj = sl.pb[ej];
-    T gx = 0, gy = 0, gz = 0;
-    pair(dj, pj, qj, ek1, v1, gx, gy, gz);
-    pair(dj, pj, qj, ek2, v2, gx, gy, gz);
-    lds_f64* gj = sl.gs + __umul24(ej, 3);
-    lds_add(gj + 0, (double)gx);
-    lds_add(gj + 1, (double)gy);
-    lds_add(gj + 2, (double)gz);
+    JSide<T> js;
+    pair(dj, pj, qj, ek1, v1, js);
+    pair(dj, pj, qj, ek2, v2, js);
+    adj_j(sl, ej, dj, js.ue * pj.w + js.h * qj.w - js.ct * (pj.x * pj.x), js);
   }
 }
 
@@ -1335,7 +1379,7 @@ __device__ __forceinline__ void pairs_adj_prog(const Slice<T>& sl, int lane, int
   it.init(lane, A0, LA, B0, LB);
   int ej, ek1, ek2;
   bool v1, v2;
-  auto pair = [&](const V& dj, const V& pj, int ek, bool v, T& gx, T& gy, T& gz) {
+  auto pair = [&](const V& dj, const V& pj, int ek, bool v, JSide<T>& js) {
     const V dk = sl.d[ek], pk = sl.pa[ek];
     T rr, c, H, Hq;
     adj_geom_sel<T, G4>(dj, dk, pj, pk, J, v, rr, c, H, Hq);
@@ -1358,25 +1402,14 @@ __device__ __forceinline__ void pairs_adj_prog(const Slice<T>& sl, int lane, int
       S0 += P * h0;
       S1 += h1;
     }
-    T Pj, Pk, Q;
-    adj_coef<T, G4>(pj, pk, rr, c, H, Hq, S0, S1, Pj, Pk, Q);
-    gx += Pj * dj.x + Q * dk.x;
-    gy += Pj * dj.y + Q * dk.y;
-    gz += Pj * dj.z + Q * dk.z;
-    lds_f64* gk = sl.gs + __umul24(ek, 3);
-    lds_add(gk + 0, (double)(Pk * dk.x + Q * dj.x));
-    lds_add(gk + 1, (double)(Pk * dk.y + Q * dj.y));
-    lds_add(gk + 2, (double)(Pk * dk.z + Q * dj.z));
+    adj_pair<T, G4>(sl, ek, dj, pj, dk, pk, rr, c, H, Hq, v, S0, S1, js);
   };
   while (it.next(ej, ek1, ek2, v1, v2)) {
     const V dj = sl.d[ej], pj = sl.pa[ej];
-    T gx = 0, gy = 0, gz = 0;
-    pair(dj, pj, ek1, v1, gx, gy, gz);
-    pair(dj, pj, ek2, v2, gx, gy, gz);
-    lds_f64* gj = sl.gs + __umul24(ej, 3);
-    lds_add(gj + 0, (double)gx);
-    lds_add(gj + 1, (double)gy);
-    lds_add(gj + 2, (double)gz);
+    JSide<T> js;
+    pair(dj, pj, ek1, v1, js);
+    pair(dj, pj, ek2, v2, js);
+    adj_j(sl, ej, dj, js.ue * pj.w + js.h - js.ct * (pj.x * pj.x), js);
   }
 }
 
