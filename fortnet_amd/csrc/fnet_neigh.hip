@@ -226,10 +226,18 @@ __device__ __forceinline__ bool near_test(double ci0, double ci1, double ci2, co
 // writes row i at i * cap (entries past cap dropped) and its full length, in one pass.
 enum { kCount = 0, kFill = 1, kPadded = 2 };
 
-// Bounded to 80 registers (6 waves per SIMD instead of the compiler's 82 and 5), which it meets
-// without spilling: 8192 Si cells 2.74 -> 2.55 ms; at 64 registers (8 waves) it spills and takes
-// 3.38 ms.
-template <int MODE, typename V>
+// Bound by the tests of its candidates (FP64, a few dozen instructions for each 64 of them).  The
+// wave's number is taken as a scalar, so that the atom, its structure and the image ranges are
+// scalars too: 80 -> 46 registers, 8 waves to a SIMD instead of 6 (123 000 atoms of 8-512-atom Si
+// cells 328 -> 259 us, 38 400 water atoms 125 -> 103 us).  Neither the writes of the hits nor the
+// strided loads bound it: queueing hits until 64 are complete and a copy of the coordinates by
+// component gained nothing.
+//
+// SPLIT: the four waves of a block share one atom, each testing every fourth 64 of its candidates;
+// a barrier per step exchanges their hit counts, so the row's order stays.  A small batch waits
+// for one atom's serial walk over its candidates (192 water atoms 13.6 -> 9.2 us, 209 atoms of a
+// request 13.6 -> 8.2 us).
+template <int MODE, typename V, bool SPLIT = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
     k_neigh(const double* __restrict__ xyz, const long long* __restrict__ off,
             const int* __restrict__ atom_struct, const StructInfo* __restrict__ sinfo,
@@ -243,7 +251,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
 #pragma clang fp contract(off)
   constexpr bool WRITE = MODE != kCount;
   const int lane = threadIdx.x & 63;
-  const long long i = a0 + ((long long)blockIdx.x * blockDim.x + threadIdx.x) / 64;
+  // (the wave's number as a scalar: everything of the atom and its structure then is one too)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int w = SPLIT ? wave : 0;  // this wave's turn in a step of 64 kW candidates
+  constexpr int kW = SPLIT ? 4 : 1;
+  const long long i = a0 + (SPLIT ? (long long)blockIdx.x : (long long)blockIdx.x * 4 + wave);
   if (i >= a1) return;
   const int s = atom_struct[i];
   if (cellinfo[s].w) return;  // structure handled by the cell-list kernels
@@ -258,9 +270,24 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
 
   // key of an entry: (image + 1) n + (j - i) mod n, which increases along the row (the image
   // index is key / n - 1); the force gather's mirror search reads it
+  __shared__ int hits[2][4];  // SPLIT: the waves' hits of this step and the one before
+  int par = 0;
   auto emit = [&](bool hit, int j, int key, double nd0, double nd1, double nd2, double d2) {
     const unsigned long long mask = __ballot(hit);
-    const int q = count + __popcll(mask & lanemask_lt(lane));
+    int before = 0, all = __popcll(mask);
+    if constexpr (SPLIT) {
+      if (lane == 0) hits[par][w] = all;
+      __syncthreads();
+      all = 0;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int h = hits[par][v];
+        before += v < w ? h : 0;
+        all += h;
+      }
+      par ^= 1;
+    }
+    const int q = count + before + __popcll(mask & lanemask_lt(lane));
     if (WRITE && hit && (MODE != kPadded || q < cap)) {
       const long long pos = base + q;
       nj[pos] = (int)(o + j);
@@ -273,12 +300,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
       nd[pos] = v;
       if (MODE == kPadded && mir) mir[pos] = -1;
     }
-    count += __popcll(mask);
+    count += all;
   };
 
   // central cell: j = i+1 .. n-1, 0 .. i-1
-  for (int t0 = 1; t0 < n; t0 += 64) {
-    const int t = t0 + lane;
+  for (int t0 = 1; t0 < n; t0 += 64 * kW) {
+    const int t = t0 + 64 * w + lane;
     int j = li + t;
     if (j >= n) j -= n;
     double nd0 = 0, nd1 = 0, nd2 = 0, d2 = 0;
@@ -293,7 +320,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
     // LDS table with their translation, then the (image, atom) pairs of the table are tested as
     // one list, 64 per step, so small cells (n << 64) still fill the wave.
     __shared__ double4 tab[4][64];  // per wave: translation L . n (x, y, z), image index (w)
-    double4* tw = tab[(threadIdx.x >> 6) & 3];
+    double4* tw = tab[wave];
     const double* L = lat + 9 * s;
     double sf[3];
     for (int a = 0; a < 3; ++a)
@@ -310,7 +337,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
     const int m23 = m2 * m3;
     const double rm23 = 1.0 / (double)m23, rm3 = 1.0 / (double)m3;
     const int qorig = ((0 - si.lo[0]) * m2 + (0 - si.lo[1])) * m3 + (0 - si.lo[2]);
-    const int qs = 64 / n, rs = 64 % n;
+    const int qs = 64 * kW / n, rs = 64 * kW % n;
     for (int q0 = 0; q0 < nq; q0 += 64) {
       const int q = q0 + lane;
       bool keep = false;
@@ -348,8 +375,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       // flat index u = slot n + t over the kept images, t = 0 .. n - 1 from the centre on
       const int tot = __popcll(km) * n;
-      int slot = lane / n, t = lane % n;
-      for (int u0 = 0; u0 < tot; u0 += 64) {
+      int slot = (64 * w + lane) / n, t = (64 * w + lane) % n;
+      for (int u0 = 64 * w; u0 - 64 * w < tot; u0 += 64 * kW) {
         double nd0 = 0, nd1 = 0, nd2 = 0, d2 = 0;
         bool hit = false;
         int j = 0, img = 0;
@@ -373,8 +400,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
   }
-  if (MODE != kFill && lane == 0) cnt[i] = count;
-  if (MODE == kPadded && lane == 0) {
+  if (MODE != kFill && lane == 0 && w == 0) cnt[i] = count;
+  if (MODE == kPadded && lane == 0 && w == 0) {
     raise_max(maxnb, count);
     if (blockIdx.x == gridDim.x - 1) stamp_now(t_end);
   }
@@ -543,22 +570,25 @@ hipError_t launch_neigh_fill(fnet_batch* b, double rc, long long a0, long long a
   return hipGetLastError();
 }
 
+// Atoms up to which the direct search gives each four waves: beyond about a wave to every SIMD the
+// barriers cost more than the shorter walk gains (3072 water atoms 21.5 us with one, 23.6 with four).
+constexpr long long kNeighSplit = 1024;
+
 hipError_t launch_neigh_pad(fnet_batch* b, double rc, int fp64, hipStream_t s, int* mir,
                             unsigned long long* stamp) {
   const long long n = b->N;
   if (n <= 0 || b->n_cell_struct == b->S) return hipSuccess;
-  const unsigned grid = (unsigned)((n + 3) / 4);
-  if (fp64) {
-    k_neigh<kPadded, double4><<<grid, 256, 0, s>>>(b->xyz, b->off, b->atom_struct, b->sinfo,
-                                                   b->lat, rc, 0, n, b->cnt, nullptr, b->pnj,
-                                                   b->pnimg, (double4*)b->pnd, b->cellinfo,
-                                                   b->nb_cap, mir, b->d_maxnb, stamp);
-  } else {
-    k_neigh<kPadded, float4><<<grid, 256, 0, s>>>(b->xyz, b->off, b->atom_struct, b->sinfo,
-                                                  b->lat, rc, 0, n, b->cnt, nullptr, b->pnj,
-                                                  b->pnimg, (float4*)b->pnd, b->cellinfo,
-                                                  b->nb_cap, mir, b->d_maxnb, stamp);
-  }
+  const bool split = n <= kNeighSplit;
+  const unsigned grid = (unsigned)(split ? n : (n + 3) / 4);
+  auto go = [&](auto* kern, auto* nd) {
+    kern<<<grid, 256, 0, s>>>(b->xyz, b->off, b->atom_struct, b->sinfo, b->lat, rc, 0, n, b->cnt,
+                              nullptr, b->pnj, b->pnimg, nd, b->cellinfo, b->nb_cap, mir,
+                              b->d_maxnb, stamp);
+  };
+  if (fp64)
+    go(split ? k_neigh<kPadded, double4, true> : k_neigh<kPadded, double4>, (double4*)b->pnd);
+  else
+    go(split ? k_neigh<kPadded, float4, true> : k_neigh<kPadded, float4>, (float4*)b->pnd);
   return hipGetLastError();
 }
 
