@@ -44,7 +44,8 @@ namespace fnet {
 namespace {
 
 __global__ void __launch_bounds__(256) k_mirror(MirrorArgs a) {
-  mirror_centre(a, a.a0 + ((long long)blockIdx.x * blockDim.x + threadIdx.x) / 64,
+  mirror_centre(a, a.a0 + (long long)blockIdx.x * (blockDim.x >> 6) +
+                          __builtin_amdgcn_readfirstlane(threadIdx.x >> 6),
                 threadIdx.x & 63);
 }
 
@@ -66,7 +67,8 @@ __global__ void __launch_bounds__(256)
     return;
   }
   const int lane = threadIdx.x & 63;
-  const long long i = a0 + ((long long)blockIdx.x * blockDim.x + threadIdx.x) / 64;
+  const long long i = a0 + (long long)blockIdx.x * (blockDim.x >> 6) +
+                          __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (i >= a1) return;
   const long long bi = rl.base(i);
   const int len = rl.len(i);

@@ -141,7 +141,8 @@ __global__ void __launch_bounds__(256) k_mlp_fwd(MlpArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   stamp(a.stamp);
   if ((int)blockIdx.x >= a.ntiles) {
-    mirror_centre(a.mr, (long long)((int)blockIdx.x - a.ntiles) * 4 + (threadIdx.x >> 6),
+    mirror_centre(a.mr, (long long)((int)blockIdx.x - a.ntiles) * 4 +
+                  __builtin_amdgcn_readfirstlane(threadIdx.x >> 6),
                   threadIdx.x & 63);
     return;
   }

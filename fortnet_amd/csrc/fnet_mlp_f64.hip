@@ -123,7 +123,8 @@ __device__ __forceinline__ void input_rows(const F64Args& a, double* X, int ld, 
 template <bool FP, typename Rows, typename Out>
 __device__ __forceinline__ void forward16(const F64Args& a, const double* P, int act, double* sm,
                                           Rows rows, Out out) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, j = lane & 15;
+  const int lane = threadIdx.x & 63, g = lane >> 4, j = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nl = a.sh.nl;
   for (int l = 0; l < nl - 1; ++l) {
     const int din = a.sh.dims[l], dout = a.sh.dims[l + 1];
@@ -175,7 +176,8 @@ __device__ __forceinline__ void reverse16(const F64Args& a, const double* P, int
 template <bool GRADIN>
 __global__ void __launch_bounds__(256) k_mlp_f64(F64Args a) {
   extern __shared__ __align__(16) double sm[];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, j = lane & 15;
+  const int lane = threadIdx.x & 63, g = lane >> 4, j = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   stamp(a.stamp);
   if ((int)blockIdx.x >= a.nblocks) {
     mirror_centre(a.mr, (long long)((int)blockIdx.x - a.nblocks) * 4 + w, lane);
@@ -224,7 +226,8 @@ __global__ void __launch_bounds__(256) k_mlp_f64(F64Args a) {
 // partial, the others add to it, each value always by the same thread.
 __global__ void __launch_bounds__(256) k_mlp_grad_f64(F64Args a) {
   extern __shared__ __align__(16) double sm[];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, j = lane & 15;
+  const int lane = threadIdx.x & 63, g = lane >> 4, j = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int tile = blockIdx.x;
   const int sp = a.tile_sp[tile], cnt = a.tile_cnt[tile];
   const int nl = a.sh.nl, act = a.sh.act[sp];
