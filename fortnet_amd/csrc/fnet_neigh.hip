@@ -229,9 +229,9 @@ enum { kCount = 0, kFill = 1, kPadded = 2 };
 // Bound by the tests of its candidates (FP64, a few dozen instructions for each 64 of them).  The
 // wave's number is taken as a scalar, so that the atom, its structure and the image ranges are
 // scalars too: 80 -> 46 registers, 8 waves to a SIMD instead of 6 (123 000 atoms of 8-512-atom Si
-// cells 328 -> 259 us, 38 400 water atoms 125 -> 103 us).  Neither the writes of the hits nor the
-// strided loads bound it: queueing hits until 64 are complete and a copy of the coordinates by
-// component gained nothing.
+// cells 328 -> 259 us, 38 400 water atoms 125 -> 103 us).  Its vector units are busy
+// all the time then; the strided loads of the coordinates do not bound it (a copy by component: no
+// gain).
 //
 // SPLIT: the four waves of a block share one atom, each testing every fourth 64 of its candidates;
 // a barrier per step exchanges their hit counts, so the row's order stays.  A small batch waits
@@ -268,13 +268,64 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
   const long long base = MODE == kFill ? rowptr[i] : (MODE == kPadded ? i * cap : 0);
   int count = 0;
 
+  __shared__ double4 tab[4][64];  // per wave: translation L . n (x, y, z), image index (w)
+  double4* tw = tab[wave];
+  auto order = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
   // key of an entry: (image + 1) n + (j - i) mod n, which increases along the row (the image
   // index is key / n - 1); the force gather's mirror search reads it
+  auto put = [&](int q, int j, int key, double nd0, double nd1, double nd2, double d2) {
+    if (MODE == kPadded && q >= cap) return;
+    const long long pos = base + q;
+    nj[pos] = (int)(o + j);
+    nimg[pos] = key;
+    V v;
+    v.x = nd0;
+    v.y = nd1;
+    v.z = nd2;
+    entry_d2(v, d2);
+    nd[pos] = v;
+    if (MODE == kPadded && mir) mir[pos] = -1;
+  };
+  // QUEUE: the hits wait in a ring of (t, slot of tab or -1: central cell) until 64 of them, or a
+  // table of images, are complete; they are then tested once more for their vectors and written
+  // one to a lane.  A step of 64 candidates has a few hits, whose write would cost all lanes half
+  // as much as the test (123 000 atoms of 8-512-atom Si cells 259 -> 235 us, 38 400 water atoms
+  // 103 -> 91 us).
+  constexpr bool QUEUE = WRITE && !SPLIT;
+  __shared__ int2 ring[QUEUE ? 4 : 1][QUEUE ? 128 : 1];
+  int2* rw = ring[QUEUE ? wave : 0];
+  int head = 0;  // hits so far; count of them are written
+  auto flush = [&](int nf) {
+    order();
+    if (lane < nf) {
+      const int2 h = rw[(count + lane) & 127];
+      double4 c = make_double4(0.0, 0.0, 0.0, -1.0);
+      if (h.y >= 0) c = tw[h.y];
+      int j = li + h.x;
+      if (j >= n) j -= n;
+      double nd0, nd1, nd2, d2;
+      near_test(ci0, ci1, ci2, X, j, c.x, c.y, c.z, rc2, nd0, nd1, nd2, d2);
+      put(count + lane, j, ((int)c.w + 1) * n + h.x, nd0, nd1, nd2, d2);
+    }
+    count += nf;
+    order();
+  };
   __shared__ int hits[2][4];  // SPLIT: the waves' hits of this step and the one before
   int par = 0;
-  auto emit = [&](bool hit, int j, int key, double nd0, double nd1, double nd2, double d2) {
+  auto emit = [&](bool hit, int j, int t, int slot, int img, double nd0, double nd1, double nd2,
+                  double d2) {
     const unsigned long long mask = __ballot(hit);
     int before = 0, all = __popcll(mask);
+    if constexpr (QUEUE) {
+      if (hit) rw[(head + __popcll(mask & lanemask_lt(lane))) & 127] = make_int2(t, slot);
+      head += all;
+      if (head - count >= 64) flush(64);
+      return;
+    }
     if constexpr (SPLIT) {
       if (lane == 0) hits[par][w] = all;
       __syncthreads();
@@ -287,19 +338,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
       }
       par ^= 1;
     }
-    const int q = count + before + __popcll(mask & lanemask_lt(lane));
-    if (WRITE && hit && (MODE != kPadded || q < cap)) {
-      const long long pos = base + q;
-      nj[pos] = (int)(o + j);
-      nimg[pos] = key;
-      V v;
-      v.x = nd0;
-      v.y = nd1;
-      v.z = nd2;
-      entry_d2(v, d2);
-      nd[pos] = v;
-      if (MODE == kPadded && mir) mir[pos] = -1;
-    }
+    if (WRITE && hit)
+      put(count + before + __popcll(mask & lanemask_lt(lane)), j, (img + 1) * n + t, nd0, nd1, nd2,
+          d2);
     count += all;
   };
 
@@ -311,7 +352,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
     double nd0 = 0, nd1 = 0, nd2 = 0, d2 = 0;
     bool hit = false;
     if (t < n) hit = near_test(ci0, ci1, ci2, X, j, 0.0, 0.0, 0.0, rc2, nd0, nd1, nd2, d2);
-    emit(hit, j, t, nd0, nd1, nd2, d2);
+    emit(hit, j, t, -1, -1, nd0, nd1, nd2, d2);
   }
   const StructInfo& si = sinfo[s];
   if (si.periodic) {
@@ -319,8 +360,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
     // skipped), 64 at a time: the ones that can hold a neighbour are compacted in order into an
     // LDS table with their translation, then the (image, atom) pairs of the table are tested as
     // one list, 64 per step, so small cells (n << 64) still fill the wave.
-    __shared__ double4 tab[4][64];  // per wave: translation L . n (x, y, z), image index (w)
-    double4* tw = tab[wave];
     const double* L = lat + 9 * s;
     double sf[3];
     for (int a = 0; a < 3; ++a)
@@ -369,10 +408,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
         tv = make_double4(cv[0], cv[1], cv[2], (double)(q > qorig ? q - 1 : q));
       }
       const unsigned long long km = __ballot(keep);
+      if (QUEUE && head != count) flush(head - count);  // (their images are still in the table)
       if (keep) tw[__popcll(km & lanemask_lt(lane))] = tv;
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      order();
       // flat index u = slot n + t over the kept images, t = 0 .. n - 1 from the centre on
       const int tot = __popcll(km) * n;
       int slot = (64 * w + lane) / n, t = (64 * w + lane) % n;
@@ -387,7 +425,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
           img = (int)c.w;
           hit = near_test(ci0, ci1, ci2, X, j, c.x, c.y, c.z, rc2, nd0, nd1, nd2, d2);
         }
-        emit(hit, j, (img + 1) * n + t, nd0, nd1, nd2, d2);
+        emit(hit, j, t, slot, img, nd0, nd1, nd2, d2);
         slot += qs;
         t += rs;
         if (t >= n) {
@@ -395,11 +433,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
           slot += 1;
         }
       }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      order();
     }
   }
+  if (QUEUE && head != count) flush(head - count);
   if (MODE != kFill && lane == 0 && w == 0) cnt[i] = count;
   if (MODE == kPadded && lane == 0 && w == 0) {
     raise_max(maxnb, count);
