@@ -15,8 +15,8 @@ against the FP64 device path (itself pinned to the oracle): energy error per ato
 eagerly launched or replayed as a HIP graph, whichever is faster; the plain path (FP64, one
 structure per launch) is timed on the same batch and reported beside it.
 
-``roofline`` is for the dominant kernel (largest stage time measured with HIP events on the
-stream the kernels run on); ``cpu_baseline`` times the FP64 C oracle in the reference's loop
+``roofline`` is for the dominant kernel (largest stage time by the clock stamps that its
+kernels write); ``cpu_baseline`` times the FP64 C oracle in the reference's loop
 shape (neighbour list rebuilt per atom and function, dense dG/dr, dense force contraction) on a
 bounded sample of the same workload.
 """

@@ -164,8 +164,8 @@ int fnet_set_graph(fnet_ctx* ctx, int enable);
 /* Waits for the batch's last step and validates it (see fnet_run). */
 int fnet_batch_sync(fnet_batch* batch);
 
-/* Device time of the whole last fnet_run / fnet_forces step in ms (HIP events on the context
- * stream); *graph = 1 if the batch's last fnet_run replayed its graph. */
+/* Device time of the whole last fnet_run / fnet_forces step in ms (clock stamps that its kernels
+ * write, or HIP events on the context stream where it was launched structure by structure); *graph = 1 if the batch's last fnet_run replayed its graph. */
 int fnet_step_time(fnet_ctx* ctx, double* ms);
 int fnet_batch_step_info(const fnet_batch* batch, int* graph);
 
@@ -242,8 +242,8 @@ int fnet_sync(fnet_ctx* ctx);
  * else an fnet_status (no reference counterpart; used by the serving loop). */
 int fnet_query(fnet_ctx* ctx);
 
-/* Timing of the last fnet_run / fnet_forces call, per stage, in milliseconds (HIP events on
- * the context stream): [0] neighbour list (with the mirror entries), [1] ACSF forward,
+/* Timing of the last fnet_run / fnet_forces call, per stage, in milliseconds (clock stamps
+ * that its kernels write, or HIP events): [0] neighbour list (with the mirror entries), [1] ACSF forward,
  * [2] networks, [3] adjoint forces (with the force gather), [4] energy reduction.
  * n = number of entries written (<= 8).  A step replayed as a graph has only its total, in [0]. */
 int fnet_stage_times(fnet_ctx* ctx, double* ms, int n);
