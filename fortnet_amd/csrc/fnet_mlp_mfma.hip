@@ -25,6 +25,7 @@
 // takes hi.hi only (8 bits; its errors are reported, not gated).  The input layer (z-scored
 // features, which can be ill-conditioned) and the output layer stay FP32.
 #include <algorithm>
+#include <type_traits>
 
 #include "../../include/fnet_hip.h"
 #include "fnet_device.hpp"
@@ -297,9 +298,11 @@ __device__ __forceinline__ bool hidden_hidden(int l, int nl) { return l >= 1 && 
 // SPLIT: the four waves of a block share 16 atoms, each taking every fourth output block, instead
 // of running 16 atoms each through all of them: a batch that leaves most of the chip idle waits
 // for one wave's chain of loads, products and activations, which this cuts to about a third.  The
-// sums are the same either way.
-template <bool GRADIN, int BF, bool SPLIT>
-__global__ void __launch_bounds__(256) k_mlp_mfma(MfmaArgs a) {
+// sums are the same either way.  kOwn: output blocks of a hidden layer that one wave holds in
+// registers, both of a layer up to 32 wide or every fourth of one up to 64, 128 or kMaxDim.
+template <bool GRADIN, int BF, bool SPLIT, int kOwn>
+__global__ void __launch_bounds__(256)
+    __attribute__((amdgpu_waves_per_eu(kOwn > 2 ? 4 : !SPLIT && BF == 3 ? 5 : 6))) k_mlp_mfma(MfmaArgs a) {
   extern __shared__ __align__(16) float smf[];
   const int lane = threadIdx.x & 63;
   // a scalar, and with it the tile and its addresses (500 boxes' weight gradients, whole iteration
@@ -331,96 +334,109 @@ __global__ void __launch_bounds__(256) k_mlp_mfma(MfmaArgs a) {
   const bool valid = j < nv;
   const long long atom = valid ? (long long)a.perm[start + a0 + j] : 0;
 
-  // input rows: standardised features (and external features), zero beyond d0 and nv
+  // input rows: standardised features (and external features), zero beyond d0 and nv; 32 lanes to
+  // a row's chunk
   const int d0 = a.sh.dims[0], K0 = r32(d0);
-  for (int idx = SPLIT ? (int)threadIdx.x : lane; idx < 16 * K0; idx += 64 * nw) {
-    const int r = idx / K0, k = idx - r * K0;
-    float v = 0.0f;
-    if (r < nv && k < d0) {
-      const long long at = a.perm[start + a0 + r];
-      v = k < a.nG ? (float)((a.G[at * a.nG + k] - a.zmean[k]) * a.zinv[k])
-                   : (float)a.ext[at * a.next + a.ext_in[k - a.nG]];
+  {
+    const int t = SPLIT ? (int)threadIdx.x : lane, kl = t & 31;
+    for (int r = t >> 5; r < 16; r += 2 * nw) {
+      const long long at = r < nv ? a.perm[start + a0 + r] : 0;
+      for (int k = kl; k < K0; k += 32) {
+        float v = 0.0f;
+        if (r < nv && k < d0)
+          v = k < a.nG ? (float)((a.G[at * a.nG + k] - a.zmean[k]) * a.zinv[k])
+                       : (float)a.ext[at * a.next + a.ext_in[k - a.nG]];
+        X[r * ldx + k] = v;
+      }
     }
-    X[r * ldx + k] = v;
   }
   sync();
 
-  // linear output layer (nout <= 16): lane group g holds outputs 4 g + r of atom j
-  auto write_out = [&](const f4& c) {
+  // this wave's output blocks of a hidden layer: q -> block (q < kOwn)
+  auto own = [&](int q) { return SPLIT ? me + 4 * q : q; };
+  float* row = X + j * ldx + 4 * g;  // a fragment's place in the rows: row + 16 * block
+  // products of a hidden layer's own blocks, added to c
+  auto product = [&](const float* Wf, const bf8* Bf, long long bsz, bool bf, int Kc, int Nb,
+                     f4 (&c)[kOwn]) {
+    if constexpr (SPLIT) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int o = 4 * g + r;
-      if (o < a.nout) a.Eatom[atom * a.nout + o] = (double)c[r];
+      for (int q = 0; q < kOwn; ++q)
+        if (own(q) < Nb) {
+          if (bf) gemm_one_bf<BF ? BF : 1>(Bf, bsz, own(q), Kc >> 1, X, ldx, lane, j, g, c[q]);
+          else gemm_one(Wf, own(q), Kc, X, ldx, lane, j, g, c[q]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+    } else {
+      if (bf) gemm_pair_bf<BF>(Bf, bsz, 0, Kc >> 1, X, ldx, lane, j, g, c[0], c[1]);
+      else gemm_pair(Wf, 0, Kc, X, ldx, lane, j, g, c[0], c[1]);
     }
   };
-  for (int l = 0; l < nl - 1; ++l) {
+
+  // hidden layers: the pre-activations stay in registers until every wave has read the layer's
+  // rows, then the next rows y = f(z) and, in fragment order, f'(z), 16 bytes at a time (through
+  // LDS value by value before: 8192 parts of 32-128-128-1 176 -> 147 us, whole step of 131 072 Si
+  // atoms 2049 -> 2034)
+  for (int l = 0; l < nl - 2; ++l) {
     const int Kc = r32(a.sh.dims[l]) >> 4, Nb = r32(a.sh.dims[l + 1]) >> 4;
-    const float* Wf = WP + a.fw[l];
     const float* Bp = WP + a.pb[l];
-    const bool hidden = l < nl - 2;
-    float* zs = FP + a.fpoff[l + 1];
-    const bool bf = BF && hidden_hidden(l, nl);
-    const bf8* Bf = a.bpack + (long long)sp * a.bk_stride + a.bfw[l];
-    if constexpr (SPLIT) {
-      // the output layer's second block holds no output
-      for (int ob = me; ob < (hidden ? Nb : 1); ob += nw) {
-        f4 c0 = *(const f4*)(Bp + 16 * ob + 4 * g);
-        if (bf) gemm_one_bf<BF ? BF : 1>(Bf, a.bsz[l], ob, Kc >> 1, X, ldx, lane, j, g, c0);
-        else gemm_one(Wf, ob, Kc, X, ldx, lane, j, g, c0);
-        if (hidden) *(f4*)(zs + (ob * 64 + lane) * 4) = c0;
-        else if (valid) write_out(c0);
-      }
-    } else {
-      for (int ob0 = 0; ob0 < Nb; ob0 += 2) {
-        f4 c0 = *(const f4*)(Bp + 16 * ob0 + 4 * g);
-        f4 c1 = *(const f4*)(Bp + 16 * ob0 + 16 + 4 * g);
-        if (bf) gemm_pair_bf<BF>(Bf, a.bsz[l], ob0, Kc >> 1, X, ldx, lane, j, g, c0, c1);
-        else gemm_pair(Wf, ob0, Kc, X, ldx, lane, j, g, c0, c1);
-        if (hidden) {
-          *(f4*)(zs + (ob0 * 64 + lane) * 4) = c0;
-          *(f4*)(zs + ((ob0 + 1) * 64 + lane) * 4) = c1;
-        } else if (valid) {
-          write_out(c0);
+    f4 c[kOwn];
+#pragma unroll
+    for (int q = 0; q < kOwn; ++q)
+      if (own(q) < Nb) c[q] = *(const f4*)(Bp + 16 * own(q) + 4 * g);
+    product(WP + a.fw[l], a.bpack + (long long)sp * a.bk_stride + a.bfw[l], a.bsz[l],
+            BF && hidden_hidden(l, nl), Kc, Nb, c);
+    sync();
+    float* ds = FP + a.fpoff[l + 1];
+#pragma unroll
+    for (int q = 0; q < kOwn; ++q)
+      if (own(q) < Nb) {
+        f4 f, d;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float fr, dr;
+          actfd(act, c[q][r], fr, dr);
+          f[r] = fr;
+          d[r] = dr;
         }
+        *(f4*)(row + 16 * own(q)) = f;
+        if (GRADIN) *(f4*)(ds + (own(q) * 64 + lane) * 4) = d;
+        __builtin_amdgcn_sched_barrier(0);  // (blocks interleaved take registers that cost waves)
       }
-    }
-    sync();  // every lane has read this layer's rows before they are overwritten
-    if (hidden) {
-      // activation: z in the fragment slots -> next rows y = f(z), slots <- f'(z); four at a
-      // time, so that their LDS reads and transcendentals overlap (the kernel's occupancy is
-      // set by its LDS, not by these registers)
-#pragma unroll 4
-      for (int q = me; q < 4 * Nb; q += nw) {
-        const int ob = q >> 2, r = q & 3;
-        float* slot = zs + (ob * 64 + lane) * 4 + r;
-        const float z = *slot;
-        float f, d;
-        actfd(act, z, f, d);
-        X[j * ldx + 16 * ob + 4 * g + r] = f;
-        *slot = d;
-      }
-      sync();
-    }
+    sync();
+  }
+  // linear output layer (nout <= 16: one block): lane group g holds outputs 4 g + r of atom j
+  if (!SPLIT || w == 0) {
+    const int l = nl - 2;
+    f4 c = *(const f4*)(WP + a.pb[l] + 4 * g);
+    gemm_one(WP + a.fw[l], 0, r32(a.sh.dims[l]) >> 4, X, ldx, lane, j, g, c);
+    if (valid)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (4 * g + r < a.nout) a.Eatom[atom * a.nout + 4 * g + r] = (double)c[r];
   }
   if (!GRADIN) return;
+  sync();
 
   // reverse sweep of the single output (input gradient = row of the Jacobian)
   double* out = a.cG + atom * a.nG;
   int m = nl - 2;
   {
     // delta of activation layer m from the one-hot output: column 0 of ww(m), times f'(z_m)
-    const int dm = a.sh.dims[m], Kb = r32(dm) >> 4;
+    const int dm = a.sh.dims[m], Nb = r32(dm) >> 4;
     const float* col = a.params_f + (long long)sp * a.sh.nparams + a.sh.woff[m];
     if (m >= 1) {
-      float* sl = FP + a.fpoff[m];
-#pragma unroll 4
-      for (int q = me; q < 4 * Kb; q += nw) {
-        const int ib = q >> 2, r = q & 3, k = 16 * ib + 4 * g + r;
-        float* slot = sl + (ib * 64 + lane) * 4 + r;
-        const float d = (k < dm ? col[k] : 0.0f) * *slot;
-        *slot = d;
-        X[j * ldx + k] = d;
-      }
+      const float* ds = FP + a.fpoff[m];
+#pragma unroll
+      for (int q = 0; q < kOwn; ++q)
+        if (own(q) < Nb) {
+          f4 d = *(const f4*)(ds + (own(q) * 64 + lane) * 4);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int k = 16 * own(q) + 4 * g + r;
+            d[r] = (k < dm ? col[k] : 0.0f) * d[r];
+          }
+          *(f4*)(row + 16 * own(q)) = d;
+        }
       sync();
     } else if (valid) {
       for (int k = 4 * g + 16 * me; k < a.nG; k += 16 * nw)
@@ -429,54 +445,46 @@ __global__ void __launch_bounds__(256) k_mlp_mfma(MfmaArgs a) {
           if (k + r < a.nG) out[k + r] = (double)col[k + r] * a.zinv[k + r];
     }
   }
-  // delta_{m-1}^T = W_{m-1} . delta_m^T (rows in X), times f'(z_{m-1}) for hidden layers; the
-  // input layer: the ACSF part of d out / d x feeds the force adjoint (FP64, z-score factor)
-  auto write_in = [&](const f4& c, int ib) {
+  // delta_{m-1}^T = W_{m-1} . delta_m^T (rows in X), times f'(z_{m-1})
+  for (; m >= 2; --m) {
+    const int Nb = r32(a.sh.dims[m - 1]) >> 4, Kc = r32(a.sh.dims[m]) >> 4;
+    f4 c[kOwn];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int f = 16 * ib + 4 * g + r;
-      if (f < a.nG) out[f] = (double)c[r] * a.zinv[f];
-    }
-  };
-  for (; m >= 1; --m) {
-    const int Mb = r32(a.sh.dims[m - 1]) >> 4, Kc = r32(a.sh.dims[m]) >> 4;
-    const float* Rf = WP + a.rw[m - 1];
-    float* sl = FP + a.fpoff[m - 1];
-    const bool bf = BF && hidden_hidden(m - 1, nl);
-    const bf8* Br = a.bpack + (long long)sp * a.bk_stride + a.brw[m - 1];
-    auto put = [&](const f4& c, int ib) {
-      if (m - 1 >= 1) {
-        f4* s0 = (f4*)(sl + (ib * 64 + lane) * 4);
-        *s0 = c * *s0;
-      } else if (valid) {
-        write_in(c, ib);
+    for (int q = 0; q < kOwn; ++q) c[q] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    product(WP + a.rw[m - 1], a.bpack + (long long)sp * a.bk_stride + a.brw[m - 1], a.bsz[m - 1],
+            BF && hidden_hidden(m - 1, nl), Kc, Nb, c);
+    sync();
+    const float* ds = FP + a.fpoff[m - 1];
+#pragma unroll
+    for (int q = 0; q < kOwn; ++q)
+      if (own(q) < Nb)
+        *(f4*)(row + 16 * own(q)) = c[q] * *(const f4*)(ds + (own(q) * 64 + lane) * 4);
+    sync();
+  }
+  // input layer: the ACSF part of d out / d x feeds the force adjoint (FP64, z-score factor)
+  if (m == 1) {
+    const int Mb = K0 >> 4, Kc = r32(a.sh.dims[1]) >> 4;
+    const float* Rf = WP + a.rw[0];
+    auto write_in = [&](const f4& c, int ib) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int f = 16 * ib + 4 * g + r;
+        if (valid && f < a.nG) out[f] = (double)c[r] * a.zinv[f];
       }
     };
     if constexpr (SPLIT) {
       for (int ib = me; ib < Mb; ib += nw) {
         f4 c0 = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (bf) gemm_one_bf<BF ? BF : 1>(Br, a.bsz[m - 1], ib, Kc >> 1, X, ldx, lane, j, g, c0);
-        else gemm_one(Rf, ib, Kc, X, ldx, lane, j, g, c0);
-        put(c0, ib);
+        gemm_one(Rf, ib, Kc, X, ldx, lane, j, g, c0);
+        write_in(c0, ib);
       }
     } else {
       for (int ib0 = 0; ib0 < Mb; ib0 += 2) {
         f4 c0 = {0.0f, 0.0f, 0.0f, 0.0f}, c1 = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (bf) gemm_pair_bf<BF>(Br, a.bsz[m - 1], ib0, Kc >> 1, X, ldx, lane, j, g, c0, c1);
-        else gemm_pair(Rf, ib0, Kc, X, ldx, lane, j, g, c0, c1);
-        put(c0, ib0);
-        put(c1, ib0 + 1);
+        gemm_pair(Rf, ib0, Kc, X, ldx, lane, j, g, c0, c1);
+        write_in(c0, ib0);
+        write_in(c1, ib0 + 1);
       }
-    }
-    sync();
-    if (m - 1 >= 1) {
-      // delta_{m-1} fragments -> rows for the next product
-#pragma unroll 4
-      for (int q = me; q < 4 * Mb; q += nw) {
-        const int ib = q >> 2, r = q & 3;
-        X[j * ldx + 16 * ib + 4 * g + r] = sl[(ib * 64 + lane) * 4 + r];
-      }
-      sync();
     }
   }
 }
@@ -943,9 +951,9 @@ hipError_t launch_mlp_grad_mfma(fnet_batch* b, const DevModel& m, hipStream_t s)
 
 // 16-atom parts up to which the waves of a block share one (SPLIT): 1132 parts 26.2 -> 24.7 us,
 // 2400 parts 27.1 -> 26.2 us; beyond that every CU has its fill of the other kind (6000 parts of
-// 32-32-32: 26.7 -> 33 us).  Networks whose rows and f'(z) let fewer than four waves of their own into
-// 64 KB share at every size: the other kind has 6 waves on a CU there (130 000 atoms of 32-128-128-1 in
-// split BF16: 294 -> 178 us).
+// 32-32-32: 26.7 -> 33 us).  Networks wider than 32, or whose rows and f'(z) let fewer than four waves
+// of their own into 64 KB, share at every size: the other kind has few waves on a CU there (7700
+// parts of 24-64-64-1: 123 -> 101 us; 8192 of 32-128-128-1 in split BF16: 294 -> 178 us).
 constexpr long long kSplitTiles = 2560;
 
 hipError_t launch_mlp_mfma(fnet_batch* b, const DevModel& m, int first_tile, int ntiles,
@@ -991,25 +999,32 @@ hipError_t launch_mlp_mfma(fnet_batch* b, const DevModel& m, int first_tile, int
   a.nsub = waves;
   a.mr = mirror_args(b, 0, b->N);
   a.stamp = stamp;
-  const bool split = (long long)ntiles * waves <= kSplitTiles ||
-                     4 * a.wave_floats * sizeof(float) > 64 * 1024;
+  bool split = (long long)ntiles * waves <= kSplitTiles ||
+               4 * a.wave_floats * sizeof(float) > 64 * 1024;
+  int width = 0;  // of the widest hidden layer
+  for (int l = 1; l + 1 < m.shape.nl; ++l) width = std::max(width, m.shape.dims[l]);
+  split = split || width > 32;
+  if (!want_grad_in) a.wave_floats = 16 * a.ldx;  // no f'(z) to keep
   const int bw = split ? 4 : waves;  // waves per block
   a.ntiles = split ? ntiles * waves : ntiles;
   const size_t lds = (size_t)(split ? 1 : waves) * a.wave_floats * sizeof(float);
   const dim3 grid((unsigned)(a.ntiles + (mirror ? (b->N + bw - 1) / bw : 0))), block(64 * bw);
-  auto go = [&](auto* sp, auto* one) {
-    if (split) sp<<<grid, block, lds, s>>>(a);
-    else one<<<grid, block, lds, s>>>(a);
+  auto run = [&](void (*kern)(MfmaArgs)) { kern<<<grid, block, lds, s>>>(a); };
+  auto go = [&](auto gradin, auto bfc) {
+    constexpr bool G = decltype(gradin)::value;
+    constexpr int B = decltype(bfc)::value;
+    if (!split) run(k_mlp_mfma<G, B, false, 2>);
+    else if (width <= 64) run(k_mlp_mfma<G, B, true, 1>);
+    else if (width <= 128) run(k_mlp_mfma<G, B, true, 2>);
+    else run(k_mlp_mfma<G, B, true, 4>);
   };
-  if (want_grad_in) {
-    if (bf == 3) go(k_mlp_mfma<true, 3, true>, k_mlp_mfma<true, 3, false>);
-    else if (bf == 1) go(k_mlp_mfma<true, 1, true>, k_mlp_mfma<true, 1, false>);
-    else go(k_mlp_mfma<true, 0, true>, k_mlp_mfma<true, 0, false>);
-  } else {
-    if (bf == 3) go(k_mlp_mfma<false, 3, true>, k_mlp_mfma<false, 3, false>);
-    else if (bf == 1) go(k_mlp_mfma<false, 1, true>, k_mlp_mfma<false, 1, false>);
-    else go(k_mlp_mfma<false, 0, true>, k_mlp_mfma<false, 0, false>);
-  }
+  auto mode = [&](auto gradin) {
+    if (bf == 3) go(gradin, std::integral_constant<int, 3>());
+    else if (bf == 1) go(gradin, std::integral_constant<int, 1>());
+    else go(gradin, std::integral_constant<int, 0>());
+  };
+  if (want_grad_in) mode(std::true_type());
+  else mode(std::false_type());
   return hipGetLastError();
 }
 
