@@ -307,7 +307,8 @@ __device__ __forceinline__ bool hidden_hidden(int l, int nl) { return l >= 1 && 
 // registers, both of a layer up to 32 wide or every fourth of one up to 64, 128 or kMaxDim.
 template <bool GRADIN, int BF, bool SPLIT, int kOwn>
 __global__ void __launch_bounds__(256)
-    __attribute__((amdgpu_waves_per_eu(kOwn > 2 ? 4 : !SPLIT && BF == 3 ? 5 : 6))) k_mlp_mfma(MfmaArgs a) {
+    __attribute__((amdgpu_waves_per_eu(kOwn > 2 ? 4 : !SPLIT && BF == 3 ? 5 : 6)))
+    k_mlp_mfma(MfmaArgs a) {
   extern __shared__ __align__(16) float smf[];
   const int lane = threadIdx.x & 63;
   // a scalar, and with it the tile and its addresses (500 boxes' weight gradients, whole iteration
@@ -498,8 +499,8 @@ __global__ void __launch_bounds__(256)
 // One block = nw waves = 16 nw atoms of one element (a tile of the MFMA layout, or a fixed part of
 // one).  Forward: every wave runs its 16 atoms through the hidden layers as above, keeping each
 // layer's pre-activation rows z_l (tanh and sigmoid: f(z_l)) for all atoms of the block in LDS (R[l];
-// R[0] holds the input rows) and otherwise its own current activations in Xw.  Backward, top layer first, with delta_out = the
-// loss gradient of each atom (nout = 1):
+// R[0] holds the input rows) and, for other activations, its own current values in Xw.  Backward,
+// top layer first, with delta_out = the loss gradient of each atom (nout = 1):
 //  * the output layer (rank one) on the vector unit: dW[0][k] = sum_at delta_out a_l[at][k],
 //    delta_l = W[0][k] delta_out f'(z_l);
 //  * every other layer l: dW_l[o][k] = sum_at delta_{l+1}[at][o] a_l[at][k] on the matrix cores
