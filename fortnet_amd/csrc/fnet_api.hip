@@ -572,7 +572,7 @@ int do_adjoint(fnet_batch* b) {
   int rc = do_mirror(b);
   if (rc) return rc;
   hipStream_t s = ctx->stream;
-  int* norph = b->d_norph;  // cleared by the first launch of the adjoint
+  int* norph = b->d_norph;  // cleared by the first launch of the adjoint (none without atoms)
   if (b->launch == FNET_PER_STRUCT) {
     for (int st = 0; st < b->S; ++st) {
       if (b->h_off[st + 1] == b->h_off[st]) continue;

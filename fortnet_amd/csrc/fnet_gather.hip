@@ -215,6 +215,9 @@ void* scratch_ptr(int device) {
 
 hipError_t launch_force_finish(fnet_batch* b, const DevModel& m, bool energies, hipStream_t s,
                                bool host, unsigned long long* stamps) {
+  // no atoms: no adjoint ran, so nothing cleared the orphan counter of an earlier batch, whose
+  // entries the kernel would follow
+  if (b->N == 0) return hipSuccess;
   const int* nj = b->nl_padded ? b->pnj : b->nj;
   const EnergyArgs en = energy_args(b, m, energies);
   const unsigned nen =
@@ -307,7 +310,6 @@ extern "C" int fnet_forces_noalloc(fnet_ctx* ctx, fnet_batch* b) {
       e = launch_mirror(b, 0, b->N, entries, s);
     }
     int* clear = norph;  // cleared by the first launch of the adjoint
-    if (b->N == 0 && e == hipSuccess) e = launch_zero_int(norph, 1, s);
     if (b->launch == FNET_PER_STRUCT) {
       for (int st = 0; st < b->S && e == hipSuccess; ++st) {
         if (b->h_off[st + 1] == b->h_off[st]) continue;
