@@ -142,8 +142,9 @@ void ladder_form(AngGroup& a) {
 }
 
 // Fills the progression form of an angular group (np = 0 when it does not have it): at most two
-// lambda values, exponents x0 + k s with x0 >= 1 (P^(x0 - 1) stays finite at P = 0) and at most
-// kProgLen of them, each (lambda, xi) once.  The automatic ACSF scheme steps xi evenly from 1
+// lambda values of at most 1 in size (P = 1 + lambda cos(theta) stays >= 0: below it, P^s has no
+// real value where integer members of the group have one), exponents x0 + k s with x0 >= 1
+// (P^(x0 - 1) stays finite at P = 0) and at most kProgLen of them, each (lambda, xi) once.  The automatic ACSF scheme steps xi evenly from 1
 // (acsf.F90:276-363); a group split at kMaxMembers continues the steps from a larger x0.  The
 // largest exponent is bounded so that the padded slots of the kernels stay finite in FP32.
 void progression_form(AngGroup& a) {
@@ -160,6 +161,7 @@ void progression_form(AngGroup& a) {
   distinct(xi);
   const int K = (int)xi.size();
   if (lam.size() > 2 || K > kProgLen || K < 1 || !(xi[0] >= 1.0)) return;
+  if (!(lam.front() >= -1.0 && lam.back() <= 1.0)) return;
   const double s = K > 1 ? (xi[K - 1] - xi[0]) / (K - 1) : 0.0;
   for (int k = 0; k < K; ++k)
     if (std::fabs(xi[k] - (xi[0] + k * s)) > 1e-14 * xi[k]) return;
