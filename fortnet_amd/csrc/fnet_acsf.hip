@@ -65,7 +65,10 @@ __device__ __forceinline__ double lit(double c) {
 // degree 13 on |r| <= ln 2 / 2 (remainder 4e-18), scaled by 2^n; 1.4e-16 relative.  20 instructions
 // without branches or large temporaries; libm's exp and cos took the FP64 kernels to 177 and 148
 // registers (now 112 and 100: 16 water boxes forward 194 -> 155 us, adjoint 327 -> 253 us).
+// Below -1000 it takes -1000 (by the high word alone), whose result is 0 too: the reduction loses r
+// beyond 1e17, and has none at -infinity.
 __device__ __forceinline__ double fexp(double x) {
+  x = __hiloint2double(x < -1000.0 ? (int)0xc08f4000 : __double2hiint(x), __double2loint(x));
   const double n = rint(x * 1.4426950408889634);
   double r = fma(-n, 0.6931471805599453, x);
   r = fma(-n, 2.3190468138462996e-17, r);
