@@ -65,10 +65,9 @@ __device__ __forceinline__ double lit(double c) {
 // degree 13 on |r| <= ln 2 / 2 (remainder 4e-18), scaled by 2^n; 1.4e-16 relative.  20 instructions
 // without branches or large temporaries; libm's exp and cos took the FP64 kernels to 177 and 148
 // registers (now 112 and 100: 16 water boxes forward 194 -> 155 us, adjoint 327 -> 253 us).
-// Below -1000 it takes -1000 (by the high word alone), whose result is 0 too: the reduction loses r
-// beyond 1e17, and has none at -infinity.
+// The reduction loses r beyond 1e17, where the result is still 0 up to 1e35 (then the polynomial
+// overflows): the model upload keeps the angular functions' arguments below that.
 __device__ __forceinline__ double fexp(double x) {
-  x = __hiloint2double(x < -1000.0 ? (int)0xc08f4000 : __double2hiint(x), __double2loint(x));
   const double n = rint(x * 1.4426950408889634);
   double r = fma(-n, 0.6931471805599453, x);
   r = fma(-n, 2.3190468138462996e-17, r);
@@ -87,6 +86,12 @@ __device__ __forceinline__ double fexp(double x) {
   p = fma(p, r, 1.0);
   p = fma(p, r, 1.0);
   return ldexp(p, __double2int_rn(n));
+}
+// fexp of any argument (radial functions, whose shift has no bound).  In the pair loops the compare
+// and selects cost 2 % of an FP64 force call.
+__device__ __forceinline__ float fexp_any(float x) { return __expf(x); }
+__device__ __forceinline__ double fexp_any(double x) {
+  return fexp(fabs(x) > 1000.0 ? copysign(1000.0, x) : x);
 }
 __device__ __forceinline__ float fcos(float x) { return __cosf(x); }
 __device__ __forceinline__ double fcos(double x) { return cos(x); }
@@ -1543,7 +1548,7 @@ __device__ __forceinline__ double radial_sum(const AcsfArgs& a, const Slice<T>& 
       }
       U term;
       if (fn.type == 1) term = fcv;
-      else if (fn.type == 2) term = fexp(-eta * ((r - rs) * (r - rs))) * fcv;
+      else if (fn.type == 2) term = fexp_any(-eta * ((r - rs) * (r - rs))) * fcv;
       else term = fcos(kap * r) * fcv;
       acc += (double)term;
     }
@@ -1779,7 +1784,7 @@ __device__ __forceinline__ void acsf_centre(const AcsfArgs& a, const long long i
             g = dfc;
           } else if (fn.type == 2) {
             const T eta = (T)fn.eta, dr = r - (T)fn.rs;
-            g = (dfc - fc * (T)2 * eta * dr) * fexp(-eta * dr * dr);
+            g = (dfc - fc * (T)2 * eta * dr) * fexp_any(-eta * dr * dr);
           } else {
             const T kap = (T)fn.kappa;
             g = fcos(kap * r) * dfc - fsin(kap * r) * fc * kap;

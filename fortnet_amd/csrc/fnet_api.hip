@@ -1126,7 +1126,10 @@ int fnet_model_upload(fnet_ctx* ctx, const fnet_model_desc* md) {
         a.same = (z1 == z2) ? 1 : 0;
         a.atomid = atomid;
         a.rc = rc;
-        a.eta = eta;
+        // exp(-eta r^2) for r up to 2 rc is 0 (or infinite) beyond this eta unless r < 1e-13 rc, and
+        // the kernels' exponential stays within its range (NaN stays NaN)
+        const double most = 1e30 / (rc * rc);
+        a.eta = eta > most ? most : eta < -most ? -most : eta;
         grp.push_back(a);
         open[key] = (int)grp.size() - 1;
         it = open.find(key);
