@@ -26,8 +26,8 @@
 //    dense array, but without forming it and with periodic images summed exactly.
 //
 // Arithmetic is T (double or float); sums over neighbours and pairs, the values G and the forces
-// are accumulated in FP64 in both modes.  FP64 evaluates exp and the cutoff's cos and sin to within
-// 3e-16 (fexp, cut_cs), roots, quotients and real powers with libm; FP32 uses the hardware instructions (v_exp_f32, v_cos_f32,
+// are accumulated in FP64 in both modes.  FP64 evaluates exp and the cutoff's cos and sin to an ulp or
+// two from polynomials (fexp, cut_cs), roots, quotients and real powers with libm; FP32 uses the hardware instructions (v_exp_f32, v_cos_f32,
 // v_sin_f32, v_sqrt_f32, v_rcp_f32: about 1 ulp, cos/sin to ~1e-6 absolute on [0, pi]).
 #include "fnet_device.hpp"
 
@@ -116,16 +116,22 @@ __device__ __forceinline__ void dist_inv(double r2, double& r, double& ir) {
 __device__ __forceinline__ double fdiv(double x, double y) { return x / y; }
 // cos and sin of the cosine cutoff's argument x = pi r / rc for r in [0, rc] (finite beyond; the
 // callers discard those).  FP32: the hardware instructions on r (pi / rc).  FP64: with
-// u = x / 2 - pi / 4 = (pi / 4)(2 r / rc - 1), |u| <= pi / 4, cos x = -2 sin u cos u and
-// sin x = 1 - 2 sin^2 u, both from Taylor polynomials (remainders 5e-17 and 2e-18) and one rounding
-// of 2 r / rc - 1 in place of those of pi r and its quotient: as close to the exact value as libm's
-// cos of the rounded argument.
+// u = x / 2 - pi / 4 = (pi / 4)(2 r / rc - 1), |u| <= pi / 4,
+//   |cos x| = 2 |sin u| cos u = 1 - (cos u - |sin u|)^2,   sin x = 1 - 2 sin^2 u,
+// sin u and cos u from Taylor polynomials (remainders 5e-17 and 2e-18).  Written as 1 less a square,
+// cos x stays within [-1, 1] and is -1 at r = rc, so that the cutoff is 0 there and nowhere negative
+// (the product 2 sin u cos u missed 1 by an ulp on either side).  cut_cs takes 2 / rc in two parts:
+// its sine needs them near the ends.  Errors over r and rc (largest, rms): cosine 3.4e-16, 7e-17
+// (cut_cos 4.6e-16, 8e-17), sine 5.8e-16, 8e-17; of the library's cosine and sine of the rounded
+// pi r / rc 4.8e-16, 10e-17 and 6.6e-16, 11e-17.
 __device__ __forceinline__ void cut_cs(float r, float rc, float pirc, float& c, float& s) {
   c = fcos(r * pirc);
   s = fsin(r * pirc);
 }
-__device__ __forceinline__ void cut_cs(double r, double rc, double pirc, double& c, double& s) {
-  const double u = fma(r, 2.0 / rc, -1.0) * 0.78539816339744831, z = u * u;
+__device__ __forceinline__ float cut_cos(float r, float rc, float pirc) { return fcos(r * pirc); }
+// sn = sin u of u = (pi / 4) t; returns cos x
+__device__ __forceinline__ double cut_quarter(double t, double& sn) {
+  const double u = t * 0.78539816339744831, z = u * u;
   double a = lit(-1.0 / 1307674368000.0);
   a = fma(a, z, lit(1.0 / 6227020800.0));
   a = fma(a, z, lit(-1.0 / 39916800.0));
@@ -133,7 +139,7 @@ __device__ __forceinline__ void cut_cs(double r, double rc, double pirc, double&
   a = fma(a, z, lit(-1.0 / 5040.0));
   a = fma(a, z, lit(1.0 / 120.0));
   a = fma(a, z, lit(-1.0 / 6.0));
-  const double sn = fma(a * z, u, u);
+  sn = fma(a * z, u, u);
   double b = lit(1.0 / 20922789888000.0);
   b = fma(b, z, lit(-1.0 / 87178291200.0));
   b = fma(b, z, lit(1.0 / 479001600.0));
@@ -142,15 +148,18 @@ __device__ __forceinline__ void cut_cs(double r, double rc, double pirc, double&
   b = fma(b, z, lit(-1.0 / 720.0));
   b = fma(b, z, lit(1.0 / 24.0));
   b = fma(b, z, -0.5);
-  const double cs = fma(b, z, 1.0);
-  c = -2.0 * sn * cs;
+  const double d = fma(b, z, 1.0) - fabs(sn);
+  return copysign(fma(-d, d, 1.0), -sn);
+}
+__device__ __forceinline__ void cut_cs(double r, double rc, double pirc, double& c, double& s) {
+  const double i2 = 2.0 / rc, low = fma(-i2, rc, 2.0) * (0.5 * i2);
+  double sn;
+  c = cut_quarter(fma(r, low, fma(r, i2, -1.0)), sn);
   s = fma(-2.0 * sn, sn, 1.0);
 }
-template <typename T>
-__device__ __forceinline__ T cut_cos(T r, T rc, T pirc) {
-  T c, s;
-  cut_cs(r, rc, pirc, c, s);
-  return c;
+__device__ __forceinline__ double cut_cos(double r, double rc, double pirc) {
+  double sn;
+  return cut_quarter(fma(r, 2.0 / rc, -1.0), sn);
 }
 
 // A wave-uniform value moved to scalar registers (values converted from FP64 on the vector
@@ -662,6 +671,7 @@ template <> struct JkConst<float> {
     c = __builtin_amdgcn_cosf(x);
     sn = __builtin_amdgcn_sinf(x);
   }
+  __device__ __forceinline__ float cosine(float r) const { return __builtin_amdgcn_cosf(r * prev); }
 };
 template <> struct JkConst<double> {
   double rc, eta, pirc;
@@ -674,6 +684,7 @@ template <> struct JkConst<double> {
   __device__ __forceinline__ void cs(double r, double& c, double& sn) const {
     cut_cs(r, rc, pirc, c, sn);
   }
+  __device__ __forceinline__ double cosine(double r) const { return cut_cos(r, rc, pirc); }
 };
 
 // adj_geom without branches: a pair that does not exist (v false) or lies beyond the cutoff
@@ -874,9 +885,7 @@ __device__ __forceinline__ T pair_base(const JkConst<T>& K, const typename Vec4<
     const T rx = dj.x - dk.x, ry = dj.y - dk.y, rz = dj.z - dk.z;
     const T r2 = rx * rx + ry * ry + rz * rz;
     const T rjk = fsqrt(r2);
-    T cx, sx;
-    K.cs(rjk, cx, sx);
-    const T fcjk = (T)0.5 * pj.z * pk.z * (cx + (T)1);
+    const T fcjk = (T)0.5 * pj.z * pk.z * (K.cosine(rjk) + (T)1);
     base *= K.ex(r2) * fcjk;
     in = in && (rjk <= K.rc);
   }
@@ -2125,7 +2134,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8)))
 
 // FP32 forward with the radial terms in FP64 (models with an ill-conditioned radial z-score); 96
 // registers, 5 waves per SIMD (130 000 Si atoms, 12 G2 + 20 G5: 780 -> 570 us with the paired groups
-// in one walk and the polynomial exp and cos)
+// in one walk and the polynomial exp and cos; one register more, and 4 waves, cost 2 % of the step)
 template <int MQ, int FORM, bool PAIRS>
 __global__ void __launch_bounds__(512) k_acsf_fwd32_r64(AcsfArgs a) {
   acsf_wave<float, false, MQ, FORM, PAIRS, true>(a);

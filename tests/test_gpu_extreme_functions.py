@@ -34,3 +34,30 @@ def test_vanishing_exponentials(ctx, mode, eta):  # noqa: F811
     assert np.abs(G - G0).max() <= (1e-10 if mode == fa.FNET_FP64 else 1e-5) * np.abs(G0).max()
     if eta < 1e100:  # (the derivative's eta r overflows beyond)
         assert np.isfinite(F).all()
+
+
+def test_cutoff_near_its_end(ctx):  # noqa: F811
+    """Pairs up to the cutoff radius itself, one function G1 = fc(r): never negative, 0 at r = rc, and
+    close to the exact value: cos x within 5e-16 (halved, and half an ulp for the sum with 1), its
+    derivative through sin x within 6e-16 (three roundings on top)."""
+    L = np.longdouble
+    pi = L("3.14159265358979323846264338327950288")
+    dims = [1, 1]
+    for rc in (RC, 7.3, 9.0):
+        u = np.nextafter(rc, np.inf) - rc
+        r = np.concatenate([rc - u * np.arange(40), rc - u * 2.0 ** np.arange(6, 48),
+                            rc * np.random.default_rng(3).uniform(0.05, 1.0, 900)])
+        p = np.array([[1.0, 0.0, 0.0, 0.0]])  # E = G1
+        g = fa.GFunctions([1], [rc])
+        ctx.upload_model(fa.Netstat(g, [14], dims, 0, p))
+        b = ctx.batch([fa.Geometry([[0.0, 0.0, 0.0], [x, 0.0, 0.0]], [14] * 2, [0] * 2) for x in r],
+                      fa.FNET_FP64)
+        G, F = b.acsf()[::2, 0], b.forces()[1::2, 0]
+        b.close()
+        x = pi * r.astype(L) / L(rc)
+        fc, dfc = (np.cos(x) + 1) / 2, -np.sin(x) * pi / (2 * L(rc))
+        print("rc", rc, "fc", float(np.abs(G - fc).max()), "min", G.min(),
+              "sin", float(np.abs(F + 2 * dfc).max() * L(rc) / pi), flush=True)
+        assert (G >= 0.0).all() and (G[r == rc] == 0.0).all() and (r == rc).any()
+        assert np.abs(G - fc).max() <= 0.5 * 5e-16 + 1.2e-16
+        assert np.abs(F + 2 * dfc).max() * L(rc) / pi <= 6e-16 + 3 * 1.2e-16  # both atoms' energies
