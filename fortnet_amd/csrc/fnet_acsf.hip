@@ -1327,31 +1327,140 @@ __device__ __forceinline__ void lad_one(CGroup& grp, CGroup* pg,
 // R = P^s and, for groups that start above xi = 1, one P^(x0 - 1) serve all members: a power
 // function per member and pair (two in the adjoint) bound the kernels before (256 Si cells, 18 113
 // atoms, 16 angular functions in steps of 15 / 7: whole FP32 step 3.50 -> 0.44 ms).
+//
+// FP32 forms P^s as the integer power and the hardware's exp2(f log2 P) of the fraction f, FP64 with
+// an integer step as products.  The products R^k carry R's error k times, which a power function of
+// each member did not have: FP64 with a real step (EXACT) forms P, ln P and R in two parts of
+// together 3e-17 (log_dd, exp_dd), and a member's own exponent, which its place in the progression
+// misses by a rounding, enters as P^delta = 1 + delta ln P.  Error of P^xi, xi = 16, at random angles
+// (rms): 2.8e-16 (lambda 1) and 6e-16 (-1) with the library's power, 7.5e-16 and 9e-16 with one-part
+// products; the step of 128 Si cells (8 965 atoms)
+// 2519 us, 370 and 462.
+
+template <typename T>
+struct ProgPow {
+  T P, R;      // P, P^s
+  T Rl, L, B;  // EXACT: the second part of R, ln P, P^(x0 - 1)
+};
 
 template <typename T> struct ProgConst {
-  int sint, bint;
+  int sint, bint;   // integer parts of s and x0 - 1 and their fractions
   T sfrac, bfrac;
 };
 
-// P^(n + f), 0 <= f < 1: integer powers as products, the fraction through exp2 and log2 (FP64:
-// exp and log; P = 0 gives 0 for f > 0).  n and f are wave-uniform.
+constexpr double kLn2Hi = 0.6931471805592082, kLn2Lo = 7.371002565167799e-13;  // 40 bits, the rest
+
+// ln(p + pl) for p in (0, 4), pl below an ulp of p, in two parts (4e-18 and an ulp of the second):
+// p = 2^e m with m in [sqrt(1/2), sqrt(2)), ln m = 2 artanh q, q = (m - 1) / (m + 1) with its
+// remainder, the odd series to q^19.
+__device__ __forceinline__ void log_dd(double p, double pl, double& hi, double& lo) {
+  double m = __builtin_amdgcn_frexp_mant(p);
+  int e = __builtin_amdgcn_frexp_exp(p);
+  const bool small = m < lit(0.70710678118654752);
+  m = small ? m + m : m;
+  e -= small ? 1 : 0;
+  const double f = m - 1.0, d = m + 1.0, dl = f - (d - 2.0);
+  double y = __builtin_amdgcn_rcp(d);
+  y = fma(fma(-d, y, 1.0), y, y);
+  y = fma(fma(-d, y, 1.0), y, y);
+  const double q = f * y, ql = (fma(-q, d, f) - q * dl) * y, z = q * q;
+  double a = lit(2.0 / 19.0);
+  a = fma(a, z, lit(2.0 / 17.0));
+  a = fma(a, z, lit(2.0 / 15.0));
+  a = fma(a, z, lit(2.0 / 13.0));
+  a = fma(a, z, lit(2.0 / 11.0));
+  a = fma(a, z, lit(2.0 / 9.0));
+  a = fma(a, z, lit(2.0 / 7.0));
+  a = fma(a, z, lit(2.0 / 5.0));
+  a = fma(a, z, lit(2.0 / 3.0));
+  const double u = (double)e * lit(kLn2Hi), v = q + q;
+  const double h = u + v, w = fma(a * z, q, ql + ql);
+  const double t = (u - h) + v +  // (u is 0 or the larger)
+                   fma((double)e, lit(kLn2Lo), fma(ldexp(pl, -e), __builtin_amdgcn_rcp(m), w));
+  hi = h + t;
+  lo = t - (hi - h);
+}
+
+// exp(x + xl) in two parts (2e-17): as fexp, the sum 1 + r + ... kept in two parts
+__device__ __forceinline__ void exp_dd(double x, double xl, double& hi, double& lo) {
+  const double n = rint(x * lit(1.4426950408889634));
+  const double r0 = fma(-n, lit(kLn2Hi), x), r1 = fma(-n, lit(kLn2Lo), xl);
+  const double r = r0 + r1, rl = (r0 - r) + r1;
+  double q = lit(1.0 / 6227020800.0);
+  q = fma(q, r, lit(1.0 / 479001600.0));
+  q = fma(q, r, lit(1.0 / 39916800.0));
+  q = fma(q, r, lit(1.0 / 3628800.0));
+  q = fma(q, r, lit(1.0 / 362880.0));
+  q = fma(q, r, lit(1.0 / 40320.0));
+  q = fma(q, r, lit(1.0 / 5040.0));
+  q = fma(q, r, lit(1.0 / 720.0));
+  q = fma(q, r, lit(1.0 / 120.0));
+  q = fma(q, r, lit(1.0 / 24.0));
+  q = fma(q, r, lit(1.0 / 6.0));
+  q = fma(q, r, 0.5);
+  const double s = r + 1.0, t = (r - (s - 1.0)) + fma(r * r, q, rl * s), h = s + t;
+  const int k = __double2int_rn(n);
+  hi = ldexp(h, k);
+  lo = ldexp(t - (h - s), k);
+}
+
+// P^(n + f), 0 <= f < 1 (P = 0 gives 0 for f > 0); n and f are wave-uniform, f is 0 in FP64
 __device__ __forceinline__ float pow_split(float P, int n, float f) {
   float r = powi(P, n);
   if (f != 0.0f) r *= __builtin_amdgcn_exp2f(f * __builtin_amdgcn_logf(P));
   return r;
 }
-__device__ __forceinline__ double pow_split(double P, int n, double f) {
-  double r = powi(P, n);
-  if (f != 0.0) r *= exp(f * log(P));
-  return r;
+__device__ __forceinline__ double pow_split(double P, int n, double f) { return powi(P, n); }
+
+template <bool EXACT, typename T>
+__device__ __forceinline__ ProgPow<T> prog_pow(T c, T lam, const ProgConst<T>& pc) {
+  ProgPow<T> w;
+  w.Rl = w.L = w.B = 0;
+  if constexpr (EXACT) {
+    w.P = fma(lam, c, 1.0);
+    const bool zero = w.P == 0.0;
+    double Ll;
+    log_dd(zero ? 1.0 : w.P, fma(lam, c, 1.0 - w.P), w.L, Ll);
+    auto power = [&](double x, double& hi, double& lo) {
+      const double y = x * w.L;
+      exp_dd(y, fma(x, w.L, -y) + x * Ll, hi, lo);
+      hi = zero ? 0.0 : hi;
+      lo = zero ? 0.0 : lo;
+    };
+    power((double)pc.sint + pc.sfrac, w.R, w.Rl);
+    if (pc.bfrac != 0.0) {
+      double lo;
+      power((double)pc.bint + pc.bfrac, w.B, lo);
+    } else {
+      w.B = powi(w.P, pc.bint);
+    }
+  } else {
+    w.P = (T)1 + lam * c;
+    w.R = pow_split(w.P, pc.sint, pc.sfrac);
+  }
+  return w;
+}
+
+// t P^(delta_k) and, in t, the next member's term
+template <bool EXACT, typename T>
+__device__ __forceinline__ T prog_term(T& t, const ProgPow<T>& w, T delta) {
+  T v = t;
+  if constexpr (EXACT) {
+    v = fma(t, delta * w.L, t);
+    t = fma(t, w.R, t * w.Rl);
+  } else {
+    t *= w.R;
+  }
+  return v;
 }
 
 // Forward: off-diagonal pairs, two per step, FP64 sums per slot; the two pairs' terms are added in
 // T before the conversion.
-template <typename T, int K, bool SAME, bool G4>
+template <typename T, int K, bool SAME, bool G4, bool EXACT>
 __device__ __forceinline__ void pairs_fwd_prog(const Slice<T>& sl, int lane, int A0, int LA, int B0,
                                                int LB, T lam0, T lam1, const JkConst<T>& J,
-                                               const ProgConst<T>& pc, double (&acc)[2][K]) {
+                                               const ProgConst<T>& pc, const T (&delta)[K],
+                                               double (&acc)[2][K]) {
   using V = typename Vec4<T>::type;
   PairWalk2<SAME> it;
   it.init(lane, A0, LA, B0, LB);
@@ -1367,30 +1476,29 @@ __device__ __forceinline__ void pairs_fwd_prog(const Slice<T>& sl, int lane, int
 #pragma unroll
     for (int l = 0; l < 2; ++l) {
       const T lam = l ? lam1 : lam0;
-      const T P1 = (T)1 + lam * c1, P2 = (T)1 + lam * c2;
-      const T R1 = pow_split(P1, pc.sint, pc.sfrac), R2 = pow_split(P2, pc.sint, pc.sfrac);
-      T t1 = b1 * P1, t2 = b2 * P2;
+      const ProgPow<T> w1 = prog_pow<EXACT>(c1, lam, pc), w2 = prog_pow<EXACT>(c2, lam, pc);
+      T t1 = b1 * w1.P, t2 = b2 * w2.P;
       if (pc.bint || pc.bfrac != (T)0) {
-        t1 *= pow_split(P1, pc.bint, pc.bfrac);
-        t2 *= pow_split(P2, pc.bint, pc.bfrac);
+        t1 *= EXACT ? w1.B : pow_split(w1.P, pc.bint, pc.bfrac);
+        t2 *= EXACT ? w2.B : pow_split(w2.P, pc.bint, pc.bfrac);
       }
 #pragma unroll
       for (int k = 0; k < K; ++k) {
-        acc[l][k] += (double)(t1 + t2);
-        t1 *= R1;
-        t2 *= R2;
+        const T u1 = prog_term<EXACT>(t1, w1, delta[k]), u2 = prog_term<EXACT>(t2, w2, delta[k]);
+        acc[l][k] += (double)(u1 + u2);
       }
     }
   }
 }
 
-// Adjoint: with H0 = sum_k c0_k R^k and H1 = sum_k c1_k R^k (Horner), S0 = P^x0 H0 and its
-// derivative in cos(theta) S1 = P^(x0 - 1) H1; c0, c1 as in pairs_adj_lad.
-template <typename T, int K, bool SAME, bool G4>
+// Adjoint: with H0 = sum_k c0_k R^k and H1 = sum_k c1_k R^k, S0 = P^x0 H0 and its derivative in
+// cos(theta) S1 = P^(x0 - 1) H1; c0, c1 as in pairs_adj_lad (EXACT: H1 from c0 and the exponents
+// lambda (x0 + k s), whose array would not fit the scalar registers beside c0).
+template <typename T, int K, bool SAME, bool G4, bool EXACT>
 __device__ __forceinline__ void pairs_adj_prog(const Slice<T>& sl, int lane, int A0, int LA, int B0,
                                                int LB, T lam0, T lam1, const T (&c0)[2][K],
                                                const T (&c1)[2][K], const JkConst<T>& J,
-                                               const ProgConst<T>& pc) {
+                                               const ProgConst<T>& pc, const T (&delta)[K]) {
   using V = typename Vec4<T>::type;
   PairWalk2<SAME> it;
   it.init(lane, A0, LA, B0, LB);
@@ -1403,20 +1511,34 @@ __device__ __forceinline__ void pairs_adj_prog(const Slice<T>& sl, int lane, int
     T S0 = 0, S1 = 0;
 #pragma unroll
     for (int l = 0; l < 2; ++l) {
-      const T P = (T)1 + (l ? lam1 : lam0) * c;
-      const T R = pow_split(P, pc.sint, pc.sfrac);
-      T h0 = c0[l][K - 1], h1 = c1[l][K - 1];
+      const T lam = l ? lam1 : lam0;
+      const ProgPow<T> w = prog_pow<EXACT>(c, lam, pc);
+      T h0, h1;
+      if constexpr (EXACT) {
+        double t = 1.0;
+        h0 = h1 = 0.0;
 #pragma unroll
-      for (int k = K - 2; k >= 0; --k) {
-        h0 = h0 * R + c0[l][k];
-        h1 = h1 * R + c1[l][k];
+        for (int k = 0; k < K; ++k) {
+          const double u = c0[l][k] * prog_term<EXACT>(t, w, delta[k]);
+          h0 += u;
+          h1 = fma((double)k, u, h1);
+        }
+        h1 = lam * fma((double)pc.sint + pc.sfrac, h1, ((double)pc.bint + pc.bfrac + 1.0) * h0);
+      } else {
+        h0 = c0[l][K - 1];
+        h1 = c1[l][K - 1];
+#pragma unroll
+        for (int k = K - 2; k >= 0; --k) {
+          h0 = h0 * w.R + c0[l][k];
+          h1 = h1 * w.R + c1[l][k];
+        }
       }
       if (pc.bint || pc.bfrac != (T)0) {
-        const T B = pow_split(P, pc.bint, pc.bfrac);
+        const T B = EXACT ? w.B : pow_split(w.P, pc.bint, pc.bfrac);
         h0 *= B;
         h1 *= B;
       }
-      S0 += P * h0;
+      S0 += w.P * h0;
       S1 += h1;
     }
     adj_pair<T, G4>(sl, ek, dj, pj, dk, pk, rr, c, H, Hq, v, S0, S1, js);
@@ -1431,10 +1553,10 @@ __device__ __forceinline__ void pairs_adj_prog(const Slice<T>& sl, int lane, int
 }
 
 // One progression group of one centre; K >= the group's exponents, the slots beyond them unused.
-template <typename T, bool ADJ, int K>
-__device__ __forceinline__ void group_prog(CGroup& grp, const Slice<T>& sl, int lane, long long i,
-                                           int A0, int L1, int B0, int L2, T rc, T eta, T pirc,
-                                           cdouble* cG, double* G, int nG) {
+template <typename T, bool ADJ, int K, bool EXACT>
+__device__ __forceinline__ void group_prog_of(CGroup& grp, const Slice<T>& sl, int lane,
+                                              long long i, int A0, int L1, int B0, int L2, T rc,
+                                              T eta, T pirc, cdouble* cG, double* G, int nG) {
   const bool g4 = grp.type == 4;
   const bool same = grp.same != 0;
   const T lam0 = uniform((T)grp.lamv[0]), lam1 = uniform((T)grp.lamv[1]);
@@ -1445,6 +1567,9 @@ __device__ __forceinline__ void group_prog(CGroup& grp, const Slice<T>& sl, int 
   pc.bint = grp.bint;
   pc.sfrac = uniform((T)grp.sfrac);
   pc.bfrac = uniform((T)grp.bfrac);
+  T delta[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) delta[k] = EXACT ? (T)grp.pdelta[k] : (T)0;
   if constexpr (!ADJ) {
     double acc[2][K];
 #pragma unroll
@@ -1460,21 +1585,17 @@ __device__ __forceinline__ void group_prog(CGroup& grp, const Slice<T>& sl, int 
         const T cjj = diag_cos(sl.d[A0 + e], (T)0);
 #pragma unroll
         for (int l = 0; l < 2; ++l) {
-          const T P = (T)1 + (l ? lam1 : lam0) * cjj;
-          const T R = pow_split(P, pc.sint, pc.sfrac);
-          T t = base * P * pow_split(P, pc.bint, pc.bfrac);
+          const ProgPow<T> w = prog_pow<EXACT>(cjj, l ? lam1 : lam0, pc);
+          T t = base * w.P * (EXACT ? w.B : pow_split(w.P, pc.bint, pc.bfrac));
 #pragma unroll
-          for (int k = 0; k < K; ++k) {
-            acc[l][k] += (double)t;
-            t *= R;
-          }
+          for (int k = 0; k < K; ++k) acc[l][k] += (double)prog_term<EXACT>(t, w, delta[k]);
         }
       }
-      if (g4) pairs_fwd_prog<T, K, true, true>(sl, lane, A0, L1, B0, L2, lam0, lam1, J, pc, acc);
-      else pairs_fwd_prog<T, K, true, false>(sl, lane, A0, L1, B0, L2, lam0, lam1, J, pc, acc);
+      if (g4) pairs_fwd_prog<T, K, true, true, EXACT>(sl, lane, A0, L1, B0, L2, lam0, lam1, J, pc, delta, acc);
+      else pairs_fwd_prog<T, K, true, false, EXACT>(sl, lane, A0, L1, B0, L2, lam0, lam1, J, pc, delta, acc);
     } else {
-      if (g4) pairs_fwd_prog<T, K, false, true>(sl, lane, A0, L1, B0, L2, lam0, lam1, J, pc, acc);
-      else pairs_fwd_prog<T, K, false, false>(sl, lane, A0, L1, B0, L2, lam0, lam1, J, pc, acc);
+      if (g4) pairs_fwd_prog<T, K, false, true, EXACT>(sl, lane, A0, L1, B0, L2, lam0, lam1, J, pc, delta, acc);
+      else pairs_fwd_prog<T, K, false, false, EXACT>(sl, lane, A0, L1, B0, L2, lam0, lam1, J, pc, delta, acc);
     }
     // the slot sums in one exchange; slot (l, k) has flat index l K + k
     constexpr int NA = pow2_at_least(2 * K);
@@ -1516,13 +1637,26 @@ __device__ __forceinline__ void group_prog(CGroup& grp, const Slice<T>& sl, int 
         sl.gs[3 * ej + 1] += gsc * dj.y;
         sl.gs[3 * ej + 2] += gsc * dj.z;
       }
-      if (g4) pairs_adj_prog<T, K, true, true>(sl, lane, A0, L1, B0, L2, lam0, lam1, c0, c1, J, pc);
-      else pairs_adj_prog<T, K, true, false>(sl, lane, A0, L1, B0, L2, lam0, lam1, c0, c1, J, pc);
+      if (g4) pairs_adj_prog<T, K, true, true, EXACT>(sl, lane, A0, L1, B0, L2, lam0, lam1, c0, c1, J, pc, delta);
+      else pairs_adj_prog<T, K, true, false, EXACT>(sl, lane, A0, L1, B0, L2, lam0, lam1, c0, c1, J, pc, delta);
     } else {
-      if (g4) pairs_adj_prog<T, K, false, true>(sl, lane, A0, L1, B0, L2, lam0, lam1, c0, c1, J, pc);
-      else pairs_adj_prog<T, K, false, false>(sl, lane, A0, L1, B0, L2, lam0, lam1, c0, c1, J, pc);
+      if (g4) pairs_adj_prog<T, K, false, true, EXACT>(sl, lane, A0, L1, B0, L2, lam0, lam1, c0, c1, J, pc, delta);
+      else pairs_adj_prog<T, K, false, false, EXACT>(sl, lane, A0, L1, B0, L2, lam0, lam1, c0, c1, J, pc, delta);
     }
   }
+}
+
+template <typename T, bool ADJ, int K>
+__device__ __forceinline__ void group_prog(CGroup& grp, const Slice<T>& sl, int lane, long long i,
+                                           int A0, int L1, int B0, int L2, T rc, T eta, T pirc,
+                                           cdouble* cG, double* G, int nG) {
+  if constexpr (std::is_same<T, double>::value) {
+    if (grp.pexact) {
+      group_prog_of<T, ADJ, K, true>(grp, sl, lane, i, A0, L1, B0, L2, rc, eta, pirc, cG, G, nG);
+      return;
+    }
+  }
+  group_prog_of<T, ADJ, K, false>(grp, sl, lane, i, A0, L1, B0, L2, rc, eta, pirc, cG, G, nG);
 }
 
 // Forward value of one radial function (G1/G2/G3, acsf.F90:1287-1373) summed over the staged

@@ -1,6 +1,7 @@
 // C-ABI of libfnet_hip.so: context, model and batch management and the stage drivers.
 // Declarations and their reference counterparts are in include/fnet_hip.h.
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -144,13 +145,14 @@ void ladder_form(AngGroup& a) {
 // Fills the progression form of an angular group (np = 0 when it does not have it): at most two
 // lambda values of at most 1 in size (P = 1 + lambda cos(theta) stays >= 0: below it, P^s has no
 // real value where integer members of the group have one), exponents x0 + k s with x0 >= 1
-// (P^(x0 - 1) stays finite at P = 0) and at most kProgLen of them, each (lambda, xi) once.  The automatic ACSF scheme steps xi evenly from 1
-// (acsf.F90:276-363); a group split at kMaxMembers continues the steps from a larger x0.  The
+// (P^(x0 - 1) stays finite at P = 0) and at most kProgLen of them, each (lambda, xi) once.  The automatic ACSF
+// scheme steps xi evenly from 1 (acsf.F90:276-363), rounded; a group split at kMaxMembers continues the steps from a larger x0.  The
 // largest exponent is bounded so that the padded slots of the kernels stay finite in FP32.
 void progression_form(AngGroup& a) {
-  a.np = a.sint = a.bint = 0;
+  a.np = a.sint = a.bint = a.pexact = 0;
   a.sfrac = a.bfrac = 0.0;
   for (int k = 0; k < 2 * kProgLen; ++k) a.pmem[k] = -1;
+  for (int k = 0; k < kProgLen; ++k) a.pdelta[k] = 0.0;
   if (a.lad) return;
   std::vector<double> lam(a.lam, a.lam + a.nmem), xi(a.xi, a.xi + a.nmem);
   auto distinct = [](std::vector<double>& v) {
@@ -163,8 +165,10 @@ void progression_form(AngGroup& a) {
   if (lam.size() > 2 || K > kProgLen || K < 1 || !(xi[0] >= 1.0)) return;
   if (!(lam.front() >= -1.0 && lam.back() <= 1.0)) return;
   const double s = K > 1 ? (xi[K - 1] - xi[0]) / (K - 1) : 0.0;
-  for (int k = 0; k < K; ++k)
-    if (std::fabs(xi[k] - (xi[0] + k * s)) > 1e-14 * xi[k]) return;
+  for (int k = 0; k < K; ++k) {
+    a.pdelta[k] = (double)((long double)xi[k] - ((long double)xi[0] + (long double)k * s));
+    if (!(std::fabs(a.pdelta[k]) <= 8 * DBL_EPSILON * xi[k])) return;
+  }
   if (!(xi[0] + kProgLen * s <= 120.0)) return;
   for (int q = 0; q < a.nmem; ++q) {
     const int i = a.lam[q] == lam[0] ? 0 : 1;
@@ -177,19 +181,14 @@ void progression_form(AngGroup& a) {
   }
   a.lamv[0] = lam[0];
   a.lamv[1] = lam.size() > 1 ? lam[1] : lam[0];
-  // an integer step (or base) within rounding is taken as one: products instead of a real power
   auto split = [](double x, int& n, double& f) {
     n = (int)std::floor(x);
     f = x - n;
-    if (f > 1.0 - 1e-14) {
-      n += 1;
-      f = 0.0;
-    } else if (f < 1e-14) {
-      f = 0.0;
-    }
   };
   split(s, a.sint, a.sfrac);
   split(xi[0] - 1.0, a.bint, a.bfrac);
+  a.pexact = a.sfrac != 0.0 || a.bfrac != 0.0;
+  for (int k = 0; k < K; ++k) a.pexact = a.pexact || a.pdelta[k] != 0.0;
   a.np = K;
 }
 

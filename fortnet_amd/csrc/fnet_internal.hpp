@@ -65,6 +65,8 @@ struct AngGroup {
   int np;
   int sint, bint;       // integer parts of s and x0 - 1
   double sfrac, bfrac;  // their fractions
+  double pdelta[kProgLen];  // xi_k - (x0 + k s), a few ulp of xi_k at most
+  int pexact;               // some exponent is no integer
   int pmem[2 * kProgLen];
   // Adjoint pass: a G5 ladder group and another one over the same lists with the same ladder
   // and lambdas but another eta are evaluated together (partner >= 0 on the first one,
