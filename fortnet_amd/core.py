@@ -358,8 +358,14 @@ class Batch:
 
     def reload(self, geos):
         """``fnet_batch_reload``: new structures in the same device buffers (serving)."""
-        d = self._describe(geos)
-        check(self.ctx.h, self.lib.fnet_batch_reload(self.h, ctypes.byref(d)), "fnet_batch_reload")
+        kept = dict(self.__dict__)
+        try:
+            d = self._describe(geos)
+            check(self.ctx.h, self.lib.fnet_batch_reload(self.h, ctypes.byref(d)),
+                  "fnet_batch_reload")
+        except Exception:
+            self.__dict__.update(kept)  # the sizes of the structures that are still loaded
+            raise
 
     def query(self):
         """True while work queued on the context is still running (``fnet_query``)."""

@@ -596,18 +596,24 @@ int do_adjoint(fnet_batch* b) {
 // searched with cell lists when that tests fewer candidates, priced at kCellCandidateCost, than
 // the direct scan (per centre: 27 bins of n / (nb_0 nb_1 nb_2) atoms, against n atoms in each of
 // the ~(1 + 2 w_a) images per axis that the scan's image pruning keeps, w_a = rc / width_a);
-// any other structure takes the direct scan.
-// `fresh`: the device tables hold nothing of this batch yet (else equal tables stay as they are).
-int setup_cells(fnet_batch* b, const double* lat, const int* per, bool fresh) {
-  fnet_ctx* ctx = b->ctx;
-  const double rc = ctx->model.rcmax;
-  std::vector<int> info(4 * (size_t)b->S, 0), coff(b->S + 1, 0);
+// any other structure takes the direct scan.  plan_cells works out (and refuses) on the host, before
+// anything of the batch changes.
+struct CellPlan {
+  std::vector<int> info, off;  // [4 S] bins per axis and 1 (0: no cell list); [S + 1] first cell
   long long total = 0, bins = 0;
   int used = 0;
   bool in_prep = true;  // every cell-list structure fits one struct-prep block
-  for (int s = 0; s < b->S; ++s) {
-    coff[s] = (int)total;
-    const long long n = b->h_off[s + 1] - b->h_off[s];
+};
+
+int plan_cells(fnet_ctx* ctx, int S, const long long* offsets, const double* lat, const int* per,
+               CellPlan& plan) {
+  const double rc = ctx->model.rcmax;
+  std::vector<int>&info = plan.info, &coff = plan.off;
+  info.assign(4 * (size_t)S, 0);
+  coff.assign(S + 1, 0);
+  for (int s = 0; s < S; ++s) {
+    coff[s] = (int)plan.total;
+    const long long n = offsets[s + 1] - offsets[s];
     if (!per[s] || n < kCellMinAtoms) continue;
     const double* L = lat + 9 * s;
     auto o = [&](int r, int c) { return L[c * 3 + r]; };
@@ -641,15 +647,24 @@ int setup_cells(fnet_batch* b, const double* lat, const int* per, bool fresh) {
     info[4 * s + 3] = 1;
     // one more than the bins: the end of the structure's last bin
     const long long nbins = (long long)nb[0] * nb[1] * nb[2];
-    total += nbins + 1;
-    bins = std::max(bins, nbins);
-    in_prep = in_prep && n <= kPrepBinAtoms && nbins <= kPrepBins;
-    ++used;
+    plan.total += nbins + 1;
+    plan.bins = std::max(plan.bins, nbins);
+    plan.in_prep = plan.in_prep && n <= kPrepBinAtoms && nbins <= kPrepBins;
+    ++plan.used;
+    if (plan.total >= (1LL << 30)) return fail(ctx, FNET_ERR_CAPACITY, "too many cells");
   }
-  b->n_cell_struct = used;
-  b->bin_lds = used && in_prep ? (int)bins : 0;
-  coff[b->S] = (int)total;
-  if (total >= (1LL << 30)) return fail(ctx, FNET_ERR_CAPACITY, "too many cells");
+  coff[S] = (int)plan.total;
+  return FNET_OK;
+}
+
+// Takes a plan for the batch.  `fresh`: the device tables hold nothing of this batch yet (else equal
+// tables stay as they are).
+int take_cells(fnet_batch* b, const CellPlan& plan, bool fresh) {
+  fnet_ctx* ctx = b->ctx;
+  const std::vector<int>&info = plan.info, &coff = plan.off;
+  const long long total = plan.total;
+  b->n_cell_struct = plan.used;
+  b->bin_lds = plan.used && plan.in_prep ? (int)plan.bins : 0;
   if (!fresh && info == b->h_cellinfo) return FNET_OK;
   if (!b->cellinfo) {
     HIPCHECK(ctx, dalloc(&b->cellinfo, (size_t)b->S));
@@ -663,6 +678,7 @@ int setup_cells(fnet_batch* b, const double* lat, const int* per, bool fresh) {
     dfree(b->cell_start);
     dfree(b->cell_scan_tmp);
     b->cell_count = b->cell_start = b->cell_scan_tmp = nullptr;
+    b->cell_cap = 0;
     HIPCHECK(ctx, dalloc(&b->cell_count, (size_t)total));
     HIPCHECK(ctx, dalloc(&b->cell_start, (size_t)total + 1));
     HIPCHECK(ctx, dalloc(&b->cell_scan_tmp, (size_t)scan_tmp_size(total)));
@@ -946,6 +962,7 @@ int check_ready(fnet_ctx* ctx, fnet_batch* b) {
   if (!b) return fail(ctx, FNET_ERR_ARG, "batch is NULL");
   if (b->ctx != ctx) return fail(ctx, FNET_ERR_ARG, "batch belongs to another context");
   if (!ctx->model.valid) return fail(ctx, FNET_ERR_STATE, "no model uploaded");
+  if (!b->loaded) return fail(ctx, FNET_ERR_STATE, "the batch's last load failed");
   HIPCHECK(ctx, hipSetDevice(ctx->device));
   // results of an earlier model (list cutoff, functions, networks) or of earlier parameters
   // are stale
@@ -1349,6 +1366,11 @@ int load_batch(fnet_ctx* ctx, fnet_batch* b, const fnet_batch_desc* d) {
     zc[i] = last_c;
     zone = zone && last_c == 0;
   }
+  CellPlan cells;
+  if (const int crc = plan_cells(ctx, S, d->offsets, lat.data(), per.data(), cells)) return crc;
+  // (what was refused so far left the batch as it was; from here on it has to get through)
+  b->loaded = false;
+  invalidate(b);
   const hipStream_t s = ctx->stream;
   // chunks of the energy reduction: kEnergyChunk atoms of one structure each
   std::vector<int> chunks(S + 1, 0);  // chunk_first, then (padded) chunk_struct
@@ -1381,6 +1403,7 @@ int load_batch(fnet_ctx* ctx, fnet_batch* b, const fnet_batch_desc* d) {
     b->atom_struct = b->species = b->zcode = b->cnt = b->rowptr = b->scan_tmp = nullptr;
     b->atom_cell = b->cell_atoms = nullptr;
     b->atom_m = nullptr;
+    b->capN = 0;
     const long long cap = std::max<long long>(N, 1);
     HIPCHECK(ctx, dalloc(&b->xyz, (size_t)3 * cap));
     HIPCHECK(ctx, dalloc(&b->atom_struct, (size_t)cap));
@@ -1397,8 +1420,10 @@ int load_batch(fnet_ctx* ctx, fnet_batch* b, const fnet_batch_desc* d) {
   if (grow_e) {
     dfree(b->ext);
     b->ext = nullptr;
-    b->capExt = std::max<long long>(N * d->n_ext, 1);
-    HIPCHECK(ctx, dalloc(&b->ext, (size_t)b->capExt));
+    b->capExt = 0;
+    const long long cap = std::max<long long>(N * d->n_ext, 1);
+    HIPCHECK(ctx, dalloc(&b->ext, (size_t)cap));
+    b->capExt = cap;
   }
   if (grow_s) {
     void* ps[] = {b->lat, b->periodic, b->off, b->sinfo, b->cellinfo, b->cell_off};
@@ -1408,6 +1433,7 @@ int load_batch(fnet_ctx* ctx, fnet_batch* b, const fnet_batch_desc* d) {
     b->off = nullptr;
     b->sinfo = nullptr;
     b->cellinfo = nullptr;
+    b->capS = 0;
     const long long cap = std::max(S, 1);
     HIPCHECK(ctx, dalloc(&b->lat, (size_t)9 * cap));
     HIPCHECK(ctx, dalloc(&b->periodic, (size_t)cap));
@@ -1455,13 +1481,13 @@ int load_batch(fnet_ctx* ctx, fnet_batch* b, const fnet_batch_desc* d) {
   HIPCHECK(ctx, stage_in(ctx, b->zcode, zc.data(), sizeof(int) * N));
   HIPCHECK(ctx, stage_in(ctx, b->chunk_tab, chunks.data(), sizeof(int) * chunks.size()));
   HIPCHECK(ctx, stage_in(ctx, b->ext, d->ext, sizeof(double) * N * d->n_ext));
-  invalidate(b);
   b->tile_atoms = 0;  // species layout changed: rebuild the network tiles
   b->result_precision = -1;
   b->gen++;
-  const int rc = setup_cells(b, lat.data(), per.data(), true);
+  const int rc = take_cells(b, cells, true);
   if (rc) return rc;
   HIPCHECK(ctx, stage_flush(ctx));
+  b->loaded = true;
   return FNET_OK;
 }
 
@@ -1520,6 +1546,7 @@ int fnet_batch_update_coords(fnet_batch* b, const double* coords, const double* 
   if (!b) return FNET_ERR_ARG;
   fnet_ctx* ctx = b->ctx;
   if (!coords) return fail(ctx, FNET_ERR_ARG, "coords is NULL");
+  if (!b->loaded) return fail(ctx, FNET_ERR_STATE, "the batch's last load failed");
   // the new cells pass the checks of a batch upload before anything is copied or launched
   if (latvecs)
     for (int st = 0; st < b->S; ++st)
@@ -1529,16 +1556,25 @@ int fnet_batch_update_coords(fnet_batch* b, const double* coords, const double* 
         if (lrc) return lrc;
       }
   HIPCHECK(ctx, hipSetDevice(ctx->device));
+  CellPlan cells;
+  if (latvecs) {
+    std::vector<double> lat = b->h_lat;
+    for (int q = 0; q < 9 * b->S; ++q)
+      if (b->h_periodic[q / 9]) lat[q] = latvecs[q];
+    const int crc = plan_cells(ctx, b->S, b->h_off.data(), lat.data(), b->h_periodic.data(), cells);
+    if (crc) return crc;
+    b->h_lat = lat;
+  }
+  b->loaded = false;  // until everything is on its way
+  invalidate(b);
   HIPCHECK(ctx, stage_in(ctx, b->xyz, coords, sizeof(double) * 3 * b->N));
   if (latvecs) {
     HIPCHECK(ctx, stage_in(ctx, b->lat, latvecs, sizeof(double) * 9 * b->S));
-    for (int q = 0; q < 9 * b->S; ++q)
-      if (b->h_periodic[q / 9]) b->h_lat[q] = latvecs[q];
-    const int crc = setup_cells(b, b->h_lat.data(), b->h_periodic.data(), false);
+    const int crc = take_cells(b, cells, false);
     if (crc) return crc;
   }
   HIPCHECK(ctx, stage_flush(ctx));
-  invalidate(b);
+  b->loaded = true;
   return FNET_OK;
 }
 

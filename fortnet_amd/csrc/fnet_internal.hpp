@@ -342,6 +342,7 @@ struct fnet_batch {
   double* h_res = nullptr;
   size_t h_res_cap = 0;
   bool host_E = false, host_F = false;
+  bool loaded = false;          // the last load or update got through
   bool pending = false;
   int pending_level = 0;        // what was computed on that list: 1 features, 2 energies, 3 forces
   long long gen = 0;            // bumped whenever a buffer the step uses is reallocated
