@@ -38,6 +38,11 @@ int fail(fnet_ctx* ctx, int code, const std::string& msg) {
   if (ctx) {
     ctx->err = msg;
     ctx->segs.n = 0;  // copies of a call that did not get through are not made
+    if (ctx->stage_direct) {
+      // ... or, as commands of their own, done before the caller takes its memory back
+      ctx->stage_direct = false;
+      (void)hipStreamSynchronize(ctx->stream);
+    }
   }
   return code;
 }
@@ -1910,6 +1915,10 @@ int fnet_train_gradients(fnet_ctx* ctx, fnet_batch* b, int n_global, const doubl
   if (n_global < 0 || n_global > m.nout) return fail(ctx, FNET_ERR_ARG, "invalid n_global");
   if (n_global > 0 && !g_targets) return fail(ctx, FNET_ERR_ARG, "g_targets missing");
   if (n_global < m.nout && !a_targets) return fail(ctx, FNET_ERR_ARG, "a_targets missing");
+  double wsum = dp_weights ? 0.0 : (double)b->S;
+  if (dp_weights)
+    for (int k = 0; k < b->S; ++k) wsum += dp_weights[k];
+  if (!(wsum > 0.0)) return fail(ctx, FNET_ERR_ARG, "datapoint weights sum to zero");
   rc = evaluate(b, 1);
   if (!rc) rc = validate_step(b);
   if (rc) return rc;
@@ -1933,18 +1942,11 @@ int fnet_train_gradients(fnet_ctx* ctx, fnet_batch* b, int n_global, const doubl
   double* at = gt + (long long)b->S * n_global;
   double* aw = at + b->N * na;
   double* dpw = aw + b->N;
-  double wsum = 0.0;
   if (n_global > 0)
     HIPCHECK(ctx, stage_in(ctx, gt, g_targets, sizeof(double) * b->S * n_global));
   if (na > 0) HIPCHECK(ctx, stage_in(ctx, at, a_targets, sizeof(double) * b->N * na));
   if (atomic_weights) HIPCHECK(ctx, stage_in(ctx, aw, atomic_weights, sizeof(double) * b->N));
-  if (dp_weights) {
-    HIPCHECK(ctx, stage_in(ctx, dpw, dp_weights, sizeof(double) * b->S));
-    for (int k = 0; k < b->S; ++k) wsum += dp_weights[k];
-  } else {
-    wsum = (double)b->S;
-  }
-  if (!(wsum > 0.0)) return fail(ctx, FNET_ERR_ARG, "datapoint weights sum to zero");
+  if (dp_weights) HIPCHECK(ctx, stage_in(ctx, dpw, dp_weights, sizeof(double) * b->S));
   HIPCHECK(ctx, stage_flush(ctx));
   double* dloss = dpw + b->S;
   const LossInput li = {n_global, ctx->loss, gt, at, atomic_weights ? aw : nullptr,

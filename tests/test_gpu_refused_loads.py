@@ -60,3 +60,21 @@ def test_refused_cell(ctx):  # noqa: F811
     b.update_coords(coords)  # the refused cells and coordinates have left nothing behind
     assert np.array_equal(b.forces(), want)
     b.close()
+
+
+def test_refused_weights(ctx):  # noqa: F811
+    """Datapoint weights that sum to zero are refused before the targets (here more than the staged
+    copies take, so a copy command of their own) are on their way; the next call is as any other."""
+    ctx.upload_model(_model())
+    rng = np.random.default_rng(4)
+    geos = [fa.Geometry([[0.0, 0.0, 0.0], [d, 0.0, 0.0]], [14] * 2, [0] * 2)
+            for d in rng.uniform(3.0, 7.0, 35000)]
+    b = ctx.batch(geos, fa.FNET_FP64)
+    at, w = rng.normal(size=(b.N, 1)), rng.uniform(0.5, 1.5, b.S)
+    want = b.train_gradients(a_targets=at, dp_weights=w, n_global=0)
+    loss = b.loss
+    with pytest.raises(fa.FnetError, match="sum to zero"):
+        b.train_gradients(a_targets=np.zeros((b.N, 1)), dp_weights=np.zeros(b.S), n_global=0)
+    got = b.train_gradients(a_targets=at, dp_weights=w, n_global=0)
+    assert b.loss == loss and all(np.array_equal(x, y) for x, y in zip(want, got))
+    b.close()
