@@ -962,6 +962,32 @@ int validate_step(fnet_batch* b) {
   return settle_list(b, nullptr);
 }
 
+int check_lattice(fnet_ctx* ctx, const double* L, double rcmax, int s, long long natoms);
+
+// A resident batch under a model uploaded after it: the checks of a load that depend on the model,
+// the element slots, and the bins for its cutoff.
+int fit_model(fnet_batch* b) {
+  fnet_ctx* ctx = b->ctx;
+  const DevModel& m = ctx->model;
+  if (m.need_ext > b->next)
+    return fail(ctx, FNET_ERR_ARG, "the model needs more external feature columns than the batch has");
+  if (b->max_species >= m.nspecies)
+    return fail(ctx, FNET_ERR_ARG, "the batch has a species index that the model has not");
+  for (int s = 0; s < b->S; ++s)
+    if (b->h_periodic[s]) {
+      const int rc = check_lattice(ctx, &b->h_lat[9 * s], m.rcmax, s, b->h_off[s + 1] - b->h_off[s]);
+      if (rc) return rc;
+    }
+  CellPlan cells;
+  int rc = plan_cells(ctx, b->S, b->h_off.data(), b->h_lat.data(), b->h_periodic.data(), cells);
+  if (rc) return rc;
+  b->loaded = false;
+  rc = take_cells(b, cells, false);
+  if (!rc && b->zcode_gen != ctx->model_gen) rc = upload_zcode(b);
+  b->loaded = rc == FNET_OK;
+  return rc;
+}
+
 int check_ready(fnet_ctx* ctx, fnet_batch* b) {
   if (!ctx) return FNET_ERR_ARG;
   if (!b) return fail(ctx, FNET_ERR_ARG, "batch is NULL");
@@ -973,11 +999,9 @@ int check_ready(fnet_ctx* ctx, fnet_batch* b) {
   // are stale
   if (b->seen_model_gen != ctx->model_gen) {
     invalidate(b);
+    const int rc = fit_model(b);
+    if (rc) return rc;
     b->seen_model_gen = ctx->model_gen;
-    if (b->zcode_gen != ctx->model_gen) {
-      const int rc = upload_zcode(b);
-      if (rc) return rc;
-    }
   } else if (b->seen_params_gen != ctx->params_gen) {
     b->have_E = b->have_F = b->host_E = b->host_F = false;
   }
@@ -1359,11 +1383,12 @@ int load_batch(fnet_ctx* ctx, fnet_batch* b, const fnet_batch_desc* d) {
     }
     for (long long i = d->offsets[s]; i < d->offsets[s + 1]; ++i) astruct[i] = s;
   }
-  int zone = m.nZ == 1;
+  int zone = m.nZ == 1, max_species = -1;
   int last_z = 0, last_c = zcode_of(m, 0);  // runs of one element look its slot up once
   for (long long i = 0; i < N; ++i) {
     if (d->species[i] < 0 || d->species[i] >= m.nspecies)
       return fail(ctx, FNET_ERR_ARG, "species index out of range");
+    max_species = std::max(max_species, d->species[i]);
     if (d->atnum[i] != last_z) {
       last_z = d->atnum[i];
       last_c = zcode_of(m, last_z);
@@ -1469,6 +1494,7 @@ int load_batch(fnet_ctx* ctx, fnet_batch* b, const fnet_batch_desc* d) {
   b->next = d->n_ext;
   b->h_off.assign(d->offsets, d->offsets + S + 1);
   b->h_species.assign(d->species, d->species + N);
+  b->max_species = max_species;
   b->h_lat = lat;
   b->h_periodic = per;
   b->nchunks = nchunks;
@@ -1492,6 +1518,7 @@ int load_batch(fnet_ctx* ctx, fnet_batch* b, const fnet_batch_desc* d) {
   const int rc = take_cells(b, cells, true);
   if (rc) return rc;
   HIPCHECK(ctx, stage_flush(ctx));
+  b->seen_model_gen = ctx->model_gen;
   b->loaded = true;
   return FNET_OK;
 }

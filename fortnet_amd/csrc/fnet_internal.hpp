@@ -235,6 +235,7 @@ struct fnet_batch {
   int res_nG = -1, res_nout = -1;
   std::vector<long long> h_off;
   std::vector<int> h_species;
+  int max_species = -1;        // largest of them
   // inputs
   double* xyz = nullptr;       // [N][3]
   double* lat = nullptr;       // [S][9]
