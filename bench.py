@@ -237,7 +237,7 @@ def serving_bench(rates, duration_s, max_requests, full):
 
 def time_steps(ctx, batch, steps, warmup, graph):
     """Wall time of ``steps`` back-to-back fnet_run steps (one synchronisation on each side),
-    then the per-stage HIP-event times of ``steps`` more eager steps (or, for graph replays,
+    then the per-stage device times of ``steps`` more eager steps (or, for graph replays,
     the device time of each step)."""
     ctx.set_graph(graph)
     for _ in range(warmup):

@@ -2201,7 +2201,7 @@ __device__ __forceinline__ void acsf_centre(const AcsfArgs& a, const long long i
 template <typename T, bool ADJ, int MQ, int FORM, bool PAIRS, bool R64 = false,
           bool PERSIST = false>
 __device__ __forceinline__ void acsf_wave(const AcsfArgs& a) {
-  // (the paired forward has no register left for it: its boundary is the search's end)
+  // (the paired forward has no register left for a stamp: its start is taken to be the search's end)
   if constexpr (ADJ) {
     stamp(a.stamp);
     if (a.norph && blockIdx.x == 0 && threadIdx.x == 0) *a.norph = 0;

@@ -109,12 +109,14 @@ __global__ void __launch_bounds__(256)
   stamp(ts);
   if (blockIdx.x > 0 && blockIdx.x <= nen) {
     energy_total(en, (long long)(blockIdx.x - 1) * 256 + threadIdx.x, 0, S);
+    if (ts) stamp_last(ts + 1);
     return;
   }
   const int cnt = *norph;
   if (blockIdx.x > 0) {
     const long long k = (long long)(blockIdx.x - 1 - nen) * 256 + threadIdx.x;
     if (cnt == 0 && k < nf) hF[k] = F[k];
+    if (ts) stamp_last(ts + 1);
     return;
   }
   for (int q = threadIdx.x; q < cnt; q += blockDim.x) {
@@ -130,7 +132,7 @@ __global__ void __launch_bounds__(256)
     for (long long k = threadIdx.x; k < nf; k += blockDim.x)
       hF[k] = __hip_atomic_load(&F[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  stamp(ts ? ts + 1 : nullptr);
+  if (ts) stamp_last(ts + 1);
 }
 
 __global__ void k_zero_int(int* __restrict__ p, int n) {

@@ -402,7 +402,7 @@ hipError_t launch_neigh_count(fnet_batch* b, double rc, long long a0, long long 
 hipError_t launch_neigh_fill(fnet_batch* b, double rc, long long a0, long long a1, int fp64,
                              hipStream_t s);
 // padded rows; a non-null mir (sized for the padded layout) gets -1 at every entry written
-// (stamp: end of the launch)
+// (stamp: end of the launch, near enough: stamp_now)
 hipError_t launch_neigh_pad(fnet_batch* b, double rc, int fp64, hipStream_t s,
                             int* mir = nullptr, unsigned long long* stamp = nullptr);
 hipError_t launch_cells_pad(fnet_batch* b, double rc, int fp64, hipStream_t s,
@@ -453,7 +453,7 @@ hipError_t launch_mirror(fnet_batch* b, long long a0, long long a1, long long fi
 hipError_t launch_force_gather(fnet_batch* b, const DevModel& m, long long a0, long long a1,
                                bool energies, hipStream_t s);
 // the orphans' part of the forces; energies: also the sums over the chunks; host: also the pinned
-// copy of the forces; stamps: {start, end} of the launch
+// copy of the forces; stamps: {start, end} of the launch (stamp_last)
 hipError_t launch_force_finish(fnet_batch* b, const DevModel& m, bool energies, hipStream_t s,
                                bool host, unsigned long long* stamps = nullptr);
 

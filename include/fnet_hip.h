@@ -245,7 +245,9 @@ int fnet_query(fnet_ctx* ctx);
 /* Timing of the last fnet_run / fnet_forces call, per stage, in milliseconds (clock stamps
  * that its kernels write, or HIP events): [0] neighbour list (with the mirror entries), [1] ACSF forward,
  * [2] networks, [3] adjoint forces (with the force gather), [4] energy reduction.
- * n = number of entries written (<= 8).  A step replayed as a graph has only its total, in [0]. */
+ * n = number of entries written (<= 8).  Stamps of a steady-state step are good to some ten
+ * microseconds (the end of the search and of the step are taken in their last blocks), and the mirror entries are
+ * searched beside the networks or the ACSF stages, not in [0].  A step replayed as a graph has only its total, in [0]. */
 int fnet_stage_times(fnet_ctx* ctx, double* ms, int n);
 
 /* Launch parameters of the batched kernels (no reference counterpart): knobs[5] = waves per
