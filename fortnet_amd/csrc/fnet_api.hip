@@ -228,7 +228,7 @@ int upload_zcode(fnet_batch* b) {
 int ensure_tiles(fnet_batch* b) {
   fnet_ctx* ctx = b->ctx;
   const DevModel& m = ctx->model;
-  const int TA = mlp_tile_atoms(m.shape, net64(b->precision), b->N);
+  const int TA = mlp_tile_atoms(b, m.shape, net64(b->precision));
   // 16 atoms per wave on the MFMA kernel; the tuned wave count when it fits
   int MW = mlp_mfma_waves(m.shape);
   if (MW && tune_of(b).mlp_waves > 0) MW = std::min(MW, tune_of(b).mlp_waves);

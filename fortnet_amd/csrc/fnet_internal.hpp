@@ -502,13 +502,13 @@ hipError_t launch_regularize(const DevModel& m, double* grad, double scale, doub
 hipError_t launch_sd_step(double* params, const double* grad, long long n, double lr,
                           double max_disp, double tol, double* scratch, int nspecies,
                           hipStream_t s);
-// atoms per generic tile of a batch of n_atoms
-int mlp_tile_atoms(const NetShape& sh, int fp64, long long n_atoms);
+// atoms per generic tile of the batch
+int mlp_tile_atoms(const fnet_batch* b, const NetShape& sh, int fp64);
 int grad_chunks(int ntiles);  // chunks of the weight-gradient reduction
 
-// launchers (fnet_mlp_f64.hip): FP64 element networks on MFMA 16x16x4 f64.  Atoms per tile for a
-// batch of n_atoms (a multiple of 16), 0 if the network is too wide for a block's LDS
-int mlp_f64_tile_atoms(const NetShape& sh, long long n_atoms);
+// launchers (fnet_mlp_f64.hip): FP64 element networks on MFMA 16x16x4 f64.  Atoms per tile of the
+// batch (a multiple of 16), 0 if the network is too wide for a block's LDS
+int mlp_f64_tile_atoms(const fnet_batch* b, const NetShape& sh);
 hipError_t launch_mlp_f64(fnet_batch* b, const DevModel& m, int first_tile, int ntiles,
                           int want_grad_in, hipStream_t s, bool mirror, unsigned long long* stamp);
 hipError_t launch_mlp_grad_f64(fnet_batch* b, const DevModel& m, hipStream_t s);

@@ -593,9 +593,9 @@ MlpArgs make_args(fnet_batch* b, const DevModel& m, int first_tile) {
 
 int grad_chunks(int ntiles) { return std::max(1, (ntiles + kGradChunk - 1) / kGradChunk); }
 
-int mlp_tile_atoms(const NetShape& sh, int fp64, long long n_atoms) {
+int mlp_tile_atoms(const fnet_batch* b, const NetShape& sh, int fp64) {
   if (fp64)
-    if (const int ta = mlp_f64_tile_atoms(sh, n_atoms)) return ta;
+    if (const int ta = mlp_f64_tile_atoms(b, sh)) return ta;
   int TA = 64;
   while (TA > 1 && (fp64 ? host_lds<double>(sh, TA) : host_lds<float>(sh, TA)) > 64 * 1024) TA >>= 1;
   return TA;
@@ -605,7 +605,7 @@ hipError_t launch_mlp_fwd(fnet_batch* b, const DevModel& m, int first_tile, int 
                           int want_grad_in, hipStream_t s, bool mirror,
                           unsigned long long* stamp) {
   if (ntiles <= 0) return hipSuccess;
-  if (fp64 && mlp_f64_tile_atoms(m.shape, b->N))
+  if (fp64 && mlp_f64_tile_atoms(b, m.shape))
     return launch_mlp_f64(b, m, first_tile, ntiles, want_grad_in, s, mirror, stamp);
   auto go = [&](auto* grad, auto* plain, MlpArgs a, size_t lds) {
     a.ntiles = ntiles;
@@ -692,7 +692,7 @@ hipError_t launch_mlp_grad(fnet_batch* b, const DevModel& m, int fp64, double* g
     const hipError_t e = launch_mlp_grad_mfma(b, m, s);
     if (e != hipSuccess) return e;
   } else if (b->ntiles > 0) {
-    if (fp64 && mlp_f64_tile_atoms(m.shape, b->N)) {
+    if (fp64 && mlp_f64_tile_atoms(b, m.shape)) {
       const hipError_t e = launch_mlp_grad_f64(b, m, s);
       if (e != hipSuccess) return e;
     } else if (fp64) {

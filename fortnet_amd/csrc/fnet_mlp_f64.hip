@@ -354,9 +354,9 @@ constexpr long long kF64Tiles = 512;
 
 }  // namespace
 
-int mlp_f64_tile_atoms(const NetShape& sh, long long n_atoms) {
-  if (layout(sh, true, nullptr) > kF64Lds) return 0;
-  const long long parts = (n_atoms + 15) / 16;
+int mlp_f64_tile_atoms(const fnet_batch* b, const NetShape& sh) {
+  if (layout(sh, true, nullptr) > std::min<size_t>(kF64Lds, b->ctx->lds_block)) return 0;
+  const long long parts = (b->N + 15) / 16;
   return 16 * (int)std::max<long long>(1, std::min<long long>(64, (parts + kF64Tiles - 1) / kF64Tiles));
 }
 
