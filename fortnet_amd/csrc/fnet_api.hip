@@ -334,6 +334,9 @@ int ensure_results(fnet_batch* b) {
     return FNET_OK;
   void* pr[] = {b->G, b->cG, b->Eatom, b->Estruct, b->F, b->lossgrad};
   for (void* p : pr) dfree(p);
+  b->G = b->cG = b->F = nullptr;
+  b->Eatom = b->Estruct = b->lossgrad = nullptr;
+  b->res_N = b->res_S = 0;
   const long long N = std::max<long long>(b->N, b->capN), S = std::max<long long>(b->S, b->capS);
   HIPCHECK(ctx, dalloc((double**)&b->G, (size_t)N * m.nG));
   HIPCHECK(ctx, dalloc((double**)&b->cG, (size_t)N * m.nout * m.nG));
@@ -426,6 +429,7 @@ int do_neighbours(fnet_batch* b) {
     dfree(b->nd);
     b->nj = b->nimg = nullptr;
     b->nd = nullptr;
+    b->pcap = 0;
     const long long cap = P + P / 8 + 1024;
     HIPCHECK(ctx, dalloc(&b->nj, cap));
     HIPCHECK(ctx, dalloc(&b->nimg, cap));
@@ -529,6 +533,7 @@ int ensure_force_buffers(fnet_batch* b) {
     dfree(b->orph);
     b->mir = b->orph = nullptr;
     b->mir_clear = false;
+    b->gv_entries = 0;
     const long long cap = entries + entries / 8 + 1024;
     HIPCHECK(ctx, dalloc(&b->mir, (size_t)cap));
     HIPCHECK(ctx, dalloc(&b->orph, (size_t)cap));
@@ -538,6 +543,7 @@ int ensure_force_buffers(fnet_batch* b) {
   if (glen > b->gv_len) {
     dfree(b->gvec);
     b->gvec = nullptr;
+    b->gv_len = 0;
     const long long cap = glen + glen / 8 + 4096;
     HIPCHECK(ctx, dalloc(&b->gvec, (size_t)cap));
     b->gv_len = cap;
@@ -1654,6 +1660,7 @@ int fnet_get_neighbours(fnet_ctx* ctx, fnet_batch* b, long long* rowptr, int* j,
       dfree(b->nd);
       b->nj = b->nimg = nullptr;
       b->nd = nullptr;
+      b->pcap = 0;
       const long long cap = (long long)P + P / 8 + 1024;
       HIPCHECK(ctx, dalloc(&b->nj, cap));
       HIPCHECK(ctx, dalloc(&b->nimg, cap));
@@ -1962,6 +1969,7 @@ int fnet_train_gradients(fnet_ctx* ctx, fnet_batch* b, int n_global, const doubl
   if (need > b->targets_cap) {
     dfree(b->d_targets);
     b->d_targets = nullptr;
+    b->targets_cap = 0;
     HIPCHECK(ctx, dalloc(&b->d_targets, (size_t)need));
     b->targets_cap = need;
   }
@@ -1983,6 +1991,7 @@ int fnet_train_gradients(fnet_ctx* ctx, fnet_batch* b, int n_global, const doubl
   if (np > ctx->grad_cap) {
     dfree(ctx->d_grad);
     ctx->d_grad = nullptr;
+    ctx->grad_cap = 0;
     HIPCHECK(ctx, dalloc(&ctx->d_grad, (size_t)np + m.nspecies));
     ctx->grad_cap = np;
   }
@@ -1994,6 +2003,7 @@ int fnet_train_gradients(fnet_ctx* ctx, fnet_batch* b, int n_global, const doubl
     if (need > b->gpart_len) {
       dfree(b->gpart);
       b->gpart = nullptr;
+      b->gpart_len = 0;
       HIPCHECK(ctx, dalloc(&b->gpart, (size_t)need));
       b->gpart_len = need;
     }
