@@ -114,23 +114,25 @@ __device__ __forceinline__ void dist_inv(double r2, double& r, double& ir) {
   ir = 1.0 / r;
 }
 __device__ __forceinline__ double fdiv(double x, double y) { return x / y; }
-// cos and sin of the cosine cutoff's argument x = pi r / rc for r in [0, rc] (finite beyond; the
-// callers discard those).  FP32: the hardware instructions on r (pi / rc).  FP64: with
-// u = x / 2 - pi / 4 = (pi / 4)(2 r / rc - 1), |u| <= pi / 4,
-//   |cos x| = 2 |sin u| cos u = 1 - (cos u - |sin u|)^2,   sin x = 1 - 2 sin^2 u,
-// sin u and cos u from Taylor polynomials (remainders 5e-17 and 2e-18).  Written as 1 less a square,
-// cos x stays within [-1, 1] and is -1 at r = rc, so that the cutoff is 0 there and nowhere negative
-// (the product 2 sin u cos u missed 1 by an ulp on either side).  cut_cs takes 2 / rc in two parts:
-// its sine needs them near the ends.  Errors over r and rc (largest, rms): cosine 3.4e-16, 7e-17
-// (cut_cos 4.6e-16, 8e-17), sine 5.8e-16, 8e-17; of the library's cosine and sine of the rounded
-// pi r / rc 4.8e-16, 10e-17 and 6.6e-16, 11e-17.
+// The cosine cutoff's 1 + cos x (cut_1cos) and, for derivatives, cos x and sin x (cut_cs), x = pi r / rc
+// with r in [0, rc] (finite beyond; the callers discard those).  FP32: the hardware instructions on
+// r (pi / rc).  FP64: with u = x / 2 - pi / 4 = (pi / 4)(2 r / rc - 1), |u| <= pi / 4, from sin u and
+// cos u, Taylor polynomials (remainders 5e-17 and 2e-18):
+//   1 + cos x = 1 - 2 sin u cos u, in one rounding, 0 at r = rc, and not below it where the product
+//     exceeds 1 by an ulp just inside;
+//   |cos x| = 1 - (cos u - |sin u|)^2, which stays within 1, and sin x = 1 - 2 sin^2 u, whose argument
+//     takes 2 / rc in two parts: the sine needs them near the ends.
+// Errors over r and rc (largest, rms): cosine 3.5e-16, 7e-17, sine 5.8e-16, 8e-17; of the library's
+// cosine and sine of the rounded pi r / rc 4.8e-16, 10e-17 and 6.6e-16, 11e-17.
+__device__ __forceinline__ float cut_1cos(float r, float rc, float pirc) {
+  return fcos(r * pirc) + 1.0f;
+}
 __device__ __forceinline__ void cut_cs(float r, float rc, float pirc, float& c, float& s) {
   c = fcos(r * pirc);
   s = fsin(r * pirc);
 }
-__device__ __forceinline__ float cut_cos(float r, float rc, float pirc) { return fcos(r * pirc); }
-// sn = sin u of u = (pi / 4) t; returns cos x
-__device__ __forceinline__ double cut_quarter(double t, double& sn) {
+// sin and cos of u = (pi / 4) t
+__device__ __forceinline__ void sc_quarter(double t, double& sn, double& cs) {
   const double u = t * 0.78539816339744831, z = u * u;
   double a = lit(-1.0 / 1307674368000.0);
   a = fma(a, z, lit(1.0 / 6227020800.0));
@@ -148,18 +150,20 @@ __device__ __forceinline__ double cut_quarter(double t, double& sn) {
   b = fma(b, z, lit(-1.0 / 720.0));
   b = fma(b, z, lit(1.0 / 24.0));
   b = fma(b, z, -0.5);
-  const double d = fma(b, z, 1.0) - fabs(sn);
-  return copysign(fma(-d, d, 1.0), -sn);
+  cs = fma(b, z, 1.0);
+}
+__device__ __forceinline__ double cut_1cos(double r, double rc, double pirc) {
+  double sn, cs;
+  sc_quarter(fma(r, 2.0 / rc, -1.0), sn, cs);
+  return r < rc ? fmax(fma(-2.0 * sn, cs, 1.0), 0.0) : 0.0;
 }
 __device__ __forceinline__ void cut_cs(double r, double rc, double pirc, double& c, double& s) {
   const double i2 = 2.0 / rc, low = fma(-i2, rc, 2.0) * (0.5 * i2);
-  double sn;
-  c = cut_quarter(fma(r, low, fma(r, i2, -1.0)), sn);
+  double sn, cs;
+  sc_quarter(fma(r, low, fma(r, i2, -1.0)), sn, cs);
+  const double d = cs - fabs(sn);
+  c = copysign(fma(-d, d, 1.0), -sn);
   s = fma(-2.0 * sn, sn, 1.0);
-}
-__device__ __forceinline__ double cut_cos(double r, double rc, double pirc) {
-  double sn;
-  return cut_quarter(fma(r, 2.0 / rc, -1.0), sn);
 }
 
 // A wave-uniform value moved to scalar registers (values converted from FP64 on the vector
@@ -608,7 +612,7 @@ __device__ __forceinline__ void pairs_fwd(const Slice<T>& sl, int lane, int A0, 
       const T rx = dj.x - dk.x, ry = dj.y - dk.y, rz = dj.z - dk.z;
       const T r2 = rx * rx + ry * ry + rz * rz;
       const T rjk = fsqrt(r2);
-      const T fcjk = (T)0.5 * pj.z * pk.z * (cut_cos(rjk, rc, pirc) + (T)1);
+      const T fcjk = (T)0.5 * pj.z * pk.z * cut_1cos(rjk, rc, pirc);
       const T f = fexp(-eta * r2) * fcjk;
       base = (rjk <= rc) ? base * f : (T)0;
     }
@@ -671,7 +675,7 @@ template <> struct JkConst<float> {
     c = __builtin_amdgcn_cosf(x);
     sn = __builtin_amdgcn_sinf(x);
   }
-  __device__ __forceinline__ float cosine(float r) const { return __builtin_amdgcn_cosf(r * prev); }
+  __device__ __forceinline__ float cos1(float r) const { return __builtin_amdgcn_cosf(r * prev) + 1.0f; }
 };
 template <> struct JkConst<double> {
   double rc, eta, pirc;
@@ -684,7 +688,7 @@ template <> struct JkConst<double> {
   __device__ __forceinline__ void cs(double r, double& c, double& sn) const {
     cut_cs(r, rc, pirc, c, sn);
   }
-  __device__ __forceinline__ double cosine(double r) const { return cut_cos(r, rc, pirc); }
+  __device__ __forceinline__ double cos1(double r) const { return cut_1cos(r, rc, pirc); }
 };
 
 // adj_geom without branches: a pair that does not exist (v false) or lies beyond the cutoff
@@ -885,7 +889,7 @@ __device__ __forceinline__ T pair_base(const JkConst<T>& K, const typename Vec4<
     const T rx = dj.x - dk.x, ry = dj.y - dk.y, rz = dj.z - dk.z;
     const T r2 = rx * rx + ry * ry + rz * rz;
     const T rjk = fsqrt(r2);
-    const T fcjk = (T)0.5 * pj.z * pk.z * (K.cosine(rjk) + (T)1);
+    const T fcjk = (T)0.5 * pj.z * pk.z * K.cos1(rjk);
     base *= K.ex(r2) * fcjk;
     in = in && (rjk <= K.rc);
   }
@@ -1687,7 +1691,7 @@ __device__ __forceinline__ double radial_sum(const AcsfArgs& a, const Slice<T>& 
         fcv = (U)*(const double*)(sl.pa + e);
       } else {
         const U qj = (U)ext_q(a.ext, a.next, fn.atomid, sl.j[e]);
-        fcv = (U)0.5 * qi * qj * (cut_cos(r, rc, pirc) + (U)1);
+        fcv = (U)0.5 * qi * qj * cut_1cos(r, rc, pirc);
       }
       U term;
       if (fn.type == 1) term = fcv;
@@ -1737,7 +1741,7 @@ __device__ __forceinline__ void acsf_centre(const AcsfArgs& a, const long long i
     sl.d[pos] = d;
     sl.j[pos] = ADJ ? e : jj;  // adjoint: the entry's index in its row, for the output
     sl.zc[pos] = key < nZ ? key : -1;
-    if (!ADJ) sl.fc[pos] = (T)0.5 * (cut_cos(d.w, rcl, pircl) + (T)1);
+    if (!ADJ) sl.fc[pos] = (T)0.5 * cut_1cos(d.w, rcl, pircl);
   };
   if (a.zone) {
     if (lane < 2) {
@@ -1814,7 +1818,7 @@ __device__ __forceinline__ void acsf_centre(const AcsfArgs& a, const long long i
       if constexpr (R64) {
         for (int e = lane; e < n; e += 64)
           *(double*)(sl.pa + e) =
-              0.5 * (cut_cos((double)sl.d[e].w, a.rclist, kPi / a.rclist) + 1.0);
+              0.5 * cut_1cos((double)sl.d[e].w, a.rclist, kPi / a.rclist);
         wave_sync();
       }
       // Lanes are (function, share of its element range) pairs.  When the functions fit one
@@ -2008,10 +2012,15 @@ __device__ __forceinline__ void acsf_centre(const AcsfArgs& a, const long long i
             }
           } else {
             qj = (T)ext_q(a.ext, a.next, grp.atomid, nbr(e));
-            T cx, sx;
-            cut_cs(r, rc, pirc, cx, sx);
-            fc = (T)0.5 * qi * qj * (cx + (T)1);
-            dfc = -(T)0.5 * qi * qj * pirc * sx;
+            if (ADJ) {
+              T cx, sx;
+              cut_cs(r, rc, pirc, cx, sx);
+              fc = (T)0.5 * qi * qj * (cx + (T)1);
+              dfc = -(T)0.5 * qi * qj * pirc * sx;
+            } else {
+              fc = (T)0.5 * qi * qj * cut_1cos(r, rc, pirc);
+              dfc = 0;
+            }
           }
           const T ex = fexp(-eta * r * r);
           E = ex * fc;
