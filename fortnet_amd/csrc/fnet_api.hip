@@ -477,9 +477,9 @@ int do_acsf(fnet_batch* b) {
 }
 
 // Batches of up to this many atoms search their mirror entries in extra blocks of the networks
-// launch, which is latency-bound there and hides them (18 113 atoms: 396 -> 382 us per step); larger
-// ones (38 400 atoms: 1587 -> 1537 us, 130 000: 2941 -> 2682) on the side stream beside the ACSF
-// forward.
+// launch, which is latency-bound there and hides them; larger ones on the side stream beside the ACSF
+// forward.  MD calls of 64-atom Si cells, side stream -> extra blocks: 8 192 atoms 151 -> 142 us, 16 384
+// 240 -> 237, 24 576 319 -> 315, 32 768 408 either way, 49 152 571 -> 576, 65 536 711 -> 725.
 constexpr long long kMirrorInline = 24576;
 
 int do_mlp(fnet_batch* b, int gradin, bool mirror = false) {

@@ -5,7 +5,7 @@
 // arrays are written into the ring instead and one kernel copies all of them to their places, on
 // the context's own stream, so nothing is waited for.  Results of small calls come back the same
 // way: one kernel gathers them in the ring, one wait, plain memory copies from there.  Large arrays
-// (kStageMax) keep their copy commands, whose bandwidth is better.
+// (kStageMax) keep their copy commands, whose bandwidth is better (1 MB up: 44 us against 50).
 //
 // The ring belongs to one context (one host thread, one stream): space is reused only after the
 // stream has drained, which a context that waits for its results does anyway.
