@@ -26,9 +26,10 @@
 //    dense array, but without forming it and with periodic images summed exactly.
 //
 // Arithmetic is T (double or float); sums over neighbours and pairs, the values G and the forces
-// are accumulated in FP64 in both modes.  FP64 evaluates exp and the cutoff's cos and sin to an ulp or
-// two from polynomials (fexp, cut_cs), roots, quotients and real powers with libm; FP32 uses the hardware instructions (v_exp_f32, v_cos_f32,
-// v_sin_f32, v_sqrt_f32, v_rcp_f32: about 1 ulp, cos/sin to ~1e-6 absolute on [0, pi]).
+// are accumulated in FP64 in both modes.  FP64 evaluates exp and the cutoff's cos and sin to an ulp
+// or two from polynomials (fexp, cut_cs), the real powers of a progression in two parts (ProgPow),
+// roots, quotients and other real powers with libm; FP32 uses the hardware instructions (v_exp_f32,
+// v_cos_f32, v_sin_f32, v_sqrt_f32, v_rcp_f32: about 1 ulp, cos/sin to ~1e-6 absolute on [0, pi]).
 #include "fnet_device.hpp"
 
 // The kernel instances are compiled in four translation units, side by side: this file (FP32
